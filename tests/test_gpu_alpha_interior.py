@@ -1,0 +1,33 @@
+"""The alpha walk runs all but the first and last groups of anti-diagonals without looking at any
+bounds.  Where those interior groups begin and end (and whether there are any) depends on the
+frames and labels of each utterance and on how the label positions are dealt to wavefronts; the
+alphas and costs must carry the oracle's bits in every case."""
+import numpy as np
+import pytest
+
+import oracle
+from util import DeviceCase, assert_same_bits, gpu_forward
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("U", [2, 3, 64, 65, 128, 129, 257, 300])
+@pytest.mark.parametrize("T", [31, 66, 97, 164])
+def test_alphas_where_the_interior_begins_and_ends(T, U):
+    V, il = 6, [T, T, T - 1, T - 2, T - 3, max(T // 2, 1), 17, 1]
+    ll = [U - 1, U // 2, max(U - 2, 0), 1, 0, min(63, U - 1), min(64, U - 1), U - 1]
+    B = len(il)
+    rng = np.random.default_rng(1000 * T + U)
+    E = rng.standard_normal((B, T, V), dtype=np.float32)
+    P = rng.standard_normal((B, U, V), dtype=np.float32)
+    P[1, :, 0] = -np.inf          # no blank anywhere: no path, through interior groups too
+    E[2, T // 2, 1:] = -np.inf    # one frame that emits nothing
+    labels = rng.integers(1, V, (B, U - 1)).astype(np.int32)
+    il, ll = np.array(il, np.int32), np.array(ll, np.int32)
+    LN = oracle.log_norms_naive(E, P, il, ll)
+    want_costs, want = oracle.forward(E, P, LN, labels, il, ll)
+    costs, alphas = gpu_forward(DeviceCase(E, P, labels, il, ll), np.nan_to_num(LN))
+    for b in range(B):
+        got, ref = alphas[b, :il[b], :ll[b] + 1], want[b, :il[b], :ll[b] + 1]
+        assert_same_bits(got, ref, "alphas of utterance %d" % b)
+    assert_same_bits(costs, want_costs, "costs")

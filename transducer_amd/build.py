@@ -16,13 +16,16 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 
-# (source, extra flags, object name).  The gradient kernels are by far the longest compile: the
-# file comes in six parts (egrads, pgrads x fp32, bf16, fp16 scores) that are compiled side by side.
-HIP_SOURCES = [("rnnt_grads.hip", ["-DRNNT_GRADS_PART=%d" % part], "rnnt_grads_%d.o" % part)
+# (source, extra flags, object name).  The gradient kernels and the lattice walks are by far the
+# longest compiles: their files come in parts (egrads, pgrads x fp32, bf16, fp16 scores; the walks
+# by kind) that are compiled side by side, the longest first.
+HIP_SOURCES = [("rnnt_dp.hip", ["-DRNNT_DP_PART=%d" % part], "rnnt_dp_%d.o" % part)
+               for part in (2, 1, 4, 3, 0)] + \
+              [("rnnt_grads.hip", ["-DRNNT_GRADS_PART=%d" % part], "rnnt_grads_%d.o" % part)
                for part in range(6)] + \
               [(src, [], src.replace(".hip", ".o"))
-               for src in ("rnnt_dp.hip", "rnnt_capi.hip", "rnnt_lse.hip", "rnnt_cand.hip",
-                           "rnnt_fused.hip", "rnnt_prep.hip")]
+               for src in ("rnnt_capi.hip", "rnnt_lse.hip", "rnnt_cand.hip", "rnnt_fused.hip",
+                           "rnnt_prep.hip")]
 
 # -ffp-contract=off: the lattice recursions must round like the reference's scalar code.
 # packed-fp32 instructions are disabled for the device pass (the host pass does not know the

@@ -13,6 +13,10 @@
 // (plane_at in rnnt_internal.h), so that four steps are one 16-byte load per lane and the lanes'
 // loads are neighbours in memory; they are requested several groups ahead.  This file is compiled with -ffp-contract=off: the rounding
 // sequence of every cell must equal the reference's.
+//
+// The file is compiled in parts side by side (-DRNNT_DP_PART=0..4: everything else, the alpha
+// walk in its narrow and its wide forms, the dalpha walk, the best-path walk; all of it without
+// the macro): a part holds the launchers that instantiate its kernels.
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -21,7 +25,14 @@
 #include "rnnt_libm.h"
 #include "rnnt_split.h"
 
+#ifndef RNNT_DP_PART
+#define RNNT_DP_PART -1
+#endif
+#define RNNT_IN_PART(n) (RNNT_DP_PART < 0 || RNNT_DP_PART == (n))
+
 namespace rnnt {
+
+int live_blocks(const Dims& d, int* waves);
 
 namespace {
 
@@ -48,20 +59,22 @@ __device__ inline float wave_shl1(float x, float fill) {
                                                     0x130 /* wave_shl:1 */, 0xf, 0xf, false));
 }
 
-// exp(x) for x <= 0 and log(w) for w in [1,2] straight on the hardware transcendental units
-// (v_exp_f32 / v_log_f32 work in base 2 and are good to about one ulp).  In the one place they
+// exp(x) for x <= 0 straight on the hardware transcendental unit
+// (v_exp_f32 and v_log_f32 work in base 2 and are good to about one ulp).  In the one place they
 // are used -- log1p(exp(-|a-b|)) below -- the rounding of x*log2(e) costs at most 2.4e-8
 // absolute in the result (it is largest where exp(x) is small), i.e. less than half an ulp of
 // the value log 2 that the result never exceeds.
 __device__ inline float exp_neg(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
-__device__ inline float log_1to2(float w) { return __builtin_amdgcn_logf(w) * 0.693147180559945309f; }
 
-// log1p(y) for y in [0,1]:  log(1+y) with the rounding error of the sum 1+y folded back in.
-// Within about one ulp of the correctly rounded value over the whole range.
+// log1p(y) for y in [0,1]:  log(1+y) with the rounding error of the sum 1+y folded back in, divided
+// by 1 + y to three digits (1 - y/2: the lost part is at most 2^-24, so a seventh of it is below a
+// tenth of the result's last bit, and two instructions stand in for a reciprocal's four-cycle
+// quarter-rate slot).  Within about one ulp of the correctly rounded value over the whole range.
 __device__ inline float log1p_unit(float y) {
   const float w = 1.0f + y;
   const float lost = y - (w - 1.0f);
-  return log_1to2(w) + lost * __builtin_amdgcn_rcpf(w);
+  return __builtin_fmaf(__builtin_amdgcn_logf(w), 0.693147180559945309f,
+                        lost * __builtin_fmaf(y, -0.5f, 1.0f));
 }
 
 // log1p(exp(d)) for d <= 0 on the hardware transcendental units: within a few ulp of the C
@@ -73,12 +86,12 @@ __device__ inline float softplus_fast(float d) { return log1p_unit(exp_neg(d)); 
 // evaluations (a few ulp of lf), the second the rounding of d * log2(e) ahead of v_exp_f32,
 // whose effect on the result grows with |d|.  The bound is not taken from data sheets: the
 // fast value is compared with the exact one for EVERY float d <= 0 (rnnt_hip_lse_bound_check,
-// run by the tests on the device itself).  Measured on gfx950, in units of 2^-23 lf: at most 2.2
-// for |d| <= 1.5, 3.9 up to 4, 6.8 up to 8, 0.46 (5 + 1.25 |d|) beyond; the constants leave an
-// eighth on top of that everywhere.  They are what decides how often a wavefront of the alpha
-// walk takes the library path (its chance per lane is bound / half the sum's spacing), so they
-// are not rounder than that: with 5 and 1.25 the walk of B=32 T=2000 U=100 was a tenth slower.
-constexpr float kFastRelA = 2.75f * 0x1p-23f;
+// run by the tests on the device itself).  Measured on gfx950, in units of 2^-23 lf: at most 2.1
+// for |d| <= 1.5, 3.6 up to 4, 5.7 up to 8, 0.91 (2.1 + 0.65 |d|) beyond; the constants leave a
+// tenth on top of that.  They are what decides how often a wavefront of the alpha walk takes the
+// library path (its chance per lane is twice the bound / the sum's spacing), so they are not
+// rounder than that: with 5 and 1.25 the walk of B=32 T=2000 U=100 was a tenth slower.
+constexpr float kFastRelA = 2.1f * 0x1p-23f;
 constexpr float kFastRelB = 0.65f * 0x1p-23f;
 // The bound for fast value lf at argument d.  The clamp keeps 0 * inf out of it at d = -inf;
 // the added 2^-125 covers d below -87.3, where the library's value is a subnormal number and
@@ -100,27 +113,38 @@ __device__ inline float lse2_libm(float a, float b, const unsigned long long* ta
 // The same bits, mostly without the library's ~100 instructions.  What the recursion keeps is
 // r = fl(hi + l) with l = log1pf(expf(d)) at most log 2, and from a few hundred steps into a
 // lattice |hi| is in the thousands: the sum's spacing is then thousands of times the
-// uncertainty of a fast l, so nearly every fast sum is provably the library's sum.  Per lane:
-//   r = fl(hi + lf), t = lf - (r - hi): the exact remainder (hi + lf) - r whenever |hi| >= lf;
-//   the library's sum rounds to the same r if |t| + bound(lf) stays below half the spacing of
-//   floats on the narrower side of r (the spacing at the float just below |r|: halves when r is
-//   a power of two).
-// Where |hi| < lf the remainder is not exact, but then |r| < 2 lf, the half spacing is below
-// 2^-23 lf and bound(lf) >= 2.75 * 2^-23 lf alone exceeds it: the test fails by itself.  r = 0, NaN
-// operands and two operands of -inf (inf - inf) fail it too.  Lanes that fail take the library
-// path; a wavefront skips it when none does (Ziv's strategy).  Either way the result is the
+// uncertainty of a fast l, so nearly every fast sum is provably the library's sum.  The library's l
+// lies in [lf - e, lf + e], e the bound above, and rounding is monotone: where fl(hi + lo) and
+// fl(hi + up) are the same float, lo = fl(lf - e) and up = fl(lf + e), that float is the library's
+// sum as well.  (l is a float, so lf - e <= l gives fl(lf - e) <= l: the rounding of the two ends
+// costs nothing.)  No exponents are looked at, and the sum itself falls out of the proof: eight
+// instructions, where forming the sum, its exact remainder and half the spacing of floats below
+// it took twelve.  NaN operands and two operands of -inf (inf - inf) fail by themselves.  When a lane
+// fails, its wavefront takes the library path (Ziv's strategy); either way the result is the
 // library's, bit for bit.
-__device__ inline float lse2_checked(float a, float b, const unsigned long long* tab) {
-  const float hi = a > b ? a : b;
+struct FastLse {
+  float lo, up;  // fl(hi + l) is the library's sum where the two are the same
+};
+// max without the two instructions that quiet its operands first (a NaN fails the proof anyway)
+__device__ inline float max_raw(float a, float b) {
+  float r;
+  asm("v_max_f32_e32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ inline FastLse lse2_fast(float a, float b) {
+  const float hi = max_raw(a, b);
   const float d = -fabsf(a - b);
   const float lf = softplus_fast(d);
-  float r = hi + lf;
-  const float t = lf - (r - hi);
-  const float bound = fast_bound(lf, d);
-  const int below = (__float_as_int(r) - 1) & 0x7f800000;  // exponent of the float below |r|
-  const float half_spacing = __int_as_float(below - (24 << 23));
-  if (!(fabsf(t) + bound < half_spacing)) r = lse2_libm(a, b, tab);
+  const float e = fast_bound(lf, d);
+  FastLse r;
+  r.lo = hi + (lf - e);
+  r.up = hi + (lf + e);
   return r;
+}
+__device__ inline float lse2_checked(float a, float b, const unsigned long long* tab) {
+  const FastLse r = lse2_fast(a, b);
+  // (all lanes take the library's value then: it is what the others hold already)
+  return __builtin_amdgcn_ballot_w64(!(r.lo == r.up)) ? lse2_libm(a, b, tab) : r.lo;
 }
 
 // The same on the hardware units alone (no check): for the chain-latency probe.
@@ -364,7 +388,13 @@ __global__ __launch_bounds__(256) void gather_cells_kernel(const TIO* __restrict
 // never read by a valid cell.
 // W > 1: the label positions are dealt to W wavefronts of one workgroup (wavefront w owns
 // positions [64 C w, 64 C (w+1))), because the walk is bound by how fast ONE wavefront issues
-// the ~22 instructions of a cell: a step costs about 30 + 65 C ns.  The only value that crosses
+// the instructions of a cell: 28, two of them at a quarter of the rate, then about 25 per group of
+// four steps for loads, store and hand-over (interior groups, below).  Measured with B=8 T=2000, one
+// cell a lane: 95 ns a step on one wavefront (64 positions), 117 on two or four (101, 256);
+// 151, 165 and 162 while every step tested its bounds, every load formed a 64-bit address and the
+// proof of the fast log-sum-exp took twelve instructions.  Of the 117, 77 are left with the proof
+// and its branch compiled out (wrong bits, timing only); the library path itself is taken in 2 % of
+// the steps (60 of 2100) and costs a tenth.  The only value that crosses
 // a wavefront boundary is the label-move score of the boundary cell, one float per step: the
 // lower wavefront leaves it in an LDS array indexed by step and then publishes how far it has
 // got; the upper one runs a few groups behind, so it finds its inputs there without waiting and
@@ -406,6 +436,7 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
   extern __shared__ __attribute__((aligned(16))) float hand[];  // [W-1][hand_stride]: entry s =
                                                                 // score handed to step s
   __shared__ int done[W];          // steps a wavefront has published
+  __shared__ __attribute__((aligned(16))) float nothing[4];
   __shared__ unsigned long long etab[32];  // expf's table (rnnt_libm.h)
   // live blocks: workgroups go round the 8 XCDs in launch order; ids i, i + 8, i + 16 .. share
   // one, and with it the L2 the boundary scores cross in.  Eight utterances take 8 live_n
@@ -468,32 +499,62 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
   if (W > 1) {
     if (threadIdx.x < W) done[threadIdx.x] = 0;
     if (threadIdx.x < W - 1) hand[threadIdx.x * hand_stride] = kOutside;  // nothing enters step 0
+    if (threadIdx.x < 4) nothing[threadIdx.x] = kNegInf;
   }
   __syncthreads();
+  // a wavefront past this utterance's labels: nobody reads what it would hand on
+  const int u_lo = u_base + wave * 64 * C;
+  if (W > 1 && u_lo >= Ub) return;
   float* hand_out = hand + wave * hand_stride;                     // wave < W-1
-  const float* hand_in = hand + (wave > 0 ? wave - 1 : 0) * hand_stride;  // wave > 0
+  // wave > 0; wavefront 0 finds there that nothing comes in (-inf: see run_group)
+  const float* hand_in = wave > 0 ? hand + (wave - 1) * hand_stride : nothing;
   // E[t,blank] for the cells of step s sits at ebp[s - u]; column c at step s = 4g+j reads
   // ebl[4g + j - c], so one run of C+3 values serves all columns of a group
-  const float* ebl = p.eb + (size_t)b * d.Tp + d.Eo - u0;
+  const float* ebl = p.eb + (size_t)b * d.Tp + d.Eo - min(u0, Ub - 1);
 
   float stay[C], emit[C], pbv[C], plv[C];
   unsigned tlim[C];  // frames of this column: T_b, or 0 for a label position past the utterance
   const float* lnp[C];
   const float* elp[C];
   float* ap[C];
+  // Operands of a position past the utterance's last one are the last one's (its label score the
+  // last label's), and its moves carry kOutside on top: whatever it meets is an ordinary number
+  // far below any alpha, so that the interior groups below need no test for it.
 #pragma unroll
   for (int c = 0; c < C; ++c) {
-    tlim[c] = (u0 + c < Ub) ? (unsigned)Tb : 0u;
-    const size_t row = plane_group0(d, b, u0 + c);  // u0 + c < Ua always
-    lnp[c] = p.lnS + row;
-    elp[c] = p.elS + row;
-    ap[c] = p.aS + row;
-    pbv[c] = p.pb[(size_t)b * d.Ua + u0 + c];
-    plv[c] = p.pl[(size_t)b * d.Ua + u0 + c];
+    const bool real = u0 + c < Ub;
+    tlim[c] = real ? (unsigned)Tb : 0u;
+    lnp[c] = p.lnS + plane_group0(d, b, min(u0 + c, Ub - 1));
+    elp[c] = p.elS + plane_group0(d, b, max(min(u0 + c, Ub - 2), 0));
+    ap[c] = p.aS + plane_group0(d, b, u0 + c);  // u0 + c < Ua always
+    pbv[c] = real ? p.pb[(size_t)b * d.Ua + u0 + c] : kOutside;
+    plv[c] = real ? p.pl[(size_t)b * d.Ua + u0 + c] : kOutside;
     // :43 alpha[0,0] = 0: cell (0,0) finds 0 coming up from below and nothing from the left
     stay[c] = (u0 + c == 0) ? 0.0f : kNegInf;
     emit[c] = kOutside;
   }
+
+  const int nwhole = nsteps >> 2;  // groups with all four steps
+  // Interior groups [in_lo, in_hi): step 4g is past the first frame of the wavefront's last
+  // position (rounded up to whole lanes), step 4g + 3 not past the last frame of its first one.
+  // Their operands are addressed by 32-bit offsets from the utterance's own (uniform) plane
+  // origins: one addition per load where 64-bit pointers took five instructions.
+  const int top = min(u_lo + 64 * C, ((Ub + C - 1) / C) * C) - 1;
+  const bool small_plane = 4ull * (unsigned long long)d.Ua * (unsigned)d.Dp < (1ull << 32);
+  const int in_lo = (top + 3) >> 2;
+  const int in_hi = (small_plane && Ub > 1) ? min((Tb + u_lo) >> 2, nwhole) : 0;
+  const char* ln_b = reinterpret_cast<const char*>(p.lnS + plane_group0(d, b, 0));
+  const char* el_b = reinterpret_cast<const char*>(p.elS + plane_group0(d, b, 0));
+  char* a_b = reinterpret_cast<char*>(p.aS + plane_group0(d, b, 0));
+  const char* eb_b = reinterpret_cast<const char*>(p.eb + (size_t)b * d.Tp);
+  unsigned ln_o[C], el_o[C], a_o[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    ln_o[c] = 16u * (unsigned)min(u0 + c, Ub - 1);
+    el_o[c] = 16u * (unsigned)max(min(u0 + c, Ub - 2), 0);
+    a_o[c] = 16u * (unsigned)(u0 + c);
+  }
+  const unsigned eb_o = 4u * (unsigned)(d.Eo - min(u0, Ub - 1) - (C - 1));
 
   struct Group {
     float4 ln[C], el[C];
@@ -532,9 +593,25 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
     // the empty asm statements only keep the compiler from moving LDS accesses across
     avail = bounded_wait(&done[wave - 1], avail, need, spin_limit, trouble);
   };
+  // What enters a wavefront above the first during a group is asked for one group ahead (its
+  // latency would otherwise stand at the head of every group), into two register sets in turn.
+  // The first wavefront's interior groups ask as well, always for the same four entries that say
+  // that nothing comes in, and never wait: no branch on the wavefront's place in the hot loop.
+  if (wave == 0) avail = 0x7fffffff;
+  auto fetch_hand = [&](int g, float4& h) {
+    if (W == 1 || g >= ngroups) return;
+    const int need = 4 * g + 3;  // the scores entering steps 4g .. 4g+3 left steps 4g-1 .. 4g+2
+    if (__builtin_expect(avail < need, 0)) wait_for(need);
+    h = *reinterpret_cast<const float4*>(hand_in + (wave > 0 ? 4 * g : 0));
+  };
   // kWhole: all four steps of the group exist (every group but the last; no test per step)
-  auto run_group = [&](int g, const Group& cur, auto whole) {
+  // kInterior: all four steps of every position of this wavefront (those past the utterance's
+  // last one aside, see above) are inside the lattice, and no bounds are looked at; that is all
+  // but the first and last 64 C steps or so.
+  auto run_group = [&](int g, const Group& cur, const float4& hand_cur, float4& hand_next,
+                       auto whole, auto interior) {
     constexpr bool kWhole = decltype(whole)::value;
+    constexpr bool kInterior = decltype(interior)::value;
     float4 aout[C];
     // what enters the wavefront's first column from the left: for the lattice's own first
     // column (u = 0) nothing, which is -inf while its cells are inside the lattice (:49-52 adds
@@ -542,7 +619,8 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
     // past the last frame (the idle lane's pair is then (kOutside, -inf) again)
     float4 hin;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) f4set(hin, j, (first_column && 4 * g + j < Tb) ? kNegInf : kOutside);
+    for (int j = 0; j < 4; ++j)
+      f4set(hin, j, (first_column && (kInterior || 4 * g + j < Tb)) ? kNegInf : kOutside);
     if constexpr (kMulti) {
       if (gin) hin = cur.gh;  // wavefront 0: from the block below
       if constexpr (kLive) {
@@ -577,45 +655,58 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
         }
       }
     }
-    if (W > 1 && wave > 0) {
-      wait_for(4 * g + 3);  // the scores entering steps 4g .. 4g+3 left steps 4g-1 .. 4g+2
-      hin = *reinterpret_cast<const float4*>(hand_in + 4 * g);
+    if constexpr (W > 1) {
+      if (kInterior && !kMulti) hin = hand_cur;
+      else if (wave > 0) hin = hand_cur;
+      fetch_hand(g + 1, hand_next);
     }
-    float hout[4];
     float gsend[4];  // what this lane's last column hands to the right after each step
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int s = 4 * g + j;
-      if constexpr (kMulti) gsend[j] = kOutside;
+      gsend[j] = kOutside;
       if (kWhole || s < nsteps) {  // uniform; a step past the last must not touch the scores
         const float from_left = wave_shr1(emit[C - 1], f4get(hin, j));  // lane 0: hin
 #pragma unroll
         for (int c = C - 1; c >= 0; --c) {
           const float left = (c == 0) ? from_left : emit[c - 1];
-          const float a = lse2_checked(left, stay[c], etab);
           const float ln = f4get(cur.ln[c], j);
-          float sb = a + cur.eb[j - c + (C - 1)];
-          sb = sb + pbv[c];
-          sb = sb - ln;
-          float se = a + f4get(cur.el[c], j);
-          se = se + plv[c];
-          se = se - ln;
+          float a, sb, se;
+          auto moves = [&](float x) {
+            a = x;
+            sb = a + cur.eb[j - c + (C - 1)];
+            sb = sb + pbv[c];
+            sb = sb - ln;
+            se = a + f4get(cur.el[c], j);
+            se = se + plv[c];
+            se = se - ln;
+          };
+          // the moves go on from the fast sum while its proof is still on its way
+          const FastLse fast = lse2_fast(left, stay[c]);
+          moves(fast.lo);
+          asm volatile("" : "+v"(sb), "+v"(se));
+          if (__builtin_expect(
+                  __builtin_amdgcn_ballot_w64(!(fast.lo == fast.up)) != 0ull, 0))
+            moves(lse2_libm(left, stay[c], etab));
           // a cell of the lattice: 0 <= t = s - u < T_b (one unsigned comparison).  Cells before
           // the first frame or past the last one hand kOutside on, so whatever the planes hold
           // outside the utterance never enters a log-sum-exp (where it would cost the whole
           // wavefront the library path).
-          const bool inside = (unsigned)(s - (u0 + c)) < tlim[c];
+          const bool inside = kInterior || (unsigned)(s - (u0 + c)) < tlim[c];
           stay[c] = inside ? sb : kNegInf;
           emit[c] = inside ? se : kOutside;
           f4set(aout[c], j, a);
         }
-        if constexpr (kMulti) gsend[j] = emit[C - 1];
+        gsend[j] = emit[C - 1];
       }
-      if (W > 1)
-        hout[j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(emit[C - 1]), 63));
     }
 #pragma unroll
-    for (int c = 0; c < C; ++c) *reinterpret_cast<float4*>(ap[c] + (size_t)g * gstride) = aout[c];
+    for (int c = 0; c < C; ++c) {
+      if constexpr (kInterior)
+        *reinterpret_cast<float4*>(a_b + (size_t)(a_o[c] + (unsigned)g * (4u * (unsigned)gstride))) = aout[c];
+      else
+        *reinterpret_cast<float4*>(ap[c] + (size_t)g * gstride) = aout[c];
+    }
     if constexpr (kMulti) {
       if (gout && wave == W - 1 && lane == 63) {  // entries 4g+1 .. 4g+4 for the block above
 #pragma unroll
@@ -630,9 +721,9 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
         }
       }
     }
-    if (W > 1 && wave < W - 1 && lane == 0) {  // entries 4g+1 .. 4g+4, then the progress
+    if (W > 1 && wave < W - 1 && lane == 63) {  // entries 4g+1 .. 4g+4, then the progress
 #pragma unroll
-      for (int j = 0; j < 4; ++j) hand_out[4 * g + 1 + j] = hout[j];
+      for (int j = 0; j < 4; ++j) hand_out[4 * g + 1 + j] = gsend[j];
       asm volatile("" ::: "memory");
       __hip_atomic_store(&done[wave], 4 * g + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
@@ -656,25 +747,59 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
   Group q0 = load_group(0), q1 = load_group(clamp_g(1)), q2 = load_group(clamp_g(2)),
         q3 = load_group(clamp_g(3));
   if (W > 1 && wave > 0) wait_for(min(4 * ngroups, 4 * (kLive ? kLiveWaveLag : 8) * wave));  // fall a few groups behind
-  const std::true_type whole;
-  const std::false_type partial;
-  const int nwhole = nsteps >> 2;  // groups with all four steps
+  const std::true_type whole, interior;
+  const std::false_type partial, edge;
+  auto load_inner = [&](int g) -> Group {
+    Group r;
+    const unsigned by = (unsigned)g * (4u * (unsigned)gstride);  // bytes
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      r.ln[c] = *reinterpret_cast<const float4*>(ln_b + (size_t)(ln_o[c] + by));
+      r.el[c] = *reinterpret_cast<const float4*>(el_b + (size_t)(el_o[c] + by));
+    }
+    const unsigned eo = eb_o + 16u * (unsigned)g;
+#pragma unroll
+    for (int k = 0; k < C + 3; ++k)
+      r.eb[k] = reinterpret_cast<const float*>(eb_b + (size_t)eo)[k];
+    if constexpr (kMulti) {
+      r.gh = make_float4(kOutside, kOutside, kOutside, kOutside);
+      if (gin) r.gh = *reinterpret_cast<const float4*>(gin + 4 * g);  // uniform
+      if constexpr (kLive) r.lv = live_load(4 * g + (lane & 3));
+    }
+    return r;
+  };
+  float4 h0 = make_float4(kOutside, kOutside, kOutside, kOutside), h1 = h0;
+  fetch_hand(0, h0);
   int g = 0;
   for (; g + 4 <= nwhole; g += 4) {
-    run_group(g, q0, whole);
+    // (with eight or sixteen positions a lane the registers are what is short)
+    if constexpr (C <= 4) {
+      for (; g >= in_lo && g + 4 <= in_hi && g + 8 <= ngroups; g += 4) {
+        run_group(g, q0, h0, h1, whole, interior);
+        q0 = load_inner(g + 4);
+        run_group(g + 1, q1, h1, h0, whole, interior);
+        q1 = load_inner(g + 5);
+        run_group(g + 2, q2, h0, h1, whole, interior);
+        q2 = load_inner(g + 6);
+        run_group(g + 3, q3, h1, h0, whole, interior);
+        q3 = load_inner(g + 7);
+      }
+      if (g + 4 > nwhole) break;
+    }
+    run_group(g, q0, h0, h1, whole, edge);
     q0 = load_group(clamp_g(g + 4));
-    run_group(g + 1, q1, whole);
+    run_group(g + 1, q1, h1, h0, whole, edge);
     q1 = load_group(clamp_g(g + 5));
-    run_group(g + 2, q2, whole);
+    run_group(g + 2, q2, h0, h1, whole, edge);
     q2 = load_group(clamp_g(g + 6));
-    run_group(g + 3, q3, whole);
+    run_group(g + 3, q3, h1, h0, whole, edge);
     q3 = load_group(clamp_g(g + 7));
   }
   // the last one to four groups, the very last of which may be partial
-  if (g < ngroups) run_group(g, q0, partial);
-  if (g + 1 < ngroups) run_group(g + 1, q1, partial);
-  if (g + 2 < ngroups) run_group(g + 2, q2, partial);
-  if (g + 3 < ngroups) run_group(g + 3, q3, partial);
+  if (g < ngroups) run_group(g, q0, h0, h1, partial, edge);
+  if (g + 1 < ngroups) run_group(g + 1, q1, h1, h0, partial, edge);
+  if (g + 2 < ngroups) run_group(g + 2, q2, h0, h1, partial, edge);
+  if (g + 3 < ngroups) run_group(g + 3, q3, h1, h0, partial, edge);
   // :73-78 the blank move out of the last cell, negated; that cell was the last one its
   // column processed
 #pragma unroll
@@ -2085,6 +2210,7 @@ __global__ __launch_bounds__(256) void lse_bound_kernel(unsigned lo, unsigned hi
 }
 }  // namespace
 
+#if RNNT_IN_PART(0)
 int launch_lse_bound_check(unsigned lo, unsigned hi, unsigned* out, hipStream_t s) {
   hipLaunchKernelGGL(lse_bound_kernel, dim3(4096), dim3(256), 0, s, lo, hi, out);
   hipError_t err = hipGetLastError();
@@ -2199,12 +2325,15 @@ void carve_planes(void* base, const Dims& d, Planes* p, bool decode_only) {
   p->hand[0] = take(bh); p->hand[1] = take(bh);
 }
 
+#endif
+
 // ------------------------------------------------------------------ launchers
 // tiles of 64 anti-diagonals x 64 label positions over all anti-diagonals t + u < T + U
 static dim3 tile_grid(const Dims& d) {
   return dim3((d.T + d.U + 62) / 64, (d.U + 63) / 64, d.B);
 }
 
+#if RNNT_IN_PART(0)
 int launch_skew(const float* src, float* dstS, const int* inLen, const int* labLen, const Dims& d,
                 hipStream_t s) {
   if (d.B == 0 || d.T == 0 || d.U == 0) return kOk;
@@ -2247,6 +2376,8 @@ int launch_gather(const f16_t* E, const f16_t* P, const int* labels, const int* 
   return gather_any(E, P, labels, inLen, labLen, p, d, s);
 }
 
+#endif
+
 // Label positions one launch of a lattice walk covers: the whole axis up to 1024, else blocks of
 // 1024 (64 lanes x 16 positions), one launch per block.
 static int block_cells_per_lane(const Dims& d) { return min(cells_per_lane(d.U), 16); }
@@ -2255,7 +2386,7 @@ static int label_blocks(const Dims& d) {
   return (d.U + width - 1) / width;
 }
 
-__global__ void clear_words_kernel(int* x, int n) {
+static __global__ void clear_words_kernel(int* x, int n) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < n) x[i] = 0;
 }
@@ -2281,6 +2412,20 @@ static int launch_live(K kernel, const Planes& p, const Dims& d, int n, int W,
   return kOk;
 }
 
+int launch_alpha_wide(const Planes& p, const int* inLen, const int* labLen, float* costs,
+                      const Dims& d, hipStream_t s, int C, int W, bool multi, size_t lds,
+                      int* trouble, int u_base, const float* ghin, float* ghout);
+#define CASE(C, W, M)                                                                        \
+  case (M ? 10000 : 0) + C * 100 + W:                                                        \
+    if (lds > 64 * 1024)                                                                     \
+      RNNT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(alpha_kernel<C, W, M>),     \
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));   \
+    hipLaunchKernelGGL((alpha_kernel<C, W, M>), dim3(d.B), dim3(64 * W), lds, s, p, inLen,  \
+                       labLen, costs, d, stride, g_spin_limit, trouble, u_base, ghin,        \
+                       ghout, nullptr, 0);                                                   \
+    break;
+
+#if RNNT_IN_PART(1)
 int launch_alpha(const Planes& p, const int* inLen, const int* labLen, float* costs,
                  const Dims& d, hipStream_t s) {
   if (d.B == 0) return kOk;
@@ -2291,8 +2436,8 @@ int launch_alpha(const Planes& p, const int* inLen, const int* labLen, float* co
   // (two wavefronts up to 128 label positions, four beyond -- one, two or four positions a lane
   // -- if their three hand-over arrays fit LDS: a step costs a wavefront one log-sum-exp per
   // position it owns, and the step is what a lattice is bound by.  B=8 T=2000, 129..256 label
-  // positions: 262 ns a step with two wavefronts of two positions, 160 with four of one, what
-  // 101 positions on two wavefronts take)
+  // positions: 117 ns a step with four wavefronts of one position, what 101 positions on two
+  // wavefronts take; two wavefronts of two positions were 1.6 times as slow as that)
   const bool single_block = nblocks == 1;
   const int W = (single_block && cpl >= 4 && 3 * stride * sizeof(float) <= 144 * 1024) ? 4
                 : (cpl >= 2 && stride * sizeof(float) <= 144 * 1024) ? 2 : 1;
@@ -2301,9 +2446,9 @@ int launch_alpha(const Planes& p, const int* inLen, const int* labLen, float* co
   RNNT_TRY(trouble_flag(&trouble));
   // From 257 label positions, with few enough utterances that the device has the CUs: blocks
   // of 256 positions side by side on as many CUs, four wavefronts of one position a lane each
-  // (B=8 T=10000, 401 positions: 176 ns a step against 235 on one CU; B=8 T=2000, 513 .. 1024
-  // positions: 523 .. 539 ns on one CU with two to four positions a lane; from about a hundred
-  // utterances on the planes' traffic holds every form, B=128 T=2000: 241 ns)
+  // (B=8 T=10000, 401 positions: 129 ns a step, 150 at T=2000 and from 513 to 1024 positions; on
+  // one CU, before the cell was shortened, 235 and 523 .. 539 against 176 and 198 side by side;
+  // from about a hundred utterances on the planes' traffic holds every form, B=128 T=2000: 235 ns)
   int live_w = 0;
   if (const int n = live_blocks(d, &live_w)) {
     if (live_w == 4)
@@ -2318,28 +2463,37 @@ int launch_alpha(const Planes& p, const int* inLen, const int* labLen, float* co
     float* ghout = k == nblocks - 1 ? nullptr : p.hand[k & 1];
     const int u_base = k * 64 * cpl;
     switch ((nblocks > 1 ? 10000 : 0) + cpl / W * 100 + W) {
-#define CASE(C, W, M)                                                                        \
-  case (M ? 10000 : 0) + C * 100 + W:                                                        \
-    if (lds > 64 * 1024)                                                                     \
-      RNNT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(alpha_kernel<C, W, M>),     \
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));   \
-    hipLaunchKernelGGL((alpha_kernel<C, W, M>), dim3(d.B), dim3(64 * W), lds, s, p, inLen,  \
-                       labLen, costs, d, stride, g_spin_limit, trouble, u_base, ghin,        \
-                       ghout, nullptr, 0);                                                   \
-    break;
-      CASE(1, 1, false) CASE(2, 1, false) CASE(4, 1, false) CASE(8, 1, false) CASE(16, 1, false)
-      CASE(1, 2, false) CASE(2, 2, false) CASE(4, 2, false) CASE(8, 2, false)
+      CASE(1, 1, false) CASE(2, 1, false) CASE(4, 1, false)
+      CASE(1, 2, false) CASE(2, 2, false) CASE(4, 2, false)
       CASE(1, 4, false) CASE(2, 4, false) CASE(4, 4, false)
-      CASE(16, 1, true) CASE(8, 2, true)  // several blocks: always 1024 positions each
-#undef CASE
       default:
-        return fail(kInvalid, "alpha: no kernel for %d label positions per lane", cpl);
+        RNNT_TRY(launch_alpha_wide(p, inLen, labLen, costs, d, s, cpl / W, W, nblocks > 1, lds,
+                                   trouble, u_base, ghin, ghout));
     }
     RNNT_LAUNCH_CHECK("alpha_kernel");
   }
   return kOk;
 }
+#endif
 
+#if RNNT_IN_PART(2)
+// eight or sixteen label positions a lane; several blocks are always 1024 positions each
+int launch_alpha_wide(const Planes& p, const int* inLen, const int* labLen, float* costs,
+                      const Dims& d, hipStream_t s, int C, int W, bool multi, size_t lds,
+                      int* trouble, int u_base, const float* ghin, float* ghout) {
+  const int stride = d.Dp;
+  switch ((multi ? 10000 : 0) + C * 100 + W) {
+    CASE(8, 1, false) CASE(16, 1, false) CASE(8, 2, false)
+    CASE(16, 1, true) CASE(8, 2, true)
+    default:
+      return fail(kInvalid, "alpha: no kernel for %d label positions per lane", C);
+  }
+  return kOk;
+}
+#endif
+#undef CASE
+
+#if RNNT_IN_PART(0)
 int launch_weights(const Planes& p, const int* inLen, const int* labLen, const Dims& d,
                    hipStream_t s) {
   if (d.B == 0 || d.T == 0 || d.U == 0) return kOk;
@@ -2349,6 +2503,9 @@ int launch_weights(const Planes& p, const int* inLen, const int* labLen, const D
   return kOk;
 }
 
+#endif
+
+#if RNNT_IN_PART(3)
 int launch_beta(const Planes& p, const int* labels, const int* inLen, const int* labLen,
                 const Dims& d, hipStream_t s) {
   if (d.B == 0 || d.T == 0 || d.U == 0) return kOk;
@@ -2403,7 +2560,9 @@ int launch_beta(const Planes& p, const int* labels, const int* inLen, const int*
   }
   return kOk;
 }
+#endif
 
+#if RNNT_IN_PART(0)
 int launch_sparse(const Planes& p, const float* bsum, const float* emT, float* egrads,
                   float* pgrads, const int* labels, const int* inLen, const int* labLen,
                   const float* scale, bool add, const Dims& d, hipStream_t s) {
@@ -2499,7 +2658,9 @@ int launch_maxplus(const f16_t* E, const f16_t* P, const int* inLen, const int* 
                    float* best, int* arg, const Dims& d, hipStream_t s, void* lists, bool force) {
   return maxplus_any(E, P, inLen, labLen, best, arg, d, s, lists, force);
 }
+#endif
 
+#if RNNT_IN_PART(4)
 // 32-step words per column of the decision table (one spare)
 static int viterbi_words(const Dims& d) { return (d.T + d.U + 31) / 32 + 1; }
 
@@ -2596,5 +2757,6 @@ int launch_viterbi(const Planes& p, const float* bestS, const float* argS,
 size_t viterbi_bits_bytes(const Dims& d) {
   return sizeof(unsigned) * (size_t)d.B * 64 * cells_per_lane(d.U) * viterbi_words(d);
 }
+#endif
 
 }  // namespace rnnt
