@@ -184,6 +184,18 @@ size_t rnnt_hip_static_scratch_bytes(void);
  * when no such call is in flight).  No counterpart in the reference. */
 int rnnt_hip_release_scratch(void);
 
+/* The reference's front end compares the longest utterance with the padded sizes before it calls
+ * the library (transducer/torch_binding.py:222-228), which waits for the device.  _begin enqueues
+ * that comparison; _end, called once the rest is enqueued, waits for its result alone (not for
+ * what was enqueued after it) and gives the ticket back: verdict is 0, or 1 if some input_length
+ * exceeds T, plus 2 if some label_length exceeds U - 1.  Every kernel clamps lengths to the
+ * padded sizes, so what is enqueued in between stays inside the arrays either way.  One _end per
+ * successful _begin, on the same stream; not capturable; any thread.  At most 256 under way:
+ * _begin then fails and enqueues nothing. */
+int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_lengths, int B, int T,
+                                 int U, rnnt_stream_t stream, int* ticket);
+int rnnt_hip_check_lengths_end(int ticket, rnnt_stream_t stream, int* verdict);
+
 /* ---- stage timing (diagnostic; no counterpart in the reference, whose only instrumentation
  * is wall-clock loops in transducer/benchmark.cpp:21-34) ---------------------------------- */
 

@@ -226,3 +226,60 @@ def test_fused_entry_points_replay_from_a_captured_graph(shape):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(costs, want[0]) and torch.equal(eg, want[1]) and torch.equal(pg, want[2])
+
+
+@pytest.mark.parametrize("B", [1, 257])
+def test_lengths_past_the_padded_sizes_are_refused_after_the_work_is_enqueued(B):
+    """The lengths are compared on the device beside the call's own kernels: the same errors in
+    the same order of precedence as a comparison made first, also for the largest integer, and
+    the next call is untouched.  More calls than there are checks that may be under way."""
+    device, gen = torch.device("cuda"), torch.Generator().manual_seed(B)
+    E, P = torch.randn(B, 6, 5, generator=gen).to(device), torch.randn(B, 4, 5, generator=gen).to(device)
+    labels = torch.randint(1, 5, (B, 3), generator=gen, dtype=torch.int32).to(device)
+    fit = [torch.full((B,), n, dtype=torch.int32, device=device) for n in (6, 3)]
+    criterion = TransducerLoss()
+    want = criterion(E, P, labels, *fit), criterion.viterbi(E, P, *fit)
+    for inputs, outputs, message in ((7, 3, "Input"), (6, 4, "Output"), (7, 4, "Input"),
+                                     (2 ** 31 - 1, 2 ** 31 - 1, "Input"), (6, 2 ** 31 - 1, "Output")):
+        il, ll = fit[0].clone(), fit[1].clone()
+        il[B - 1], ll[B - 1] = inputs, outputs
+        with pytest.raises(ValueError, match=message + " length mismatch"):
+            criterion(E, P, labels, il, ll)
+        with pytest.raises(ValueError, match=message + " length mismatch"):
+            criterion.viterbi(E, P, il, ll)
+        with pytest.raises(ValueError, match=message + " length mismatch"):
+            TransducerLoss(blank=5)(E, P, labels, il, ll)
+    with pytest.raises(ValueError, match="blank must lie in"):
+        TransducerLoss(blank=5)(E, P, labels, *fit)
+    for _ in range(300):
+        costs = criterion(E, P, labels, *fit)
+    assert torch.equal(costs, want[0])
+    assert torch.equal(criterion.viterbi(E, P, *fit), want[1])
+
+
+def test_lengths_are_checked_on_each_threads_own_stream():
+    import threading
+    device, gen = torch.device("cuda"), torch.Generator().manual_seed(3)
+    E, P = torch.randn(3, 40, 9, generator=gen).to(device), torch.randn(3, 8, 9, generator=gen).to(device)
+    labels = torch.randint(1, 9, (3, 7), generator=gen, dtype=torch.int32).to(device)
+    il = torch.tensor([40, 31, 7], dtype=torch.int32, device=device)
+    ll = torch.tensor([7, 2, 0], dtype=torch.int32, device=device)
+    want = TransducerLoss()(E, P, labels, il, ll)
+    torch.cuda.synchronize()
+    wrong = []
+
+    def caller(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for i in range(50):
+                try:
+                    costs = TransducerLoss()(E, P, labels, il + (k + i) % 2, ll)
+                    ok = (k + i) % 2 == 0 and torch.equal(costs, want)
+                except ValueError as error:
+                    ok = (k + i) % 2 == 1 and "Input length mismatch" in str(error)
+                if not ok:
+                    wrong.append((k, i))
+
+    threads = [threading.Thread(target=caller, args=(k,)) for k in range(4)]
+    for t in threads: t.start()
+    for t in threads: t.join()
+    assert not wrong

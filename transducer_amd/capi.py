@@ -30,6 +30,8 @@ SIGNATURES = {
     "rnnt_hip_viterbi_decode_static": (_I, [_F] * 5 + [_I] * 5 + [_F]),
     "rnnt_hip_static_scratch_bytes": (_Z, []),
     "rnnt_hip_release_scratch": (_I, []),
+    "rnnt_hip_check_lengths_begin": (_I, [_F] * 2 + [_I] * 3 + [_F] * 2),
+    "rnnt_hip_check_lengths_end": (_I, [_I] + [_F] * 2),
     "rnnt_hip_viterbi_decode_bf16": (_I, [_F] * 5 + [_I] * 5 + [_F]),
     "rnnt_hip_viterbi_decode_f16": (_I, [_F] * 5 + [_I] * 5 + [_F]),
     "rnnt_hip_check_kernels": (_I, [_F]),

@@ -245,6 +245,31 @@ PYBIND11_MODULE(_transducer, m) {
         "batch_size"_a, "max_input_length"_a, "max_label_length"_a, "alphabet_size"_a, "blank"_a,
         "stream"_a = 0);
 
+  // -> ticket, or -1 where the check could not be enqueued (the caller then compares by itself)
+  m.def("check_lengths_begin",
+        [](ptr_t input_lengths, ptr_t label_lengths, int batch_size, int max_input_length,
+           int max_label_length, ptr_t stream) {
+          int ticket = -1;
+          const int status = rnnt_hip_check_lengths_begin(
+              as<const int>(input_lengths), as<const int>(label_lengths), batch_size,
+              max_input_length, max_label_length, as<void>(stream), &ticket);
+          return status == RNNT_OK ? ticket : -1;
+        },
+        "input_lengths"_a, "label_lengths"_a, "batch_size"_a, "max_input_length"_a,
+        "max_label_length"_a, "stream"_a);
+
+  m.def("check_lengths_end",
+        [](int ticket, ptr_t stream) {
+          int verdict = 0, status;
+          {
+            py::gil_scoped_release unlocked;
+            status = rnnt_hip_check_lengths_end(ticket, as<void>(stream), &verdict);
+          }
+          raise_on(status);
+          return verdict;
+        },
+        "ticket"_a, "stream"_a);
+
 #ifdef VERSION_INFO
   m.attr("__version__") = VERSION_INFO;
 #else

@@ -93,7 +93,7 @@ __device__ inline int clampi(int x, int lo, int hi) { return x < lo ? lo : (x > 
 __device__ inline void utt_extent(const int* inLen, const int* labLen, int b, int T, int U,
                                   int& Tb, int& Ub) {
   Tb = inLen ? clampi(inLen[b], 0, T) : T;
-  Ub = labLen ? clampi(labLen[b] + 1, 0, U) : U;
+  Ub = labLen ? clampi(labLen[b], -1, U - 1) + 1 : U;
 }
 
 // Label of position u of utterance b, forced into the vocabulary.  The reference indexes its

@@ -109,7 +109,7 @@ __global__ __launch_bounds__(256) void rowmax_pick_p_kernel(const TIO* __restric
   const int lane = threadIdx.x & 63;
   if (row >= (long)d.B * d.U) return;
   const int b = (int)(row / d.U), u = (int)(row - (long)b * d.U);
-  const int Ub = min(max(labLen[b], 0) + 1, d.U);
+  const int Ub = clampi(labLen[b], 0, d.U - 1) + 1;
   if (u >= Ub) {
     if (lane == 0) mP[row] = 0.0f;
     return;
