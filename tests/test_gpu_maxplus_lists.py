@@ -316,3 +316,36 @@ def test_16bit_decode_same_labels_in_both_modes(dtype):
 def test_mode_is_validated():
     with pytest.raises(Exception):
         capi.call("rnnt_hip_set_maxplus_mode", 3)
+
+
+@pytest.mark.parametrize("V", [2, 33, 127, 128, 129, 515, 1056])
+@pytest.mark.parametrize("B,T,U", [(1, 1, 1), (2, 129, 65), (3, 63, 4), (1, 200, 130)])
+def test_ranges_of_columns_side_by_side(B, T, U, V):
+    """Every column for every cell, the columns dealt to workgroups in ranges: one to sixteen of
+    them here.  Quantised scores tie within a chunk, across chunks and across ranges; rows of -inf
+    win nowhere; the blank sits at a range's edge."""
+    rng = np.random.default_rng(V * 1000 + T)
+    E = rng.integers(-2, 3, (B, T, V)).astype(np.float32)
+    P = rng.integers(-2, 3, (B, U, V)).astype(np.float32)
+    E[0, T // 2] = -np.inf
+    E[B - 1, 0, V // 2] = np.inf
+    P[0, U // 2] = -np.inf
+    il, ll = lengths(rng, B, T, U)
+    for blank in (0, V // 2, V - 1):
+        check(E, P, il, ll, blank, modes=(1,))
+
+
+def test_ranges_of_columns_give_way_where_the_scratch_is_fixed():
+    """The decode with built-in scratch takes fewer ranges where the rest of its scratch leaves no
+    room for all of them; its labels are the allocating decode's."""
+    import torch
+    B, T, U, V = 8, 2000, 101, 1000
+    rng = np.random.default_rng(5)
+    E, P = dev(rng.standard_normal((B, T, V), dtype=np.float32)), dev(
+        rng.standard_normal((B, U, V), dtype=np.float32))
+    il, ll = (dev(x) for x in lengths(rng, B, T, U))
+    out = [torch.full((B, U - 1), -1, dtype=torch.int32, device=E.device) for _ in range(2)]
+    for entry, o in zip(("rnnt_hip_viterbi_decode_static", "rnnt_hip_viterbi_decode"), out):
+        capi.call(entry, ptr(E), ptr(P), ptr(il), ptr(ll), ptr(o), B, T, U, V, 0, None)
+    torch.cuda.synchronize()
+    assert torch.equal(*out)

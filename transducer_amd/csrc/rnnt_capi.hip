@@ -143,6 +143,11 @@ class Scratch {
     size_ = bytes;
     return kOk;
   }
+  // what an allocation of this many bytes leaves in a fixed region, rounded down to whole pieces
+  size_t room(size_t bytes) const {
+    if (!fixed_) return ~(size_t)0;
+    return bytes < capacity_ ? (capacity_ - bytes) & ~(size_t)255 : 0;
+  }
   void* take(size_t bytes) {
     void* p = static_cast<char*>(base_) + used_;
     used_ += align_up(bytes);
@@ -331,24 +336,23 @@ void release_check_slot(int slot) {
 }
 
 // Scratch the best-path stages need (planes, the two max-plus planes, the decision table).
-// `lists`: whether this call builds its table of best labels from candidate lists (asked once
-// per call, so that what is reserved and what is taken agree whatever another thread sets).
-size_t viterbi_scratch_bytes(const Dims& d, bool lists) {
+// `plan`: how this call builds its table of best labels (asked once per call, so that what is
+// reserved and what is taken agree whatever another thread sets).
+size_t viterbi_scratch_bytes(const Dims& d, const MaxplusPlan& plan) {
   const size_t plane = sizeof(float) * (size_t)d.B * d.Ua * d.Dp + 64;
   return align_up(planes_bytes(d, true)) + 2 * align_up(plane) +
          align_up(viterbi_bits_bytes(d)) +
-         (lists ? align_up(maxplus_lists_bytes(d)) : 0);
+         align_up(plan.bytes);
 }
 
-// `scratch` has viterbi_scratch_bytes(d, with_lists) left to take (one allocation per call, made by the caller
+// `scratch` has viterbi_scratch_bytes(d, plan) left to take (one allocation per call, made by the caller
 // together with whatever else it needs: the allocator calls are a visible part of a small decode).
 // With `ready`, the lattice planes were carved by the caller and already hold LN and the blank
 // scores (the log-normaliser left them there): no transposing copy, no gather.
 template <typename TIO>
 int viterbi_impl(const TIO* E, const TIO* P, const float* LN, int* labels,
                         const int* inLen, const int* labLen, const Dims& d, Scratch& scratch,
-                        hipStream_t s, int plan, const Planes* ready = nullptr) {
-  const bool with_lists = plan != 0;
+                        hipStream_t s, const MaxplusPlan& plan, const Planes* ready = nullptr) {
   const size_t plane = sizeof(float) * (size_t)d.B * d.Ua * d.Dp + 64;
   Planes p;
   if (ready) p = *ready;
@@ -357,9 +361,9 @@ int viterbi_impl(const TIO* E, const TIO* P, const float* LN, int* labels,
   float* argS = static_cast<float*>(scratch.take(plane));
   unsigned long long* bits =
       static_cast<unsigned long long*>(scratch.take(viterbi_bits_bytes(d)));
-  void* lists = with_lists ? scratch.take(maxplus_lists_bytes(d)) : nullptr;
+  void* table = plan.bytes ? scratch.take(plan.bytes) : nullptr;
   RNNT_STAGE(kMaxplus, launch_maxplus(E, P, inLen, labLen, bestS, reinterpret_cast<int*>(argS), d,
-                                      s, lists, plan == 2));
+                                      s, table, plan));
   if (!ready) {
     RNNT_STAGE(kSkew, launch_skew(LN, p.lnS, inLen, labLen, d, s));
     // blank scores only: the label planes of the gather are not needed here
@@ -476,11 +480,10 @@ int lowp_viterbi_decode(const TIO* E, const TIO* P, const int* inLen, const int*
   if (!lse_stream_supported(E, d)) return fail(kInvalid, "%s: B*T*U too large", who);
   Scratch scratch(s);
   const size_t yb = lse_scratch_bytes(d);
-  const int plan = maxplus_plan(d);
-  const bool with_lists = plan != 0;
+  const MaxplusPlan plan = maxplus_plan(d);
   RNNT_TRY(scratch.reserve(align_up(sizeof(float) * (size_t)B * T) +
                            align_up(sizeof(float) * (size_t)B * U) + align_up(yb) +
-                           viterbi_scratch_bytes(d, with_lists)));
+                           viterbi_scratch_bytes(d, plan)));
   float* mE = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * T));
   float* mP = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * U));
   void* ys = scratch.take(yb);
@@ -507,13 +510,13 @@ int decode_fp32(const float* E, const float* P, const int* inLen, const int* lab
   const Dims d = make_dims(B, T, U, V, blank);
   if (!lse_stream_supported(E, d)) return fail(kInvalid, "%s: B*T*U too large", who);
   const size_t yb = lse_scratch_bytes(d);
-  const int plan = maxplus_plan(d);
-  const bool with_lists = plan != 0;
   // LN and the blank scores go straight into the lattice planes, as in the whole-loss path
   // (no row-major LN, no transposing copy, no gather)
-  RNNT_TRY(scratch.reserve(align_up(sizeof(float) * (size_t)B * T) +
-                           align_up(sizeof(float) * (size_t)B * U) + align_up(yb) +
-                           viterbi_scratch_bytes(d, with_lists)));
+  const size_t base = align_up(sizeof(float) * (size_t)B * T) +
+                      align_up(sizeof(float) * (size_t)B * U) + align_up(yb) +
+                      viterbi_scratch_bytes(d, MaxplusPlan());
+  const MaxplusPlan plan = maxplus_plan(d, scratch.room(base));
+  RNNT_TRY(scratch.reserve(base + align_up(plan.bytes)));
   float* mE = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * T));
   float* mP = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * U));
   void* ys = scratch.take(yb);
@@ -616,21 +619,19 @@ int rnnt_hip_maxplus_table(const float* E, const float* P, const int* inLen, con
   hipStream_t s = static_cast<hipStream_t>(stream);
   const Dims d = make_dims(B, T, U, V, blank);
   const size_t plane = sizeof(float) * (size_t)d.B * d.Ua * d.Dp + 64;
-  const int plan = maxplus_plan(d);
-  const bool with_lists = plan != 0;
+  const MaxplusPlan plan = maxplus_plan(d);
   Scratch scratch(s);
-  RNNT_TRY(scratch.reserve(2 * align_up(plane) +
-                           (with_lists ? align_up(maxplus_lists_bytes(d)) : 0)));
+  RNNT_TRY(scratch.reserve(2 * align_up(plane) + align_up(plan.bytes)));
   float* bestS = static_cast<float*>(scratch.take(plane));
   int* argS = static_cast<int*>(scratch.take(plane));
-  void* lists = with_lists ? scratch.take(maxplus_lists_bytes(d)) : nullptr;
-  RNNT_STAGE(kMaxplus, launch_maxplus(E, P, inLen, labLen, bestS, argS, d, s, lists, plan == 2));
+  void* table = plan.bytes ? scratch.take(plan.bytes) : nullptr;
+  RNNT_STAGE(kMaxplus, launch_maxplus(E, P, inLen, labLen, bestS, argS, d, s, table, plan));
   return launch_table_out(bestS, argS, inLen, labLen, best, arg, d, s);
 }
 
 int rnnt_hip_maxplus_tries_lists(int B, int T, int U, int V) {
   if (B <= 0 || T <= 0 || U <= 0 || V <= 0) return 0;
-  return maxplus_plan(make_dims(B, T, U, V, 0)) != 0 ? 1 : 0;
+  return maxplus_plan(make_dims(B, T, U, V, 0)).lists != 0 ? 1 : 0;
 }
 
 int rnnt_hip_set_fused_grads(int mode) {
@@ -771,9 +772,8 @@ int rnnt_hip_viterbi(const float* E, const float* P, const float* LN, int* label
   const Dims d = make_dims(B, T, U, V, blank);
   hipStream_t s = static_cast<hipStream_t>(stream);
   Scratch scratch(s);
-  const int plan = maxplus_plan(d);
-  const bool with_lists = plan != 0;
-  RNNT_TRY(scratch.reserve(viterbi_scratch_bytes(d, with_lists)));
+  const MaxplusPlan plan = maxplus_plan(d);
+  RNNT_TRY(scratch.reserve(viterbi_scratch_bytes(d, plan)));
   return viterbi_impl(E, P, LN, labels, inLen, labLen, d, scratch, s, plan);
 }
 

@@ -17,6 +17,7 @@
 // The file is compiled in parts side by side (-DRNNT_DP_PART=0..4: everything else, the alpha
 // walk in its narrow and its wide forms, the dalpha walk, the best-path walk; all of it without
 // the macro): a part holds the launchers that instantiate its kernels.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -1628,11 +1629,57 @@ __global__ __launch_bounds__(256) void sparse_p_kernel(Planes p, float* __restri
 // Wavefronts whose label positions lie past the utterance only help staging.
 constexpr int kMpT = 128, kMpK = 32, kMpPitch = 36, kMpRows = 8;
 constexpr int kMpWaves = 8, kMpU = kMpWaves * kMpRows, kMpThreads = 64 * kMpWaves;
+// As many ranges of columns as bring the grid to kMpWanted workgroups (two fit a CU at a time, and
+// the padded tiles of short utterances end at once), each range at least kMpMinChunks chunks long.
+// The table of B=16 T=1500 U=81 V=2001 (384 tiles): 495 us before ranges, 344 with two, 359 with five;
+// B=8 T=2000 U=101 V=1000 (256): 191, 146 with four, 158 with eight; B=32 of the same (1024): 641,
+// 546 with one, 539 with two.
+constexpr long kMpWanted = 1024, kMpMinChunks = 2, kMpMaxParts = 16;
 constexpr int kMpEPasses = kMpT * (kMpK / 4) / kMpThreads;  // 16-byte pieces of the E chunk per thread
 
+// The lowest column of a chunk at which a cell reaches its maximum `want`: the chunk's 32 columns
+// of the cell's two rows come in as sixteen 16-byte loads, all requested before the first is
+// looked at, and the sums are compared in registers.  (Looked up column by column, the way the
+// reference scans, this was two dependent loads and a wait per column and cell: five hundred
+// memory round trips in a row at the end of every wavefront.)
+template <bool kVec, typename TIO>
+__device__ inline int chunk_argmax(const TIO* __restrict__ e, const TIO* __restrict__ q, int chunk,
+                                   float want, const Dims& d) {
+  const int v0 = max(chunk, 0) * kMpK;
+  float4 ev[kMpK / 4], pv[kMpK / 4];
+#pragma unroll
+  for (int g = 0; g < kMpK / 4; ++g) {
+    const int v = v0 + 4 * g;
+    // (kVec: a group of four is inside the row or past it as a whole, and one past it is
+    // never looked at, so the clamped start only keeps the load inside the array)
+    ev[g] = kVec ? load4(e + min(v, d.V - 4)) : load4_any(e, min(v, d.V - 1), d.V);
+    pv[g] = kVec ? load4(q + min(v, d.V - 4)) : load4_any(q, min(v, d.V - 1), d.V);
+  }
+  int at = 0;  // :160 the scan starts from index 0 and keeps it if nothing beats -inf
+  if (chunk >= 0) {
+    // from the last column down, so that the lowest match is what remains
+#pragma unroll
+    for (int g = kMpK / 4 - 1; g >= 0; --g) {
+      const float sum[4] = {ev[g].x + pv[g].x, ev[g].y + pv[g].y, ev[g].z + pv[g].z,
+                            ev[g].w + pv[g].w};
+#pragma unroll
+      for (int j = 3; j >= 0; --j) {
+        const int v = v0 + 4 * g + j;
+        if (v < d.V && v != d.blank && sum[j] == want) at = v;
+      }
+    }
+  }
+  return at;
+}
+
+// kParts: a workgroup takes one of parts.n ranges of columns and leaves its cells' maxima and
+// chunks in `parts` (maxplus_index_kernel goes on from there); without, it takes all columns and
+// finishes its cells: that form redoes single tiles after the list pass.  Each workgroup walks its
+// columns alone, so with one range few tiles are a long walk on a few CUs: the table of B=1 T=500
+// U=41 V=1000 (four tiles) 124 -> 31 us with sixteen ranges.
 // kVec: V is a multiple of 4, so four consecutive elements never straddle a row's end and every
 // group of four is naturally aligned (16 bytes in fp32, 8 in bf16).
-template <bool kVec, typename TIO>
+template <bool kVec, bool kParts, typename TIO>
 __global__ __launch_bounds__(kMpThreads) void maxplus_kernel(const TIO* __restrict__ E,
                                                        const TIO* __restrict__ P,
                                                        const int* __restrict__ inLen,
@@ -1641,10 +1688,12 @@ __global__ __launch_bounds__(kMpThreads) void maxplus_kernel(const TIO* __restri
                                                        int* __restrict__ arg, Dims d,
                                                        const int* __restrict__ tile_fail,
                                                        const int* __restrict__ lists_on,
-                                                       int fail_limit) {
+                                                       int fail_limit, MaxplusParts parts) {
   __shared__ __attribute__((aligned(16))) float Es[2][kMpT * kMpPitch];
   __shared__ __attribute__((aligned(16))) float Ps[2][kMpU * kMpK];
-  const int b = blockIdx.z, t0 = blockIdx.x * kMpT, u0 = blockIdx.y * kMpU;
+  const int part = kParts ? (int)(blockIdx.z % (unsigned)parts.n) : 0;
+  const int b = kParts ? (int)(blockIdx.z / (unsigned)parts.n) : (int)blockIdx.z;
+  const int t0 = blockIdx.x * kMpT, u0 = blockIdx.y * kMpU;
   // after the list pass (if it went past its sample): only the tiles in which too many cells
   // failed its test are redone
   if (tile_fail && lists_on[0] != 0 &&
@@ -1717,11 +1766,13 @@ __global__ __launch_bounds__(kMpThreads) void maxplus_kernel(const TIO* __restri
 #pragma unroll
     for (int r = 0; r < kMpRows; ++r) { top[i][r] = kNegInf; chunk[i][r] = -1; }
 
-  const int nchunks = (d.V + kMpK - 1) / kMpK;
+  const int all = (d.V + kMpK - 1) / kMpK;
+  const int first = kParts ? (int)((long)all * part / parts.n) : 0;
+  const int nchunks = kParts ? (int)((long)all * (part + 1) / parts.n) : all;
   int cur = 0;
-  stash(0, 0, fetch_all(0));
+  stash(0, first, fetch_all(first));
   __syncthreads();
-  for (int k = 0; k < nchunks; ++k) {
+  for (int k = first; k < nchunks; ++k) {
     const int kn = min(k + 1, nchunks - 1);  // the last chunk re-reads its own
     const Staged nxt = fetch_all(kn);
     if (active) {
@@ -1766,52 +1817,108 @@ __global__ __launch_bounds__(kMpThreads) void maxplus_kernel(const TIO* __restri
     cur ^= 1;
   }
   if (!active) return;
-  // Recover the lowest index inside the winning chunk: the chunk's 32 columns of the cell's two
-  // rows come in as sixteen 16-byte loads, all requested before the first is looked at, and the
-  // sums are compared in registers.  (Looked up column by column, the way the reference scans,
-  // this was two dependent loads and a wait per column and cell: five hundred memory round
-  // trips in a row at the end of every wavefront.)  Every lane goes through the loads with
-  // clamped rows; only cells of the utterance are written.
+  if constexpr (kParts) {  // maxplus_index_kernel compares the parts and looks the column up
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < kMpRows; ++r) {
+        const int t = t0 + lane + 64 * i, u = ur0 + r;
+        if (t < Tb && u < Ub) {
+          const size_t o = parts.n > 1 ? (((size_t)part * d.B + b) * d.U + u) * d.T + t
+                                       : plane_at(d, b, u, t + u);
+          parts.top[o] = top[i][r];
+          parts.chunk[o] = chunk[i][r];
+        }
+      }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int r = 0; r < kMpRows; ++r) {
       const int t = t0 + lane + 64 * i, u = ur0 + r;
-      const bool cell = t < Tb && u < Ub;
-      const int v0 = max(chunk[i][r], 0) * kMpK;
-      const TIO* e = Eb + (size_t)min(t, Tb - 1) * d.V;
-      const TIO* q = Pb + (size_t)min(u, Ub - 1) * d.V;
-      float4 ev[kMpK / 4], pv[kMpK / 4];
-#pragma unroll
-      for (int g = 0; g < kMpK / 4; ++g) {
-        const int v = v0 + 4 * g;
-        // (kVec: a group of four is inside the row or past it as a whole, and one past it is
-        // never looked at, so the clamped start only keeps the load inside the array)
-        ev[g] = kVec ? load4(e + min(v, d.V - 4)) : load4_any(e, min(v, d.V - 1), d.V);
-        pv[g] = kVec ? load4(q + min(v, d.V - 4)) : load4_any(q, min(v, d.V - 1), d.V);
-      }
-      int at = 0;  // :160 the scan starts from index 0 and keeps it if nothing beats -inf
-      if (chunk[i][r] >= 0) {
-        const float want = top[i][r];
-        // from the last column down, so that the lowest match is what remains
-#pragma unroll
-        for (int g = kMpK / 4 - 1; g >= 0; --g) {
-          const float sum[4] = {ev[g].x + pv[g].x, ev[g].y + pv[g].y, ev[g].z + pv[g].z,
-                                ev[g].w + pv[g].w};
-#pragma unroll
-          for (int j = 3; j >= 0; --j) {
-            const int v = v0 + 4 * g + j;
-            if (v < d.V && v != d.blank && sum[j] == want) at = v;
-          }
-        }
-      }
-      if (cell) {
+      // every lane goes through the loads with clamped rows; only cells of the utterance are written
+      const int at = chunk_argmax<kVec>(Eb + (size_t)min(t, Tb - 1) * d.V,
+                                        Pb + (size_t)min(u, Ub - 1) * d.V, chunk[i][r], top[i][r], d);
+      if (t < Tb && u < Ub) {
         // straight into the skewed planes the lattice walk reads
         const size_t o = plane_at(d, b, u, t + u);
         best[o] = top[i][r];
         arg[o] = at;
       }
     }
+}
+
+// The table from what maxplus_kernel<.., true> left: the first range of columns that holds the
+// largest maximum, then the lowest column of its chunk that reaches it.  A wavefront takes 64 frames
+// of one label position.  Eight lanes look at a cell, four columns each, so that a load brings in
+// eight cells' 128 contiguous bytes: with one lane to a cell every load touched 64 cache lines,
+// and the look-up took as long as the maxima (365 of 668 us at B=32 T=2000 U=101 V=1000, as it
+// did at the end of maxplus_kernel itself).
+template <bool kVec, typename TIO>
+__global__ __launch_bounds__(256) void maxplus_index_kernel(const TIO* __restrict__ E,
+                                                            const TIO* __restrict__ P,
+                                                            const int* __restrict__ inLen,
+                                                            const int* __restrict__ labLen,
+                                                            float* best, int* arg, Dims d,
+                                                            MaxplusParts parts) {
+  const int b = blockIdx.z, lane = threadIdx.x & 63, t0 = blockIdx.x * 64;
+  const int u = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int Tb, Ub;
+  utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
+  if (t0 >= Tb || u >= Ub) return;  // uniform
+  const int t = t0 + lane, tc = min(t, Tb - 1);
+  const size_t w = plane_at(d, b, u, tc + u);
+  float top;
+  int chunk;
+  if (parts.n > 1) {
+    const size_t stride = (size_t)d.B * d.U * d.T;
+    const size_t o = ((size_t)b * d.U + u) * d.T + tc;
+    top = parts.top[o];
+    chunk = parts.chunk[o];
+    for (int s = 1; s < parts.n; ++s) {
+      const float x = parts.top[s * stride + o];
+      const int c = parts.chunk[s * stride + o];
+      if (x > top) { top = x; chunk = c; }
+    }
+  } else {
+    top = parts.top[w];
+    chunk = parts.chunk[w];
+  }
+  const TIO* Eb = E + (size_t)b * d.T * d.V;
+  const TIO* q = P + ((size_t)b * d.U + u) * d.V;
+  float4 ev[8], pv[8];
+  int v0[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {  // cells 8 i .. 8 i + 7
+    const int cell = 8 * i + (lane >> 3);
+    v0[i] = max(__shfl(chunk, cell), 0) * kMpK + 4 * (lane & 7);
+    const TIO* e = Eb + (size_t)min(t0 + cell, Tb - 1) * d.V;
+    // columns past V: see chunk_argmax
+    ev[i] = kVec ? load4(e + min(v0[i], d.V - 4)) : load4_any(e, min(v0[i], d.V - 1), d.V);
+    pv[i] = kVec ? load4(q + min(v0[i], d.V - 4)) : load4_any(q, min(v0[i], d.V - 1), d.V);
+  }
+  int at = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float want = __shfl(top, 8 * i + (lane >> 3));
+    const float sum[4] = {ev[i].x + pv[i].x, ev[i].y + pv[i].y, ev[i].z + pv[i].z,
+                          ev[i].w + pv[i].w};
+    int found = 0x7fffffff;
+#pragma unroll
+    for (int j = 3; j >= 0; --j) {
+      const int v = v0[i] + j;
+      if (v < d.V && v != d.blank && sum[j] == want) found = v;
+    }
+    found = min(found, __shfl_xor(found, 1));
+    found = min(found, __shfl_xor(found, 2));
+    found = min(found, __shfl_xor(found, 4));
+    const int got = __shfl(found, 8 * (lane & 7));
+    at = (lane >> 3) == i ? got : at;
+  }
+  if (t >= Tb) return;
+  best[w] = top;
+  arg[w] = chunk < 0 ? 0 : at;  // :160 the scan starts from index 0 and keeps it
 }
 
 // ------------------------------------------------------------------ viterbi
@@ -2614,49 +2721,90 @@ int launch_post_beta(const Planes& p, const float* mE, const float* mP, float* W
 // column for every cell; 2: lists wherever the shape allows (tests run small shapes through them)
 static std::atomic<int> g_maxplus_mode{0};
 void set_maxplus_mode(int mode) { g_maxplus_mode.store(mode); }
-int maxplus_plan(const Dims& d) {
+// Ranges of columns for maxplus_kernel<.., kParts>.
+int maxplus_parts(const Dims& d) {
+  const long tiles = (long)((d.T + kMpT - 1) / kMpT) * ((d.U + kMpU - 1) / kMpU) * d.B;
+  const long all = (d.V + kMpK - 1) / kMpK;
+  if (tiles == 0) return 1;
+  const long n = std::min(std::min(kMpWanted / tiles, all / kMpMinChunks), (long)kMpMaxParts);
+  return n < 1 ? 1 : (int)n;
+}
+size_t maxplus_parts_bytes(const Dims& d, int n) {
+  return n > 1 ? (size_t)n * 2 * sizeof(float) * d.B * d.U * d.T : 0;
+}
+
+MaxplusPlan maxplus_plan(const Dims& d, size_t room) {
   const int mode = g_maxplus_mode.load();  // read once per call: the plan is what the call follows
-  if (mode == 1 || !maxplus_lists_possible(d)) return 0;
-  if (mode == 2) return 2;
-  return maxplus_lists_pay(d) ? 1 : 0;
+  MaxplusPlan p;
+  if (mode != 1 && maxplus_lists_possible(d)) p.lists = mode == 2 ? 2 : maxplus_lists_pay(d) ? 1 : 0;
+  if (p.lists) {
+    p.bytes = maxplus_lists_bytes(d);
+  } else {
+    p.parts = maxplus_parts(d);
+    while (maxplus_parts_bytes(d, p.parts) > room) --p.parts;
+    p.bytes = maxplus_parts_bytes(d, p.parts);
+  }
+  return p;
 }
 
 template <typename TIO>
 static int maxplus_any(const TIO* E, const TIO* P, const int* inLen, const int* labLen,
-                       float* best, int* arg, const Dims& d, hipStream_t s, void* lists,
-                       bool force) {
+                       float* best, int* arg, const Dims& d, hipStream_t s, void* scratch,
+                       const MaxplusPlan& plan) {
   if (d.B == 0 || d.T == 0 || d.U == 0) return kOk;
   static_assert(kMpT == 128 && kMpU == 64, "the list pass counts failures per tile of this kernel");
   const int *tile_fail = nullptr, *lists_on = nullptr;
-  if (lists) {  // (the caller made the plan, and reserved `lists` if it says lists)
-    RNNT_TRY(launch_maxplus_lists(E, P, inLen, labLen, best, arg, d, lists, force, s));
-    maxplus_lists_counters(lists, d, &tile_fail, &lists_on);
+  if (plan.lists) {  // (the caller made the plan, and reserved what it says)
+    RNNT_TRY(launch_maxplus_lists(E, P, inLen, labLen, best, arg, d, scratch, plan.lists == 2, s));
+    maxplus_lists_counters(scratch, d, &tile_fail, &lists_on);
   }
-  const dim3 grid((d.T + kMpT - 1) / kMpT, (d.U + kMpU - 1) / kMpU, d.B);
+  MaxplusParts parts;  // one range: the maxima and chunks wait in the table itself
+  parts.n = plan.lists ? 1 : plan.parts;
+  parts.top = parts.n > 1 ? static_cast<float*>(scratch) : best;
+  parts.chunk = parts.n > 1
+      ? reinterpret_cast<int*>(parts.top + (size_t)parts.n * d.B * d.U * d.T) : arg;
+  const dim3 grid((d.T + kMpT - 1) / kMpT, (d.U + kMpU - 1) / kMpU, d.B * parts.n);
   const bool vec = d.V % 4 == 0 &&
                    ((reinterpret_cast<uintptr_t>(E) | reinterpret_cast<uintptr_t>(P)) &
                     (4 * sizeof(TIO) - 1)) == 0;
-  if (vec)
-    hipLaunchKernelGGL((maxplus_kernel<true, TIO>), grid, dim3(kMpThreads), 0, s, E, P, inLen,
-                       labLen, best, arg, d, tile_fail, lists_on, maxplus_tile_limit());
-  else
-    hipLaunchKernelGGL((maxplus_kernel<false, TIO>), grid, dim3(kMpThreads), 0, s, E, P, inLen,
-                       labLen, best, arg, d, tile_fail, lists_on, maxplus_tile_limit());
-  RNNT_LAUNCH_CHECK("maxplus_kernel");
-  if (tile_fail) RNNT_TRY(launch_maxplus_cells(E, P, inLen, labLen, best, arg, d, lists, s));
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kMpThreads), 0, s, E, P, inLen, labLen, best, arg, d,
+                       tile_fail, lists_on, maxplus_tile_limit(), parts);
+  };
+  if (plan.lists) {
+    if (vec) launch(maxplus_kernel<true, false, TIO>);
+    else launch(maxplus_kernel<false, false, TIO>);
+    RNNT_LAUNCH_CHECK("maxplus_kernel");
+  } else {
+    if (vec) launch(maxplus_kernel<true, true, TIO>);
+    else launch(maxplus_kernel<false, true, TIO>);
+    RNNT_LAUNCH_CHECK("maxplus_kernel");
+    const dim3 cells((d.T + 63) / 64, (d.U + 3) / 4, d.B);
+    if (vec)
+      hipLaunchKernelGGL((maxplus_index_kernel<true, TIO>), cells, dim3(256), 0, s, E, P, inLen,
+                         labLen, best, arg, d, parts);
+    else
+      hipLaunchKernelGGL((maxplus_index_kernel<false, TIO>), cells, dim3(256), 0, s, E, P, inLen,
+                         labLen, best, arg, d, parts);
+    RNNT_LAUNCH_CHECK("maxplus_index_kernel");
+  }
+  if (tile_fail) RNNT_TRY(launch_maxplus_cells(E, P, inLen, labLen, best, arg, d, scratch, s));
   return kOk;
 }
 int launch_maxplus(const float* E, const float* P, const int* inLen, const int* labLen,
-                   float* best, int* arg, const Dims& d, hipStream_t s, void* lists, bool force) {
-  return maxplus_any(E, P, inLen, labLen, best, arg, d, s, lists, force);
+                   float* best, int* arg, const Dims& d, hipStream_t s, void* scratch,
+                   const MaxplusPlan& plan) {
+  return maxplus_any(E, P, inLen, labLen, best, arg, d, s, scratch, plan);
 }
 int launch_maxplus(const bf16_t* E, const bf16_t* P, const int* inLen, const int* labLen,
-                   float* best, int* arg, const Dims& d, hipStream_t s, void* lists, bool force) {
-  return maxplus_any(E, P, inLen, labLen, best, arg, d, s, lists, force);
+                   float* best, int* arg, const Dims& d, hipStream_t s, void* scratch,
+                   const MaxplusPlan& plan) {
+  return maxplus_any(E, P, inLen, labLen, best, arg, d, s, scratch, plan);
 }
 int launch_maxplus(const f16_t* E, const f16_t* P, const int* inLen, const int* labLen,
-                   float* best, int* arg, const Dims& d, hipStream_t s, void* lists, bool force) {
-  return maxplus_any(E, P, inLen, labLen, best, arg, d, s, lists, force);
+                   float* best, int* arg, const Dims& d, hipStream_t s, void* scratch,
+                   const MaxplusPlan& plan) {
+  return maxplus_any(E, P, inLen, labLen, best, arg, d, s, scratch, plan);
 }
 #endif
 

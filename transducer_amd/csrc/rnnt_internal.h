@@ -195,25 +195,35 @@ int launch_post_beta(const Planes& p, const float* mE, const float* mP, float* W
                      float* bsum, float* emT, const int* labels, const int* inLen,
                      const int* labLen, const Dims& d, hipStream_t s,
                      const WImages& img = WImages());
-// best / arg: skewed planes (see plane_at), written for valid cells only.
+// How a call of this shape builds its table of best labels under the current mode, decided ONCE
+// per call (the mode is process-wide and another thread may change it).  lists: 0 over every
+// column, 1 from candidate lists (rnnt_cand.hip: only the cells whose bound test fails are
+// evaluated over every column) if a sample of cells agrees, 2 from lists unconditionally.
+// parts: ranges of columns that go to workgroups of their own (without lists).  bytes: scratch.
+struct MaxplusPlan {
+  int lists = 0, parts = 1;
+  size_t bytes = 0;
+};
+// room: parts take no more scratch than this.
+MaxplusPlan maxplus_plan(const Dims& d, size_t room = ~(size_t)0);
+// [n][B][U][T]: the maximum of a range of columns and the chunk of columns that reached it first
+struct MaxplusParts {
+  int n = 1;
+  float* top = nullptr;
+  int* chunk = nullptr;
+};
+// best / arg: skewed planes (see plane_at), written for valid cells only; scratch: plan.bytes.
 int launch_maxplus(const float* E, const float* P, const int* inLen, const int* labLen,
-                   float* best, int* arg, const Dims& d, hipStream_t s, void* lists = nullptr,
-                   bool force = false);
+                   float* best, int* arg, const Dims& d, hipStream_t s, void* scratch,
+                   const MaxplusPlan& plan);
 int launch_maxplus(const bf16_t* E, const bf16_t* P, const int* inLen, const int* labLen,
-                   float* best, int* arg, const Dims& d, hipStream_t s, void* lists = nullptr,
-                   bool force = false);
+                   float* best, int* arg, const Dims& d, hipStream_t s, void* scratch,
+                   const MaxplusPlan& plan);
 int launch_maxplus(const f16_t* E, const f16_t* P, const int* inLen, const int* labLen,
-                   float* best, int* arg, const Dims& d, hipStream_t s, void* lists = nullptr,
-                   bool force = false);
-// `lists`: maxplus_lists_bytes(d) bytes of scratch, or null (plan 0); force: plan 2.  With it, and where
-// maxplus_plan(d) says so, most cells are settled from short candidate lists
-// (rnnt_cand.hip) and only the cells whose bound test fails are evaluated over every column.
+                   float* best, int* arg, const Dims& d, hipStream_t s, void* scratch,
+                   const MaxplusPlan& plan);
 bool maxplus_lists_possible(const Dims& d);
 bool maxplus_lists_pay(const Dims& d);
-// How a call of this shape builds its table under the current mode, decided ONCE per call (the
-// mode is process-wide and another thread may change it): 0 over every column, 1 from lists if
-// the sample of cells agrees, 2 from lists unconditionally.
-int maxplus_plan(const Dims& d);
 size_t maxplus_lists_bytes(const Dims& d);
 void set_maxplus_mode(int mode);
 int maxplus_tile_limit();
