@@ -780,3 +780,36 @@ def test_pgrads_split_over_frames_gives_the_bits_of_the_unsplit_walk():
     want = oracle.loss_and_grads(E, P, labels, il, ll)
     assert_close(one[0], want["costs"], what="costs")
     assert_close(one[2], want["pgrads"], what="pgrads")
+
+
+@pytest.mark.parametrize("U", [1, 33, 129, 161])
+@pytest.mark.parametrize("T", [256, 257, 513, 800])
+def test_pgrads_of_tiles_whose_frames_are_split(T, U):
+    """Chunks of 256 frames summed in workgroups of their own: the last chunk of one frame or of 32
+    slabs, chunks past an utterance, blocks of 32 label positions past one, a vocabulary that ends
+    inside a tile; whole loss, and added to what the caller's array holds.  A batch too large to
+    be split gives the same bits."""
+    V, rng = 131, np.random.default_rng(T * 1000 + U)
+    il = np.array([T, 1, min(T, 255)], np.int32)
+    ll = np.array([U - 1, U // 2, 0], np.int32)
+    E = rng.standard_normal((3, T, V), dtype=np.float32)
+    P = rng.standard_normal((3, U, V), dtype=np.float32)
+    labels = rng.integers(1, V, (3, max(U - 1, 0))).astype(np.int32)
+    few = gpu_loss(DeviceCase(E, P, labels, il, ll), deltas=np.array([1, 2, 0.5], np.float32))
+    rep = lambda a: np.tile(a, (28,) + (1,) * (a.ndim - 1))
+    many = gpu_loss(DeviceCase(rep(E), rep(P), rep(labels), rep(il), rep(ll)),
+                    deltas=rep(np.array([1, 2, 0.5], np.float32)))
+    for got, want in zip(many, few):
+        assert np.array_equal(got[:3], want) and np.array_equal(got[-3:], want)
+    c = DeviceCase(E, P, labels, il, ll)
+    lng = rng.standard_normal((3, T, U)).astype(np.float32)
+    LN = oracle.log_norms_naive(E, P, il, ll)
+    held = rng.standard_normal((3, U, V)).astype(np.float32)
+    _, got = gpu_dense_grads(c, np.zeros_like(E), held, lng, np.nan_to_num(LN))
+    for b in range(3):
+        n, m = il[b], ll[b] + 1
+        w = lng[b, :n, :m, None].astype(np.float64) * np.exp(
+            E[b, :n, None].astype(np.float64) + P[b, None, :m] - LN[b, :n, :m, None])
+        # the exponents' rounding, about 2^-21, on every one of the n terms
+        assert np.abs(got[b, :m] - (held[b, :m] + w.sum(0))).max() <= 4e-6 * np.abs(w).sum(0).max() + 1e-6
+        assert np.array_equal(got[b, m:], held[b, m:])

@@ -251,16 +251,17 @@ size_t loss_workspace_layout(const Dims& d, void* base, LossWorkspace* w) {
   float* Wt = Wn ? reinterpret_cast<float*>(reinterpret_cast<char*>(Wn) + wb) : nullptr;
   float* bsum = take(sizeof(float) * (size_t)d.B * d.T);
   float* emT = take(btu);  // label-move terms of egrads, [B][U][T]
-  void* ys = take(lse_scratch_bytes(d));  // forward only
-  void* ps = take(pgrads_split_bytes(d));  // backward only
+  // the Y pieces (forward only) and the partial sums of pgrads (backward only) share memory
+  const size_t yb = lse_scratch_bytes(d), sb = pgrads_split_bytes(d);
+  void* ys = take(yb > sb ? yb : sb);
   if (base) {
     w->mE = mE; w->mP = mP; w->LN = LN; w->Wn = Wn; w->Wt = Wt; w->bsum = bsum; w->emT = emT;
     if (images) {
       w->img.e = reinterpret_cast<unsigned*>(Wn);
       w->img.p = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(Wn) + ie);
     }
-    w->lse_scratch = lse_scratch_bytes(d) ? ys : nullptr;
-    w->psplit = pgrads_split_bytes(d) ? ps : nullptr;
+    w->lse_scratch = yb ? ys : nullptr;
+    w->psplit = sb ? ys : nullptr;
   }
   return off;
 }

@@ -463,14 +463,12 @@ __global__ __launch_bounds__(256, 2) void egrads_stream_kernel(
 
 // Splitting a tile's frames over several workgroups (small grids: one utterance with a small
 // vocabulary is a single tile, whose workgroup would walk all frames alone).  Workgroup c of
-// `chunks` sums slabs [c*per, (c+1)*per) and leaves its sums in `partial`; the one that arrives
-// last at the tile's counter adds all of them up in chunk order (so the result does not depend
-// on who was last) and writes the tile.  Nobody waits for anybody.  per == kPsFlush, always:
-// see pgrads_split_plan.
+// `chunks` sums slabs [c*per, (c+1)*per) and leaves its sums in `partial`; pgrads_combine_kernel
+// adds them up in chunk order and writes the tile.  per == kPsFlush, always: see
+// pgrads_split_plan.
 struct PSplit {
   int chunks = 1, per = 0;
   float* partial = nullptr;  // [tile][chunk][4 blocks][16 registers][256 threads]
-  int* counter = nullptr;    // [tile], zero before the launch
 };
 constexpr int kPsPartialFloats = 4 * 16 * 256;
 
@@ -483,8 +481,8 @@ __device__ __forceinline__ void pgrads_tile(
     const float* __restrict__ mP, const float* __restrict__ Wt, const float* __restrict__ deltas,
     TIO* __restrict__ pgrads, unsigned short (*As)[3][kPsPlane], float (*Ms)[32], const Dims& d,
     int Up, int Tw, int b, int u0, int Tb, int Ub, const PRowTerms* rt, const PSplit& split,
-    int chunk, int tile, int* last_flag) {
-  if (kSplit && NMB == 0 && chunk > 0) return;  // nothing to sum: chunk 0 alone writes the zeros
+    int chunk, int tile) {
+  if (kSplit && NMB == 0) return;  // nothing to sum
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, h = lane >> 5;
   const int vcol = blockIdx.x * 128 + wave * 32 + l32;
   const bool vok = vcol < d.V;
@@ -624,29 +622,7 @@ __device__ __forceinline__ void pgrads_tile(
     for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mine[(mb * 16 + r) * 256 + tid] = acc[mb][r];
-    __threadfence();  // the sums are out before the arrival is counted
-    __syncthreads();
-    if (tid == 0) {
-      const int before = __hip_atomic_fetch_add(&split.counter[tile], 1, __ATOMIC_ACQ_REL,
-                                                __HIP_MEMORY_SCOPE_AGENT);
-      *last_flag = before == split.chunks - 1;
-    }
-    __syncthreads();
-    if (!*last_flag) return;
-    __threadfence();  // the others' sums are visible after their arrivals were seen
-    const float* all = split.partial + (size_t)tile * split.chunks * kPsPartialFloats;
-#pragma unroll
-    for (int mb = 0; mb < NMB; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mb][r] = 0.0f;
-    for (int c = 0; c < split.chunks; ++c) {
-      const float* src = all + (size_t)c * kPsPartialFloats;
-#pragma unroll
-      for (int mb = 0; mb < NMB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          acc[mb][r] += __builtin_nontemporal_load(&src[(mb * 16 + r) * 256 + tid]);
-    }
+    return;
   }
 
   const TIO* Pb = P + (size_t)b * d.U * d.V;
@@ -690,6 +666,18 @@ __device__ __forceinline__ void pgrads_tile(
     }
 }
 
+// Blank / label terms of the rows of tile row u0 for the threads of a workgroup to stage (k < 128):
+// blank total, label and label total; rows without one get a label that matches no column.
+__device__ inline void stage_row_terms(PRowTerms& Rt, const SparsePTerms& sp, const Dims& d, int b,
+                                       int u0, int Tb, int Ub, int k) {
+  const int u = u0 + k;
+  const bool valid = Tb > 0 && u < Ub, has_label = valid && u + 1 < Ub;
+  const int l = has_label ? label_at(sp.labels, d, b, u) : d.blank;
+  Rt.gB[k] = valid ? sp.gB[(size_t)b * d.Ua + u] : 0.0f;
+  Rt.gL[k] = has_label ? sp.gL[(size_t)b * d.Ua + u] : 0.0f;
+  Rt.label[k] = (has_label && l != d.blank) ? l : -1;
+}
+
 template <bool kAccumulate, bool kSplit, typename TIO>
 __global__ __launch_bounds__(256, 2) void pgrads_stream_kernel(
     const TIO* __restrict__ E, const TIO* __restrict__ P, const float* __restrict__ mE,
@@ -699,7 +687,6 @@ __global__ __launch_bounds__(256, 2) void pgrads_stream_kernel(
   __shared__ __attribute__((aligned(16))) unsigned short As[2][3][kPsPlane];
   __shared__ __attribute__((aligned(16))) float Ms[2][32];
   __shared__ PRowTerms Rt;
-  __shared__ int last_flag;
   const int b = blockIdx.z;
   const int ut = kSplit ? blockIdx.y / split.chunks : blockIdx.y;
   const int chunk = kSplit ? blockIdx.y - ut * split.chunks : 0;
@@ -708,23 +695,16 @@ __global__ __launch_bounds__(256, 2) void pgrads_stream_kernel(
   const int u0 = ut * 128;
   int Tb, Ub;
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
-  const bool folding = !kAccumulate && sp.gB != nullptr;
-  if (folding && threadIdx.x < 128) {
-    // this tile's rows: blank total, label and label total; rows without one get a label that
-    // matches no column.  Visible to all after the barriers of the walk (or the one below).
-    const int k = threadIdx.x, u = u0 + k;
-    const bool valid = Tb > 0 && u < Ub, has_label = valid && u + 1 < Ub;
-    const int l = has_label ? label_at(sp.labels, d, b, u) : d.blank;
-    Rt.gB[k] = valid ? sp.gB[(size_t)b * d.Ua + u] : 0.0f;
-    Rt.gL[k] = has_label ? sp.gL[(size_t)b * d.Ua + u] : 0.0f;
-    Rt.label[k] = (has_label && l != d.blank) ? l : -1;
-  }
+  const bool folding = !kAccumulate && !kSplit && sp.gB != nullptr;
+  // visible to all after the barrier below
+  if (folding && threadIdx.x < 128)
+    stage_row_terms(Rt, sp, d, b, u0, Tb, Ub, threadIdx.x);
   if (folding) __syncthreads();
   const PRowTerms* rt = folding ? &Rt : nullptr;
   const int nmb = (u0 < Ub && Tb > 0) ? min(4, (Ub - u0 + 31) >> 5) : 0;  // 32-row blocks in use
 #define RNNT_PG_TILE(NMB)                                                                   \
   pgrads_tile<NMB, kAccumulate, kSplit>(E, P, mE, mP, Wt, deltas, pgrads, As, Ms, d, Up, Tw, \
-                                        b, u0, Tb, Ub, rt, split, chunk, tile, &last_flag)
+                                        b, u0, Tb, Ub, rt, split, chunk, tile)
   switch (nmb) {
     case 0: RNNT_PG_TILE(0); break;
     case 1: RNNT_PG_TILE(1); break;
@@ -733,6 +713,73 @@ __global__ __launch_bounds__(256, 2) void pgrads_stream_kernel(
     default: RNNT_PG_TILE(4); break;
   }
 #undef RNNT_PG_TILE
+}
+
+// Adds the chunks' sums of a tile up, in chunk order, and writes the tile: one workgroup per block
+// of 32 label positions.  Bound by the partial sums it reads (16 KB a chunk, all of a chunk's asked
+// for together).  Doing this in the walk's own launch, by whichever workgroup arrives last, took a
+// release and an acquire at device scope per workgroup; each writes back an XCD's L2 and the launch
+// grew with their number (B=8 T=2000 U=101 V=1000, 512 workgroups: 144 us, 46 with the two
+// launches, 106 unsplit).
+template <bool kAccumulate, typename TIO>
+__global__ __launch_bounds__(256) void pgrads_combine_kernel(
+    const TIO* __restrict__ P, const float* __restrict__ mP, const float* __restrict__ deltas,
+    TIO* __restrict__ pgrads, const int* __restrict__ inLen, const int* __restrict__ labLen, Dims d,
+    SparsePTerms sp, PSplit split) {
+  __shared__ PRowTerms Rt;
+  const int b = blockIdx.z, ut = blockIdx.y >> 2, mb = blockIdx.y & 3, u0 = ut * 128;
+  const int tile = (b * (gridDim.y >> 2) + ut) * gridDim.x + blockIdx.x;
+  int Tb, Ub;
+  utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
+  const bool folding = !kAccumulate && sp.gB != nullptr;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, h = lane >> 5;
+  if (folding) {
+    if (tid < 128) stage_row_terms(Rt, sp, d, b, u0, Tb, Ub, tid);
+    __syncthreads();
+  }
+  const int vcol = blockIdx.x * 128 + wave * 32 + l32;
+  if (u0 + 32 * mb >= d.U) return;
+  const bool vok = vcol < d.V;
+  const int vc = vok ? vcol : d.V - 1;
+  const float delta = deltas ? deltas[b] : 1.0f;
+  const bool summed = Tb > 0 && u0 + 32 * mb < Ub;  // uniform: the walk left sums for this block
+  float praw[16], mraw[16], acc[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int uc = min(u0 + 32 * mb + mfma_row(r, h), d.U - 1);
+    praw[r] = ldf(P + ((size_t)b * d.U + uc) * d.V + vc);
+    mraw[r] = mP[(size_t)b * d.U + uc];
+    acc[r] = 0.0f;
+  }
+  if (summed) {
+    const float* src = split.partial + (size_t)tile * split.chunks * kPsPartialFloats +
+                       mb * 16 * 256 + tid;
+    // (chunks past the utterance hold zeros)
+#pragma unroll 2
+    for (int c = 0; c < split.chunks; ++c) {
+      float x[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        x[r] = __builtin_nontemporal_load(&src[(size_t)c * kPsPartialFloats + r * 256]);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] += x[r];
+    }
+  }
+  TIO* out = pgrads + (size_t)b * d.U * d.V;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int k = 32 * mb + mfma_row(r, h), u = u0 + k;
+    const float g = u < Ub && summed ? __expf(praw[r] - mraw[r]) * acc[r] : 0.0f;
+    if (u < d.U && vok) {
+      TIO* o = out + (size_t)u * d.V + vcol;
+      float res = delta * (kAccumulate ? ldf(o) + g : g);
+      if (folding) {  // as in pgrads_tile
+        if (vcol == d.blank) res += delta * Rt.gB[k];
+        else if (vcol == Rt.label[k]) res += delta * Rt.gL[k];
+      }
+      stf(o, res);
+    }
+  }
 }
 
 }  // namespace
@@ -880,15 +927,18 @@ int launch_egrads_stream(const f16_t* E, const f16_t* P, const float* mE, const 
 // period at which the unsplit walk moves its running sum into the second-level sum: the
 // chunks' sums, added in chunk order, then go through exactly the additions the unsplit walk
 // performs, so split and unsplit results are the same bits and an utterance's gradient does
-// not depend on the batch it is computed in.  Split only when the device would otherwise be
-// nearly empty (at most one workgroup per CU after the split): each chunk pays a start-up, a
-// device-scope fence and a share of the final addition.
+// not depend on the batch it is computed in.  Split only when the tiles would leave CUs empty: each
+// chunk pays a start-up and 64 KB of sums written and read back.  pgrads in us, unsplit and split:
+// 64 tiles (B=8 T=2000 U=101 V=1000) 106 and 46, 128 (V=2000) 115 and 75, B=4 T=1000 U=201 V=2000 69
+// and 42; 256 (B=16 of the second) 127 and 138, B=32 T=300 U=101 V=1000 35 and 44.  At most 256 MB of
+// sums (64 tiles of T=10000, B=2 U=101 V=4000, are 160 MB: 523 and 165).
+constexpr long kPsSplitTiles = 160, kPsSplitMost = 4096;
 static void pgrads_split_plan(const Dims& d, int& chunks, int& per) {
   const long tiles = (long)((d.V + 127) / 128) * ((d.U + 127) / 128) * d.B;
   const int nk = (d.T + 31) / 32;
   per = kPsFlush;
   chunks = (nk + per - 1) / per;
-  if (chunks < 2 || tiles * chunks > 256) chunks = 1;
+  if (chunks < 2 || tiles > kPsSplitTiles || tiles * chunks > kPsSplitMost) chunks = 1;
 }
 
 #if RNNT_IN_PART(3)
@@ -898,14 +948,9 @@ size_t pgrads_split_bytes(const Dims& d) {
   pgrads_split_plan(d, chunks, per);
   if (chunks <= 1) return 0;
   const size_t tiles = (size_t)((d.V + 127) / 128) * ((d.U + 127) / 128) * d.B;
-  return tiles * chunks * kPsPartialFloats * sizeof(float) + ((tiles * sizeof(int) + 255) & ~(size_t)255);
+  return tiles * chunks * kPsPartialFloats * sizeof(float);
 }
 #endif
-
-static __global__ void zero_ints_kernel(int* x, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) x[i] = 0;
-}
 
 template <typename TIO>
 static int pgrads_stream_any(const TIO* E, const TIO* P, const float* mE, const float* mP,
@@ -919,23 +964,20 @@ static int pgrads_stream_any(const TIO* E, const TIO* P, const float* mE, const 
   PSplit split;
   if (split_ws != nullptr) pgrads_split_plan(d, split.chunks, split.per);
   if (split.chunks > 1) {
-    // counters first (256-byte multiple), partial sums behind them; cleared by a kernel, not a
-    // memset node, so that the call can be captured into a graph
-    const int tiles = vtiles * utiles * d.B;
-    split.counter = static_cast<int*>(split_ws);
-    split.partial = reinterpret_cast<float*>(static_cast<char*>(split_ws) +
-                                             ((tiles * sizeof(int) + 255) & ~(size_t)255));
-    hipLaunchKernelGGL(zero_ints_kernel, dim3((tiles + 255) / 256), dim3(256), 0, s,
-                       split.counter, tiles);
-    RNNT_LAUNCH_CHECK("zero_ints_kernel");
+    split.partial = static_cast<float*>(split_ws);
+    // (what the walk would write out is the combining kernel's business: no forms of its own for it)
     const dim3 grid(vtiles, utiles * split.chunks, d.B);
-    if (accumulate)
-      hipLaunchKernelGGL((pgrads_stream_kernel<true, true, TIO>), grid, dim3(256), 0, s, E, P, mE,
-                         mP, Wt, deltas, pgrads, inLen, labLen, d, Up, Tw, sp, split);
-    else
-      hipLaunchKernelGGL((pgrads_stream_kernel<false, true, TIO>), grid, dim3(256), 0, s, E, P, mE,
-                         mP, Wt, deltas, pgrads, inLen, labLen, d, Up, Tw, sp, split);
+    hipLaunchKernelGGL((pgrads_stream_kernel<false, true, TIO>), grid, dim3(256), 0, s, E, P, mE,
+                       mP, Wt, deltas, pgrads, inLen, labLen, d, Up, Tw, sp, split);
     RNNT_LAUNCH_CHECK("pgrads_stream_kernel (split)");
+    const dim3 blocks(vtiles, utiles * 4, d.B);
+    if (accumulate)
+      hipLaunchKernelGGL((pgrads_combine_kernel<true, TIO>), blocks, dim3(256), 0, s, P, mP, deltas,
+                         pgrads, inLen, labLen, d, sp, split);
+    else
+      hipLaunchKernelGGL((pgrads_combine_kernel<false, TIO>), blocks, dim3(256), 0, s, P, mP,
+                         deltas, pgrads, inLen, labLen, d, sp, split);
+    RNNT_LAUNCH_CHECK("pgrads_combine_kernel");
     return kOk;
   }
   const dim3 grid(vtiles, utiles, d.B);
