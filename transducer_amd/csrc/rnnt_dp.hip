@@ -1960,6 +1960,7 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
   static_assert(!kLive || (kMulti && !kLdsBits), "live blocks keep their columns in global memory");
   extern __shared__ __attribute__((aligned(16))) int dyn[];
   __shared__ int done[W];  // steps a wavefront has published
+  __shared__ __attribute__((aligned(16))) float nothing[4];
   const int live_block = kLive ? (int)(blockIdx.x >> 3) % live_n : 0;
   const int b = kLive ? (int)(blockIdx.x / (8 * live_n)) * 8 + (blockIdx.x & 7) : blockIdx.x;
   const int lane = threadIdx.x & 63, tidx = threadIdx.x;
@@ -2016,12 +2017,14 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
   if (W > 1) {
     if (tidx < W) done[tidx] = 0;
     if (tidx < W - 1) hand[tidx * hand_stride] = kNegInf;  // nothing enters step 0
+    if (tidx < 4) nothing[tidx] = kNegInf;
   }
   if (!kLive)
     for (int u = tidx; u < Ub; u += 64 * W) taken[u] = -1;
   __syncthreads();
   float* hand_out = hand + wave * hand_stride;                            // wave < W-1
-  const float* hand_in = hand + (wave > 0 ? wave - 1 : 0) * hand_stride;  // wave > 0
+  // wave > 0; wavefront 0 finds there that nothing comes in
+  const float* hand_in = wave > 0 ? hand + (wave - 1) * hand_stride : nothing;
   // (a launch that only traces asks for its first groups' operands like any other, and never
   // uses them: it asks where the lowest block would, inside the arrays)
   const int u0 = (walks ? u_base : 0) + (wave * 64 + lane) * C;
@@ -2045,6 +2048,20 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
     emit[c] = kNegInf;
     wbits[c] = 0u;
   }
+  // Groups from in_lo on need not ask whether a cell has started: step 4g is past the first frame of
+  // the wavefront's last position (positions past the utterance are never consulted, whatever
+  // they run on).  Their operands are addressed by 32-bit offsets from the utterance's own (uniform) plane
+  // origins.
+  const int u_lo = (walks ? u_base : 0) + wave * 64 * C;
+  const bool small_plane = 4ull * (unsigned long long)d.Ua * (unsigned)d.Dp < (1ull << 32);
+  const int in_lo = small_plane ? (max(min(u_lo + 64 * C, Ub) - 1, 1) + 3) >> 2 : 0x7fffffff;
+  const char* ln_b = reinterpret_cast<const char*>(p.lnS + plane_group0(d, b, 0));
+  const char* bs_b = reinterpret_cast<const char*>(bestS + plane_group0(d, b, 0));
+  const char* eb_b = reinterpret_cast<const char*>(p.eb + (size_t)b * d.Tp);
+  unsigned row_o[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) row_o[c] = 16u * (unsigned)min(u0 + c, d.U - 1);
+  const unsigned eb_o = 4u * (unsigned)(d.Eo - u0 - (C - 1));
   struct Group {
     float4 ln[C], bs[C];
     float eb[C + 3];
@@ -2068,13 +2085,44 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
     }
     return r;
   };
+  auto load_inner = [&](int g) -> Group {
+    Group r;
+    const unsigned by = (unsigned)g * (4u * (unsigned)gstride);  // bytes
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      r.ln[c] = *reinterpret_cast<const float4*>(ln_b + (size_t)(row_o[c] + by));
+      r.bs[c] = *reinterpret_cast<const float4*>(bs_b + (size_t)(row_o[c] + by));
+    }
+    const unsigned eo = eb_o + 16u * (unsigned)g;
+#pragma unroll
+    for (int k = 0; k < C + 3; ++k)
+      r.eb[k] = reinterpret_cast<const float*>(eb_b + (size_t)eo)[k];
+    if constexpr (kMulti) {
+      r.gh = make_float4(kNegInf, kNegInf, kNegInf, kNegInf);
+      if (gin) r.gh = *reinterpret_cast<const float4*>(gin + 4 * g);  // uniform
+      if constexpr (kLive) r.lv = live_load(4 * g + (lane & 3));
+    }
+    return r;
+  };
   int avail = 0;  // steps the wavefront below is known to have published (see alpha_kernel)
   auto wait_for = [&](int need) {
     avail = bounded_wait(&done[wave - 1], avail, need, spin_limit, trouble);
   };
+  // what enters a wavefront above the first is asked for a group ahead, as in alpha_kernel (the
+  // first one asks for the four entries that say that nothing comes in)
+  if (wave == 0) avail = 0x7fffffff;
+  auto fetch_hand = [&](int g, float4& h) {
+    if (W == 1 || g >= ngroups) return;
+    const int need = 4 * g + 3;
+    if (__builtin_expect(avail < need, 0)) wait_for(need);
+    h = *reinterpret_cast<const float4*>(hand_in + (wave > 0 ? 4 * g : 0));
+  };
   // A cell that has not started (t < 0) keeps -inf scores and never takes a label; cells past
   // the utterance run on whatever the planes hold and are never consulted by the backtrace.
-  auto run_group = [&](int g, const Group& cur) {
+  // The decision bits of 32 steps are shifted in from the right, one addition with carry a cell.
+  auto run_group = [&](int g, const Group& cur, const float4& hand_cur, float4& hand_next,
+                       auto interior) {
+    constexpr bool kInterior = decltype(interior)::value;
     float4 hin = {kNegInf, kNegInf, kNegInf, kNegInf};
     if constexpr (kMulti) hin = cur.gh;  // wavefront 0: from the block below (or nothing)
     if constexpr (kLive) {
@@ -2100,38 +2148,34 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
         live_sink ^= (unsigned)cur.lv;
       }
     }
-    if (W > 1 && wave > 0) {
-      wait_for(4 * g + 3);
-      hin = *reinterpret_cast<const float4*>(hand_in + 4 * g);
+    if constexpr (W > 1) {
+      if (!kMulti) hin = hand_cur;
+      else if (wave > 0) hin = hand_cur;
+      fetch_hand(g + 1, hand_next);
     }
-    float hout[4];
     float gsend[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int s = 4 * g + j;
-      const unsigned sbit = 1u << (s & 31);  // uniform
-      float from_left = wave_shr1(emit[C - 1], kNegInf);
-      if (W > 1 || kMulti) from_left = (lane == 0) ? f4get(hin, j) : from_left;
+      const float from_left = wave_shr1(emit[C - 1], f4get(hin, j));  // lane 0: hin
 #pragma unroll
       for (int c = C - 1; c >= 0; --c) {
         const float left = (c == 0) ? from_left : emit[c - 1];
         const bool take = left > stay[c];  // :200-206 ties go to blank
         float x = take ? left : stay[c];
-        if (j == 0 && g == 0) x = (u0 + c == 0) ? 0.0f : x;
-        wbits[c] |= take ? sbit : 0u;
+        if (!kInterior && j == 0 && g == 0) x = (u0 + c == 0) ? 0.0f : x;
+        wbits[c] = wbits[c] + wbits[c] + (take ? 1u : 0u);
         const float ln = f4get(cur.ln[c], j);
         float sb = x + cur.eb[j - c + (C - 1)];
         sb = sb + pbv[c];
         sb = sb - ln;
         float se = x + f4get(cur.bs[c], j);
         se = se - ln;
-        const bool started = s >= u0 + c;
+        const bool started = kInterior || s >= u0 + c;
         stay[c] = started ? sb : kNegInf;
         emit[c] = started ? se : kNegInf;
       }
-      if constexpr (kMulti) gsend[j] = emit[C - 1];
-      if (W > 1)
-        hout[j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(emit[C - 1]), 63));
+      gsend[j] = emit[C - 1];
     }
     if constexpr (kMulti) {
       if (gout && wave == W - 1 && lane == 63) {  // entries 4g+1 .. 4g+4 for the block above
@@ -2150,13 +2194,14 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
     if ((g & 7) == 7 || g == ngroups - 1) {  // uniform: a word of 32 steps is complete
 #pragma unroll
       for (int c = 0; c < C; ++c) {
-        cols[(size_t)(u0 + c) * nw + (g >> 3)] = wbits[c];
+        // (the last word may hold fewer steps: the first of them goes to bit 0 all the same)
+        cols[(size_t)(u0 + c) * nw + (g >> 3)] = __brev(wbits[c] << (28 - 4 * (g & 7)));
         wbits[c] = 0u;
       }
     }
-    if (W > 1 && wave < W - 1 && lane == 0) {  // entries 4g+1 .. 4g+4, then the progress
+    if (W > 1 && wave < W - 1 && lane == 63) {  // entries 4g+1 .. 4g+4, then the progress
 #pragma unroll
-      for (int j = 0; j < 4; ++j) hand_out[4 * g + 1 + j] = hout[j];
+      for (int j = 0; j < 4; ++j) hand_out[4 * g + 1 + j] = gsend[j];
       asm volatile("" ::: "memory");
       __hip_atomic_store(&done[wave], 4 * g + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
@@ -2181,14 +2226,30 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
   const int nwalk = walks ? ngroups : 0;  // a block past the utterance's labels only traces
   if (W > 1 && wave > 0 && walks)
     wait_for(min(4 * ngroups, 4 * (kLive ? kLiveWaveLag : 8) * wave));  // fall a few groups behind
+  const std::true_type inner;
+  const std::false_type edge;
+  float4 h0 = make_float4(kNegInf, kNegInf, kNegInf, kNegInf), h1 = h0;
+  if (walks) fetch_hand(0, h0);
   for (int g = 0; g < nwalk; g += 4) {
-    run_group(g, q0);
+    if constexpr (C <= 4) {  // (beyond, the registers are what is short)
+      for (; g >= in_lo && g + 8 <= ngroups; g += 4) {
+        run_group(g, q0, h0, h1, inner);
+        q0 = load_inner(g + 4);
+        run_group(g + 1, q1, h1, h0, inner);
+        q1 = load_inner(g + 5);
+        run_group(g + 2, q2, h0, h1, inner);
+        q2 = load_inner(g + 6);
+        run_group(g + 3, q3, h1, h0, inner);
+        q3 = load_inner(g + 7);
+      }
+    }
+    run_group(g, q0, h0, h1, edge);
     q0 = load_group(clamp_g(g + 4));
-    if (g + 1 < ngroups) run_group(g + 1, q1);
+    if (g + 1 < ngroups) run_group(g + 1, q1, h1, h0, edge);
     q1 = load_group(clamp_g(g + 5));
-    if (g + 2 < ngroups) run_group(g + 2, q2);
+    if (g + 2 < ngroups) run_group(g + 2, q2, h0, h1, edge);
     q2 = load_group(clamp_g(g + 6));
-    if (g + 3 < ngroups) run_group(g + 3, q3);
+    if (g + 3 < ngroups) run_group(g + 3, q3, h1, h0, edge);
     q3 = load_group(clamp_g(g + 7));
   }
   if constexpr (kLive) {
