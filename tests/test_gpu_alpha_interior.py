@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle
-from util import DeviceCase, assert_same_bits, gpu_forward
+from util import DeviceCase, assert_same_bits, gpu_backward, gpu_forward
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +31,23 @@ def test_alphas_where_the_interior_begins_and_ends(T, U):
         got, ref = alphas[b, :il[b], :ll[b] + 1], want[b, :il[b], :ll[b] + 1]
         assert_same_bits(got, ref, "alphas of utterance %d" % b)
     assert_same_bits(costs, want_costs, "costs")
+
+
+@pytest.mark.parametrize("U", [1, 2, 63, 64, 65, 130])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 70])
+def test_dalphas_where_groups_of_four_meet_the_lattices_edges(T, U):
+    """The transition weights are formed four anti-diagonals at a time: lattices that begin or end
+    inside such a group, shorter than one, and utterances of one frame or without labels."""
+    V, il, ll = 5, [T, T, max(T - 1, 1), 1], [U - 1, 0, U // 2, U - 1]
+    rng = np.random.default_rng(100 * T + U)
+    E = rng.standard_normal((4, T, V), dtype=np.float32)
+    P = rng.standard_normal((4, U, V), dtype=np.float32)
+    labels = rng.integers(1, V, (4, U - 1)).astype(np.int32)
+    il, ll = np.array(il, np.int32), np.array(ll, np.int32)
+    LN = oracle.log_norms_naive(E, P, il, ll)
+    c = DeviceCase(E, P, labels, il, ll)
+    _, alphas = gpu_forward(c, np.nan_to_num(LN))
+    got = gpu_backward(c, np.nan_to_num(alphas), np.nan_to_num(LN))
+    want = oracle.backward(E, P, np.nan_to_num(alphas), LN, labels, il, ll)
+    for g, w, what in zip(got, want, ("egrads", "pgrads", "lngrads")):
+        assert_same_bits(g, w, what)
