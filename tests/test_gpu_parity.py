@@ -813,3 +813,26 @@ def test_pgrads_of_tiles_whose_frames_are_split(T, U):
         # the exponents' rounding, about 2^-21, on every one of the n terms
         assert np.abs(got[b, :m] - (held[b, :m] + w.sum(0))).max() <= 4e-6 * np.abs(w).sum(0).max() + 1e-6
         assert np.array_equal(got[b, m:], held[b, m:])
+
+
+@pytest.mark.parametrize("V", [2, 63, 255, 256, 511, 512])
+@pytest.mark.parametrize("T,U", [(1, 2), (33, 40), (64, 33), (129, 97)])
+def test_sparse_terms_either_side_of_every_split_of_frames_and_positions(T, U, V):
+    """Blank and label terms through the three-call interface: label positions dealt to wavefronts
+    eight at a time, frames to workgroups by 64 or 32 rows of the vocabulary, repeated labels,
+    labels that are the blank; enough utterances for both forms of the per-frame sums."""
+    rng = np.random.default_rng(T + V)
+    for B in (3, 100):
+        E = rng.standard_normal((B, T, V), dtype=np.float32)
+        P = rng.standard_normal((B, U, V), dtype=np.float32)
+        labels = rng.integers(0, min(V, 7), (B, U - 1)).astype(np.int32)
+        il = rng.integers(1, T + 1, B).astype(np.int32)
+        ll = rng.integers(0, U, B).astype(np.int32)
+        il[0], ll[0] = T, U - 1
+        LN = oracle.log_norms_naive(E, P, il, ll)
+        c = DeviceCase(E, P, labels, il, ll)
+        _, alphas = gpu_forward(c, np.nan_to_num(LN))
+        got = gpu_backward(c, np.nan_to_num(alphas), np.nan_to_num(LN))
+        want = oracle.backward(E, P, np.nan_to_num(alphas), LN, labels, il, ll)
+        for g, w, what in zip(got, want, ("egrads", "pgrads", "lngrads")):
+            assert_same_bits(g, w, what)

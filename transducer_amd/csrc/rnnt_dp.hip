@@ -1268,60 +1268,72 @@ __global__ __launch_bounds__(256) void sparse_e_kernel(const float* __restrict__
 // The same terms for a small vocabulary, added (times scale[b]) onto an egrads that holds the
 // dense part.  With few columns the hardware adds of sparse_e_kernel all land in a few cache
 // lines per row and queue up at L2 (B=8, T=2000, U=100, V=100: 0.08 ms for 1.6 M adds), so
-// here a wavefront keeps its 64 frames' rows in LDS (64 x V floats, odd pitch: lane t owns row
-// t, all lanes hit column l together, no conflicts), subtracts the terms there in the
-// reference's order, and then adds the rows to egrads with row-contiguous accesses.
-// Dynamic LDS: 64 * (V | 1) floats.
-__global__ __launch_bounds__(64) void sparse_e_rows_kernel(const float* __restrict__ bsum,
-                                                           const float* __restrict__ emT,
-                                                           float* __restrict__ egrads,
-                                                           const int* __restrict__ labels,
-                                                           const int* __restrict__ inLen,
-                                                           const int* __restrict__ labLen,
-                                                           const float* __restrict__ scale,
-                                                           Dims d) {
+// here a workgroup keeps its frames' rows in LDS (64 x V floats, odd pitch: lane t owns row t, all
+// lanes hit column l together, no conflicts).  Its first wavefront subtracts the terms there in the
+// reference's order, the next sixteen requested ahead; then all four add the rows to egrads, which are
+// one contiguous piece of memory (B=8 T=2000 U=101 V=100: 34 us with one wavefront doing it all, a
+// round trip per eight rows and 64 columns, 21 now).
+// `frames` (at most 64) rows a workgroup; 32 where the LDS of 64 would pass 64 KB (B=16 T=2000 U=101
+// V=500: 162 us with hardware adds, 58 so).  Dynamic LDS: frames * (V | 1) floats.
+__global__ __launch_bounds__(256) void sparse_e_rows_kernel(const float* __restrict__ bsum,
+                                                            const float* __restrict__ emT,
+                                                            float* __restrict__ egrads,
+                                                            const int* __restrict__ labels,
+                                                            const int* __restrict__ inLen,
+                                                            const int* __restrict__ labLen,
+                                                            const float* __restrict__ scale,
+                                                            Dims d, int frames) {
   extern __shared__ float rows[];
-  const int b = blockIdx.y, t0 = blockIdx.x * 64, lane = threadIdx.x;
+  const int b = blockIdx.y, t0 = blockIdx.x * frames, tid = threadIdx.x;
   int Tb, Ub;
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
   if (Ub == 0 || t0 >= Tb) return;
   const int pitch = d.V | 1;
-  for (int i = lane; i < 64 * pitch; i += 64) rows[i] = 0.0f;
+  for (int i = tid; i < frames * pitch; i += 256) rows[i] = 0.0f;
   __syncthreads();
-  const int t = min(t0 + lane, Tb - 1);  // lanes past the utterance walk its last frame, unused
-  float* mine = rows + lane * pitch;
-  const int* __restrict__ lab = labels + (size_t)b * (d.U - 1);
-  const float* __restrict__ em = emT + (size_t)b * d.U * d.T + t;
-  constexpr int kChunk = 16;
-  for (int uhi = Ub - 2; uhi >= 0; uhi -= kChunk) {
-    float e[kChunk];
+  if (tid < frames) {
+    const int t = min(t0 + tid, Tb - 1);  // lanes past the utterance walk its last frame, unused
+    float* mine = rows + tid * pitch;
+    const int* __restrict__ lab = labels + (size_t)b * (d.U - 1);
+    const float* __restrict__ em = emT + (size_t)b * d.U * d.T + t;
+    constexpr int kChunk = 16;
+    struct Terms { float e[kChunk]; };
+    auto request = [&](int uhi) -> Terms {
+      Terms r;
 #pragma unroll
-    for (int k = 0; k < kChunk; ++k) e[k] = em[(size_t)max(uhi - k, 0) * d.T];
+      for (int k = 0; k < kChunk; ++k) r.e[k] = em[(size_t)max(uhi - k, 0) * d.T];
+      return r;
+    };
+    const float blanks = bsum[(size_t)b * d.T + t];
+    Terms cur = request(Ub - 2);
+    for (int uhi = Ub - 2; uhi >= 0; uhi -= kChunk) {
+      const Terms nxt = request(uhi - kChunk);
 #pragma unroll
-    for (int k = 0; k < kChunk; ++k) {
-      const int u = uhi - k;
-      if (u >= 0) {  // uniform
-        const int l = clampi(lab[u], 0, d.V - 1);
-        if (l != d.blank) mine[l] -= e[k];
+      for (int k = 0; k < kChunk; ++k) {
+        const int u = uhi - k;
+        if (u >= 0) {  // uniform
+          const int l = clampi(lab[u], 0, d.V - 1);
+          if (l != d.blank) mine[l] -= cur.e[k];
+        }
       }
+      cur = nxt;
     }
+    mine[d.blank] += blanks;
   }
-  mine[d.blank] += bsum[(size_t)b * d.T + t];
   __syncthreads();
   const float sc = scale ? scale[b] : 1.0f;
-  const int nrows = min(64, Tb - t0);
-  // eight rows at a time, their loads requested together (a row-by-row read-add-write would pay
-  // one round trip per row)
+  const int n = min(frames, Tb - t0) * d.V;
   float* base = egrads + ((size_t)b * d.T + t0) * d.V;
-  for (int v = lane; v < d.V; v += 64) {
-    for (int r0 = 0; r0 < nrows; r0 += 8) {
-      float have[8];
+  for (int i0 = tid; i0 < n; i0 += 8 * 256) {
+    float have[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) have[k] = base[(size_t)min(r0 + k, nrows - 1) * d.V + v];
+    for (int k = 0; k < 8; ++k) have[k] = base[min(i0 + 256 * k, n - 1)];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const float x = rows[min(r0 + k, nrows - 1) * pitch + v];
-        if (r0 + k < nrows && x != 0.0f) base[(size_t)(r0 + k) * d.V + v] = have[k] + sc * x;
+    for (int k = 0; k < 8; ++k) {
+      const int i = i0 + 256 * k;
+      if (i < n) {
+        const float x = rows[i / d.V * pitch + i % d.V];
+        if (x != 0.0f) base[i] = have[k] + sc * x;
       }
     }
   }
@@ -1336,11 +1348,18 @@ __global__ __launch_bounds__(64) void sparse_e_rows_kernel(const float* __restri
 //   emT[b][u][t]  the label move's dalpha[t,u+1] wE[t,u] of every cell ([B][U][T]: the kernel that
 //                 folds them in reads one label position's frames in a row).
 // One lane per frame subtracts its frame's terms in the reference's order, label positions last
-// to first; a wavefront takes 64 frames and works alone (no workgroup barrier).  The operands
-// come through LDS: for eight label positions at a time the wavefront copies the groups of
-// anti-diagonals its 64 frames meet there -- 128 contiguous bytes a group and plane -- with
-// 16-byte loads, requested one chunk ahead, and each lane then picks its own cells (read straight
-// from the planes, the 64 frames would touch 17 cache lines per load).
+// to first.  The operands come through LDS: for eight label positions at a time a wavefront copies the
+// groups of anti-diagonals its 64 frames meet there -- 128 contiguous bytes a group and plane --
+// with 16-byte loads, requested one round ahead, and each lane then picks its own cells (read
+// straight from the planes, the 64 frames would touch 17 cache lines per load).
+// kShared: a workgroup takes 64 frames and 32 label positions a round, eight to a wavefront; the
+// wavefronts form the products side by side and leave those of the blank moves in LDS, where the
+// first one subtracts them in order.  Without: a wavefront takes 64 frames and all their positions by
+// itself, without barriers.  The latter moves more bytes at a time where there are workgroups enough
+// (us for post_beta_kernel at B=32 T=2000 U=101 47 against 65, B=8 T=10000 U=401 249 against 290), and
+// is thirteen round trips one after the other where there are not (B=8 T=2000 U=101 30 against
+// 21, B=32 T=400 U=102 31 against 23; B=16 T=2000 U=101, 128
+// workgroups of the other kind, 34 against 37): shared up to 96 of them.
 constexpr int kBsFrames = 64, kBsPos = 8;
 constexpr int kBsGroups = (kBsFrames + kBsPos + 3) / 4 + 1;  // groups of four anti-diagonals a chunk meets
 // floats per staged group; the pitches put the 16-byte pieces of consecutive groups on different banks
@@ -1349,7 +1368,12 @@ constexpr int kBsPitchD = 4 * (kBsPos + 1) + 8;  // dalpha: nine (a cell's label
 constexpr int kBsPieces = (kBsGroups * kBsPos + 63) / 64;         // 16-byte pieces a lane copies per plane
 constexpr int kBsPiecesD = (kBsGroups * (kBsPos + 1) + 63) / 64;
 constexpr int kBsWave = kBsGroups * (2 * kBsPitch + kBsPitchD);   // floats of LDS a wavefront stages in
-constexpr int kPostBetaLds = 4 * kBsWave > 64 * 65 ? 4 * kBsWave : 64 * 65;  // floats: either kind of block
+constexpr int kBsSums = 2 * 4 * kBsPos * kBsFrames;  // floats: the products of a round, stay and label moves
+constexpr int kBsAll = 4 * kBsWave + kBsSums;
+constexpr int post_beta_lds(bool shared) {  // floats: either kind of block
+  return std::max(shared ? kBsAll : 4 * kBsWave, 64 * 65);
+}
+template <bool kShared>
 __device__ __forceinline__ void frame_terms_block(const Planes& p, float* __restrict__ bsum,
                                                   float* __restrict__ emT,
                                                   const int* __restrict__ labels,
@@ -1357,10 +1381,10 @@ __device__ __forceinline__ void frame_terms_block(const Planes& p, float* __rest
                                                   const int* __restrict__ labLen, const Dims& d,
                                                   int bx, int b, float* __restrict__ lds) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int t0 = (4 * bx + wave) * kBsFrames, t = t0 + lane;
+  const int t0 = (kShared ? bx : 4 * bx + wave) * kBsFrames, t = t0 + lane;
   int Tb, Ub;
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
-  if (Ub == 0 || t0 >= Tb) return;  // the whole wavefront
+  if (Ub == 0 || t0 >= Tb) return;  // the whole workgroup (wavefront)
   const bool active = t < Tb;
   const int* __restrict__ lab = labels + (size_t)b * (d.U - 1);
   const float* __restrict__ dS = p.dS;
@@ -1369,6 +1393,8 @@ __device__ __forceinline__ void frame_terms_block(const Planes& p, float* __rest
   float* stW = lds + wave * kBsWave;        // wB of anti-diagonal groups gbase ..
   float* stE = stW + kBsGroups * kBsPitch;  // wE
   float* stD = stE + kBsGroups * kBsPitch;  // dalpha
+  float* stays = lds + 4 * kBsWave;                 // [position of the round][frame]
+  float* emits = stays + 4 * kBsPos * kBsFrames;    // where the label is the blank
   const size_t plane_b = (size_t)b * d.Ua * d.Dp;
   const int ngroups_plane = d.Dp >> 2;
   const bool has_stay = t + 1 < Tb;
@@ -1402,10 +1428,14 @@ __device__ __forceinline__ void frame_terms_block(const Planes& p, float* __rest
     }
     return r;
   };
-  const int ua_first = (Ub - 1) & ~(kBsPos - 1);
-  Pieces cur = request(ua_first);
-  for (int ua = ua_first; ua >= 0; ua -= kBsPos) {
-    const int gbase = (t0 + ua) >> 2;
+  // round by round from the last positions down; this wavefront's eight may lie past the
+  // utterance's last one (their cells hold zeros or nothing and are not looked at)
+  constexpr int kRound = (kShared ? 4 : 1) * kBsPos;
+  const int u_off = kShared ? kBsPos * wave : 0;
+  const int first = (Ub - 1) & ~(kRound - 1);
+  Pieces cur = request(first + u_off);
+  for (int u_round = first; u_round >= 0; u_round -= kRound) {
+    const int ua = u_round + u_off, gbase = (t0 + ua) >> 2;
     // (LDS serves a wavefront's accesses in order; the fences only hold the compiler to it)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -1427,7 +1457,7 @@ __device__ __forceinline__ void frame_terms_block(const Planes& p, float* __rest
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    cur = request(ua - kBsPos);
+    cur = request(ua - kRound);
     if (active) {
 #pragma unroll
       for (int k = kBsPos - 1; k >= 0; --k) {
@@ -1438,15 +1468,33 @@ __device__ __forceinline__ void frame_terms_block(const Planes& p, float* __rest
           const int next = (((dd + 1) >> 2) - gbase) * kBsPitchD + 4 * k + ((dd + 1) & 3);
           const float ne = stD[next] * stW[here];      // dalpha[t+1,u] wB[t,u]
           const float em = stD[next + 4] * stE[here];  // dalpha[t,u+1] wE[t,u]
-          acc -= has_stay ? ne : 0.0f;
           const bool has_label = u + 1 < Ub;
-          if (has_label && clampi(lab[u], 0, d.V - 1) == d.blank) acc -= em;
+          if constexpr (kShared) {
+            stays[(u_off + k) * kBsFrames + lane] = has_stay ? ne : 0.0f;
+            emits[(u_off + k) * kBsFrames + lane] = em;
+          } else {
+            acc -= has_stay ? ne : 0.0f;
+            if (has_label && clampi(lab[u], 0, d.V - 1) == d.blank) acc -= em;
+          }
           emT[((size_t)b * d.U + u) * d.T + t] = has_label ? em : 0.0f;
         }
       }
     }
+    if constexpr (kShared) {
+      __syncthreads();
+      if (wave == 0) {
+#pragma unroll 8
+        for (int k = min(kRound, Ub - u_round) - 1; k >= 0; --k) {
+          acc -= stays[k * kBsFrames + lane];
+          const int u = u_round + k;
+          if (u + 1 < Ub && clampi(lab[u], 0, d.V - 1) == d.blank)
+            acc -= emits[k * kBsFrames + lane];
+        }
+      }
+      __syncthreads();
+    }
   }
-  if (active) bsum[(size_t)b * d.T + t] = acc;
+  if (active && (!kShared || wave == 0)) bsum[(size_t)b * d.T + t] = acc;
 }
 
 // W from the skewed planes the lattice kernels leave behind (dalpha and LN): no un-skewed copy of
@@ -1564,6 +1612,7 @@ __device__ __forceinline__ void wimages_block(
 // instead of waiting behind a kernel boundary.  The last nw blocks form W (tile bx, by of
 // utterance b; with `img` the tiles are 64 frames x 64 label positions and go to the slab images
 // instead), the blocks before them the per-frame terms bsum and emT (bsum == nullptr: none).
+template <bool kShared>
 __global__ __launch_bounds__(256) void post_beta_kernel(Planes p, const float* __restrict__ mE,
                                                         const float* __restrict__ mP,
                                                         float* __restrict__ Wn,
@@ -1575,7 +1624,7 @@ __global__ __launch_bounds__(256) void post_beta_kernel(Planes p, const float* _
                                                         const int* __restrict__ labLen, Dims d,
                                                         int Up, int Tw, int wx, int wy, int nw,
                                                         int sx, WImages img) {
-  __shared__ __attribute__((aligned(16))) float lds[kPostBetaLds];
+  __shared__ __attribute__((aligned(16))) float lds[post_beta_lds(kShared)];
   float (*tile)[65] = reinterpret_cast<float (*)[65]>(lds);
   // the per-frame blocks come first in the grid: each runs longer than a W tile, and started
   // last they would be the kernel's tail
@@ -1590,7 +1639,7 @@ __global__ __launch_bounds__(256) void post_beta_kernel(Planes p, const float* _
                            r / wx, b);
   } else {
     const int m = blockIdx.x;
-    frame_terms_block(p, bsum, emT, labels, inLen, labLen, d, m % sx, m / sx, lds);
+    frame_terms_block<kShared>(p, bsum, emT, labels, inLen, labLen, d, m % sx, m / sx, lds);
   }
 }
 
@@ -2748,13 +2797,15 @@ int launch_sparse(const Planes& p, const float* bsum, const float* emT, float* e
                   const float* scale, bool add, const Dims& d, hipStream_t s) {
   if (d.B == 0 || d.T == 0 || d.U == 0) return kOk;
   if (!bsum || !emT) return fail(kInvalid, "sparse terms: the per-frame terms were not formed");
-  const size_t rows_bytes = sizeof(float) * 64 * (size_t)(d.V | 1);
+  const int frames = 64 * (size_t)(d.V | 1) * sizeof(float) <= 64 * 1024 ? 64 : 32;
+  const size_t rows_bytes = sizeof(float) * frames * (size_t)(d.V | 1);
   // (a small vocabulary also when the terms are to be stored: the arrays are zero-filled then,
   // and adding to zeros leaves the same bits -- B=8 T=10000 U=400 V=32: 1.67 ms with one
   // hardware add per term, all of them into 128 bytes a frame)
   if (rows_bytes <= 64 * 1024 && labels != nullptr) {
-    hipLaunchKernelGGL(sparse_e_rows_kernel, dim3((d.T + 63) / 64, d.B), dim3(64), rows_bytes, s,
-                       bsum, emT, egrads, labels, inLen, labLen, add ? scale : nullptr, d);
+    hipLaunchKernelGGL(sparse_e_rows_kernel, dim3((d.T + frames - 1) / frames, d.B), dim3(256),
+                       rows_bytes, s, bsum, emT, egrads, labels, inLen, labLen,
+                       add ? scale : nullptr, d, frames);
     RNNT_LAUNCH_CHECK("sparse_e_rows_kernel");
   } else {
     hipLaunchKernelGGL(sparse_e_kernel, dim3((d.T + 255) / 256, d.B), dim3(256), 0, s, bsum, emT,
@@ -2782,10 +2833,16 @@ int launch_post_beta(const Planes& p, const float* mE, const float* mP, float* W
   const int nw = (Wn || img.e) ? wx * wy * d.B : 0;
   if ((bsum == nullptr) != (emT == nullptr))
     return fail(kInvalid, "post_beta: the blank totals and the label-move terms come together");
-  const int sx = (d.T + 4 * kBsFrames - 1) / (4 * kBsFrames), ns = bsum ? sx * d.B : 0;
+  const int alone = (d.T + 4 * kBsFrames - 1) / (4 * kBsFrames);
+  const bool shared = (long)alone * d.B <= 96;
+  const int sx = shared ? (d.T + kBsFrames - 1) / kBsFrames : alone, ns = bsum ? sx * d.B : 0;
   if (nw + ns == 0) return kOk;
-  hipLaunchKernelGGL(post_beta_kernel, dim3(nw + ns), dim3(256), 0, s, p, mE, mP, Wn, Wt, bsum,
-                     emT, labels, inLen, labLen, d, Up, Tw, wx, wy, nw, sx, img);
+  if (shared)
+    hipLaunchKernelGGL(post_beta_kernel<true>, dim3(nw + ns), dim3(256), 0, s, p, mE, mP, Wn, Wt,
+                       bsum, emT, labels, inLen, labLen, d, Up, Tw, wx, wy, nw, sx, img);
+  else
+    hipLaunchKernelGGL(post_beta_kernel<false>, dim3(nw + ns), dim3(256), 0, s, p, mE, mP, Wn, Wt,
+                       bsum, emT, labels, inLen, labLen, d, Up, Tw, wx, wy, nw, sx, img);
   RNNT_LAUNCH_CHECK("post_beta_kernel");
   return kOk;
 }
