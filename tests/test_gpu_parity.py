@@ -836,3 +836,27 @@ def test_sparse_terms_either_side_of_every_split_of_frames_and_positions(T, U, V
         want = oracle.backward(E, P, np.nan_to_num(alphas), LN, labels, il, ll)
         for g, w, what in zip(got, want, ("egrads", "pgrads", "lngrads")):
             assert_same_bits(g, w, what)
+
+
+@pytest.mark.parametrize("U,V", [(113, 512), (130, 514), (250, 700), (401, 515)])
+def test_label_terms_of_label_axes_of_several_slices(U, V):
+    """Dozens of labels in one block of 32 columns, the same label many times, labels that are the
+    blank, transcripts that end inside a block: the egrads write-out adds their terms up in LDS,
+    fourteen of them asked for ahead.  With the device's log-normaliser on both sides, at the
+    tolerance of the other whole-loss tests."""
+    rng = np.random.default_rng(U)
+    B, T = 3, 70
+    E = rng.standard_normal((B, T, V), dtype=np.float32)
+    P = rng.standard_normal((B, U, V), dtype=np.float32)
+    labels = rng.integers(0, V, (B, U - 1)).astype(np.int32)
+    labels[1] = rng.integers(0, 40, U - 1)
+    il, ll = np.array([T, T - 1, 33], np.int32), np.array([U - 1, U - 2, 5], np.int32)
+    c = DeviceCase(E, P, labels, il, ll)
+    costs, eg, pg = gpu_loss(c)
+    LN = np.nan_to_num(gpu_log_norms(c))
+    want_costs, alphas = oracle.forward(E, P, LN, labels, il, ll)
+    weg, wpg, lng = oracle.backward(E, P, np.nan_to_num(alphas), LN, labels, il, ll)
+    weg, wpg = oracle.accumulate_grads(E, P, weg, wpg, lng, LN, il, ll)
+    assert_close(costs, want_costs, what="costs")
+    assert_close(eg, weg, what="egrads")
+    assert_close(pg, wpg, what="pgrads")

@@ -78,7 +78,8 @@ __device__ __forceinline__ void egrads_walk(
     const float* __restrict__ mP, const float* __restrict__ Wn, const float* __restrict__ deltas,
     TOUT* __restrict__ egrads, unsigned short (*As)[3][kEsPlane], float (*Ms)[32], const Dims& d,
     int Up, int Tw, int tiles_per_chunk, int u_lo, int b, int Tb, int Ub, const SparseTerms& sp,
-    const unsigned short* match, int nmatch, float (*Sp)[32], const EgradsWindow& win) {
+    const unsigned short* match, int nmatch, float (*Sp)[32], float* block,
+    const EgradsWindow& win) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, h = lane >> 5;
   const int wave_col0 = blockIdx.x * 128 + wave * 32;  // this wavefront's 32 columns
   const int vcol = wave_col0 + l32;
@@ -182,12 +183,17 @@ __device__ __forceinline__ void egrads_walk(
   if (tile_lo < tile_valid) store_slab(0, fetch_slab(tile_lo));
   __syncthreads();
 
-  // the first kEsPrefetch matches, resolved once: label position and target lane
-  int mu[kEsPrefetch], mc[kEsPrefetch];
+  // the first matches, resolved once: label position and target lane.  (kBlocks: each half of the
+  // wavefront keeps every second one)
+  constexpr bool kBlocks = kManyLabels && kMode == kEgFinal;
+  constexpr int kPre = kBlocks ? kEsManyPrefetch : kEsPrefetch;
+  constexpr int kPerReg = kBlocks ? 2 : 1;
+  int mu[kPre], mc[kPre];
 #pragma unroll
-  for (int i = 0; i < kEsPrefetch; ++i) {
-    mu[i] = (sp.labels && i < nmatch) ? match[i] : 0;
-    mc[i] = (sp.labels && i < nmatch) ? label_at(sp.labels, d, b, mu[i]) - wave_col0 : -1;
+  for (int i = 0; i < kPre; ++i) {
+    const int m = kPerReg * i + (kBlocks ? h : 0);
+    mu[i] = (sp.labels && m < nmatch) ? match[m] : 0;
+    mc[i] = (sp.labels && m < nmatch) ? label_at(sp.labels, d, b, mu[i]) - wave_col0 : -1;
   }
 
   // bf16 only: with half the bytes the kernel is held by how long a request takes, not by how
@@ -254,14 +260,15 @@ __device__ __forceinline__ void egrads_walk(
         }
       }
     }
-    // sparse terms of this tile for up to kEsPrefetch labels that fall into this wavefront's
-    // columns: one coalesced load per plane, requested here so it arrives under the matrix work
-    float sd[kEsPrefetch], sbl = 0.0f;
+    // sparse terms of this tile for the first labels that fall into this wavefront's columns: one coalesced load per plane, requested here so it arrives under the matrix work
+    float sd[kPre], sbl = 0.0f;
     if (kSparse && (nmatch > 0 || blank_lane >= 0)) {
       const int tr = min(t0 + l32, Tb - 1);
 #pragma unroll
-      for (int i = 0; i < kEsPrefetch; ++i) {
-        sd[i] = sp.emT[((size_t)b * d.U + mu[i]) * d.T + tr];
+      for (int i = 0; i < kPre; ++i) {
+        sd[i] = 0.0f;
+        if (!kBlocks || kPerReg * i < nmatch)
+          sd[i] = sp.emT[((size_t)b * d.U + mu[i]) * d.T + tr];
       }
       if (blank_lane >= 0) sbl = sp.bsum[(size_t)b * d.T + tr];
     }
@@ -324,16 +331,64 @@ __device__ __forceinline__ void egrads_walk(
           }
         }
       };
+      if constexpr (kBlocks) {
+        // label axes of several slices (400 labels and 1000 columns put a dozen into every block):
+        // the terms are added up in a 32 x 32 block in LDS, a label to each half of the wavefront
+        // at a time and nothing waited for, and a lane takes its column's sixteen frames from
+        // there once; the first fourteen are asked for before the matrix block.  All slices of
+        // egrads at B=8 T=10000 U=401 V=1000 1026 -> 934 us, B=4 T=2000 U=300 V=2000 145 -> 126; with
+        // one slice there are few labels a block, and filling and reading it costs more than it
+        // saves (B=32 T=2000 U=101 V=1000: 197 -> 213).
+        if (nmatch > 0) {
 #pragma unroll
-      for (int i = 0; i < kEsPrefetch; ++i)
-        if (i < nmatch) apply(row_ok ? sd[i] : 0.0f, mc[i], -1.0f);
+          for (int k = 0; k < (32 * kEsBlockPitch / 4 + 63) / 64; ++k)
+            if (64 * k + lane < 32 * kEsBlockPitch / 4)
+              reinterpret_cast<float4*>(block)[64 * k + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int i = 0; i < kPre; ++i)
+            if (2 * i < nmatch && mc[i] >= 0 && row_ok)
+              unsafeAtomicAdd(&block[mc[i] * kEsBlockPitch + l32], sd[i]);
+          constexpr int kBatch = 4;
+          for (int i0 = 2 * kPre; i0 < nmatch; i0 += 2 * kBatch) {
+            float term[kBatch];
+            int col[kBatch];
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+              const int m = i0 + 2 * k + h, u = match[min(m, nmatch - 1)];
+              term[k] = sp.emT[((size_t)b * d.U + u) * d.T + min(t0 + l32, Tb - 1)];
+              col[k] = m < nmatch ? label_at(sp.labels, d, b, u) - wave_col0 : -1;
+            }
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k)
+              if (col[k] >= 0 && row_ok)
+                unsafeAtomicAdd(&block[col[k] * kEsBlockPitch + l32], term[k]);
+          }
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const float4 x =
+                *reinterpret_cast<const float4*>(&block[l32 * kEsBlockPitch + 8 * g + 4 * h]);
+            v[4 * g + 0] -= x.x;
+            v[4 * g + 1] -= x.y;
+            v[4 * g + 2] -= x.z;
+            v[4 * g + 3] -= x.w;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < kEsPrefetch; ++i)
+          if (i < nmatch) apply(row_ok ? sd[i] : 0.0f, mc[i], -1.0f);
+      }
       // more labels in one 32-column block
-      if constexpr (kManyLabels) {
-        // long transcripts over a small vocabulary (400 labels and 1000 columns put a dozen into
-        // every block): their terms are asked for four at a time, so that a tile waits one
-        // memory round trip per four, not one per label (B=8 T=10000 U=400 V=1000: 1.21 ->
-        // 1.02 ms).  A kernel of its own: compiled into the kernel of the large vocabularies,
-        // where it hardly ever runs, it cost that one 1 % (B=32 T=2000 U=100 V=10000).
+      if constexpr (kBlocks) {
+      } else if constexpr (kManyLabels) {
+        // long transcripts over a small vocabulary: their terms are asked for four at a time, so
+        // that a tile waits one memory round trip per four, not one per label.  A kernel of its
+        // own: compiled into the kernel of the large vocabularies, where it hardly ever runs, it
+        // cost that one 1 % (B=32 T=2000 U=100 V=10000).
         constexpr int kBatch = 4;
         for (int i0 = kEsPrefetch; i0 < nmatch; i0 += kBatch) {
           float term[kBatch];
@@ -419,6 +474,9 @@ __global__ __launch_bounds__(256, 2) void egrads_stream_kernel(
   __shared__ __attribute__((aligned(16))) unsigned short As[2][3][kEsPlane];
   __shared__ __attribute__((aligned(16))) float Ms[2][32];  // mE * log2(e) of the slab's frames
   __shared__ __attribute__((aligned(16))) float Strip[4][32];  // per wavefront: sparse terms
+  constexpr bool kBlocks = kManyLabels && kMode == kEgFinal;
+  __shared__ __attribute__((aligned(16))) float Block[kBlocks ? 4 : 1]
+                                                     [kBlocks ? 32 * kEsBlockPitch : 1];
   __shared__ unsigned short Match[4][kMaxLabels];  // per wavefront: label positions whose label
                                                    // is one of its 32 columns
   const int b = blockIdx.z;
@@ -450,7 +508,7 @@ __global__ __launch_bounds__(256, 2) void egrads_stream_kernel(
 #define RNNT_EG_WALK(NS)                                                                      \
   egrads_walk<NS, kMode, kManyLabels>(E, P, mE, mP, Wn, deltas, egrads, As, Ms, d, Up, Tw,   \
                                tiles_per_chunk, u_lo, b, Tb, Ub, sp, Match[threadIdx.x >> 6], \
-                               nmatch, &Strip[threadIdx.x >> 6], win)
+                               nmatch, &Strip[threadIdx.x >> 6], Block[kBlocks ? threadIdx.x >> 6 : 0], win)
   if (nsteps <= 2) RNNT_EG_WALK(2);
   else if (nsteps <= 4) RNNT_EG_WALK(4);
   else if (nsteps == 5) RNNT_EG_WALK(5);
