@@ -996,8 +996,12 @@ int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_leng
     std::lock_guard<std::mutex> lock(g_check_mutex);
     if (g_check_words == nullptr) {
       void* p = nullptr;
-      RNNT_HIP(hipHostMalloc(&p, sizeof(int) * kSlotInts * kCheckSlots,
-                             hipHostMallocPortable | hipHostMallocMapped));
+      const hipError_t e = hipHostMalloc(&p, sizeof(int) * kSlotInts * kCheckSlots,
+                                         hipHostMallocPortable | hipHostMallocMapped);
+      if (e != hipSuccess) {
+        (void)hipGetLastError();  // the caller may go on without: no later launch reports this
+        return check_hip(e, "hipHostMalloc", __FILE__, __LINE__);
+      }
       g_check_words = static_cast<int*>(p);
       for (int i = 0; i < kCheckSlots; ++i) g_check_free[i] = i;
       g_check_nfree = kCheckSlots;
