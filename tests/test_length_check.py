@@ -1,0 +1,71 @@
+"""The host side of rnnt_hip_check_lengths_begin / _end, on a stand-in for the HIP runtime
+(length_check_runtime.cpp): which device is asked, which tickets are honoured, what becomes of a
+slot when something fails.  No device is needed; the kernel itself is tested in test_gpu_torch.py."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+LIB = os.path.join(os.path.dirname(HERE), "transducer_amd", "librnnt_hip.so")
+
+PRELUDE = r"""
+import ctypes, sys
+rt = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+def knob(name): return ctypes.c_int.in_dll(rt, name)
+lib.rnnt_hip_last_error.restype = ctypes.c_char_p
+P, I = ctypes.c_void_p, ctypes.c_int
+lib.rnnt_hip_check_lengths_begin.argtypes = [P, P, I, I, I, P, P]
+lib.rnnt_hip_check_lengths_end.argtypes = [I, P, P]
+keep = []
+def begin(inputs=(6, 6), labels=(3, 3), stream=None, T=6, U=4):
+    arrays = [(I * len(x))(*x) for x in (inputs, labels)]
+    keep.append(arrays)
+    ticket = I(-7)
+    status = lib.rnnt_hip_check_lengths_begin(arrays[0], arrays[1], len(inputs), T, U, stream,
+                                              ctypes.byref(ticket))
+    return status, ticket.value
+def end(ticket, stream=None):
+    verdict = I(-7)
+    status = lib.rnnt_hip_check_lengths_end(ticket, stream, ctypes.byref(verdict))
+    return status, verdict.value
+OK, INVALID, HIP_ERROR = 0, 1, 2
+"""
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("runtime") / "libruntime.so")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-o", out,
+                           os.path.join(HERE, "length_check_runtime.cpp")])
+    return out
+
+
+def run(runtime, body):
+    """`body` in a process of its own, the stand-in loaded ahead of the library."""
+    subprocess.run([sys.executable, "-c", PRELUDE + body, runtime, LIB], check=True, timeout=60)
+
+
+def test_the_stream_is_asked_on_the_device_of_the_check(runtime):
+    """The null stream's handle is the same on every device: with another device current when the
+    answer is waited for, an idle stream of that one says nothing about the check."""
+    run(runtime, r"""
+knob("current_device").value = 1
+status, ticket = begin(inputs=(6, 7))
+assert status == OK
+knob("current_device").value = 0
+knob("delay").value = 3
+assert end(ticket) == (OK, 1), lib.rnnt_hip_last_error()
+assert knob("asked").value == 4 and knob("current_device").value == 0
+""")
+
+
+def test_verdicts(runtime):
+    run(runtime, r"""
+for inputs, labels, want in (((6, 6), (3, 3), 0), ((7, 1), (3, 3), 1), ((6, 6), (0, 4), 2),
+                             ((1, 2**31 - 1), (4, 4), 3), ((-5, 0), (-1, 0), 0)):
+    status, ticket = begin(inputs, labels)
+    assert status == OK and end(ticket) == (OK, want)
+""")

@@ -313,6 +313,7 @@ constexpr int kPending = -1, kInputTooLong = 1, kLabelsTooLong = 2;
 std::mutex g_check_mutex;
 int* g_check_words = nullptr;
 int g_check_free[kCheckSlots], g_check_nfree = 0;
+int g_check_device[kCheckSlots];  // whose stream the check went to (a null stream is every device's)
 
 __global__ __launch_bounds__(256) void check_lengths_kernel(const int* __restrict__ inLen,
                                                             const int* __restrict__ labLen, int B,
@@ -334,6 +335,19 @@ __global__ __launch_bounds__(256) void check_lengths_kernel(const int* __restric
 void release_check_slot(int slot) {
   std::lock_guard<std::mutex> lock(g_check_mutex);
   g_check_free[g_check_nfree++] = slot;
+}
+
+// hipStreamQuery with `device` current (the caller's current device may have changed since the
+// check was enqueued, and a handle of 0 means the current device's null stream).  Leaves no error
+// behind: "not ready" counts as one.
+hipError_t query_on(int device, hipStream_t s) {
+  int current = 0;
+  hipError_t e = hipGetDevice(&current);
+  if (e == hipSuccess && current != device) e = hipSetDevice(device);
+  if (e == hipSuccess) e = hipStreamQuery(s);
+  if (e != hipSuccess) (void)hipGetLastError();
+  if (current != device) (void)hipSetDevice(current);
+  return e;
 }
 
 // Scratch the best-path stages need (planes, the two max-plus planes, the decision table).
@@ -991,7 +1005,8 @@ int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_leng
                                  int U, rnnt_stream_t stream, int* ticket) {
   if (!ticket || !input_lengths || !label_lengths || B < 1)
     return fail(kInvalid, "check_lengths: null argument or empty batch");
-  int slot;
+  int slot, device = 0;
+  RNNT_HIP(hipGetDevice(&device));
   {
     std::lock_guard<std::mutex> lock(g_check_mutex);
     if (g_check_words == nullptr) {
@@ -1009,6 +1024,7 @@ int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_leng
     if (g_check_nfree == 0)
       return fail(kInvalid, "check_lengths: %d checks under way already", kCheckSlots);
     slot = g_check_free[--g_check_nfree];
+    g_check_device[slot] = device;
   }
   int* word = g_check_words + (size_t)slot * kSlotInts;
   __atomic_store_n(word, kPending, __ATOMIC_RELEASE);
@@ -1029,12 +1045,10 @@ int rnnt_hip_check_lengths_end(int ticket, rnnt_stream_t stream, int* verdict) {
   int* word = g_check_words + (size_t)ticket * kSlotInts;
   int v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
   // The wait ends with the kernel's word, or when the stream reports an error or that it has
-  // run out of work (asked now and then; the query leaves "not ready" behind as an error, which
-  // is taken back).
+  // run out of work (asked now and then).
   for (unsigned spins = 1; v == kPending; ++spins) {
     if (spins % 4096 == 0) {
-      const hipError_t q = hipStreamQuery(static_cast<hipStream_t>(stream));
-      if (q != hipSuccess) (void)hipGetLastError();
+      const hipError_t q = query_on(g_check_device[ticket], static_cast<hipStream_t>(stream));
       v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
       if (v != kPending) break;
       // (another thread's capture may forbid the question for a while: that is no answer)
