@@ -69,3 +69,35 @@ for inputs, labels, want in (((6, 6), (3, 3), 0), ((7, 1), (3, 3), 1), ((6, 6), 
     status, ticket = begin(inputs, labels)
     assert status == OK and end(ticket) == (OK, want)
 """)
+
+
+def test_an_error_somebody_else_left_behind_does_not_release_a_slot_in_use(runtime):
+    """The kernel is enqueued although an earlier call in this thread failed: its slot must not
+    go to the next check while it is still to be written."""
+    run(runtime, r"""
+knob("delay").value = 1 << 30
+knob("last_error").value = 1
+status, first = begin(inputs=(7, 7))
+assert status == OK and knob("launches").value == 1
+assert knob("last_error").value == 1      # it is not this call's to take back
+second = begin()
+assert second[0] == OK and second[1] != first
+knob("delay").value = 0
+assert end(first) == (OK, 1) and end(second[1]) == (OK, 0)
+""")
+
+
+def test_a_launch_that_fails_gives_its_slot_back_only_after_a_wait(runtime):
+    run(runtime, r"""
+knob("launch_error").value = 98
+for _ in range(1000):                     # the stream could be waited for: no slot is lost
+    assert begin()[0] == HIP_ERROR
+    assert knob("last_error").value == 0  # nor is an error left for the next launch to report
+knob("launch_error").value = 0
+assert begin()[0] == OK
+knob("launch_error").value, knob("sync_error").value = 98, 98
+for _ in range(255):                      # it could not: the slots stay out of use
+    assert begin()[0] == HIP_ERROR
+knob("launch_error").value = 0
+assert begin()[0] == INVALID and b"under way" in lib.rnnt_hip_last_error()
+""")

@@ -1005,6 +1005,7 @@ int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_leng
                                  int U, rnnt_stream_t stream, int* ticket) {
   if (!ticket || !input_lengths || !label_lengths || B < 1)
     return fail(kInvalid, "check_lengths: null argument or empty batch");
+  hipStream_t s = static_cast<hipStream_t>(stream);
   int slot, device = 0;
   RNNT_HIP(hipGetDevice(&device));
   {
@@ -1028,12 +1029,17 @@ int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_leng
   }
   int* word = g_check_words + (size_t)slot * kSlotInts;
   __atomic_store_n(word, kPending, __ATOMIC_RELEASE);
-  hipLaunchKernelGGL(check_lengths_kernel, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream),
-                     input_lengths, label_lengths, B, T, U, word);
-  const int status = check_hip(hipGetLastError(), "launch check_lengths_kernel", __FILE__, __LINE__);
-  if (status != kOk) {  // nothing was enqueued: nobody will write the slot
-    release_check_slot(slot);
-    return status;
+  // (the launch's own status: the thread's last error may be somebody else's, left behind before,
+  // and says nothing about whether this kernel is going to write the slot)
+  void* args[] = {&input_lengths, &label_lengths, &B, &T, &U, &word};
+  const hipError_t launched = hipLaunchKernel(reinterpret_cast<const void*>(check_lengths_kernel),
+                                              dim3(1), dim3(256), args, 0, s);
+  if (launched != hipSuccess) {
+    (void)hipGetLastError();
+    // the slot goes to another check only if nothing can be on its way to it any more
+    if (hipStreamSynchronize(s) == hipSuccess) release_check_slot(slot);
+    else (void)hipGetLastError();
+    return check_hip(launched, "launch check_lengths_kernel", __FILE__, __LINE__);
   }
   *ticket = slot;
   return kOk;
