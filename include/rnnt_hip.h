@@ -190,8 +190,10 @@ int rnnt_hip_release_scratch(void);
  * what was enqueued after it) and gives the ticket back: verdict is 0, or 1 if some input_length
  * exceeds T, plus 2 if some label_length exceeds U - 1.  Every kernel clamps lengths to the
  * padded sizes, so what is enqueued in between stays inside the arrays either way.  One _end per
- * successful _begin, on the same stream; not capturable; any thread, whichever device is current.
- * At most 256 under way: _begin then fails and enqueues nothing. */
+ * successful _begin, on the same stream, in any thread, whichever device is current; an _end for
+ * any other ticket or stream is refused.  An _end that fails after its wait has spent the ticket
+ * too.  _begin fails and enqueues nothing on a stream that is being captured and with 256 checks
+ * under way. */
 int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_lengths, int B, int T,
                                  int U, rnnt_stream_t stream, int* ticket);
 int rnnt_hip_check_lengths_end(int ticket, rnnt_stream_t stream, int* verdict);

@@ -40,20 +40,25 @@ struct Call {
 extern "C" {
 
 int current_device = 0;
-int delay = 0;         // questions a launch stays unfinished for
-int asked = 0;         // hipStreamQuery calls
-int launches = 0;      // kernels enqueued
-int last_error = 0;    // what hipGetLastError reports next
-int launch_error = 0;  // what hipLaunchKernel returns (and enqueues nothing)
-int sync_error = 0;    // what hipStreamSynchronize returns
-int query_error = 0;   // what hipStreamQuery returns instead of an answer
-int capturing = 0;     // hipStreamCaptureStatus of every stream
+int delay = 0;          // questions a launch stays unfinished for
+int asked = 0;          // hipStreamQuery calls
+int launches = 0;       // kernels enqueued
+int last_error = 0;     // what hipGetLastError reports next
+int launch_error = 0;   // what hipLaunchKernel returns (and enqueues nothing)
+int sync_error = 0;     // what hipStreamSynchronize returns
+int query_error = 0;    // what hipStreamQuery returns instead of an answer
+int capturing = 0;      // hipStreamCaptureStatus of every stream
+int capture_error = 0;  // what hipStreamIsCapturing returns instead
+int lose = 0;           // launches are accepted and never run
 
 int hipGetDevice(int* d) { *d = current_device; return 0; }
 int hipSetDevice(int d) { current_device = d; return 0; }
 int hipHostMalloc(void** p, size_t n, unsigned) { *p = calloc(n, 1); return *p ? 0 : 2; }
 int hipGetLastError() { const int e = last_error; last_error = 0; return e; }
-int hipStreamIsCapturing(void*, int* status) { *status = capturing; return 0; }
+int hipStreamIsCapturing(void*, int* status) {
+  *status = capturing;
+  return capture_error ? last_error = capture_error : 0;
+}
 
 int __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, void* stream) {
   pushed = Call{grid, block, lds, stream};
@@ -66,6 +71,7 @@ int __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, void** strea
 int hipLaunchKernel(const void*, dim3, dim3, void** args, size_t, void* stream) {
   if (launch_error) return last_error = launch_error;
   ++launches;
+  if (lose) return 0;
   waiting[{current_device, stream}].push_back(
       Launch{*(const int**)args[0], *(const int**)args[1], *(int*)args[2], *(int*)args[3],
              *(int*)args[4], *(int**)args[5]});

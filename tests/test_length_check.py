@@ -101,3 +101,63 @@ for _ in range(255):                      # it could not: the slots stay out of 
 knob("launch_error").value = 0
 assert begin()[0] == INVALID and b"under way" in lib.rnnt_hip_last_error()
 """)
+
+
+def test_a_ticket_is_good_for_one_end(runtime):
+    run(runtime, r"""
+assert end(0)[0] == INVALID               # nothing was ever begun
+a, b = begin(inputs=(7, 7))[1], begin()[1]
+for never in (-1, 256, 255 - a if 255 - a not in (a, b) else 17):
+    assert end(never)[0] == INVALID
+assert end(a) == (OK, 1)
+for _ in range(300):                      # (each of these once put the slot on the free list)
+    assert end(a)[0] == INVALID
+tickets = [begin() for _ in range(255)]   # with b 256 under way, each on a slot of its own
+assert all(t[0] == OK for t in tickets)
+assert len({t[1] for t in tickets} | {b}) == 256
+assert begin()[0] == INVALID and b"under way" in lib.rnnt_hip_last_error()
+assert all(end(t[1]) == (OK, 0) for t in tickets) and end(b) == (OK, 0)
+assert begin()[0] == OK
+""")
+
+
+def test_a_ticket_belongs_to_its_stream(runtime):
+    run(runtime, r"""
+a = begin(stream=0x10, inputs=(7, 7))[1]
+assert end(a, stream=0x20)[0] == INVALID and end(a)[0] == INVALID
+assert end(a, stream=0x10) == (OK, 1)
+""")
+
+
+def test_a_ticket_is_spent_by_an_end_that_fails(runtime):
+    """A stream that reports an error ends the wait; what is on its way to the slot is not known
+    then, so the slot stays out of use.  Where the stream has run out of work without the check, the
+    slot is free again."""
+    run(runtime, r"""
+a = begin()[1]
+knob("query_error").value = 719
+assert end(a)[0] == HIP_ERROR and knob("last_error").value == 0
+knob("query_error").value = 0
+assert end(a)[0] == INVALID
+others = [begin() for _ in range(255)]
+assert all(t[0] == OK and t[1] != a for t in others) and begin()[0] == INVALID
+for t in others: assert end(t[1]) == (OK, 0)
+knob("lose").value = 1
+for _ in range(300):
+    status, t = begin()
+    assert status == OK and end(t)[0] == HIP_ERROR and b"idle" in lib.rnnt_hip_last_error()
+""")
+
+
+def test_a_capturing_stream_is_refused(runtime):
+    """The verdict of a captured kernel never comes: _end would wait for good."""
+    run(runtime, r"""
+for status in (1, 2):
+    knob("capturing").value = status
+    assert begin()[0] == INVALID and b"captur" in lib.rnnt_hip_last_error()
+assert knob("launches").value == 0
+knob("capturing").value = 0
+assert end(begin()[1]) == (OK, 0)
+knob("capture_error").value = 906         # the null stream while another thread captures
+assert begin()[0] == HIP_ERROR and knob("last_error").value == 0 and knob("launches").value == 1
+""")

@@ -306,14 +306,21 @@ int fill(float* x, float v, int n, hipStream_t s) {
 // host waits: two reductions, two copies and two synchronisations ahead of the first kernel left
 // it idle for 30 to 45 us of every call (B=1 T=500 U=40 V=1000 best path: 252 -> 208 us, a training
 // step of B=4 T=50 U=10 V=32: 199 -> 166).
-// One slot per check under way, a cache line each; a slot is taken from the list by _begin and put back
-// by _end, which only returns once the kernel has written it or the stream has nothing left.
+// One slot per check under way, a cache line of pinned memory each.  _begin takes a slot from the
+// list and opens it; one _end claims it (closes it), and puts it back on the list when nothing can
+// write it any more: the kernel has, or its stream has nothing left.  A slot for which that cannot
+// be told stays off the list.
 constexpr int kCheckSlots = 256, kSlotInts = 16;
 constexpr int kPending = -1, kInputTooLong = 1, kLabelsTooLong = 2;
-std::mutex g_check_mutex;
+struct CheckSlot {
+  bool open = false;
+  int device = 0;  // whose stream it is (a null stream is every device's)
+  hipStream_t stream = nullptr;
+};
+std::mutex g_check_mutex;  // of all of these
 int* g_check_words = nullptr;
+CheckSlot g_check_slots[kCheckSlots];
 int g_check_free[kCheckSlots], g_check_nfree = 0;
-int g_check_device[kCheckSlots];  // whose stream the check went to (a null stream is every device's)
 
 __global__ __launch_bounds__(256) void check_lengths_kernel(const int* __restrict__ inLen,
                                                             const int* __restrict__ labLen, int B,
@@ -1008,6 +1015,14 @@ int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_leng
   hipStream_t s = static_cast<hipStream_t>(stream);
   int slot, device = 0;
   RNNT_HIP(hipGetDevice(&device));
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (const hipError_t e = hipStreamIsCapturing(s, &capture); e != hipSuccess) {
+    (void)hipGetLastError();  // the caller may go on without: no later launch reports this
+    return check_hip(e, "hipStreamIsCapturing", __FILE__, __LINE__);
+  }
+  if (capture != hipStreamCaptureStatusNone)
+    return fail(kInvalid, "check_lengths: the stream is being captured");
+  int* word;
   {
     std::lock_guard<std::mutex> lock(g_check_mutex);
     if (g_check_words == nullptr) {
@@ -1015,7 +1030,7 @@ int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_leng
       const hipError_t e = hipHostMalloc(&p, sizeof(int) * kSlotInts * kCheckSlots,
                                          hipHostMallocPortable | hipHostMallocMapped);
       if (e != hipSuccess) {
-        (void)hipGetLastError();  // the caller may go on without: no later launch reports this
+        (void)hipGetLastError();  // as above
         return check_hip(e, "hipHostMalloc", __FILE__, __LINE__);
       }
       g_check_words = static_cast<int*>(p);
@@ -1025,10 +1040,9 @@ int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_leng
     if (g_check_nfree == 0)
       return fail(kInvalid, "check_lengths: %d checks under way already", kCheckSlots);
     slot = g_check_free[--g_check_nfree];
-    g_check_device[slot] = device;
+    word = g_check_words + (size_t)slot * kSlotInts;
+    __atomic_store_n(word, kPending, __ATOMIC_RELEASE);
   }
-  int* word = g_check_words + (size_t)slot * kSlotInts;
-  __atomic_store_n(word, kPending, __ATOMIC_RELEASE);
   // (the launch's own status: the thread's last error may be somebody else's, left behind before,
   // and says nothing about whether this kernel is going to write the slot)
   void* args[] = {&input_lengths, &label_lengths, &B, &T, &U, &word};
@@ -1041,25 +1055,43 @@ int rnnt_hip_check_lengths_begin(const int* input_lengths, const int* label_leng
     else (void)hipGetLastError();
     return check_hip(launched, "launch check_lengths_kernel", __FILE__, __LINE__);
   }
+  {
+    std::lock_guard<std::mutex> lock(g_check_mutex);
+    g_check_slots[slot].device = device;
+    g_check_slots[slot].stream = s;
+    g_check_slots[slot].open = true;
+  }
   *ticket = slot;
   return kOk;
 }
 
 int rnnt_hip_check_lengths_end(int ticket, rnnt_stream_t stream, int* verdict) {
-  if (!verdict || ticket < 0 || ticket >= kCheckSlots || g_check_words == nullptr)
-    return fail(kInvalid, "check_lengths: no such check");
-  int* word = g_check_words + (size_t)ticket * kSlotInts;
+  if (!verdict) return fail(kInvalid, "check_lengths: null argument");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  int* word;
+  int device;
+  {
+    std::lock_guard<std::mutex> lock(g_check_mutex);
+    CheckSlot* slot = ticket >= 0 && ticket < kCheckSlots ? &g_check_slots[ticket] : nullptr;
+    if (!slot || !slot->open || slot->stream != s)
+      return fail(kInvalid, "check_lengths: no check %d is under way on this stream", ticket);
+    slot->open = false;  // this call's alone from here on
+    device = slot->device;
+    word = g_check_words + (size_t)ticket * kSlotInts;
+  }
   int v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
   // The wait ends with the kernel's word, or when the stream reports an error or that it has
   // run out of work (asked now and then).
   for (unsigned spins = 1; v == kPending; ++spins) {
     if (spins % 4096 == 0) {
-      const hipError_t q = query_on(g_check_device[ticket], static_cast<hipStream_t>(stream));
+      const hipError_t q = query_on(device, s);
       v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
       if (v != kPending) break;
-      // (another thread's capture may forbid the question for a while: that is no answer)
-      if (q == hipSuccess)
+      if (q == hipSuccess) {
+        release_check_slot(ticket);
         return fail(kHipError, "check_lengths: the stream is idle and the check has not run");
+      }
+      // (another thread's capture may forbid the question for a while: that is no answer)
       if (q != hipErrorNotReady && q != hipErrorStreamCaptureUnsupported &&
           q != hipErrorStreamCaptureImplicit)
         return check_hip(q, "check_lengths", __FILE__, __LINE__);
