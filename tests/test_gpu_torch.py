@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import oracle
-from transducer_amd import TransducerLoss
+from transducer_amd import TransducerLoss, torch_binding
 from transducer_amd.synthetic import make_inputs, small_config
 from util import assert_close, reference_vectors
 
@@ -187,7 +187,7 @@ def test_loss_on_a_side_stream_matches_the_default_stream():
 
 
 # the second shape has 19 slabs of frames on few tiles: the prediction-gradient walk splits over
-# frames there, and its arrival counters must be cleared again inside every replay; the last two
+# frames there, in a launch that sums and one that adds the sums up; the last two
 # have 300 and 700 labels: the lattice walks run blocks of the label axis side by side, whose
 # tagged entries must be cleared inside every replay too (and the emission gradients of 700
 # labels add up over several launches)
@@ -228,11 +228,19 @@ def test_fused_entry_points_replay_from_a_captured_graph(shape):
         assert torch.equal(costs, want[0]) and torch.equal(eg, want[1]) and torch.equal(pg, want[2])
 
 
+def no_comparison_made_first(monkeypatch):
+    def fell_back(*args):
+        raise AssertionError("the lengths were compared ahead of the call")
+    monkeypatch.setattr(torch_binding, "_certify_lengths", fell_back)
+
+
 @pytest.mark.parametrize("B", [1, 257])
-def test_lengths_past_the_padded_sizes_are_refused_after_the_work_is_enqueued(B):
+def test_lengths_past_the_padded_sizes_are_refused_after_the_work_is_enqueued(B, monkeypatch):
     """The lengths are compared on the device beside the call's own kernels: the same errors in
     the same order of precedence as a comparison made first, also for the largest integer, and
-    the next call is untouched.  More calls than there are checks that may be under way."""
+    the next call is untouched.  More calls than there are checks that may be under way, none of
+    which falls back to the comparison made first."""
+    no_comparison_made_first(monkeypatch)
     device, gen = torch.device("cuda"), torch.Generator().manual_seed(B)
     E, P = torch.randn(B, 6, 5, generator=gen).to(device), torch.randn(B, 4, 5, generator=gen).to(device)
     labels = torch.randint(1, 5, (B, 3), generator=gen, dtype=torch.int32).to(device)
@@ -257,8 +265,54 @@ def test_lengths_past_the_padded_sizes_are_refused_after_the_work_is_enqueued(B)
     assert torch.equal(criterion.viterbi(E, P, *fit), want[1])
 
 
-def test_lengths_are_checked_on_each_threads_own_stream():
+def test_length_check_tickets_on_the_device():
+    """Every verdict, by the C interface: more checks than there are slots one after the other, all
+    slots under way at once, a ticket that is spent, a stream under capture."""
+    import ctypes
+    from transducer_amd import capi
+    device = torch.device("cuda")
+    lengths = lambda *x: torch.tensor(x, dtype=torch.int32, device=device)
+    fits, over = lengths(1, 6, 0), lengths(6, 7, 1)
+    cases = [((fits, 6, fits, 7), 0), ((over, 6, fits, 7), 1), ((fits, 6, over, 7), 2),
+             ((over, 6, over, 7), 3)]
+    torch.cuda.synchronize()
+
+    def begin(stream, il, T, ll, U):
+        ticket = ctypes.c_int(-1)
+        capi.call("rnnt_hip_check_lengths_begin", ctypes.c_void_p(il.data_ptr()),
+                  ctypes.c_void_p(ll.data_ptr()), 3, T, U, stream, ctypes.byref(ticket))
+        assert ticket.value >= 0
+        return ticket.value
+
+    def end(stream, ticket):
+        verdict = ctypes.c_int(-1)
+        capi.call("rnnt_hip_check_lengths_end", ticket, stream, ctypes.byref(verdict))
+        return verdict.value
+
+    side = torch.cuda.Stream()
+    for stream in (None, ctypes.c_void_p(side.cuda_stream)):
+        for k in range(300):
+            assert end(stream, begin(stream, *cases[k % 4][0])) == cases[k % 4][1]
+        open_ = [begin(stream, *cases[k % 4][0]) for k in range(256)]
+        assert len(set(open_)) == 256
+        with pytest.raises(capi.RnntHipError, match="under way already"):
+            begin(stream, *cases[0][0])
+        assert [end(stream, t) for t in open_] == [cases[k % 4][1] for k in range(256)]
+        with pytest.raises(capi.RnntHipError, match="no check"):
+            end(stream, open_[0])
+    graph, x = torch.cuda.CUDAGraph(), torch.zeros(4, device=device)
+    with torch.cuda.graph(graph):
+        x.add_(1)
+        with pytest.raises(capi.RnntHipError, match="captured"):
+            begin(ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), *cases[0][0])
+    graph.replay()
+    torch.cuda.synchronize()
+    assert x.tolist() == [1, 1, 1, 1]
+
+
+def test_lengths_are_checked_on_each_threads_own_stream(monkeypatch):
     import threading
+    no_comparison_made_first(monkeypatch)
     device, gen = torch.device("cuda"), torch.Generator().manual_seed(3)
     E, P = torch.randn(3, 40, 9, generator=gen).to(device), torch.randn(3, 8, 9, generator=gen).to(device)
     labels = torch.randint(1, 9, (3, 7), generator=gen, dtype=torch.int32).to(device)
