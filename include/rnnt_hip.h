@@ -106,7 +106,9 @@ int rnnt_hip_loss_forward(const float* emissions, const float* predictions, cons
                           int blank, rnnt_stream_t stream);
 
 /* Replaces Transducer.backward (transducer/torch_binding.py:60-90): full egrads[B,T,V] and
- * pgrads[B,U,V] (sparse + dense parts, times deltas[b]); every element is written. */
+ * pgrads[B,U,V] (sparse + dense parts, times deltas[b]); every element is written.  The two may
+ * overlap no other array: egrads holds partial sums of pgrads for a while where the workspace has
+ * no room for them. */
 int rnnt_hip_loss_backward(const float* emissions, const float* predictions, const int* labels,
                            const int* input_lengths, const int* label_lengths,
                            const float* deltas, float* egrads, float* pgrads, void* workspace,

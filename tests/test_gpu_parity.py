@@ -11,7 +11,7 @@ import oracle
 from transducer_amd.synthetic import CONFIGS, make_inputs, small_config
 from util import (DeviceCase, assert_close, assert_same_bits, check_close_reference, gpu_backward, gpu_dense_grads,
                   gpu_forward, gpu_log_norms, gpu_loss, gpu_viterbi, ref_cases, reference_vectors,
-                  vector_case, violations)
+                  ptr, vector_case, violations)
 
 pytestmark = pytest.mark.gpu
 
@@ -813,6 +813,49 @@ def test_pgrads_of_tiles_whose_frames_are_split(T, U):
         # the exponents' rounding, about 2^-21, on every one of the n terms
         assert np.abs(got[b, :m] - (held[b, :m] + w.sum(0))).max() <= 4e-6 * np.abs(w).sum(0).max() + 1e-6
         assert np.array_equal(got[b, m:], held[b, m:])
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("T,U,V", [(2100, 100, 5001), (2049, 40, 12800), (1500, 330, 2000),
+                                   (2049, 130, 10000)])
+def test_pgrads_sums_that_overflow_the_workspace(T, U, V, dtype):
+    """24, 29, 17 and 58 MB of partial sums: 16 of them in the workspace, the next in the dalpha
+    walk's planes (none, one or two chunks), the rest, but in the third shape, in the array of egrads,
+    which is then filled (in the last shape, in 16 bits, by way of the workspace).  Both gradients, twice from one
+    forward pass, are the bits of the unsplit walk (a batch of too many tiles to be split), also
+    into an array one element on from an allocation's start."""
+    import torch
+    from transducer_amd import TransducerLoss, capi
+    dt, gen = getattr(torch, dtype), torch.Generator(device="cuda").manual_seed(T)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").to(dt)
+    E, P = rand(1, T, V), rand(1, U, V)
+    labels = torch.randint(1, V, (1, U - 1), generator=gen, device="cuda", dtype=torch.int32)
+    il, ll = torch.tensor([T - 3], device="cuda").int(), torch.tensor([U - 2], device="cuda").int()
+    one = [x.clone().requires_grad_() for x in (E, P)]
+    cost = TransducerLoss(allow_bf16=True, allow_fp16=True)(*one, labels, il, ll)
+    first = torch.autograd.grad(cost.sum(), one, retain_graph=True)
+    again = torch.autograd.grad(cost.sum(), one)
+    n = 161 // ((V + 127) // 128 * ((U + 127) // 128)) + 1
+    rep = lambda x: x.expand(n, *x.shape[1:]).contiguous()
+    many = [rep(x).requires_grad_() for x in (E, P)]
+    costs = TransducerLoss(allow_bf16=True, allow_fp16=True)(*many, rep(labels), rep(il), rep(ll))
+    unsplit = torch.autograd.grad(costs.sum(), many)
+    assert torch.equal(costs, cost.expand(n))
+    for got, twice, want in zip(first, again, unsplit):
+        assert torch.equal(got, twice)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[0], want[n - 1])
+    suffix = {"float32": "", "bfloat16": "_bf16", "float16": "_f16"}[dtype]
+    nbytes = capi.load().rnnt_hip_loss_workspace_bytes(1, T, U, V)
+    ws, costs = torch.empty(nbytes, dtype=torch.uint8, device="cuda"), torch.empty(1, device="cuda")
+    eg = torch.full((T * V + 2,), 7.0, dtype=dt, device="cuda")
+    pg = torch.empty_like(P)
+    capi.call("rnnt_hip_loss_forward" + suffix, ptr(E), ptr(P), ptr(labels), ptr(il), ptr(ll),
+              ptr(costs), ptr(ws), nbytes, 1, T, U, V, 0, None)
+    capi.call("rnnt_hip_loss_backward" + suffix, ptr(E), ptr(P), ptr(labels), ptr(il), ptr(ll), None,
+              ptr(eg[1:]), ptr(pg), ptr(ws), nbytes, 1, T, U, V, 0, None)
+    torch.cuda.synchronize()
+    assert torch.equal(eg[1:-1].view(1, T, V), first[0]) and torch.equal(pg, first[1])
+    assert eg[0] == 7 and eg[-1] == 7
 
 
 @pytest.mark.parametrize("V", [2, 63, 255, 256, 511, 512])

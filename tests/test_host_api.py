@@ -94,8 +94,8 @@ def test_front_end_refuses_a_blank_outside_the_vocabulary():
 def test_workspace_has_no_BTV_or_BTUV_term():
     """O(B*T*U) lattice planes plus one O(B*U*V) entry (the pieces of exp(P - mP), 6 bytes per
     element of predictions with U rounded up to 32): growing V by dV adds exactly that much, for
-    any T.  Small problems (at most 256 workgroups after splitting a tile's frames) add a bounded
-    scratch for the partial sums of pgrads: at most 256 x 64 KB."""
+    any T.  Where workgroups share a tile's frames, the partial sums of pgrads add a bounded
+    scratch: at most 256 x 64 KB."""
     from transducer_amd import capi
     lib = capi.load()
     f = lib.rnnt_hip_loss_workspace_bytes
@@ -106,6 +106,21 @@ def test_workspace_has_no_BTV_or_BTUV_term():
     for T in (500, 2000):
         extra = f(8, T, 101, 32) - (f(8, T, 101, 4096) - y_bytes(32, 4096))
         assert 0 < extra <= 256 * 64 * 1024 + 4096
+
+
+@pytest.mark.parametrize("B,T,U,V", [(1, 10000, 11, 10000), (1, 6000, 21, 20000),
+                                     (2, 10000, 101, 4000), (8, 2000, 101, 1000),
+                                     (1, 32000, 401, 4000), (4, 600, 33, 5000)])
+def test_workspace_bound_holds_where_frames_of_a_tile_are_shared(B, T, U, V):
+    """9 to 160 tiles of 128 x 128 and many frames: the partial sums of pgrads are a B*T*V term,
+    and the workspace, which is held from forward to backward, holds 16 MB of them at most."""
+    from transducer_amd import capi
+    f = capi.load().rnnt_hip_loss_workspace_bytes
+    up32 = lambda n: (n + 31) // 32 * 32
+    lattice = f(B, T, U, 1) - 6 * B * up32(U) * 32
+    pieces = 6 * B * up32(U) * up32(V)
+    assert f(B, T, U, V) <= lattice + max(pieces, 16 * 2**20) + 4096
+
 
 def test_pybind_module_has_the_reference_keyword_names():
     from transducer_amd import _transducer

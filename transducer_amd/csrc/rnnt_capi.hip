@@ -5,6 +5,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -221,8 +222,10 @@ struct LossWorkspace {
   float *mE, *mP, *LN, *Wn, *Wt, *bsum, *emT;
   WImages img;  // shares its memory with Wn / Wt: a backward call writes one form or the other
   void* lse_scratch;
-  void* psplit;  // pgrads_split_bytes(d) bytes, or null
+  SumsRooms sums;  // of pgrads
 };
+// What the workspace may hold for partial sums of pgrads alone.
+constexpr size_t kOwnSumsBytes = (size_t)16 << 20;
 
 size_t loss_workspace_layout(const Dims& d, void* base, LossWorkspace* w) {
   char* c = static_cast<char*>(base);
@@ -251,9 +254,14 @@ size_t loss_workspace_layout(const Dims& d, void* base, LossWorkspace* w) {
   float* Wt = Wn ? reinterpret_cast<float*>(reinterpret_cast<char*>(Wn) + wb) : nullptr;
   float* bsum = take(sizeof(float) * (size_t)d.B * d.T);
   float* emT = take(btu);  // label-move terms of egrads, [B][U][T]
-  // the Y pieces (forward only) and the partial sums of pgrads (backward only) share memory
-  const size_t yb = lse_scratch_bytes(d), sb = pgrads_split_bytes(d);
-  void* ys = take(yb > sb ? yb : sb);
+  // One piece of memory with three uses after one another on the call's stream: the Y pieces
+  // (forward pass), the first partial sums of pgrads, the fp32 window of 16-bit egrads.  Sums past
+  // its end go where nothing else is wanted any more once W is formed: the dalpha walk's planes
+  // (which every backward pass forms anew), then the array of egrads (both_gradients).  So the
+  // workspace has no B*T*V term for them, however long the utterances.
+  const size_t yb = lse_scratch_bytes(d), sb = std::min(pgrads_sums_bytes(d), kOwnSumsBytes);
+  const size_t shared = yb > sb ? yb : sb;
+  void* ys = take(shared);
   if (base) {
     w->mE = mE; w->mP = mP; w->LN = LN; w->Wn = Wn; w->Wt = Wt; w->bsum = bsum; w->emT = emT;
     if (images) {
@@ -261,9 +269,28 @@ size_t loss_workspace_layout(const Dims& d, void* base, LossWorkspace* w) {
       w->img.p = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(Wn) + ie);
     }
     w->lse_scratch = yb ? ys : nullptr;
-    w->psplit = sb ? ys : nullptr;
+    const size_t plane = (char*)w->planes.dS - (char*)w->planes.wE;
+    w->sums.room[0] = {ys, shared};
+    w->sums.room[1] = {w->planes.wB, 3 * plane};
   }
   return off;
+}
+
+// The two gradient stages of a backward pass.  Where pgrads' partial sums take more room than the
+// workspace has, pgrads goes first and leaves the rest of them in the array that egrads then
+// fills (whole floats inside it).
+template <typename TIO, typename F, typename G>
+int both_gradients(TIO* egrads, const Dims& d, SumsRooms& sums, F egrads_stage, G pgrads_stage) {
+  bool first = false;
+  if (!pgrads_sums_fit(d, sums)) {
+    const uintptr_t lo = (reinterpret_cast<uintptr_t>(egrads) + 3) & ~(uintptr_t)3;
+    const uintptr_t hi = reinterpret_cast<uintptr_t>(egrads + (size_t)d.B * d.T * d.V);
+    if (hi > lo) sums.room[2] = {reinterpret_cast<void*>(lo), hi - lo};
+    first = pgrads_sums_fit(d, sums);
+  }
+  if (first) RNNT_TRY(pgrads_stage());
+  RNNT_TRY(egrads_stage());
+  return first ? kOk : pgrads_stage();
 }
 
 // cost = +inf for every utterance when the padded frame axis is empty (transducer_cpu.cpp:39-41)
@@ -476,14 +503,20 @@ int lowp_loss_backward(const TIO* E, const TIO* P, const int* labels, const int*
   sp.emT = w.emT; sp.bsum = w.bsum; sp.labels = lab;
   SparsePTerms spp;
   spp.gB = w.planes.gB; spp.gL = w.planes.gL; spp.labels = lab;
-  // a label axis of more than one slice: the slices add up in fp32, in the part of the workspace
-  // that held the log-normaliser's Y pieces during the forward pass (free by now)
-  RNNT_STAGE(kEgrads, launch_egrads_stream(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen,
-                                           d, false, sp, s, static_cast<float*>(w.lse_scratch),
-                                           lse_scratch_bytes(d)));
-  RNNT_STAGE(kPgrads, launch_pgrads_stream(E, P, w.mE, w.mP, w.Wt, deltas, pgrads, inLen, labLen,
-                                           d, false, spp, w.psplit, s));
-  return kOk;
+  auto dense = [&]() -> int {
+    // a label axis of more than one slice: the slices add up in fp32, in the part of the workspace
+    // that held the log-normaliser's Y pieces during the forward pass (free by now)
+    RNNT_STAGE(kEgrads, launch_egrads_stream(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen,
+                                             d, false, sp, s, static_cast<float*>(w.lse_scratch),
+                                             lse_scratch_bytes(d)));
+    return kOk;
+  };
+  auto across = [&]() -> int {
+    RNNT_STAGE(kPgrads, launch_pgrads_stream(E, P, w.mE, w.mP, w.Wt, deltas, pgrads, inLen, labLen,
+                                             d, false, spp, w.sums, s));
+    return kOk;
+  };
+  return both_gradients(egrads, d, w.sums, dense, across);
 }
 
 template <typename TIO>
@@ -828,22 +861,25 @@ int rnnt_hip_dense_grads(const float* E, const float* P, float* egrads, float* p
   hipStream_t s = static_cast<hipStream_t>(stream);
   const Dims d = make_dims(B, T, U, V, 0);
   const size_t wb = sizeof(float) * (size_t)B * wplane_tw(T) * wplane_up(U);
+  const size_t sb = pgrads_sums_bytes(d, wb);  // besides Wn, which only egrads reads
   Scratch scratch(s);
   RNNT_TRY(scratch.reserve(align_up(sizeof(float) * (size_t)B * T) +
                            align_up(sizeof(float) * (size_t)B * U) + 2 * align_up(wb) +
-                           align_up(pgrads_split_bytes(d))));
+                           align_up(sb)));
   float* mE = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * T));
   float* mP = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * U));
   float* Wn = static_cast<float*>(scratch.take(wb));
   float* Wt = static_cast<float*>(scratch.take(wb));
-  void* psplit = pgrads_split_bytes(d) ? scratch.take(pgrads_split_bytes(d)) : nullptr;
+  SumsRooms sums;
+  sums.room[0] = {Wn, wb};
+  sums.room[1] = {scratch.take(sb), sb};
   RNNT_STAGE(kRowmax, launch_rowmax(E, mE, (long)B * T, V, T, inLen, 0, s));
   RNNT_STAGE(kRowmax, launch_rowmax(P, mP, (long)B * U, V, U, labLen, 1, s));
   RNNT_STAGE(kWplanes, launch_wplanes(lngrads, LN, mE, mP, Wn, Wt, inLen, labLen, d, s));
   RNNT_STAGE(kEgrads, launch_egrads(E, P, mE, mP, Wn, deltas, egrads, inLen, labLen, d, true,
                                     SparseTerms(), s));
   RNNT_STAGE(kPgrads, launch_pgrads(E, P, mE, mP, Wt, deltas, pgrads, inLen, labLen, d, true,
-                                    SparsePTerms(), psplit, s));
+                                    SparsePTerms(), sums, s));
   return kOk;
 }
 
@@ -936,10 +972,17 @@ int rnnt_hip_loss_backward(const float* E, const float* P, const int* labels, co
                                           inLen, labLen, d, sp, spp, s));
     return kOk;
   }
-  RNNT_STAGE(kEgrads, launch_egrads(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen, d, false,
-                                    sp, s));
-  RNNT_STAGE(kPgrads, launch_pgrads(E, P, w.mE, w.mP, w.Wt, deltas, pgrads, inLen, labLen, d, false,
-                                    spp, w.psplit, s));
+  auto dense = [&]() -> int {
+    RNNT_STAGE(kEgrads, launch_egrads(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen, d,
+                                      false, sp, s));
+    return kOk;
+  };
+  auto across = [&]() -> int {
+    RNNT_STAGE(kPgrads, launch_pgrads(E, P, w.mE, w.mP, w.Wt, deltas, pgrads, inLen, labLen, d,
+                                      false, spp, w.sums, s));
+    return kOk;
+  };
+  RNNT_TRY(both_gradients(egrads, d, w.sums, dense, across));
   if (!fold)
     RNNT_STAGE(kSparse, launch_sparse(w.planes, w.bsum, w.emT, egrads, nullptr, labels, inLen,
                                       labLen, deltas, true, d, s));

@@ -521,14 +521,26 @@ __global__ __launch_bounds__(256, 2) void egrads_stream_kernel(
 
 // Splitting a tile's frames over several workgroups (small grids: one utterance with a small
 // vocabulary is a single tile, whose workgroup would walk all frames alone).  Workgroup c of
-// `chunks` sums slabs [c*per, (c+1)*per) and leaves its sums in `partial`; pgrads_combine_kernel
+// `chunks` sums slabs [c*per, (c+1)*per) and leaves its sums for pgrads_combine_kernel, which
 // adds them up in chunk order and writes the tile.  per == kPsFlush, always: see
 // pgrads_split_plan.
 struct PSplit {
   int chunks = 1, per = 0;
-  float* partial = nullptr;  // [tile][chunk][4 blocks][16 registers][256 threads]
+  int blocks = 0;            // of 32 label positions
+  size_t chunk_floats = 0;   // a chunk's sums: [B][tile of 128 columns][block][16 registers][256 threads]
+  float* base[kSumsRooms] = {};
+  int end[kSumsRooms] = {};  // chunks end[r-1] .. end[r]-1 lie one after the other at base[r]
 };
-constexpr int kPsPartialFloats = 4 * 16 * 256;
+constexpr int kPsBlockFloats = 16 * 256;
+
+__device__ __forceinline__ float* chunk_sums(const PSplit& split, int chunk) {
+  float* base = split.base[0];
+  int first = 0;
+#pragma unroll
+  for (int r = 1; r < kSumsRooms; ++r)
+    if (chunk >= split.end[r - 1]) { base = split.base[r]; first = split.end[r - 1]; }
+  return base + (size_t)(chunk - first) * split.chunk_floats;
+}
 
 // One workgroup's 128 x 128 tile with NMB 32-row blocks of label positions in use (a template
 // parameter, so the matrix instructions of a slice form one straight-line block).  Products are
@@ -539,7 +551,7 @@ __device__ __forceinline__ void pgrads_tile(
     const float* __restrict__ mP, const float* __restrict__ Wt, const float* __restrict__ deltas,
     TIO* __restrict__ pgrads, unsigned short (*As)[3][kPsPlane], float (*Ms)[32], const Dims& d,
     int Up, int Tw, int b, int u0, int Tb, int Ub, const PRowTerms* rt, const PSplit& split,
-    int chunk, int tile) {
+    int chunk, int block0) {
   if (kSplit && NMB == 0) return;  // nothing to sum
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, h = lane >> 5;
   const int vcol = blockIdx.x * 128 + wave * 32 + l32;
@@ -675,7 +687,7 @@ __device__ __forceinline__ void pgrads_tile(
     for (int r = 0; r < 16; ++r) acc[mb][r] += tot[mb][r];
 
   if (kSplit && NMB > 0) {
-    float* mine = split.partial + ((size_t)tile * split.chunks + chunk) * kPsPartialFloats;
+    float* mine = chunk_sums(split, chunk) + (size_t)block0 * kPsBlockFloats;
 #pragma unroll
     for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
@@ -748,8 +760,7 @@ __global__ __launch_bounds__(256, 2) void pgrads_stream_kernel(
   const int b = blockIdx.z;
   const int ut = kSplit ? blockIdx.y / split.chunks : blockIdx.y;
   const int chunk = kSplit ? blockIdx.y - ut * split.chunks : 0;
-  const int utiles = kSplit ? gridDim.y / split.chunks : gridDim.y;
-  const int tile = (b * utiles + ut) * gridDim.x + blockIdx.x;
+  const int block0 = (b * gridDim.x + blockIdx.x) * split.blocks + 4 * ut;
   const int u0 = ut * 128;
   int Tb, Ub;
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
@@ -762,7 +773,7 @@ __global__ __launch_bounds__(256, 2) void pgrads_stream_kernel(
   const int nmb = (u0 < Ub && Tb > 0) ? min(4, (Ub - u0 + 31) >> 5) : 0;  // 32-row blocks in use
 #define RNNT_PG_TILE(NMB)                                                                   \
   pgrads_tile<NMB, kAccumulate, kSplit>(E, P, mE, mP, Wt, deltas, pgrads, As, Ms, d, Up, Tw, \
-                                        b, u0, Tb, Ub, rt, split, chunk, tile)
+                                        b, u0, Tb, Ub, rt, split, chunk, block0)
   switch (nmb) {
     case 0: RNNT_PG_TILE(0); break;
     case 1: RNNT_PG_TILE(1); break;
@@ -786,7 +797,7 @@ __global__ __launch_bounds__(256) void pgrads_combine_kernel(
     SparsePTerms sp, PSplit split) {
   __shared__ PRowTerms Rt;
   const int b = blockIdx.z, ut = blockIdx.y >> 2, mb = blockIdx.y & 3, u0 = ut * 128;
-  const int tile = (b * (gridDim.y >> 2) + ut) * gridDim.x + blockIdx.x;
+  const int block = (b * gridDim.x + blockIdx.x) * split.blocks + blockIdx.y;
   int Tb, Ub;
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
   const bool folding = !kAccumulate && sp.gB != nullptr;
@@ -796,7 +807,6 @@ __global__ __launch_bounds__(256) void pgrads_combine_kernel(
     __syncthreads();
   }
   const int vcol = blockIdx.x * 128 + wave * 32 + l32;
-  if (u0 + 32 * mb >= d.U) return;
   const bool vok = vcol < d.V;
   const int vc = vok ? vcol : d.V - 1;
   const float delta = deltas ? deltas[b] : 1.0f;
@@ -810,15 +820,13 @@ __global__ __launch_bounds__(256) void pgrads_combine_kernel(
     acc[r] = 0.0f;
   }
   if (summed) {
-    const float* src = split.partial + (size_t)tile * split.chunks * kPsPartialFloats +
-                       mb * 16 * 256 + tid;
     // (chunks past the utterance hold zeros)
 #pragma unroll 2
     for (int c = 0; c < split.chunks; ++c) {
+      const float* src = chunk_sums(split, c) + (size_t)block * kPsBlockFloats + tid;
       float x[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        x[r] = __builtin_nontemporal_load(&src[(size_t)c * kPsPartialFloats + r * 256]);
+      for (int r = 0; r < 16; ++r) x[r] = __builtin_nontemporal_load(&src[r * 256]);
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[r] += x[r];
     }
@@ -986,9 +994,9 @@ int launch_egrads_stream(const f16_t* E, const f16_t* P, const float* mE, const 
 // chunks' sums, added in chunk order, then go through exactly the additions the unsplit walk
 // performs, so split and unsplit results are the same bits and an utterance's gradient does
 // not depend on the batch it is computed in.  Split only when the tiles would leave CUs empty: each
-// chunk pays a start-up and 64 KB of sums written and read back.  pgrads in us, unsplit and split:
-// 64 tiles (B=8 T=2000 U=101 V=1000) 106 and 46, 128 (V=2000) 115 and 75, B=4 T=1000 U=201 V=2000 69
-// and 42; 256 (B=16 of the second) 127 and 138, B=32 T=300 U=101 V=1000 35 and 44.  At most 256 MB of
+// chunk pays a start-up and up to 64 KB of sums written and read back.  pgrads in us, unsplit and
+// split: 64 tiles (B=8 T=2000 U=101 V=1000) 106 and 46, 128 (V=2000) 115 and 75, B=4 T=1000 U=201 V=2000
+// 69 and 42; 256 (B=16 of the second) 127 and 138, B=32 T=300 U=101 V=1000 35 and 44.  At most 256 MB of
 // sums (64 tiles of T=10000, B=2 U=101 V=4000, are 160 MB: 523 and 165).
 constexpr long kPsSplitTiles = 160, kPsSplitMost = 4096;
 static void pgrads_split_plan(const Dims& d, int& chunks, int& per) {
@@ -999,14 +1007,34 @@ static void pgrads_split_plan(const Dims& d, int& chunks, int& per) {
   if (chunks < 2 || tiles > kPsSplitTiles || tiles * chunks > kPsSplitMost) chunks = 1;
 }
 
+static size_t pgrads_chunk_floats(const Dims& d) {
+  return (size_t)d.B * ((d.V + 127) / 128) * ((d.U + 31) / 32) * kPsBlockFloats;
+}
+
+// Deals the chunks' sums to the rooms: end[r] = one past the last chunk in room r.  Whether all fit.
+static bool place_chunks(const Dims& d, const SumsRooms& rooms, int chunks, int* end) {
+  const size_t each = pgrads_chunk_floats(d) * sizeof(float);
+  int placed = 0;
+  for (int r = 0; r < kSumsRooms; ++r) {
+    placed += (int)std::min<size_t>(rooms.room[r].bytes / each, chunks - placed);
+    end[r] = placed;
+  }
+  return placed == chunks;
+}
+
 #if RNNT_IN_PART(3)
-size_t pgrads_split_bytes(const Dims& d) {
+bool pgrads_sums_fit(const Dims& d, const SumsRooms& rooms) {
+  if (pgrads_sums_bytes(d) == 0) return true;
+  int chunks, per, end[kSumsRooms];
+  pgrads_split_plan(d, chunks, per);
+  return place_chunks(d, rooms, chunks, end);
+}
+size_t pgrads_sums_bytes(const Dims& d, size_t have) {
   if (d.B == 0 || d.T == 0 || d.U == 0 || d.V == 0) return 0;
   int chunks, per;
   pgrads_split_plan(d, chunks, per);
-  if (chunks <= 1) return 0;
-  const size_t tiles = (size_t)((d.V + 127) / 128) * ((d.U + 127) / 128) * d.B;
-  return tiles * chunks * kPsPartialFloats * sizeof(float);
+  const size_t each = pgrads_chunk_floats(d) * sizeof(float), n = have / each;
+  return chunks > 1 && n < (size_t)chunks ? (chunks - n) * each : 0;
 }
 #endif
 
@@ -1014,21 +1042,23 @@ template <typename TIO>
 static int pgrads_stream_any(const TIO* E, const TIO* P, const float* mE, const float* mP,
                              const float* Wt, const float* deltas, TIO* pgrads, const int* inLen,
                              const int* labLen, const Dims& d, bool accumulate,
-                             const SparsePTerms& sp, void* split_ws, hipStream_t s) {
+                             const SparsePTerms& sp, const SumsRooms& rooms, hipStream_t s) {
   if (sp.gB && accumulate)
     return fail(kInvalid, "sparse-term folding and accumulation are mutually exclusive");
   const int Up = wplane_up(d.U), Tw = wplane_tw(d.T);
   const int vtiles = (d.V + 127) / 128, utiles = (d.U + 127) / 128;
   PSplit split;
-  if (split_ws != nullptr) pgrads_split_plan(d, split.chunks, split.per);
-  if (split.chunks > 1) {
-    split.partial = static_cast<float*>(split_ws);
+  pgrads_split_plan(d, split.chunks, split.per);
+  split.blocks = (d.U + 31) / 32;
+  split.chunk_floats = pgrads_chunk_floats(d);
+  for (int r = 0; r < kSumsRooms; ++r) split.base[r] = static_cast<float*>(rooms.room[r].base);
+  if (split.chunks > 1 && place_chunks(d, rooms, split.chunks, split.end)) {
     // (what the walk would write out is the combining kernel's business: no forms of its own for it)
     const dim3 grid(vtiles, utiles * split.chunks, d.B);
     hipLaunchKernelGGL((pgrads_stream_kernel<false, true, TIO>), grid, dim3(256), 0, s, E, P, mE,
                        mP, Wt, deltas, pgrads, inLen, labLen, d, Up, Tw, sp, split);
     RNNT_LAUNCH_CHECK("pgrads_stream_kernel (split)");
-    const dim3 blocks(vtiles, utiles * 4, d.B);
+    const dim3 blocks(vtiles, split.blocks, d.B);
     if (accumulate)
       hipLaunchKernelGGL((pgrads_combine_kernel<true, TIO>), blocks, dim3(256), 0, s, P, mP, deltas,
                          pgrads, inLen, labLen, d, sp, split);
@@ -1052,30 +1082,30 @@ static int pgrads_stream_any(const TIO* E, const TIO* P, const float* mE, const 
 int launch_pgrads_stream(const float* E, const float* P, const float* mE, const float* mP,
                          const float* Wt, const float* deltas, float* pgrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
-                         const SparsePTerms& sp, void* split_ws,
+                         const SparsePTerms& sp, const SumsRooms& rooms,
                          hipStream_t s) {
   return pgrads_stream_any(E, P, mE, mP, Wt, deltas, pgrads, inLen, labLen, d, accumulate, sp,
-                           split_ws, s);
+                           rooms, s);
 }
 #endif
 #if RNNT_IN_PART(4)
 int launch_pgrads_stream(const bf16_t* E, const bf16_t* P, const float* mE, const float* mP,
                          const float* Wt, const float* deltas, bf16_t* pgrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
-                         const SparsePTerms& sp, void* split_ws,
+                         const SparsePTerms& sp, const SumsRooms& rooms,
                          hipStream_t s) {
   return pgrads_stream_any(E, P, mE, mP, Wt, deltas, pgrads, inLen, labLen, d, accumulate, sp,
-                           split_ws, s);
+                           rooms, s);
 }
 #endif
 #if RNNT_IN_PART(5)
 int launch_pgrads_stream(const f16_t* E, const f16_t* P, const float* mE, const float* mP,
                          const float* Wt, const float* deltas, f16_t* pgrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
-                         const SparsePTerms& sp, void* split_ws,
+                         const SparsePTerms& sp, const SumsRooms& rooms,
                          hipStream_t s) {
   return pgrads_stream_any(E, P, mE, mP, Wt, deltas, pgrads, inLen, labLen, d, accumulate, sp,
-                           split_ws, s);
+                           rooms, s);
 }
 #endif
 

@@ -332,13 +332,24 @@ int launch_egrads(const float* E, const float* P, const float* mE, const float* 
                   const float* Wn, const float* deltas, float* egrads, const int* inLen,
                   const int* labLen, const Dims& d, bool accumulate, const SparseTerms& sparse,
                   hipStream_t s);
-// split_ws: pgrads_split_bytes(d) bytes of scratch that let several workgroups share a tile's
-// frames when the grid is small (null: one workgroup per tile).
-size_t pgrads_split_bytes(const Dims& d);
+// Where the workgroups that share a tile's frames may leave their sums, chunk by chunk: as many whole
+// chunks as fit into the first room, then the next (4-byte aligned; written before they are
+// read).  With less room than pgrads_sums_bytes(d) a tile has one workgroup; the results are the
+// same bits.
+constexpr int kSumsRooms = 3;
+struct SumsRooms {
+  struct Room {
+    void* base = nullptr;
+    size_t bytes = 0;
+  } room[kSumsRooms];
+};
+bool pgrads_sums_fit(const Dims& d, const SumsRooms& rooms);  // (also where there are none)
+// Bytes of room the sums take besides a room of `have` bytes; 0 where frames are not shared.
+size_t pgrads_sums_bytes(const Dims& d, size_t have = 0);
 int launch_pgrads(const float* E, const float* P, const float* mE, const float* mP,
                   const float* Wt, const float* deltas, float* pgrads, const int* inLen,
                   const int* labLen, const Dims& d, bool accumulate, const SparsePTerms& sparse,
-                  void* split_ws, hipStream_t s);
+                  const SumsRooms& rooms, hipStream_t s);
 
 
 // ---------------------------------------------------------------- launchers (rnnt_grads.hip)
@@ -372,17 +383,17 @@ int launch_egrads_stream(const f16_t* E, const f16_t* P, const float* mE, const 
 int launch_pgrads_stream(const float* E, const float* P, const float* mE, const float* mP,
                          const float* Wt, const float* deltas, float* pgrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
-                         const SparsePTerms& sparse, void* split_ws,
+                         const SparsePTerms& sparse, const SumsRooms& rooms,
                          hipStream_t s);
 int launch_pgrads_stream(const bf16_t* E, const bf16_t* P, const float* mE, const float* mP,
                          const float* Wt, const float* deltas, bf16_t* pgrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
-                         const SparsePTerms& sparse, void* split_ws,
+                         const SparsePTerms& sparse, const SumsRooms& rooms,
                          hipStream_t s);
 int launch_pgrads_stream(const f16_t* E, const f16_t* P, const float* mE, const float* mP,
                          const float* Wt, const float* deltas, f16_t* pgrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
-                         const SparsePTerms& sparse, void* split_ws,
+                         const SparsePTerms& sparse, const SumsRooms& rooms,
                          hipStream_t s);
 
 }  // namespace rnnt
