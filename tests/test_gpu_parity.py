@@ -893,6 +893,7 @@ def test_label_terms_of_label_axes_of_several_slices(U, V):
     P = rng.standard_normal((B, U, V), dtype=np.float32)
     labels = rng.integers(0, V, (B, U - 1)).astype(np.int32)
     labels[1] = rng.integers(0, 40, U - 1)
+    labels[1, ::3] = 21
     il, ll = np.array([T, T - 1, 33], np.int32), np.array([U - 1, U - 2, 5], np.int32)
     c = DeviceCase(E, P, labels, il, ll)
     costs, eg, pg = gpu_loss(c)
@@ -903,3 +904,5 @@ def test_label_terms_of_label_axes_of_several_slices(U, V):
     assert_close(costs, want_costs, what="costs")
     assert_close(eg, weg, what="egrads")
     assert_close(pg, wpg, what="pgrads")
+    for _ in range(4):  # the same bits on every call, also where a label meets itself
+        assert_same_bits(gpu_loss(c)[1], eg, "egrads")

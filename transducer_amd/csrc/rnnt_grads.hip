@@ -195,6 +195,16 @@ __device__ __forceinline__ void egrads_walk(
     mu[i] = (sp.labels && m < nmatch) ? match[m] : 0;
     mc[i] = (sp.labels && m < nmatch) ? label_at(sp.labels, d, b, mu[i]) - wave_col0 : -1;
   }
+  // (kBlocks) pairs that are the same label twice: bit i
+  unsigned twins = 0;
+  auto is_twin = [&](int col) {
+    const int other = __shfl_xor(col, 32);  // (by all lanes: one that is off would hand over 0)
+    return __ballot(col >= 0 && other == col) != 0;  // uniform
+  };
+  if constexpr (kBlocks) {
+#pragma unroll
+    for (int i = 0; i < kPre; ++i) twins |= is_twin(mc[i]) ? 1u << i : 0u;
+  }
 
   // bf16 only: with half the bytes the kernel is held by how long a request takes, not by how
   // many bytes move, so a tile's emissions are requested one whole tile before their use
@@ -335,10 +345,19 @@ __device__ __forceinline__ void egrads_walk(
         // label axes of several slices (400 labels and 1000 columns put a dozen into every block):
         // the terms are added up in a 32 x 32 block in LDS, a label to each half of the wavefront
         // at a time and nothing waited for, and a lane takes its column's sixteen frames from
-        // there once; the first fourteen are asked for before the matrix block.  All slices of
-        // egrads at B=8 T=10000 U=401 V=1000 1026 -> 934 us, B=4 T=2000 U=300 V=2000 145 -> 126; with
-        // one slice there are few labels a block, and filling and reading it costs more than it
-        // saves (B=32 T=2000 U=101 V=1000: 197 -> 213).
+        // there once; the first fourteen are asked for before the matrix block.  The order of the
+        // additions is the order of the pairs: LDS takes a wavefront's instructions one after the
+        // other, and a pair of the same label, whose halves would meet at one address within an
+        // instruction, is added up first and goes in from the lower half alone (13 us of the 4754 of
+        // a training step of B=8 T=10000 U=400 V=1000).  All slices of egrads at B=8 T=10000 U=401
+        // V=1000 1026 -> 934 us before that, B=4 T=2000 U=300 V=2000 145 -> 126; with one slice there are
+        // few labels a block, and filling and reading it costs more than it saves (B=32 T=2000 U=101
+        // V=1000: 197 -> 213).
+        auto add_pair = [&](int col, float x, bool twin) {
+          if (twin) x += __shfl_xor(x, 32);
+          if (col >= 0 && row_ok && !(twin && h))
+            unsafeAtomicAdd(&block[col * kEsBlockPitch + l32], x);
+        };
         if (nmatch > 0) {
 #pragma unroll
           for (int k = 0; k < (32 * kEsBlockPitch / 4 + 63) / 64; ++k)
@@ -348,8 +367,7 @@ __device__ __forceinline__ void egrads_walk(
           __builtin_amdgcn_wave_barrier();
 #pragma unroll
           for (int i = 0; i < kPre; ++i)
-            if (2 * i < nmatch && mc[i] >= 0 && row_ok)
-              unsafeAtomicAdd(&block[mc[i] * kEsBlockPitch + l32], sd[i]);
+            if (2 * i < nmatch) add_pair(mc[i], sd[i], (twins >> i) & 1u);
           constexpr int kBatch = 4;
           for (int i0 = 2 * kPre; i0 < nmatch; i0 += 2 * kBatch) {
             float term[kBatch];
@@ -361,9 +379,7 @@ __device__ __forceinline__ void egrads_walk(
               col[k] = m < nmatch ? label_at(sp.labels, d, b, u) - wave_col0 : -1;
             }
 #pragma unroll
-            for (int k = 0; k < kBatch; ++k)
-              if (col[k] >= 0 && row_ok)
-                unsafeAtomicAdd(&block[col[k] * kEsBlockPitch + l32], term[k]);
+            for (int k = 0; k < kBatch; ++k) add_pair(col[k], term[k], is_twin(col[k]));
           }
           __builtin_amdgcn_wave_barrier();
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
