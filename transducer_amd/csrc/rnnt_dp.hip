@@ -87,11 +87,11 @@ __device__ inline float softplus_fast(float d) { return log1p_unit(exp_neg(d)); 
 // evaluations (a few ulp of lf), the second the rounding of d * log2(e) ahead of v_exp_f32,
 // whose effect on the result grows with |d|.  The bound is not taken from data sheets: the
 // fast value is compared with the exact one for EVERY float d <= 0 (rnnt_hip_lse_bound_check,
-// run by the tests on the device itself).  Measured on gfx950, in units of 2^-23 lf: at most 2.1
-// for |d| <= 1.5, 3.6 up to 4, 5.7 up to 8, 0.91 (2.1 + 0.65 |d|) beyond; the constants leave a
-// tenth on top of that.  They are what decides how often a wavefront of the alpha walk takes the
-// library path (its chance per lane is twice the bound / the sum's spacing), so they are not
-// rounder than that: with 5 and 1.25 the walk of B=32 T=2000 U=100 was a tenth slower.
+// run by the tests on the device itself).  Measured on gfx950, the largest distance as a share of
+// the bound: 0.84 for |d| <= 1.5, 0.87 up to 4, 0.90 from there to 87, 0.50 beyond; the tests let it be
+// 0.95.  The constants are what decides how often a wavefront of the alpha walk takes the library
+// path (its chance per lane is twice the bound / the sum's spacing), so they are not rounder than
+// that: with 5 and 1.25 the walk of B=32 T=2000 U=100 takes 255 us instead of 226.
 constexpr float kFastRelA = 2.1f * 0x1p-23f;
 constexpr float kFastRelB = 0.65f * 0x1p-23f;
 // The bound for fast value lf at argument d.  The clamp keeps 0 * inf out of it at d = -inf;
@@ -2409,7 +2409,7 @@ __global__ __launch_bounds__(256) void libm_probe_kernel(const float* __restrict
 }  // namespace
 
 namespace {
-// For every float d with bit pattern in [lo, hi] (d <= 0): does the bound of lse2_checked cover
+// For every float d with bit pattern in [lo, hi] (d <= 0): does the bound of lse2_fast cover
 // the distance between the fast and the library value of log1p(exp(d))?  out[0] counts the
 // patterns where it does not, out[1] keeps the largest ratio distance / bound (as float bits;
 // ratios are non-negative, so their bit patterns order like integers).
