@@ -331,8 +331,8 @@ int fill(float* x, float v, int n, hipStream_t s) {
 // Do the lengths fit the padded arrays?  The answer goes to a word of pinned host memory that the
 // caller looks at after it has enqueued the rest of the call, so the device has work while the
 // host waits: two reductions, two copies and two synchronisations ahead of the first kernel left
-// it idle for 30 to 45 us of every call (B=1 T=500 U=40 V=1000 best path: 252 -> 208 us, a training
-// step of B=4 T=50 U=10 V=32: 199 -> 166).
+// it idle for 30 to 45 us of every call (B=1 T=500 U=40 V=1000 best path: 252 -> 208 us; the forward
+// half of a training step of B=4 T=50 U=10 V=32, on the host: 91 -> 43 to 63 us).
 // One slot per check under way, a cache line of pinned memory each.  _begin takes a slot from the
 // list and opens it; one _end claims it (closes it), and puts it back on the list when nothing can
 // write it any more: the kernel has, or its stream has nothing left.  A slot for which that cannot
