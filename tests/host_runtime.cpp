@@ -1,7 +1,8 @@
-// A stand-in for the few HIP runtime calls that the length check of librnnt_hip.so makes, for
-// tests without a device.  Loaded with RTLD_GLOBAL ahead of the library, so that the library binds
-// to it.  A launch is kept until its (device, stream) has been asked about `delay` times; only
-// then does "the kernel" write its verdict.  The test sets the knobs below.
+// A stand-in for the HIP runtime calls that the C entry points of librnnt_hip.so make, for tests
+// without a device.  Loaded with RTLD_GLOBAL ahead of the library, so that the library binds to it.
+// A launch of the length check is kept until its (device, stream) has been asked about `delay`
+// times; only then does "the kernel" write its verdict.  Other kernels must be launched with
+// `lose` set: nothing runs, and device pointers are never looked at.  The test sets the knobs below.
 #include <stdint.h>
 #include <stdlib.h>
 
@@ -50,6 +51,8 @@ int query_error = 0;    // what hipStreamQuery returns instead of an answer
 int capturing = 0;      // hipStreamCaptureStatus of every stream
 int capture_error = 0;  // what hipStreamIsCapturing returns instead
 int lose = 0;           // launches are accepted and never run
+uint64_t pool_limit = UINT64_MAX;  // the largest allocation a memory pool grants
+uint64_t pool_last = 0;            // the last one it granted
 
 int hipGetDevice(int* d) { *d = current_device; return 0; }
 int hipSetDevice(int d) { current_device = d; return 0; }
@@ -59,6 +62,18 @@ int hipStreamIsCapturing(void*, int* status) {
   *status = capturing;
   return capture_error ? last_error = capture_error : 0;
 }
+
+int hipMemPoolCreate(void** pool, const void*) { *pool = &pool_limit; return 0; }
+int hipMemPoolSetAttribute(void*, int, void*) { return 0; }
+int hipMallocFromPoolAsync(void** p, size_t n, void*, void*) {
+  if (n > pool_limit) return last_error = 2;  // hipErrorOutOfMemory
+  pool_last = n;
+  *p = reinterpret_cast<void*>(uintptr_t{1} << 40);
+  return 0;
+}
+int hipFreeAsync(void*, void*) { return 0; }
+int hipGetSymbolAddress(void** p, const void*) { *p = reinterpret_cast<void*>(uintptr_t{1} << 32); return 0; }
+int hipFuncSetAttribute(const void*, int, int) { return 0; }
 
 int __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, void* stream) {
   pushed = Call{grid, block, lds, stream};

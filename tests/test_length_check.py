@@ -1,5 +1,5 @@
 """The host side of rnnt_hip_check_lengths_begin / _end, on a stand-in for the HIP runtime
-(length_check_runtime.cpp): which device is asked, which tickets are honoured, what becomes of a
+(host_runtime.cpp): which device is asked, which tickets are honoured, what becomes of a
 slot when something fails.  No device is needed; the kernel itself is tested in test_gpu_torch.py."""
 import os
 import subprocess
@@ -39,7 +39,7 @@ OK, INVALID, HIP_ERROR = 0, 1, 2
 def runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("runtime") / "libruntime.so")
     subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-o", out,
-                           os.path.join(HERE, "length_check_runtime.cpp")])
+                           os.path.join(HERE, "host_runtime.cpp")])
     return out
 
 

@@ -144,6 +144,15 @@ class Scratch {
     size_ = bytes;
     return kOk;
   }
+  // The same for `bytes` and, if they are to be had, `extra` more (*got) that the call is faster with.
+  int reserve(size_t bytes, size_t extra, bool* got) {
+    *got = true;
+    if (extra == 0) return reserve(bytes);
+    if (reserve(bytes + extra) == kOk) return kOk;
+    (void)hipGetLastError();  // the caller goes on without: no later launch reports this
+    *got = false;
+    return reserve(bytes);
+  }
   // what an allocation of this many bytes leaves in a fixed region, rounded down to whole pieces
   size_t room(size_t bytes) const {
     if (!fixed_) return ~(size_t)0;
@@ -384,17 +393,25 @@ hipError_t query_on(int device, hipStream_t s) {
   return e;
 }
 
-// Scratch the best-path stages need (planes, the two max-plus planes, the decision table).
-// `plan`: how this call builds its table of best labels (asked once per call, so that what is
-// reserved and what is taken agree whatever another thread sets).
-size_t viterbi_scratch_bytes(const Dims& d, const MaxplusPlan& plan) {
+// Scratch the best-path stages need besides their plan's (planes, the two max-plus planes, the
+// decision table).  The plan, how this call builds its table of best labels, is asked for once per
+// call, so that what is reserved and what is taken agree whatever another thread sets.
+size_t viterbi_scratch_bytes(const Dims& d) {
   const size_t plane = sizeof(float) * (size_t)d.B * d.Ua * d.Dp + 64;
-  return align_up(planes_bytes(d, true)) + 2 * align_up(plane) +
-         align_up(viterbi_bits_bytes(d)) +
-         align_up(plan.bytes);
+  return align_up(planes_bytes(d, true)) + 2 * align_up(plane) + align_up(viterbi_bits_bytes(d));
 }
 
-// `scratch` has viterbi_scratch_bytes(d, plan) left to take (one allocation per call, made by the caller
+// Reserves `base` bytes and what the plan takes.  Ranges of columns are given up where there is no
+// memory for their table (up to 64 MB).
+int reserve_for(Scratch& scratch, size_t base, MaxplusPlan* plan) {
+  if (plan->lists) return scratch.reserve(base + align_up(plan->bytes));
+  bool got;
+  RNNT_TRY(scratch.reserve(base, align_up(plan->bytes), &got));
+  if (!got) *plan = MaxplusPlan();
+  return kOk;
+}
+
+// `scratch` has viterbi_scratch_bytes(d) and plan.bytes left to take (one allocation per call, made by the caller
 // together with whatever else it needs: the allocator calls are a visible part of a small decode).
 // With `ready`, the lattice planes were carved by the caller and already hold LN and the blank
 // scores (the log-normaliser left them there): no transposing copy, no gather.
@@ -535,10 +552,10 @@ int lowp_viterbi_decode(const TIO* E, const TIO* P, const int* inLen, const int*
   if (!lse_stream_supported(E, d)) return fail(kInvalid, "%s: B*T*U too large", who);
   Scratch scratch(s);
   const size_t yb = lse_scratch_bytes(d);
-  const MaxplusPlan plan = maxplus_plan(d);
-  RNNT_TRY(scratch.reserve(align_up(sizeof(float) * (size_t)B * T) +
-                           align_up(sizeof(float) * (size_t)B * U) + align_up(yb) +
-                           viterbi_scratch_bytes(d, plan)));
+  MaxplusPlan plan = maxplus_plan(d);
+  RNNT_TRY(reserve_for(scratch, align_up(sizeof(float) * (size_t)B * T) +
+                       align_up(sizeof(float) * (size_t)B * U) + align_up(yb) +
+                       viterbi_scratch_bytes(d), &plan));
   float* mE = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * T));
   float* mP = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * U));
   void* ys = scratch.take(yb);
@@ -569,9 +586,9 @@ int decode_fp32(const float* E, const float* P, const int* inLen, const int* lab
   // (no row-major LN, no transposing copy, no gather)
   const size_t base = align_up(sizeof(float) * (size_t)B * T) +
                       align_up(sizeof(float) * (size_t)B * U) + align_up(yb) +
-                      viterbi_scratch_bytes(d, MaxplusPlan());
-  const MaxplusPlan plan = maxplus_plan(d, scratch.room(base));
-  RNNT_TRY(scratch.reserve(base + align_up(plan.bytes)));
+                      viterbi_scratch_bytes(d);
+  MaxplusPlan plan = maxplus_plan(d, scratch.room(base));
+  RNNT_TRY(reserve_for(scratch, base, &plan));
   float* mE = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * T));
   float* mP = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * U));
   void* ys = scratch.take(yb);
@@ -674,9 +691,9 @@ int rnnt_hip_maxplus_table(const float* E, const float* P, const int* inLen, con
   hipStream_t s = static_cast<hipStream_t>(stream);
   const Dims d = make_dims(B, T, U, V, blank);
   const size_t plane = sizeof(float) * (size_t)d.B * d.Ua * d.Dp + 64;
-  const MaxplusPlan plan = maxplus_plan(d);
+  MaxplusPlan plan = maxplus_plan(d);
   Scratch scratch(s);
-  RNNT_TRY(scratch.reserve(2 * align_up(plane) + align_up(plan.bytes)));
+  RNNT_TRY(reserve_for(scratch, 2 * align_up(plane), &plan));
   float* bestS = static_cast<float*>(scratch.take(plane));
   int* argS = static_cast<int*>(scratch.take(plane));
   void* table = plan.bytes ? scratch.take(plan.bytes) : nullptr;
@@ -827,8 +844,8 @@ int rnnt_hip_viterbi(const float* E, const float* P, const float* LN, int* label
   const Dims d = make_dims(B, T, U, V, blank);
   hipStream_t s = static_cast<hipStream_t>(stream);
   Scratch scratch(s);
-  const MaxplusPlan plan = maxplus_plan(d);
-  RNNT_TRY(scratch.reserve(viterbi_scratch_bytes(d, plan)));
+  MaxplusPlan plan = maxplus_plan(d);
+  RNNT_TRY(reserve_for(scratch, viterbi_scratch_bytes(d), &plan));
   return viterbi_impl(E, P, LN, labels, inLen, labLen, d, scratch, s, plan);
 }
 
@@ -863,16 +880,17 @@ int rnnt_hip_dense_grads(const float* E, const float* P, float* egrads, float* p
   const size_t wb = sizeof(float) * (size_t)B * wplane_tw(T) * wplane_up(U);
   const size_t sb = pgrads_sums_bytes(d, wb);  // besides Wn, which only egrads reads
   Scratch scratch(s);
+  bool got;
   RNNT_TRY(scratch.reserve(align_up(sizeof(float) * (size_t)B * T) +
-                           align_up(sizeof(float) * (size_t)B * U) + 2 * align_up(wb) +
-                           align_up(sb)));
+                           align_up(sizeof(float) * (size_t)B * U) + 2 * align_up(wb),
+                           align_up(sb), &got));
   float* mE = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * T));
   float* mP = static_cast<float*>(scratch.take(sizeof(float) * (size_t)B * U));
   float* Wn = static_cast<float*>(scratch.take(wb));
   float* Wt = static_cast<float*>(scratch.take(wb));
   SumsRooms sums;
   sums.room[0] = {Wn, wb};
-  sums.room[1] = {scratch.take(sb), sb};
+  if (got) sums.room[1] = {scratch.take(sb), sb};
   RNNT_STAGE(kRowmax, launch_rowmax(E, mE, (long)B * T, V, T, inLen, 0, s));
   RNNT_STAGE(kRowmax, launch_rowmax(P, mP, (long)B * U, V, U, labLen, 1, s));
   RNNT_STAGE(kWplanes, launch_wplanes(lngrads, LN, mE, mP, Wn, Wt, inLen, labLen, d, s));
