@@ -574,7 +574,7 @@ def main():
     walks_ms = per_launch.get("alpha", 0.0) + per_launch.get("beta", 0.0)
     if walks_ms > mfma_kernels[dom]:
         a = chain["alpha"]
-        roofline = {"bound": "chain-latency", "kernel": "alpha_kernel",
+        roofline = {"bound": "chain-latency", "kernel": "alpha_walk_kernel",
                     "achieved": a["ns_per_step"], "peak": a["floor_ns_per_step"],
                     "unit": "ns/step (lower is better; frac = peak / achieved)",
                     "frac": a["frac"], "traffic": None,

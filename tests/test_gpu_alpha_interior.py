@@ -33,6 +33,34 @@ def test_alphas_where_the_interior_begins_and_ends(T, U):
     assert_same_bits(costs, want_costs, "costs")
 
 
+@pytest.mark.parametrize("U", [65, 128, 193, 256, 520])
+@pytest.mark.parametrize("T", [191, 253, 256, 517])
+def test_alphas_where_the_hand_over_between_wavefronts_wraps(T, U):
+    """What crosses from one wavefront to the next goes through rings of 256 steps: lattices of
+    about that many steps and of several times as many, utterances that end in any of the
+    wavefronts or blocks, one of them with scores so large that a step's proof never fails and one
+    with scores so small that it nearly always does."""
+    V = 5
+    il = [T, T - 1, T - 2, T - 3, T, max(T - 60, 1)]
+    ll = [U - 1, U // 2, min(64, U - 1), 0, U - 1, min(63, U - 1)]
+    B = len(il)
+    rng = np.random.default_rng(7000 * T + U)
+    E = rng.standard_normal((B, T, V), dtype=np.float32)
+    P = rng.standard_normal((B, U, V), dtype=np.float32)
+    E[1] *= 40.0
+    E[4] *= 0.01
+    P[4] *= 0.01
+    labels = rng.integers(1, V, (B, U - 1)).astype(np.int32)
+    il, ll = np.array(il, np.int32), np.array(ll, np.int32)
+    LN = oracle.log_norms_naive(E, P, il, ll)
+    want_costs, want = oracle.forward(E, P, LN, labels, il, ll)
+    costs, alphas = gpu_forward(DeviceCase(E, P, labels, il, ll), np.nan_to_num(LN))
+    for b in range(B):
+        got, ref = alphas[b, :il[b], :ll[b] + 1], want[b, :il[b], :ll[b] + 1]
+        assert_same_bits(got, ref, "alphas of utterance %d" % b)
+    assert_same_bits(costs, want_costs, "costs")
+
+
 @pytest.mark.parametrize("U", [1, 2, 63, 64, 65, 130])
 @pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 70])
 def test_dalphas_where_groups_of_four_meet_the_lattices_edges(T, U):

@@ -34,6 +34,7 @@
 namespace rnnt {
 
 int live_blocks(const Dims& d, int* waves);
+int alpha_blocks(const Dims& d);
 
 namespace {
 
@@ -94,16 +95,17 @@ __device__ inline float softplus_fast(float d) { return log1p_unit(exp_neg(d)); 
 // that: with 5 and 1.25 the walk of B=32 T=2000 U=100 takes 255 us instead of 226.
 constexpr float kFastRelA = 2.1f * 0x1p-23f;
 constexpr float kFastRelB = 0.65f * 0x1p-23f;
-// The bound for fast value lf at argument d.  The clamp keeps 0 * inf out of it at d = -inf;
-// the added 2^-125 covers d below -87.3, where the library's value is a subnormal number and
-// the hardware units return 0.
+// The bound for fast value lf at argument d.  The clamp to 1 (free: an output modifier of the
+// multiply-add) keeps 0 * inf out of it at d = -inf; the added 2^-125 covers d below -87.3, where the
+// library's value is a subnormal number and the hardware units return 0.
 __device__ inline float fast_bound(float lf, float d) {
-  return __builtin_fmaf(lf, __builtin_fmaf(-kFastRelB, fmaxf(d, -256.0f), kFastRelA), 0x1p-125f);
+  const float rel = __builtin_fmaf(fabsf(d), kFastRelB, kFastRelA);
+  return __builtin_fmaf(lf, fminf(rel, 1.0f), 0x1p-125f);
 }
 
 // transducer/transducer_cpu.cpp:16-24 with the C library's own expf and log1pf (rnnt_libm.h):
 // the same bits as the reference's CPU backend for every pair of operands.
-__device__ inline float lse2_libm(float a, float b, const unsigned long long* tab) {
+__device__ __forceinline__ float lse2_libm(float a, float b, const unsigned long long* tab) {
   // One operand -inf: |a - b| = inf, expf gives 0, log1pf(0) = 0 and the sum is the other
   // operand exactly, as the reference's early returns have it; only both -inf needs a guard.
   const float hi = a > b ? a : b;
@@ -142,20 +144,6 @@ __device__ inline FastLse lse2_fast(float a, float b) {
   r.up = hi + (lf + e);
   return r;
 }
-__device__ inline float lse2_checked(float a, float b, const unsigned long long* tab) {
-  const FastLse r = lse2_fast(a, b);
-  // (all lanes take the library's value then: it is what the others hold already)
-  return __builtin_amdgcn_ballot_w64(!(r.lo == r.up)) ? lse2_libm(a, b, tab) : r.lo;
-}
-
-// The same on the hardware units alone (no check): for the chain-latency probe.
-__device__ inline float lse2(float a, float b) {
-  // One operand -inf: |a - b| = inf, exp gives 0, log1p(0) = 0 and the sum is the other operand
-  // exactly, as the reference's early returns have it; only both -inf (inf - inf) needs a guard.
-  const float hi = fmaxf(a, b);
-  const float r = hi + log1p_unit(exp_neg(-fabsf(a - b)));
-  return (hi == kNegInf) ? kNegInf : r;
-}
 
 // Raises the device's trouble flag.  A store to GLOBAL memory by its address space: through a
 // generic pointer it would be a flat instruction, which may go to LDS as well, and with one of
@@ -177,7 +165,8 @@ __device__ inline int bounded_wait(const int* counter, int have, int need, int s
                                    int* __restrict__ trouble) {
   int spins = 0;
   while (have < need) {
-    have = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    have = __builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
     asm volatile("" ::: "memory");
     if (have < need) {
       if (spins++ >= spin_limit) {
@@ -387,15 +376,11 @@ __global__ __launch_bounds__(256) void gather_cells_kernel(const TIO* __restrict
 // cases (:49-60), also when that operand is -inf (both operands are then -inf and the library
 // path returns -inf).  Cells past the utterance (t >= T_b, u >= U_b) hand on the same and are
 // never read by a valid cell.
+// This kernel takes several label positions a lane: label axes past 256 positions that
+// alpha_walk_kernel (one a lane, below) does not take side by side.
 // W > 1: the label positions are dealt to W wavefronts of one workgroup (wavefront w owns
 // positions [64 C w, 64 C (w+1))), because the walk is bound by how fast ONE wavefront issues
-// the instructions of a cell: 28, two of them at a quarter of the rate, then about 25 per group of
-// four steps for loads, store and hand-over (interior groups, below).  Measured with B=8 T=2000, one
-// cell a lane: 95 ns a step on one wavefront (64 positions), 117 on two or four (101, 256);
-// 151, 165 and 162 while every step tested its bounds, every load formed a 64-bit address and the
-// proof of the fast log-sum-exp took twelve instructions.  Of the 117, 77 are left with the proof
-// and its branch compiled out (wrong bits, timing only); the library path itself is taken in 2 % of
-// the steps (60 of 2100) and costs a tenth.  The only value that crosses
+// the instructions of its cells.  The only value that crosses
 // a wavefront boundary is the label-move score of the boundary cell, one float per step: the
 // lower wavefront leaves it in an LDS array indexed by step and then publishes how far it has
 // got; the upper one runs a few groups behind, so it finds its inputs there without waiting and
@@ -408,47 +393,24 @@ __global__ __launch_bounds__(256) void gather_cells_kernel(const TIO* __restrict
 // null for the last block) and the next one reads them from `ghin` (null for the first block).
 // kMulti: this launch is one of several blocks (the hand-over code is compiled in only then: in
 // the single-block kernel even an unused hand-over load costs the walk its prefetch distance).
-// kLive (with kMulti): the live_n blocks of 64 C W positions of a label axis run at the same
-// time, as live_n workgroups on as many CUs of one XCD (with few utterances and many label
-// positions one CU's wavefronts are what holds the walk).  The scores of a boundary column then
-// cross in `live` (live_n - 1 arrays of [B][hand_stride] 64-bit words, zero before the launch):
-// entry s is the score entering step s with s + 1 in its upper half, so that a reader can tell
-// a written entry by itself -- one store, no fence, no separate counter.  A block asks for the
-// entries of the block below it four groups ahead like every other operand (lane j for entry
-// 4g + j), checks the tags when it comes to use them, and asks again (bounded, like the waits
-// inside a workgroup) if the block below has not got there yet; it starts kLiveLag groups
-// behind it, so that in the steady state what it asks for has long been written.  Workgroups
-// are dispatched in launch order and a block has a smaller index than the block above it, so
-// the block that is waited for is always running or done.
-constexpr int kLiveLag = 12;
+constexpr int kLiveLag = 12;      // groups between blocks that the best-path walk runs side by side
 constexpr int kBetaLiveLag = 24;  // (the dalpha walk asks eight groups ahead, not four)
 constexpr int kLiveWaveLag = 2;  // groups between the wavefronts of a live block at the start (8 elsewhere)
-template <int C, int W, bool kMulti, bool kLive = false>
+template <int C, int W, bool kMulti>
 __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __restrict__ inLen,
                                                        const int* __restrict__ labLen,
                                                        float* __restrict__ costs, Dims d,
                                                        int hand_stride, int spin_limit,
                                                        int* __restrict__ trouble, int u_base,
                                                        const float* __restrict__ ghin,
-                                                       float* __restrict__ ghout,
-                                                       unsigned long long* __restrict__ live,
-                                                       int live_n) {
-  static_assert(kMulti || !kLive, "live blocks are blocks");
+                                                       float* __restrict__ ghout) {
   extern __shared__ __attribute__((aligned(16))) float hand[];  // [W-1][hand_stride]: entry s =
                                                                 // score handed to step s
   __shared__ int done[W];          // steps a wavefront has published
   __shared__ __attribute__((aligned(16))) float nothing[4];
   __shared__ unsigned long long etab[32];  // expf's table (rnnt_libm.h)
-  // live blocks: workgroups go round the 8 XCDs in launch order; ids i, i + 8, i + 16 .. share
-  // one, and with it the L2 the boundary scores cross in.  Eight utterances take 8 live_n
-  // consecutive ids, block by block, lowest block first.
-  const int live_block = kLive ? (int)(blockIdx.x >> 3) % live_n : 0;
-  const int b = kLive ? (int)(blockIdx.x / (8 * live_n)) * 8 + (blockIdx.x & 7) : blockIdx.x;
+  const int b = blockIdx.x;
   const int lane = threadIdx.x & 63;
-  if (kLive) {
-    if (b >= d.B) return;
-    u_base = live_block * 64 * C * W;
-  }
   const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   int Tb, Ub;
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
@@ -462,40 +424,9 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
   const int u0 = u_base + (wave * 64 + lane) * C;
   const int gstride = plane_group_stride(d);
   const bool first_column = u_base == 0 && wave == 0;  // lane 0 owns the lattice's column u = 0
-  const float* gin = (kMulti && !kLive && ghin) ? ghin + (size_t)b * hand_stride : nullptr;
-  float* gout = (kMulti && !kLive && ghout) ? ghout + (size_t)b * hand_stride : nullptr;
+  const float* gin = (kMulti && ghin) ? ghin + (size_t)b * hand_stride : nullptr;
+  float* gout = (kMulti && ghout) ? ghout + (size_t)b * hand_stride : nullptr;
   if (kMulti && gout && threadIdx.x == 0) gout[0] = kOutside;  // nothing enters step 0
-  // live blocks: block h reads the entries of boundary h - 1 and writes those of boundary h
-  // (live_n - 1 arrays of [B][hand_stride] entries; the lowest block asks at its own boundary,
-  // for nothing)
-  const bool live_in = kLive && live_block > 0, live_out = kLive && live_block < live_n - 1;
-  const unsigned long long* lrow =
-      kLive ? live + ((size_t)max(live_block - 1, 0) * d.B + b) * hand_stride : nullptr;
-  unsigned long long* lrow_out =
-      kLive ? live + ((size_t)min(live_block, max(live_n - 2, 0)) * d.B + b) * hand_stride
-            : nullptr;
-  auto live_entry = [](int s, float x) -> unsigned long long {
-    return ((unsigned long long)(unsigned)(s + 1) << 32) | (unsigned long long)__float_as_uint(x);
-  };
-  auto live_load = [&](int s) -> unsigned long long {
-    return __hip_atomic_load(lrow + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  // Asking again for an entry that was not there yet: the load and its wait are one opaque
-  // statement, so that the compiler's count of the loads in flight in the walk's main loop (the
-  // operands of the next four groups) stays exact -- a loop around a load it knows of makes it
-  // wait for all of them at every use.
-  auto live_reload = [&](int s) -> unsigned long long {
-    unsigned long long e;
-    const unsigned long long* q = lrow + s;
-    asm volatile("global_load_dwordx2 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)"
-                 : "=&v"(e)
-                 : "v"(q)
-                 : "memory");
-    return e;
-  };
-  if (live_out && threadIdx.x == 0)  // nothing enters step 0
-    __hip_atomic_store(lrow_out, live_entry(0, kOutside), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
   exp2_table_to_lds(etab);
   if (W > 1) {
     if (threadIdx.x < W) done[threadIdx.x] = 0;
@@ -561,7 +492,6 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
     float4 ln[C], el[C];
     float eb[C + 3];
     float4 gh;  // scores entering the block's first column from the block below
-    unsigned long long lv;  // the same, tagged, from the block running beside this one: lane j holds entry 4g + j
   };
   auto load_group = [&](int g) -> Group {
     Group r;
@@ -575,18 +505,10 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
     if constexpr (kMulti) {
       r.gh = make_float4(kOutside, kOutside, kOutside, kOutside);
       if (gin) r.gh = *reinterpret_cast<const float4*>(gin + 4 * g);  // uniform
-      if constexpr (kLive) {
-        // every wavefront of both blocks asks (only wavefront 0 of the upper block takes the
-        // answer): a load under a condition would have its result copied, hence waited for,
-        // right where it is asked for -- and so would a load from an address all lanes share,
-        // which the compiler moves to scalar registers at once
-        r.lv = live_load(4 * g + (lane & 3));
-      }
     }
     return r;
   };
 
-  unsigned live_sink = 0;
   int avail = 0;  // steps the wavefront below is known to have published
   auto wait_for = [&](int need) {
     // LDS serves a wavefront's requests in order, so no hardware fence is needed on either
@@ -624,37 +546,6 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
       f4set(hin, j, (first_column && (kInterior || 4 * g + j < Tb)) ? kNegInf : kOutside);
     if constexpr (kMulti) {
       if (gin) hin = cur.gh;  // wavefront 0: from the block below
-      if constexpr (kLive) {
-        // Wavefront 0 of the upper block takes what it asked for: lanes 0 .. 3 hold the four
-        // entries and check their tags.  Every other wavefront folds the answer into a word
-        // that is looked at once, at the very end: a result nobody reads would have its
-        // registers reused at once, and that reuse waits for the load.
-        if (live_in && wave == 0) {  // uniform
-          unsigned long long e = cur.lv;
-          if (__builtin_amdgcn_ballot_w64(lane < 4 &&
-                                          (unsigned)(e >> 32) != (unsigned)(4 * g + lane + 1))) {
-            // An entry was not written when it was asked for: the lower block is closer than it
-            // should be.  Let it get kLiveLag groups ahead again (or finish) before going on --
-            // asking only for what is missing would leave this block right behind it, late at
-            // every group.  Lanes 0 .. 3 ask for their entries again, the others for the far one.
-            const int mine = lane < 4 ? 4 * g + lane : min(4 * ngroups, 4 * (g + kLiveLag));
-            int spins = 0;
-            do {
-              if (spins++ >= spin_limit) {
-                if (lane == 0) raise_trouble(trouble);
-                break;
-              }
-              __builtin_amdgcn_s_sleep(4);
-              e = live_reload(mine);
-            } while (__builtin_amdgcn_ballot_w64((unsigned)(e >> 32) != (unsigned)(mine + 1)));
-          }
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            f4set(hin, j, __int_as_float(__builtin_amdgcn_readlane((int)(unsigned)e, j)));
-        } else {
-          live_sink ^= (unsigned)cur.lv;
-        }
-      }
     }
     if constexpr (W > 1) {
       if (kInterior && !kMulti) hin = hand_cur;
@@ -713,14 +604,6 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
 #pragma unroll
         for (int j = 0; j < 4; ++j) gout[4 * g + 1 + j] = gsend[j];
       }
-      if constexpr (kLive) {
-        if (live_out && wave == W - 1 && lane == 63) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            __hip_atomic_store(lrow_out + 4 * g + 1 + j, live_entry(4 * g + 1 + j, gsend[j]),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
     }
     if (W > 1 && wave < W - 1 && lane == 63) {  // entries 4g+1 .. 4g+4, then the progress
 #pragma unroll
@@ -732,22 +615,9 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
   // four register sets rotate (no copies): a group's loads are requested four groups (16
   // steps, more than a microsecond) ahead -- the planes of a long batch do not fit L2
   auto clamp_g = [&](int g) { return g < ngroups ? g : ngroups - 1; };
-  if constexpr (kLive) {
-    if (live_in && wave == 0) {  // the upper block starts kLiveLag groups behind (or when the lower is done)
-      const int far = min(4 * ngroups, 4 * kLiveLag);
-      int spins = 0;
-      while ((unsigned)(live_load(far) >> 32) != (unsigned)(far + 1)) {
-        if (spins++ >= spin_limit) {
-          if (lane == 0) raise_trouble(trouble);
-          break;
-        }
-        __builtin_amdgcn_s_sleep(8);
-      }
-    }
-  }
   Group q0 = load_group(0), q1 = load_group(clamp_g(1)), q2 = load_group(clamp_g(2)),
         q3 = load_group(clamp_g(3));
-  if (W > 1 && wave > 0) wait_for(min(4 * ngroups, 4 * (kLive ? kLiveWaveLag : 8) * wave));  // fall a few groups behind
+  if (W > 1 && wave > 0) wait_for(min(4 * ngroups, 4 * 8 * wave));  // fall a few groups behind
   const std::true_type whole, interior;
   const std::false_type partial, edge;
   auto load_inner = [&](int g) -> Group {
@@ -765,7 +635,6 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
     if constexpr (kMulti) {
       r.gh = make_float4(kOutside, kOutside, kOutside, kOutside);
       if (gin) r.gh = *reinterpret_cast<const float4*>(gin + 4 * g);  // uniform
-      if constexpr (kLive) r.lv = live_load(4 * g + (lane & 3));
     }
     return r;
   };
@@ -806,11 +675,454 @@ __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __re
 #pragma unroll
   for (int c = 0; c < C; ++c)
     if (u0 + c == Ub - 1) costs[b] = -stay[c];
-  if constexpr (kLive) {
-    if (spin_limit < 0 && live_sink == 1u) raise_trouble(trouble);  // never
+}
+
+// ------------------------------------------------------------------ hand-over between wavefronts
+// A lattice walk deals 64 neighbouring label positions to a wavefront, one a lane.  The one value
+// a step that crosses from a wavefront to the next goes through a ring in LDS, four steps (a
+// "quad") at a time: entry g of boundary w is what wavefront w takes in for group g.  prog[w + 1]
+// counts the groups wavefront w has handed on; prog[w] is what it may take, and prog[w + 2] says
+// how far the taker of its own quads has got, so a quad is overwritten only once it has been read.
+// Wavefronts that have no neighbour on a side find kForever there.
+// Every lane writes the quad, lane `from` into the ring and the others into a dump that nobody
+// reads: a branch around the write would cost the walk 5.4 ns, whether taken or not, and switching
+// lanes off and on again as much.  A group's quad is written during the next group, after the
+// operands of that group's hand-over have arrived: LDS answers a wavefront in order, and a write
+// right ahead of a wait for a read would be waited for as well.
+constexpr int kRingGroups = 64;   // a power of two and a multiple of four
+constexpr int kForever = 0x3fffffff;
+// entries of 64 bits per utterance and boundary of blocks that run side by side: the value of a
+// step and the step + 1 above it, so that a reader can tell a written entry by itself -- one store,
+// no fence, no separate counter
+__device__ inline unsigned long long live_entry(int s, float x) {
+  return ((unsigned long long)(unsigned)(s + 1) << 32) | (unsigned long long)__float_as_uint(x);
+}
+__device__ inline int prog_load(const int* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline void prog_store(int* p, int x) {
+  __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// The wavefront beside the walking ones of a block that runs side by side with others: brings what
+// the block before it has left in memory (`src`) into the ring of the first walking wavefront, and
+// takes what the last one hands on out to `dst`, up to sixteen quads at a time.  It keeps the
+// tagged entries, their waits and their addresses out of the walk.  at(g, i): the step of value
+// i = 0..3 of group g.  Groups are numbered in walking order, n of them on either side.  Bounded
+// like every wait here: when nothing has moved for spin_limit turns it raises the trouble flag and
+// lets everybody go on with whatever the rings hold.
+template <typename At>
+__device__ inline void live_carrier(const unsigned long long* __restrict__ src,
+                                    unsigned long long* __restrict__ dst, int n, At at,
+                                    float* ring_in, int* prog_in, const int* prog_first,
+                                    const float* ring_out, const int* prog_last, int* prog_out,
+                                    int spin_limit, int* __restrict__ trouble) {
+  const int lane = threadIdx.x & 63, quad = lane >> 2;
+  int in = src ? 0 : n, out = dst ? 0 : n, idle = 0;
+  while (in < n || out < n) {
+    bool moved = false;
+    if (out < n) {
+      const int have = min(prog_load(prog_last), n) - out;
+      asm volatile("" ::: "memory");
+      if (have > 0) {
+        const int g = out + quad, m = min(have, 16);
+        if (quad < m) {
+          const float x = ring_out[4 * (g & (kRingGroups - 1)) + (lane & 3)];
+          const int s = at(g, lane & 3);
+          if (s >= 0) __hip_atomic_store(dst + s, live_entry(s, x), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+        }
+        out += m;
+        asm volatile("" ::: "memory");
+        if (lane == 0) prog_store(prog_out, out);
+        moved = true;
+      }
+    }
+    if (in < n) {
+      const int room = min(prog_load(prog_first) + kRingGroups - 4, n) - in;
+      if (room > 0) {
+        const int g = in + quad, m = min(room, 16);
+        const int s = at(min(g, n - 1), lane & 3);
+        const unsigned long long e =
+            __hip_atomic_load(src + max(s, 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool here = quad < m && (s < 0 || (unsigned)(e >> 32) == (unsigned)(s + 1));
+        const unsigned long long missing = __builtin_amdgcn_ballot_w64(!here);
+        const int ready = missing ? __builtin_ctzll(missing) >> 2 : 16;
+        if (ready > 0) {
+          if (quad < ready)
+            ring_in[4 * (g & (kRingGroups - 1)) + (lane & 3)] = __uint_as_float((unsigned)e);
+          in += ready;
+          asm volatile("" ::: "memory");  // (LDS serves a wavefront's requests in order)
+          if (lane == 0) prog_store(prog_in, in);
+          moved = true;
+        }
+      }
+    }
+    if (moved) {
+      idle = 0;
+    } else if (idle++ >= spin_limit) {
+      if (lane == 0) {
+        raise_trouble(trouble);
+        prog_store(prog_in, kForever);
+        prog_store(prog_out, kForever);
+      }
+      return;
+    } else {
+      __builtin_amdgcn_s_sleep(2);
+    }
   }
 }
 
+// ------------------------------------------------------------------ alpha, one position a lane
+// One cell on the fast path of lse2_fast and the two moves out of it, in an order of its own: a
+// lone wavefront issues an instruction every four cycles (1.67 ns), dependent or not, exp and log
+// take two turns, and a branch on a mask that was compared just before it stalls for 6 ns.  So what
+// counts is the number of instructions -- 25, fifteen for the sum, four for its proof, six for the
+// moves -- and that the comparison stands ahead of the moves.  Between a transcendental and the use of its result,
+// and between the last write of `emit` and the lane shift that follows this block, stand the
+// independent instructions the hardware asks for.
+struct AlphaCell {
+  float a, stay, emit;
+  unsigned long long fail;  // lanes whose sum is not proven to be the library's
+};
+__device__ inline AlphaCell alpha_cell(float left, float stay, float eb, float el, float pb,
+                                       float pl, float ln) {
+  AlphaCell r;
+  float t, y, k, w, l, hi;
+  asm volatile(
+      "v_sub_f32_e32 %[t], %[left], %[stay]\n\t"
+      "v_mul_f32_e64 %[y], |%[t]|, %[nl2e]\n\t"
+      "v_exp_f32_e32 %[y], %[y]\n\t"
+      "v_max_f32_e32 %[hi], %[left], %[stay]\n\t"
+      "v_fma_f32 %[k], |%[t]|, %[relb], %[rela] clamp\n\t"
+      "v_add_f32_e32 %[w], 1.0, %[y]\n\t"
+      "v_log_f32_e32 %[l], %[w]\n\t"
+      "v_add_f32_e32 %[w], -1.0, %[w]\n\t"
+      "v_fma_f32 %[t], %[y], -0.5, 1.0\n\t"
+      "v_sub_f32_e32 %[w], %[y], %[w]\n\t"
+      "v_mul_f32_e32 %[t], %[w], %[t]\n\t"
+      "v_fmac_f32_e32 %[t], 0x3f317218, %[l]\n\t"         // log1p(exp(-|left - stay|))
+      "v_fmaak_f32 %[k], %[t], %[k], 0x01000000\n\t"      // its bound (fast_bound)
+      "v_sub_f32_e32 %[w], %[t], %[k]\n\t"
+      "v_add_f32_e32 %[t], %[t], %[k]\n\t"
+      "v_add_f32_e32 %[a], %[hi], %[w]\n\t"
+      "v_add_f32_e32 %[hi], %[hi], %[t]\n\t"
+      "v_cmp_neq_f32_e64 %[fail], %[a], %[hi]\n\t"
+      "v_add_f32_e32 %[em], %[el], %[a]\n\t"
+      "v_add_f32_e32 %[st], %[eb], %[a]\n\t"
+      "v_add_f32_e32 %[em], %[pl], %[em]\n\t"
+      "v_sub_f32_e32 %[em], %[em], %[ln]\n\t"
+      "v_add_f32_e32 %[st], %[pb], %[st]\n\t"
+      "v_sub_f32_e32 %[st], %[st], %[ln]"
+      : [a] "=&v"(r.a), [st] "=&v"(r.stay), [em] "=&v"(r.emit), [fail] "=&s"(r.fail), [t] "=&v"(t),
+        [y] "=&v"(y), [k] "=&v"(k), [w] "=&v"(w), [l] "=&v"(l), [hi] "=&v"(hi)
+      : [left] "v"(left), [stay] "v"(stay), [eb] "v"(eb), [el] "v"(el), [pb] "v"(pb), [pl] "v"(pl),
+        [ln] "v"(ln), [nl2e] "s"(-1.44269504088896341f), [relb] "s"(kFastRelB),
+        [rela] "v"(kFastRelA));
+  return r;
+}
+
+typedef float quad_t __attribute__((ext_vector_type(4)));
+typedef float quad4_t __attribute__((ext_vector_type(4), aligned(4)));
+// A piece of memory addressed as a buffer: an access takes a lane's own constant offset and a scalar
+// one that walks, and no address is formed in vector registers.
+struct Buffer {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ Buffer(const void* p, size_t bytes) {
+    int n = (int)(unsigned)bytes, flags = 0x00020000;
+    // (opaque: words that several descriptors have in common would be copied around at every use)
+    asm volatile("" : "+s"(n), "+s"(flags));
+    r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, n, flags);
+  }
+  __device__ quad_t load(unsigned lane_off, unsigned off) const {
+    return __builtin_bit_cast(quad_t, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, 0));
+  }
+  __device__ void store(unsigned lane_off, unsigned off, quad_t x) const {
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, lane_off, off, 0);
+  }
+};
+
+// The walk of one utterance with one label position a lane: W wavefronts of 64 positions; kLive:
+// live_n such blocks of the label axis at the same time, as many workgroups on as many CUs of one
+// XCD, with a wavefront more that carries the scores between them (live_carrier).  Workgroups are
+// dispatched in launch order and a block has a smaller index than the block above it, so the block
+// that is waited for is always running or done.
+// A step is 25 instructions, the lane shift, a branch (5.4 ns, whether taken or not) and 40
+// instructions per group of four for operands, hand-over and progress: 59 ns measured on one
+// wavefront, 65 with a neighbour.  A step with a lane whose sum is not proven takes about 0.3 us
+// more (the chance falls with the size of the alphas: nearly every step up to 100 or so, one in
+// ten at 1000, one in a hundred at 10000).  Whole walks, B=8 T=2000: 85 ns a step at 51 positions, 92
+// at 101 (93 and 111 with 29 instructions, the comparison right ahead of its branch, whole
+// hand-over arrays in LDS whose writes the next group waited for); B=8 T=10000, 401
+// positions 84 (128 with the entries between blocks asked for and checked inside the walk).
+template <int W, bool kLive>
+__global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
+    Planes p, const int* __restrict__ inLen, const int* __restrict__ labLen,
+    float* __restrict__ costs, Dims d, int spin_limit, int* __restrict__ trouble,
+    unsigned long long* __restrict__ live, int live_n) {
+  constexpr bool kHand = W > 1 || kLive;
+  __shared__ __attribute__((aligned(16))) float ring[W + 1][kHand ? 4 * kRingGroups : 4];
+  __shared__ __attribute__((aligned(16))) float nothing[16];
+  __shared__ __attribute__((aligned(16))) float dump[kHand ? 4 * 64 + 16 : 4];
+  __shared__ int prog[W + 2];
+  __shared__ unsigned long long etab[32];  // expf's table (rnnt_libm.h)
+  // live blocks: workgroups go round the 8 XCDs in launch order; ids i, i + 8, i + 16 .. share
+  // one, and with it the L2 the boundary scores cross in.  Eight utterances take 8 live_n
+  // consecutive ids, block by block, lowest block first.
+  const int live_block = kLive ? (int)(blockIdx.x >> 3) % live_n : 0;
+  const int b = kLive ? (int)(blockIdx.x / (8 * live_n)) * 8 + (blockIdx.x & 7) : blockIdx.x;
+  if (kLive && b >= d.B) return;
+  const int u_base = live_block * 64 * W;
+  const int lane = threadIdx.x & 63;
+  const int wave = (W > 1 || kLive) ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  int Tb, Ub;
+  utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
+  if (Tb == 0 || Ub == 0) {  // :39-41
+    if (threadIdx.x == 0 && u_base == 0) costs[b] = kPosInf;
+    return;
+  }
+  if (u_base >= Ub) return;  // a block past this utterance's labels: nobody reads what it would leave
+  const int nsteps = Tb + Ub - 1;
+  const int ngroups = (nsteps + 3) >> 2;
+  // a block below and a block above this one (for this utterance)
+  const bool live_in = kLive && live_block > 0;
+  const bool live_out = kLive && live_block < live_n - 1 && u_base + 64 * W < Ub;
+  exp2_table_to_lds(etab);
+  if (threadIdx.x < 16) nothing[threadIdx.x] = kNegInf;
+  if (threadIdx.x < W + 2) {
+    const int w = (int)threadIdx.x - 1;  // the wavefront whose progress this is
+    prog[threadIdx.x] = w < 0 ? (live_in ? 0 : kForever)
+                        : w == W ? (live_out ? 0 : kForever)
+                                 : (u_base + 64 * w < Ub ? 0 : kForever);
+  }
+  __syncthreads();
+  if (kLive && wave == W) {
+    const unsigned long long* src =
+        live_in ? live + ((size_t)(live_block - 1) * d.B + b) * d.Dp : nullptr;
+    unsigned long long* dst = live_out ? live + ((size_t)live_block * d.B + b) * d.Dp : nullptr;
+    // what enters step s: value i of group g is what enters step 4g + 1 + i (nothing enters step 0)
+    live_carrier(src, dst, ngroups, [](int g, int i) { return 4 * g + 1 + i; }, ring[0], &prog[0],
+                 &prog[1], ring[W], &prog[W], &prog[W + 1], spin_limit, trouble);
+    return;
+  }
+  const int u_lo = u_base + wave * 64;
+  if (u_lo >= Ub) return;  // a wavefront past this utterance's labels
+  if (kLive) __builtin_amdgcn_s_setprio(3);  // ahead of the carrier on the same SIMD
+  const int u = u_lo + lane;
+  const bool real = u < Ub;
+  const bool first_column = u_lo == 0;  // lane 0 owns the lattice's column u = 0
+  // Operands of a position past the utterance's last one are the last one's (its label score the
+  // last label's), and its moves carry kOutside on top: whatever it meets is an ordinary number
+  // far below any alpha, so that the interior groups below need no test for it.
+  // (loaded in every lane: a branch here would leave the uniform sizes behind it in vector registers)
+  float pb = p.pb[(size_t)b * d.Ua + u], pl = p.pl[(size_t)b * d.Ua + u];  // u < Ua
+  asm volatile("" : "+v"(pb), "+v"(pl));
+  pb = real ? pb : kOutside;
+  pl = real ? pl : kOutside;
+  const unsigned tlim = real ? (unsigned)Tb : 0u;
+  // :43 alpha[0,0] = 0: cell (0,0) finds 0 coming up from below and nothing from the left
+  float stay = u == 0 ? 0.0f : kNegInf, emit = kOutside, final = 0.0f;
+
+  // Interior groups [in_lo, in_hi): step 4g is past the first frame of the wavefront's last
+  // position, step 4g + 3 not past the last frame of its first one.
+  const unsigned gbytes = kLive ? 16u * (unsigned)d.Ua : 1024u * W;  // from a group to the next
+  const int in_lo = (min(u_lo + 64, Ub) + 2) >> 2;
+  const int in_hi = Ub > 1 ? min((Tb + u_lo) >> 2, ngroups - 1) : 0;
+  // The planes as buffers that begin at group `origin` of the utterance (moved on before an offset
+  // would outgrow 32 bits).  E[t,blank] of step s, lane by lane, sits at eb[Eo + s - u].
+  const size_t plane = (size_t)gbytes * (unsigned)(d.Dp / 4);
+  const char* ln_b = reinterpret_cast<const char*>(p.lnS + plane_group0(d, b, 0));
+  const char* el_b = reinterpret_cast<const char*>(p.elS + plane_group0(d, b, 0));
+  char* a_b = reinterpret_cast<char*>(p.aS + plane_group0(d, b, 0));
+  const Buffer eb_q(p.eb + (size_t)b * d.Tp, 4ull * d.Tp);
+  Buffer ln_q(ln_b, plane), el_q(el_b, plane), a_q(a_b, plane);
+  int origin = 0;
+  const int span = (int)((1u << 30) / gbytes);
+  auto move_on = [&](int g) {
+    origin = g;
+    const size_t by = (size_t)g * gbytes;
+    ln_q = Buffer(ln_b + by, plane - by);
+    el_q = Buffer(el_b + by, plane - by);
+    a_q = Buffer(a_b + by, plane - by);
+  };
+  const unsigned ln_o = 16u * (unsigned)min(u, Ub - 1);
+  const unsigned el_o = 16u * (unsigned)max(min(u, Ub - 2), 0);
+  const unsigned a_o = 16u * (unsigned)u;
+  const unsigned eb_o = 4u * (unsigned)(d.Eo - min(u, Ub - 1));
+  struct Ops {
+    quad_t ln, el, eb;
+  };
+  auto load = [&](int g) -> Ops {
+    const unsigned by = (unsigned)(g - origin) * gbytes;
+    Ops r;
+    r.ln = ln_q.load(ln_o, by);
+    r.el = el_q.load(el_o, by);
+    r.eb = eb_q.load(eb_o, 16u * (unsigned)g);
+    return r;
+  };
+  auto load_to_end = [&](int g) -> Ops { return load(min(g, ngroups - 1)); };
+
+  // ---- hand-over
+  int ok = kHand ? -1 : kForever;  // groups up to here may run without looking at the neighbours
+  int have_in = 0, have_out = 0;
+  // before groups g and g + 1, which ask for the quads up to g + 2 and write those up to g + 1
+  auto refresh = [&](int g) {
+    have_in = bounded_wait(&prog[wave], have_in, min(g + 5, ngroups), spin_limit, trouble);
+    have_out = bounded_wait(&prog[wave + 2], have_out, g + 18 - kRingGroups, spin_limit, trouble);
+    ok = min(have_in >= ngroups ? kForever : have_in - 3,
+             min(have_out, kForever) + kRingGroups - 4);
+  };
+  const float* take = kHand ? (first_column ? nothing : ring[wave]) : nullptr;
+  const int take_mask = first_column ? 0 : kRingGroups / 4 - 1;
+  float* give = kHand ? (lane == 63 ? ring[wave + 1] : dump + 4 * lane) : nullptr;
+  const int give_mask = lane == 63 ? kRingGroups / 4 - 1 : 0;
+  int* give_prog = lane == 63 ? &prog[wave + 1] : reinterpret_cast<int*>(dump + 4 * lane);
+  quad_t pend = {kOutside, kOutside, kOutside, kOutside};  // what the last group handed on
+  quad_t hand = {kNegInf, kNegInf, kNegInf, kNegInf};      // what enters the running group
+  float carry = first_column ? kNegInf : kOutside;         // ... and its first step
+
+  // A group: hands on what the last one left, asks for what the next one takes in, four steps.
+  // kInner: an interior group, which needs no bounds.  At the lattice's edges every cell is asked
+  // whether it is inside, and the blank move out of a position's last cell stays in `final`.
+  auto run_group = [&](int g, const Ops& q, const float* take_next, float* give_last, auto tell,
+                       auto inner) {
+    constexpr bool kTell = decltype(tell)::value, kInner = decltype(inner)::value;
+    quad_t next = hand;
+    if constexpr (kHand) {
+      *reinterpret_cast<quad_t*>(give_last) = pend;
+      asm volatile("" ::: "memory");  // (LDS serves a wavefront's requests in order)
+      if constexpr (kTell) prog_store(give_prog, g);
+      next = *reinterpret_cast<const quad_t*>(take_next);
+    }
+    float in[4] = {carry, hand[0], hand[1], hand[2]};
+    unsigned long long inside[4];
+    if constexpr (!kHand || !kInner) {
+      if constexpr (!kHand) in[0] = in[1] = in[2] = in[3] = kNegInf;
+      if constexpr (!kInner) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          // a cell of the lattice: 0 <= t = s - u < T_b (one unsigned comparison)
+          inside[j] = __builtin_amdgcn_ballot_w64((unsigned)(4 * g + j - u) < tlim);
+          // what enters the lattice's own first column: nothing, which is -inf while its cells are
+          // inside the lattice (:49-52 adds nothing there, so a -inf blank score must come out as
+          // -inf) and kOutside once they are past the last frame (see kOutside)
+          if (first_column && 4 * g + j >= Tb) in[j] = kOutside;
+        }
+      }
+      // (set well ahead of the lane shifts that fill lane 0 from them)
+      asm volatile("" : "+v"(in[0]), "+v"(in[1]), "+v"(in[2]), "+v"(in[3]));
+    }
+    quad_t a;
+    quad_t em;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float left = wave_shr1(emit, in[j]);
+      const AlphaCell c = alpha_cell(left, stay, q.eb[j], q.el[j], pb, pl, q.ln[j]);
+      float x = c.a, sb = c.stay, se = c.emit;
+      if (__builtin_expect(c.fail != 0ull, 0)) {
+        x = lse2_libm(left, stay, etab);
+        sb = x + q.eb[j];
+        sb = sb + pb;
+        sb = sb - q.ln[j];
+        se = x + q.el[j];
+        se = se + pl;
+        se = se - q.ln[j];
+      }
+      if constexpr (kInner) {
+        stay = sb;
+        emit = se;
+      } else {
+        const bool is = __builtin_amdgcn_inverse_ballot_w64(inside[j]);
+        final = is ? sb : final;
+        stay = is ? sb : kNegInf;
+        emit = is ? se : kOutside;
+      }
+      a[j] = x;
+      em[j] = emit;
+    }
+    a_q.store(a_o, (unsigned)(g - origin) * gbytes, a);
+    pend = em;
+    carry = hand[3];
+    hand = next;
+  };
+
+  // four sets of operands rotate: a group's loads are requested four groups (16 steps, more than a
+  // microsecond) ahead -- the planes of a long batch do not fit L2
+  Ops q0 = load_to_end(0), q1 = load_to_end(1), q2 = load_to_end(2), q3 = load_to_end(3);
+  if constexpr (kHand) {
+    if (!first_column) {
+      refresh(0);
+      hand = *reinterpret_cast<const quad_t*>(take);
+    }
+  }
+  const std::true_type yes;
+  const std::false_type no;
+  int g = 0;
+  auto block = [&](auto inner) {
+    constexpr bool kInner = decltype(inner)::value;
+    const float *tk = nullptr, *tk_next = nullptr;
+    float *gv = nullptr, *gv_last = nullptr;
+    if constexpr (kHand) {
+      tk = take + 16 * ((g >> 2) & take_mask);
+      tk_next = take + 16 * (((g >> 2) + 1) & take_mask);
+      gv = give + 16 * ((g >> 2) & give_mask);
+      gv_last = give + 16 * (((g >> 2) - 1) & give_mask) + 12;
+      if (__builtin_expect(g > ok, 0)) refresh(g);
+    }
+    auto ahead = [&](int k) -> Ops {
+      if constexpr (kInner) return load(g + 4 + k);
+      return load_to_end(g + 4 + k);
+    };
+    run_group(g, q0, tk + 4, gv_last, yes, inner);
+    q0 = ahead(0);
+    run_group(g + 1, q1, tk + 8, gv, no, inner);
+    q1 = ahead(1);
+    if constexpr (kHand) {
+      if (__builtin_expect(g + 2 > ok, 0)) refresh(g + 2);
+    }
+    run_group(g + 2, q2, tk + 12, gv + 4, yes, inner);
+    q2 = ahead(2);
+    run_group(g + 3, q3, tk_next, gv + 8, no, inner);
+    q3 = ahead(3);
+    // everything LDS was asked for is there by now; said here, the head of the next block need not
+    // wait for what it has itself just asked for
+    if constexpr (kHand) __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    g += 4;
+  };
+  while (g + 4 < ngroups) {
+    if (g - origin >= span) move_on(g);
+    if (g >= in_lo && g + 4 <= in_hi && g + 8 <= ngroups) {
+      const int end = min(min(in_hi, ngroups - 4), origin + span);
+      do block(yes);
+      while (g + 4 <= end);
+    } else {
+      block(no);
+    }
+  }
+  // the last one to four groups
+  while (g < ngroups) {
+    const float* tk = nullptr;
+    float* gv = nullptr;
+    if constexpr (kHand) {
+      tk = take + 16 * (((g + 1) >> 2) & take_mask) + 4 * ((g + 1) & 3);
+      gv = give + 16 * (((g - 1) >> 2) & give_mask) + 4 * ((g - 1) & 3);
+      if (__builtin_expect(g > ok, 0)) refresh(g);
+    }
+    run_group(g, q0, tk, gv, yes, no);
+    q0 = q1;
+    q1 = q2;
+    q2 = q3;
+    ++g;
+  }
+  if constexpr (kHand) {
+    *reinterpret_cast<quad_t*>(give + 16 * (((ngroups - 1) >> 2) & give_mask) + 4 * ((ngroups - 1) & 3)) = pend;
+    asm volatile("" ::: "memory");
+    prog_store(give_prog, ngroups);
+  }
+  // :73-78 the blank move out of the last cell, negated
+  if (u == Ub - 1) costs[b] = -final;
+}
 
 // ------------------------------------------------------------------ transition weights
 // Everything of the dalpha recursion that does not depend on dalpha itself
@@ -2351,9 +2663,9 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
 // ------------------------------------------------------------------ chain-latency floor
 // What ONE step of a lattice walk costs when nothing but its dependent chain is left: operands
 // in registers, no loads, no stores, no bookkeeping, one wavefront alone on its SIMD.
-//   kind 0: a cell of alpha_kernel -- DPP hand-over, log-sum-exp on the hardware units with
-//           the check that its sum is the C library's (lse2_checked; the operands are large, so
-//           no lane falls back), then the three additions of a move;
+//   kind 0: a cell of alpha_walk_kernel -- DPP hand-over, log-sum-exp on the hardware units with
+//           the check that its sum is the C library's (alpha_cell; the operands are large, so no lane
+//           falls back), the additions of its two moves;
 //   kind 1: a cell of beta_kernel -- DPP hand-over, two multiplies and an add;
 //   kind 2: kind 0 with every lane on the library path (rnnt_libm.h: ~100 instructions, two of
 //           them divisions): what a step costs while any lane of the wavefront falls back.
@@ -2367,26 +2679,37 @@ __global__ __launch_bounds__(64) void chain_floor_kernel(float* __restrict__ sin
   __syncthreads();
   const int lane = threadIdx.x;
   float stay = -5000.0f - 0.37f * lane, emit = -5000.0f - 0.61f * lane, dcol = 1.0f / (1 + lane);
-#pragma unroll 4
-  for (int s = 0; s < steps; ++s) {
+  auto step = [&]() {
     if (kKind != 1) {
       const float left = wave_shr1(emit, kOutside);
-      const float a = kKind == 0 ? lse2_checked(left, stay, etab) : lse2_libm(left, stay, etab);
-      float sb = a + e;
-      sb = sb + p;
-      sb = sb - ln;
-      float se = a + p;
-      se = se + e;
-      se = se - ln;
-      stay = sb;
-      emit = se;
+      AlphaCell c = alpha_cell(left, stay, e, p, p, e, ln);
+      if (kKind == 2 || __builtin_expect(c.fail != 0ull, 0)) {
+        const float a = lse2_libm(left, stay, etab);
+        c.stay = a + e;
+        c.stay = c.stay + p;
+        c.stay = c.stay - ln;
+        c.emit = a + p;
+        c.emit = c.emit + e;
+        c.emit = c.emit - ln;
+      }
+      stay = c.stay;
+      emit = c.emit;
     } else {
       const float right = wave_shl1(dcol, 0.0f);
       const float ne = dcol * w;
       const float em = right * w;
       dcol = ne + em;
     }
+  };
+  // four at a time by hand: the compiler leaves a loop around the hand-written cell as it is
+  int s = 0;
+  for (; s + 4 <= steps; s += 4) {
+    step();
+    step();
+    step();
+    step();
   }
+  for (; s < steps; ++s) step();
   sink[lane] = kKind != 1 ? stay + emit : dcol;
 }
 
@@ -2523,11 +2846,17 @@ int live_blocks(const Dims& d, int* waves) {
   if (d.B * n > 192 && d.U <= 1024) return 0;
   return n;
 }
+// Blocks of 256 label positions that the alpha walk runs side by side (1: none), by the same
+// rule; its hand-over needs no LDS that grows with the utterance.
+int alpha_blocks(const Dims& d) {
+  const int n = (d.U + 255) / 256;
+  if (n < 2 || n > 16 || (d.B * n > 192 && d.U <= 1024)) return 1;
+  return n;
+}
 // The two hand-over vectors of the planes hold the walks' tagged 64-bit entries as well: one
 // array of [B][Dp] entries per boundary between live blocks.  In units of [B][Dp] floats each.
 static int hand_arrays(const Dims& d) {
-  const int n = live_blocks(d, nullptr);
-  return n > 2 ? n - 1 : 1;
+  return std::max(1, std::max(live_blocks(d, nullptr), alpha_blocks(d)) - 1);
 }
 
 size_t planes_bytes(const Dims& d, bool decode_only) {
@@ -2651,10 +2980,35 @@ int launch_alpha_wide(const Planes& p, const int* inLen, const int* labLen, floa
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));   \
     hipLaunchKernelGGL((alpha_kernel<C, W, M>), dim3(d.B), dim3(64 * W), lds, s, p, inLen,  \
                        labLen, costs, d, stride, g_spin_limit, trouble, u_base, ghin,        \
-                       ghout, nullptr, 0);                                                   \
+                       ghout);                                                               \
     break;
 
 #if RNNT_IN_PART(1)
+static int launch_alpha_walk(const Planes& p, const int* inLen, const int* labLen, float* costs,
+                             const Dims& d, hipStream_t s, int* trouble) {
+  unsigned long long* live = reinterpret_cast<unsigned long long*>(p.hand[0]);
+  const int n = alpha_blocks(d);
+  if (n > 1) {
+    const int words = 2 * d.B * d.Dp * (n - 1);
+    hipLaunchKernelGGL(clear_words_kernel, dim3((words + 255) / 256), dim3(256), 0, s,
+                       reinterpret_cast<int*>(live), words);
+    RNNT_LAUNCH_CHECK("clear_words_kernel");
+    hipLaunchKernelGGL((alpha_walk_kernel<4, true>), dim3(8 * n * ((d.B + 7) / 8)), dim3(320), 0, s,
+                       p, inLen, labLen, costs, d, g_spin_limit, trouble, live, n);
+  } else if (d.U <= 64) {
+    hipLaunchKernelGGL((alpha_walk_kernel<1, false>), dim3(d.B), dim3(64), 0, s, p, inLen, labLen,
+                       costs, d, g_spin_limit, trouble, live, 1);
+  } else if (d.U <= 128) {
+    hipLaunchKernelGGL((alpha_walk_kernel<2, false>), dim3(d.B), dim3(128), 0, s, p, inLen, labLen,
+                       costs, d, g_spin_limit, trouble, live, 1);
+  } else {
+    hipLaunchKernelGGL((alpha_walk_kernel<4, false>), dim3(d.B), dim3(256), 0, s, p, inLen, labLen,
+                       costs, d, g_spin_limit, trouble, live, 1);
+  }
+  RNNT_LAUNCH_CHECK("alpha_walk_kernel");
+  return kOk;
+}
+
 int launch_alpha(const Planes& p, const int* inLen, const int* labLen, float* costs,
                  const Dims& d, hipStream_t s) {
   if (d.B == 0) return kOk;
@@ -2662,39 +3016,25 @@ int launch_alpha(const Planes& p, const int* inLen, const int* labLen, float* co
   // array (one float per step and boundary) fits LDS
   const int cpl = block_cells_per_lane(d), nblocks = label_blocks(d);
   const int stride = d.Dp;
-  // (two wavefronts up to 128 label positions, four beyond -- one, two or four positions a lane
-  // -- if their three hand-over arrays fit LDS: a step costs a wavefront one log-sum-exp per
-  // position it owns, and the step is what a lattice is bound by.  B=8 T=2000, 129..256 label
-  // positions: 117 ns a step with four wavefronts of one position, what 101 positions on two
-  // wavefronts take; two wavefronts of two positions were 1.6 times as slow as that)
+  // (two or four positions a lane on four wavefronts if their three hand-over arrays fit LDS: a
+  // step costs a wavefront one log-sum-exp per position it owns, and the step is what a lattice
+  // is bound by)
   const bool single_block = nblocks == 1;
   const int W = (single_block && cpl >= 4 && 3 * stride * sizeof(float) <= 144 * 1024) ? 4
                 : (cpl >= 2 && stride * sizeof(float) <= 144 * 1024) ? 2 : 1;
   const size_t lds = W > 1 ? sizeof(float) * (size_t)(W - 1) * stride : 0;
   int* trouble = nullptr;
   RNNT_TRY(trouble_flag(&trouble));
-  // From 257 label positions, with few enough utterances that the device has the CUs: blocks
-  // of 256 positions side by side on as many CUs, four wavefronts of one position a lane each
-  // (B=8 T=10000, 401 positions: 129 ns a step, 150 at T=2000 and from 513 to 1024 positions; on
-  // one CU, before the cell was shortened, 235 and 523 .. 539 against 176 and 198 side by side;
-  // from about a hundred utterances on the planes' traffic holds every form, B=128 T=2000: 235 ns)
-  int live_w = 0;
-  if (const int n = live_blocks(d, &live_w)) {
-    if (live_w == 4)
-      return launch_live(alpha_kernel<1, 4, true, true>, p, d, n, 4, s, p, inLen, labLen, costs,
-                         d, stride, g_spin_limit, trouble, 0, (const float*)nullptr,
-                         (float*)nullptr);
-    return launch_live(alpha_kernel<1, 2, true, true>, p, d, n, 2, s, p, inLen, labLen, costs, d,
-                       stride, g_spin_limit, trouble, 0, (const float*)nullptr, (float*)nullptr);
-  }
+  // one position a lane wherever 256 positions, or blocks of 256 side by side, cover the label axis
+  // (B=8 T=10000, 401 positions: 84 ns a step; on one CU with two positions a lane 235)
+  if (d.U <= 256 || alpha_blocks(d) > 1)
+    return launch_alpha_walk(p, inLen, labLen, costs, d, s, trouble);
   for (int k = 0; k < nblocks; ++k) {  // lowest block first
     const float* ghin = k == 0 ? nullptr : p.hand[(k - 1) & 1];
     float* ghout = k == nblocks - 1 ? nullptr : p.hand[k & 1];
     const int u_base = k * 64 * cpl;
     switch ((nblocks > 1 ? 10000 : 0) + cpl / W * 100 + W) {
-      CASE(1, 1, false) CASE(2, 1, false) CASE(4, 1, false)
-      CASE(1, 2, false) CASE(2, 2, false) CASE(4, 2, false)
-      CASE(1, 4, false) CASE(2, 4, false) CASE(4, 4, false)
+      CASE(4, 2, false) CASE(2, 4, false) CASE(4, 4, false)
       default:
         RNNT_TRY(launch_alpha_wide(p, inLen, labLen, costs, d, s, cpl / W, W, nblocks > 1, lds,
                                    trouble, u_base, ghin, ghout));
