@@ -79,3 +79,28 @@ def test_dalphas_where_groups_of_four_meet_the_lattices_edges(T, U):
     want = oracle.backward(E, P, np.nan_to_num(alphas), LN, labels, il, ll)
     for g, w, what in zip(got, want, ("egrads", "pgrads", "lngrads")):
         assert_same_bits(g, w, what)
+
+
+@pytest.mark.parametrize("U", [65, 128, 193, 256, 300, 520])
+@pytest.mark.parametrize("T", [31, 191, 253, 256, 517])
+def test_dalphas_where_the_hand_over_between_wavefronts_wraps(T, U):
+    """The same rings, in the other direction: lattices of about 256 steps and of several times as
+    many, utterances whose last label lies in any wavefront or block, one whose labels are all the
+    blank (one accumulator for both sums)."""
+    V = 5
+    il = [T, T - 1, T - 2, T - 3, max(T - 60, 1), T]
+    ll = [U - 1, U // 2, min(64, U - 1), 0, min(63, U - 1), min(129, U - 1)]
+    B = len(il)
+    rng = np.random.default_rng(9000 * T + U)
+    E = rng.standard_normal((B, T, V), dtype=np.float32)
+    P = rng.standard_normal((B, U, V), dtype=np.float32)
+    labels = rng.integers(1, V, (B, U - 1)).astype(np.int32)
+    labels[1] = 0
+    il, ll = np.array(il, np.int32), np.array(ll, np.int32)
+    LN = oracle.log_norms_naive(E, P, il, ll)
+    _, alphas = oracle.forward(E, P, LN, labels, il, ll)
+    alphas, LN = np.nan_to_num(alphas, posinf=0.0, neginf=0.0), np.nan_to_num(LN)
+    got = gpu_backward(DeviceCase(E, P, labels, il, ll), alphas, LN)
+    want = oracle.backward(E, P, alphas, LN, labels, il, ll)
+    for g, w, what in zip(got, want, ("egrads", "pgrads", "lngrads")):
+        assert_same_bits(g, w, what)

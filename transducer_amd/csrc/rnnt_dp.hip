@@ -35,6 +35,7 @@ namespace rnnt {
 
 int live_blocks(const Dims& d, int* waves);
 int alpha_blocks(const Dims& d);
+int beta_blocks(const Dims& d, int* waves);
 
 namespace {
 
@@ -394,7 +395,6 @@ __global__ __launch_bounds__(256) void gather_cells_kernel(const TIO* __restrict
 // kMulti: this launch is one of several blocks (the hand-over code is compiled in only then: in
 // the single-block kernel even an unused hand-over load costs the walk its prefetch distance).
 constexpr int kLiveLag = 12;      // groups between blocks that the best-path walk runs side by side
-constexpr int kBetaLiveLag = 24;  // (the dalpha walk asks eight groups ahead, not four)
 constexpr int kLiveWaveLag = 2;  // groups between the wavefronts of a live block at the start (8 elsewhere)
 template <int C, int W, bool kMulti>
 __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __restrict__ inLen,
@@ -706,58 +706,70 @@ __device__ inline void prog_store(int* p, int x) {
 
 // The wavefront beside the walking ones of a block that runs side by side with others: brings what
 // the block before it has left in memory (`src`) into the ring of the first walking wavefront, and
-// takes what the last one hands on out to `dst`, up to sixteen quads at a time.  It keeps the
+// takes what the last one hands on out to `dst`, up to 64 quads in a turn.  It keeps the
 // tagged entries, their waits and their addresses out of the walk.  at(g, i): the step of value
-// i = 0..3 of group g.  Groups are numbered in walking order, n of them on either side.  Bounded
+// i = 0..3 of group g (four steps in a row).  Groups are numbered in walking order, n of them on either side; group g's quad
+// lies in slot g + kShift of a ring.  Bounded
 // like every wait here: when nothing has moved for spin_limit turns it raises the trouble flag and
 // lets everybody go on with whatever the rings hold.
-template <typename At>
+template <int kShift, typename At>
 __device__ inline void live_carrier(const unsigned long long* __restrict__ src,
                                     unsigned long long* __restrict__ dst, int n, At at,
                                     float* ring_in, int* prog_in, const int* prog_first,
                                     const float* ring_out, const int* prog_last, int* prog_out,
                                     int spin_limit, int* __restrict__ trouble) {
-  const int lane = threadIdx.x & 63, quad = lane >> 2;
+  const int lane = threadIdx.x & 63, quad = lane >> 2, value = lane & 3;
   int in = src ? 0 : n, out = dst ? 0 : n, idle = 0;
   while (in < n || out < n) {
     bool moved = false;
+    unsigned long long e[4];
+    const int room = in < n ? min(prog_load(prog_first) + kRingGroups - 4, n) - in : 0;
+    asm volatile("" ::: "memory");
+    if (room > 0) {  // (asked for ahead of the other side's work: the answer takes a microsecond)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        e[k] = __hip_atomic_load(src + at(min(in + 16 * k + quad, n - 1), value), __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+    }
     if (out < n) {
-      const int have = min(prog_load(prog_last), n) - out;
+      const int m = min(min(prog_load(prog_last), n) - out, 64);
       asm volatile("" ::: "memory");
-      if (have > 0) {
-        const int g = out + quad, m = min(have, 16);
-        if (quad < m) {
-          const float x = ring_out[4 * (g & (kRingGroups - 1)) + (lane & 3)];
-          const int s = at(g, lane & 3);
-          if (s >= 0) __hip_atomic_store(dst + s, live_entry(s, x), __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int g = out + 16 * k + quad;
+        if (16 * k + quad < m) {
+          const float x = ring_out[4 * ((g + kShift) & (kRingGroups - 1)) + value];
+          const int s = at(g, value);
+          __hip_atomic_store(dst + s, live_entry(s, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
+      }
+      if (m > 0) {
         out += m;
         asm volatile("" ::: "memory");
         if (lane == 0) prog_store(prog_out, out);
         moved = true;
       }
     }
-    if (in < n) {
-      const int room = min(prog_load(prog_first) + kRingGroups - 4, n) - in;
-      if (room > 0) {
-        const int g = in + quad, m = min(room, 16);
-        const int s = at(min(g, n - 1), lane & 3);
-        const unsigned long long e =
-            __hip_atomic_load(src + max(s, 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool here = quad < m && (s < 0 || (unsigned)(e >> 32) == (unsigned)(s + 1));
+    if (room > 0) {
+      int ready = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int g = in + 16 * k + quad;
+        const bool here = 16 * k + quad < room && (unsigned)(e[k] >> 32) == (unsigned)(at(g, value) + 1);
         const unsigned long long missing = __builtin_amdgcn_ballot_w64(!here);
-        const int ready = missing ? __builtin_ctzll(missing) >> 2 : 16;
-        if (ready > 0) {
-          if (quad < ready)
-            ring_in[4 * (g & (kRingGroups - 1)) + (lane & 3)] = __uint_as_float((unsigned)e);
-          in += ready;
-          asm volatile("" ::: "memory");  // (LDS serves a wavefront's requests in order)
-          if (lane == 0) prog_store(prog_in, in);
-          moved = true;
-        }
+        if (ready == 16 * k) ready += missing ? __builtin_ctzll(missing) >> 2 : 16;
+        if (16 * k + quad < ready)
+          ring_in[4 * ((g + kShift) & (kRingGroups - 1)) + value] = __uint_as_float((unsigned)e[k]);
+      }
+      if (ready > 0) {
+        in += ready;
+        asm volatile("" ::: "memory");  // (LDS serves a wavefront's requests in order)
+        if (lane == 0) prog_store(prog_in, in);
+        moved = true;
       }
     }
+    // (not more often than pays: its requests go the same way as the walk's operands)
+    __builtin_amdgcn_s_sleep(16);
     if (moved) {
       idle = 0;
     } else if (idle++ >= spin_limit) {
@@ -767,8 +779,6 @@ __device__ inline void live_carrier(const unsigned long long* __restrict__ src,
         prog_store(prog_out, kForever);
       }
       return;
-    } else {
-      __builtin_amdgcn_s_sleep(2);
     }
   }
 }
@@ -902,7 +912,7 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
         live_in ? live + ((size_t)(live_block - 1) * d.B + b) * d.Dp : nullptr;
     unsigned long long* dst = live_out ? live + ((size_t)live_block * d.B + b) * d.Dp : nullptr;
     // what enters step s: value i of group g is what enters step 4g + 1 + i (nothing enters step 0)
-    live_carrier(src, dst, ngroups, [](int g, int i) { return 4 * g + 1 + i; }, ring[0], &prog[0],
+    live_carrier<0>(src, dst, ngroups, [](int g, int i) { return 4 * g + 1 + i; }, ring[0], &prog[0],
                  &prog[1], ring[W], &prog[W], &prog[W + 1], spin_limit, trouble);
     return;
   }
@@ -1202,38 +1212,21 @@ constexpr int beta_depth(int C) { return C <= 2 ? 8 : C <= 4 ? 4 : 3; }
 // wavefront below reads them one group later (the same hand-over as between blocks, with the
 // bounded wait of alpha_kernel).  Every wavefront runs all groups, past the utterance's labels
 // too (zeros), so nobody waits for a wavefront that has left.
-// kLive: the live_n blocks of 64 C W positions of a label axis as live_n workgroups running at
-// the same time, as in alpha_kernel with the directions turned round: the HIGHEST block leads
-// (and has the smallest workgroup index, so it is dispatched first), lane 0 of a block's
-// wavefront 0 leaves dalpha of the block's first column in `live` (entry s: the value on
-// diagonal s, s + 1 in the upper word; zero before the launch), and the highest wavefront of the
-// block below asks for them, lane j for entry 4g + 1 + j, with its weights, checks the tags when
-// it uses them and asks again, bounded, for what was not there yet.  A block above an
-// utterance's last label leaves at once, and the utterance's highest block takes nothing.
-template <int C, int W, bool kMulti, bool kLive = false>
+template <int C, int W, bool kMulti>
 __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __restrict__ labels,
                                                       const int* __restrict__ inLen,
                                                       const int* __restrict__ labLen, Dims d,
                                                       int hand_stride, int u_base,
                                                       const float* __restrict__ ghin,
                                                       float* __restrict__ ghout, int spin_limit,
-                                                      int* __restrict__ trouble,
-                                                      unsigned long long* __restrict__ live,
-                                                      int live_n) {
+                                                      int* __restrict__ trouble) {
   static_assert(W == 1 || !kMulti, "several wavefronts only when one launch covers the label axis");
-  static_assert(!kLive || (!kMulti && W > 1), "live halves are dealt to several wavefronts");
   extern __shared__ __attribute__((aligned(16))) float hand[];  // [W-1][hand_stride]: entry s =
                                                                 // dalpha on diagonal s
   __shared__ int done[W];  // groups a wavefront has published
-  // live blocks: as in alpha_kernel, the highest block first
-  const int live_block = kLive ? live_n - 1 - (int)(blockIdx.x >> 3) % live_n : 0;
-  const int b = kLive ? (int)(blockIdx.x / (8 * live_n)) * 8 + (blockIdx.x & 7) : blockIdx.x;
+  const int b = blockIdx.x;
   const int lane = threadIdx.x & 63;
   const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
-  if (kLive) {
-    if (b >= d.B) return;
-    u_base = live_block * 64 * C * W;
-  }
   int Tb, Ub;
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
   if (Tb == 0 || Ub == 0) return;  // :92-94
@@ -1265,33 +1258,6 @@ __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __res
   const float* gin =
       (kMulti && ghin && u_base + 64 * C < Ub) ? ghin + (size_t)b * hand_stride : nullptr;
   float* gout = (kMulti && ghout) ? ghout + (size_t)b * hand_stride : nullptr;
-  // live halves: the upper one writes the entries; the highest wavefront of the lower one takes
-  // them if the utterance has an upper half at all
-  // block h writes the entries of boundary h - 1 and takes those of boundary h, if the utterance
-  // has a block above it at all (the highest block asks at its own boundary, for nothing)
-  const unsigned long long* lrow =
-      kLive ? live + ((size_t)min(live_block, max(live_n - 2, 0)) * d.B + b) * hand_stride
-            : nullptr;
-  unsigned long long* lrow_out =
-      kLive ? live + ((size_t)max(live_block - 1, 0) * d.B + b) * hand_stride : nullptr;
-  const bool live_out = kLive && live_block > 0;
-  const bool live_takes = kLive && live_block < live_n - 1 && wave == W - 1 &&
-                          u_base + 64 * C * W < Ub;
-  auto live_load = [&](int s) -> unsigned long long {
-    return __hip_atomic_load(lrow + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  // (one opaque statement: see alpha_kernel)
-  auto live_reload = [&](int s) -> unsigned long long {
-    unsigned long long e;
-    const unsigned long long* q = lrow + s;
-    asm volatile("global_load_dwordx2 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)"
-                 : "=&v"(e)
-                 : "v"(q)
-                 : "memory");
-    return e;
-  };
-  unsigned live_sink = 0;
-
   float dcol[C], accB[C], accL[C];
   bool fold[C];  // label of this position equals blank: both sums share one accumulator
   const float* wbp[C];
@@ -1313,8 +1279,6 @@ __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __res
   struct Group {
     float4 wb[C], we[C];
     float gh[4];  // dalpha of the block above's first column on diagonals 4g+1 .. 4g+4
-    unsigned long long lv;  // the same, tagged, from the half running beside this one: lane j
-                            // holds the entry of diagonal 4g + 1 + j
   };
   auto load_group = [&](int g) -> Group {
     Group r;
@@ -1328,7 +1292,6 @@ __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __res
 #pragma unroll
       for (int j = 0; j < 4; ++j) r.gh[j] = gin ? gin[4 * gc + 1 + j] : 0.0f;  // uniform
     }
-    if constexpr (kLive) r.lv = live_load(4 * gc + 1 + (lane & 3));  // every wavefront asks
     return r;
   };
   // steps last-1 .. 0 are computed; the slot of step `last` receives the seed and the slots
@@ -1351,33 +1314,6 @@ __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __res
 #pragma unroll
       for (int j = 0; j < 4; ++j) hh[j] = hand_in[4 * g + 1 + j];  // uniform
     }
-    if constexpr (kLive) {
-      if (live_takes) {  // uniform
-        // diagonals past the seed's group are never written, and never used either
-        const int top = 4 * g_first + 3;
-        unsigned long long e = w.lv;
-        if (__builtin_amdgcn_ballot_w64(lane < 4 && 4 * g + 1 + lane <= top &&
-                                        (unsigned)(e >> 32) != (unsigned)(4 * g + 2 + lane))) {
-          // (as in alpha_kernel: let the upper half get kBetaLiveLag groups ahead again)
-          const int mine = (lane < 4 && 4 * g + 1 + lane <= top) ? 4 * g + 1 + lane
-                                                                 : 4 * max(g - kBetaLiveLag, 0);
-          int spins = 0;
-          do {
-            if (spins++ >= spin_limit) {
-              if (lane == 0) raise_trouble(trouble);
-              break;
-            }
-            __builtin_amdgcn_s_sleep(4);
-            e = live_reload(mine);
-          } while (__builtin_amdgcn_ballot_w64((unsigned)(e >> 32) != (unsigned)(mine + 1)));
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          hh[j] = __int_as_float(__builtin_amdgcn_readlane((int)(unsigned)e, j));
-      } else {
-        live_sink ^= (unsigned)w.lv;  // (kept until the end: see alpha_kernel)
-      }
-    }
 #pragma unroll
     for (int j = 3; j >= 0; --j) {
       const int s = 4 * g + j;
@@ -1392,7 +1328,7 @@ __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __res
         float right[C];
         float above = 0.0f;  // right of the wavefront's last position
         if constexpr (kMulti) above = gin ? w.gh[j] : 0.0f;
-        if (W > 1) above = (wave < W - 1 || live_takes) ? hh[j] : 0.0f;
+        if (W > 1) above = wave < W - 1 ? hh[j] : 0.0f;
         if constexpr (kSpread) {
 #pragma unroll
           for (int c = 0; c < C; ++c) {
@@ -1432,16 +1368,6 @@ __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __res
         for (int j = 0; j < 4; ++j) gout[4 * g + j] = gsend[j];
       }
     }
-    if constexpr (kLive) {
-      if (live_out && wave == 0 && lane == 0) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          __hip_atomic_store(lrow_out + 4 * g + j,
-                             ((unsigned long long)(unsigned)(4 * g + j + 1) << 32) |
-                                 (unsigned long long)__float_as_uint(gsend[j]),
-                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
     if (W > 1 && wave > 0 && lane == 0) {  // entries 4g .. 4g+3, then the progress
 #pragma unroll
       for (int j = 0; j < 4; ++j) hand_out[4 * g + j] = gsend[j];
@@ -1458,25 +1384,12 @@ __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __res
   auto walk = [&](auto with_fold) __attribute__((always_inline)) {
     constexpr int kBetaDepth = beta_depth(C);
     int g = g_first;
-    if constexpr (kLive) {
-      if (live_takes) {  // start kBetaLiveLag groups behind the upper half (or when it is done)
-        const int far = 4 * max(g_first - kBetaLiveLag, 0);
-        int spins = 0;
-        while ((unsigned)(live_load(far) >> 32) != (unsigned)(far + 1)) {
-          if (spins++ >= spin_limit) {
-            if (lane == 0) raise_trouble(trouble);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(8);
-        }
-      }
-    }
     Group q[kBetaDepth];
 #pragma unroll
     for (int i = 0; i < kBetaDepth; ++i) q[i] = load_group(g - i);
     // fall a few groups behind the wavefront above, so that the wait per group finds its
     // counter there already
-    if (W > 1 && wave < W - 1) wait_for(min(g_first + 1, (kLive ? kLiveWaveLag : 8) * (W - 1 - wave)));
+    if (W > 1 && wave < W - 1) wait_for(min(g_first + 1, 8 * (W - 1 - wave)));
     // the first round, whose first group holds the seed (a short lattice may end inside it)
     const std::true_type seeded;
     const std::false_type plain;
@@ -1513,8 +1426,251 @@ __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __res
       p.gL[(size_t)b * d.Ua + u] = accL[c];
     }
   }
-  if constexpr (kLive) {
-    if (spin_limit < 0 && live_sink == 1u) raise_trouble(trouble);  // never
+}
+
+// ------------------------------------------------------------------ dalpha, one position a lane
+// The same recursion with one label position a lane, dealt to wavefronts and to blocks side by side
+// like alpha_walk_kernel's with the directions turned round: the HIGHEST wavefront leads (and the
+// highest block has the smallest workgroup index); what crosses is dalpha of a wavefront's first
+// column, quads of four diagonals through the rings.  Groups are counted in walking order, i = 0 the
+// one that holds the seed; group i's quad lies in slot i + 3 of the ring, so that the groups after
+// the seed's come in aligned blocks of four slots.
+// A step is six instructions, a group of four about twenty more, and the hand-over as many again: 19 ns
+// a step on one wavefront, 33 with a neighbour (20 and 36 when two positions a lane shared one
+// wavefront, every load formed an address and was asked for eight groups ahead).  Beyond, the walk
+// waits for memory, 12 bytes a cell: kDepth register sets rotate, a group's weights being requested
+// that many groups ahead (a microsecond is about twelve groups).  B=8, 201 positions T=2000: 124 ->
+// 80 us (the weights of a group used to be waited for together with what had just been handed
+// over); 401 positions T=2000 193 -> 100, T=10000 766 -> 372.  The weight planes hold zeros
+// wherever there is no move, so nothing asks for bounds.
+template <int W, bool kLive>
+__global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void beta_walk_kernel(
+    Planes p, const int* __restrict__ labels, const int* __restrict__ inLen,
+    const int* __restrict__ labLen, Dims d, int spin_limit, int* __restrict__ trouble,
+    unsigned long long* __restrict__ live, int live_n) {
+  constexpr bool kHand = W > 1 || kLive;
+  constexpr int kDepth = W == 1 ? 16 : 12;
+  __shared__ __attribute__((aligned(16))) float ring[W + 1][kHand ? 4 * kRingGroups : 4];
+  __shared__ __attribute__((aligned(16))) float nothing[16];
+  __shared__ __attribute__((aligned(16))) float dump[kHand ? 4 * 64 + 16 : 4];
+  __shared__ int prog[W + 2];
+  const int live_block = kLive ? live_n - 1 - (int)(blockIdx.x >> 3) % live_n : 0;
+  const int b = kLive ? (int)(blockIdx.x / (8 * live_n)) * 8 + (blockIdx.x & 7) : blockIdx.x;
+  if (kLive && b >= d.B) return;
+  const int u_base = live_block * 64 * W;
+  const int lane = threadIdx.x & 63;
+  const int wave = kHand ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  int Tb, Ub;
+  utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
+  if (Tb == 0 || Ub == 0) return;  // :92-94
+  if (u_base >= Ub) return;        // a block past this utterance's labels
+  const int last = Tb + Ub - 2;    // diagonal of the last cell
+  const int g_first = last >> 2;   // the group that holds the seed
+  const int n = g_first + 1;
+  const bool live_in = kLive && live_block < live_n - 1 && u_base + 64 * W < Ub;
+  const bool live_out = kLive && live_block > 0;
+  if constexpr (kHand) {
+    if (threadIdx.x < 16) nothing[threadIdx.x] = 0.0f;
+    if (threadIdx.x < W + 2) {
+      const int r = (int)threadIdx.x - 1;  // the wavefront, in walking order, whose progress this is
+      prog[threadIdx.x] = r < 0 ? (live_in ? 0 : kForever)
+                          : r == W ? (live_out ? 0 : kForever)
+                                   : (u_base + 64 * (W - 1 - r) < Ub ? 0 : kForever);
+    }
+    __syncthreads();
+  }
+  if (kLive && wave == W) {
+    const unsigned long long* src =
+        live_in ? live + ((size_t)live_block * d.B + b) * d.Dp : nullptr;
+    unsigned long long* dst =
+        live_out ? live + ((size_t)(live_block - 1) * d.B + b) * d.Dp : nullptr;
+    live_carrier<3>(src, dst, n, [&](int i, int k) { return 4 * (g_first - i) + k; }, ring[0],
+                    &prog[0], &prog[1], ring[W], &prog[W], &prog[W + 1], spin_limit, trouble);
+    return;
+  }
+  const int u_lo = u_base + wave * 64;
+  if (u_lo >= Ub) return;  // a wavefront past this utterance's labels
+  if (kLive) __builtin_amdgcn_s_setprio(3);  // ahead of the carrier on the same SIMD
+  const int order = W - 1 - wave;
+  const bool leads = !live_in && u_lo + 64 >= Ub;  // nothing comes in from above
+  const int u = u_lo + lane;
+  float dcol = u == Ub - 1 ? 1.0f : 0.0f;   // :95
+  float accB = u == Ub - 1 ? -1.0f : 0.0f;  // :97
+  float accL = 0.0f;
+  // label of this position equals blank: both sums share one accumulator
+  bool fold = false;
+  if (d.U > 1) {  // (read in every lane: no divergent branch, see alpha_walk_kernel)
+    const int label = label_at(labels, d, b, min(u, d.U - 2));
+    fold = (u + 1 < Ub) & (label == d.blank);
+  }
+
+  const unsigned gbytes = kLive ? 16u * (unsigned)d.Ua : 1024u * W;  // from a group to the next
+  const unsigned lane_o = 16u * (unsigned)u;
+  // the planes as buffers that begin at group `origin` (moved down as the walk goes on, so that no
+  // offset outgrows 32 bits)
+  const int span = (int)((1u << 30) / gbytes);
+  int origin = max(0, g_first - span);
+  const char* wb_b = reinterpret_cast<const char*>(p.wB + plane_group0(d, b, 0));
+  const char* we_b = reinterpret_cast<const char*>(p.wE + plane_group0(d, b, 0));
+  char* d_b = reinterpret_cast<char*>(p.dS + plane_group0(d, b, 0));
+  const size_t plane = (size_t)gbytes * (unsigned)(d.Dp / 4);
+  const size_t by0 = (size_t)origin * gbytes;
+  Buffer wb_q(wb_b + by0, plane - by0), we_q(we_b + by0, plane - by0), d_q(d_b + by0, plane - by0);
+  auto move_to = [&](int g) {
+    origin = g;
+    const size_t by = (size_t)g * gbytes;
+    wb_q = Buffer(wb_b + by, plane - by);
+    we_q = Buffer(we_b + by, plane - by);
+    d_q = Buffer(d_b + by, plane - by);
+  };
+  struct Ops {
+    quad_t wb, we;
+  };
+  auto load = [&](int i) -> Ops {  // (what is asked for past the last group is never used)
+    const unsigned by = (unsigned)(max(g_first - i, 0) - origin) * gbytes;
+    Ops r;
+    r.wb = wb_q.load(lane_o, by);
+    r.we = we_q.load(lane_o, by);
+    return r;
+  };
+
+  // ---- hand-over (see alpha_walk_kernel)
+  int ok = kHand ? -1 : kForever;
+  int have_in = 0, have_out = 0;
+  auto refresh = [&](int i) {
+    have_in = bounded_wait(&prog[order], have_in, min(i + 5, n), spin_limit, trouble);
+    have_out = bounded_wait(&prog[order + 2], have_out, i + 18 - kRingGroups, spin_limit, trouble);
+    ok = min(have_in >= n ? kForever : have_in - 3, min(have_out, kForever) + kRingGroups - 4);
+  };
+  const float* take = kHand ? (leads ? nothing : ring[order]) : nullptr;
+  const int take_mask = leads ? 0 : kRingGroups / 4 - 1;
+  float* give = kHand ? (lane == 0 ? ring[order + 1] : dump + 4 * lane) : nullptr;
+  const int give_mask = lane == 0 ? kRingGroups / 4 - 1 : 0;
+  int* give_prog = lane == 0 ? &prog[order + 1] : reinterpret_cast<int*>(dump + 4 * lane);
+  quad_t pend = {0.0f, 0.0f, 0.0f, 0.0f}, hand = pend;
+  float carry = 0.0f;
+  // dalpha of the position to the right on the diagonal just done: the next lane's, and for lane 63
+  // what was handed over
+  auto from_right = [&](float x, float in) {
+    if constexpr (!kHand)
+      return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130 /* wave_shl:1 */,
+                                                        0xf, 0xf, true));
+    return wave_shl1(x, in);
+  };
+  auto cell = [&](float wb, float we, float in, auto with_fold) {
+    const float right = from_right(dcol, in);
+    const float ne = dcol * wb;
+    const float em = right * we;
+    dcol = ne + em;
+    if constexpr (decltype(with_fold)::value) {
+      const float em_b = fold ? em : 0.0f, em_l = fold ? 0.0f : em;
+      accB = (accB - ne) - em_b;
+      accL = accL - em_l;
+    } else {
+      accB = accB - ne;
+      accL = accL - em;
+    }
+  };
+  // with_fold: some position of this wavefront has the blank as its label.  Real transcripts have
+  // none, and the walk without the two selects per cell is shorter (x - 0 is x, so the sums come
+  // out the same bits either way).
+  auto walk = [&](auto with_fold) __attribute__((always_inline)) {
+    // the group that holds the seed: the slot of diagonal `last` receives it, those after it zeros
+    Ops first = load(0);
+    Ops q[kDepth];
+#pragma unroll
+    for (int k = 0; k < kDepth; ++k) q[k] = load(1 + k);
+    if constexpr (kHand) {
+      if (!leads) {
+        refresh(0);
+        hand = *reinterpret_cast<const quad_t*>(take + 12);
+      }
+    }
+    {
+      quad_t out, next = hand;
+      if constexpr (kHand) next = *reinterpret_cast<const quad_t*>(take + 16 * (1 & take_mask));
+      const float in[4] = {hand[1], hand[2], hand[3], carry};
+#pragma unroll
+      for (int j = 3; j >= 0; --j) {
+        const int s = 4 * g_first + j;
+        if (s < last) cell(first.wb[j], first.we[j], in[j], with_fold);  // uniform
+        out[j] = s <= last ? dcol : 0.0f;
+      }
+      d_q.store(lane_o, (unsigned)(g_first - origin) * gbytes, out);
+      pend = out;
+      carry = hand[0];
+      hand = next;
+    }
+    auto run_group = [&](int i, const Ops& w, const float* take_next, float* give_last, auto tell) {
+      quad_t next = hand;
+      if constexpr (kHand) {
+        *reinterpret_cast<quad_t*>(give_last) = pend;
+        asm volatile("" ::: "memory");  // (LDS serves a wavefront's requests in order)
+        if constexpr (decltype(tell)::value) prog_store(give_prog, i);
+        next = *reinterpret_cast<const quad_t*>(take_next);
+        __builtin_amdgcn_sched_barrier(0);  // (asked for ahead of the steps, not among them)
+      }
+      const float in[4] = {hand[1], hand[2], hand[3], carry};
+      quad_t out;
+#pragma unroll
+      for (int j = 3; j >= 0; --j) {
+        cell(w.wb[j], w.we[j], in[j], with_fold);
+        out[j] = dcol;
+      }
+      d_q.store(lane_o, (unsigned)(g_first - i - origin) * gbytes, out);
+      pend = out;
+      carry = hand[0];
+      hand = next;
+    };
+    // groups i .. i + 3, an aligned block of slots; kWhole: all of them exist, and sixteen more are asked for
+    auto four = [&](int i, Ops* w, auto whole) {
+      constexpr bool kWhole = decltype(whole)::value;
+      const float *tk = nullptr, *tk_next = nullptr;
+      float *gv = nullptr, *gv_last = nullptr;
+      const int slot = (i + 3) >> 2;
+      if constexpr (kHand) {
+        tk = take + 16 * (slot & take_mask);
+        tk_next = take + 16 * ((slot + 1) & take_mask);
+        gv = give + 16 * (slot & give_mask);
+        gv_last = give + 16 * ((slot - 1) & give_mask) + 12;
+        if (__builtin_expect(i > ok, 0)) refresh(i);
+      }
+      run_group(i, w[0], tk + 4, gv_last, std::true_type{});
+      if (kWhole) w[0] = load(i + kDepth);
+      if (kWhole || i + 1 < n) run_group(i + 1, w[1], tk + 8, gv, std::false_type{});
+      if (kWhole) w[1] = load(i + 1 + kDepth);
+      if (kWhole || i + 2 < n) {
+        if constexpr (kHand) {
+          if (__builtin_expect(i + 2 > ok, 0)) refresh(i + 2);
+        }
+        run_group(i + 2, w[2], tk + 12, gv + 4, std::true_type{});
+      }
+      if (kWhole) w[2] = load(i + 2 + kDepth);
+      if (kWhole || i + 3 < n) run_group(i + 3, w[3], tk_next, gv + 8, std::false_type{});
+      if (kWhole) w[3] = load(i + 3 + kDepth);
+      if constexpr (kHand && kWhole) __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): see alpha
+    };
+    int i = 1;
+    for (; i + kDepth <= n; i += kDepth) {
+      const int lowest = max(0, g_first - i - 2 * kDepth);
+      if (lowest < origin) move_to(max(0, lowest - span));
+#pragma unroll
+      for (int k = 0; k < kDepth; k += 4) four(i + k, &q[k], std::true_type{});
+    }
+#pragma unroll
+    for (int k = 0; k < kDepth; k += 4)
+      if (i + k < n) four(i + k, &q[k], std::false_type{});
+    if constexpr (kHand) {
+      *reinterpret_cast<quad_t*>(give + 16 * (((n + 2) >> 2) & give_mask) + 4 * ((n + 2) & 3)) = pend;
+      asm volatile("" ::: "memory");
+      prog_store(give_prog, n);
+    }
+  };
+  if (__ballot(fold) != 0) walk(std::true_type{});
+  else walk(std::false_type{});
+  if (u < Ub) {
+    p.gB[(size_t)b * d.Ua + u] = accB;
+    p.gL[(size_t)b * d.Ua + u] = accL;
   }
 }
 
@@ -2846,24 +3002,49 @@ int live_blocks(const Dims& d, int* waves) {
   if (d.B * n > 192 && d.U <= 1024) return 0;
   return n;
 }
-// Blocks of 256 label positions that the alpha walk runs side by side (1: none), by the same
-// rule; its hand-over needs no LDS that grows with the utterance.
+// Blocks of 256 label positions that the alpha walk runs side by side (1: none).  Up to 1024
+// positions the other way is one workgroup with two or four positions a lane, whose one CU holds it:
+// T=2000, 401 positions 663 -> 381 us at B=128, 1000 positions 1724 -> 541 at B=64.  With more
+// workgroups than fit two to a CU side by side (about three if the axis takes three blocks or more,
+// which leaves the other way as many cells a lane) the walks only share issue slots: T=500,
+// 300 positions, B=300: 307 -> 413.  Past 1024 positions the other way is a launch per 1024, many
+// times slower whatever the batch; workgroups beyond the device's CUs queue in order.
 int alpha_blocks(const Dims& d) {
   const int n = (d.U + 255) / 256;
-  if (n < 2 || n > 16 || (d.B * n > 192 && d.U <= 1024)) return 1;
+  if (n < 2 || n > 16 || ((long)d.B * n > (n == 2 ? 512 : 900) && d.U <= 1024)) return 1;
   return n;
 }
+// Blocks that the dalpha walk runs side by side, and the wavefronts (64 positions each) of a block.
+// A cell is six instructions and 12 bytes, and what one CU's memory path moves holds the walk, so
+// blocks are narrower than alpha's: 128 positions (B=8 T=10000, 401 positions: 610 us with blocks
+// of 256, 372 with 128; T=2000 100 either way).  129 to 256 positions, which four wavefronts
+// of one workgroup can take as well, go side by side where the three planes of the walk are more
+// than the memory-side cache keeps beside everything else (B=8, 201 positions: T=2000 80 us on one
+// workgroup, 84 as two; T=4000 142 and 142; T=6000 314 and 202; B=32 T=2000 152 and 106).
+// Up to 512 positions that holds for any batch (B=512 T=300, 300 positions: 378 -> 266 against two
+// positions a lane on one CU); on longer axes with more than 512 such blocks, alpha's.
+int beta_blocks(const Dims& d, int* waves) {
+  const int n2 = (d.U + 127) / 128;
+  *waves = 2;
+  if (d.U > 256 && n2 <= 16 && (d.U <= 512 || (long)d.B * n2 <= 512)) return n2;
+  if (d.U > 128 && d.U <= 256 && 12ull * d.B * d.Ua * d.Dp > 100ull << 20) return n2;
+  *waves = 4;
+  return alpha_blocks(d);
+}
 // The two hand-over vectors of the planes hold the walks' tagged 64-bit entries as well: one
-// array of [B][Dp] entries per boundary between live blocks.  In units of [B][Dp] floats each.
-static int hand_arrays(const Dims& d) {
-  return std::max(1, std::max(live_blocks(d, nullptr), alpha_blocks(d)) - 1);
+// array of [B][Dp] entries per boundary between blocks side by side.  In units of [B][Dp] floats
+// each.
+static int hand_arrays(const Dims& d, bool decode_only) {
+  int w, n = live_blocks(d, nullptr);
+  if (!decode_only) n = std::max(n, std::max(alpha_blocks(d), beta_blocks(d, &w)));
+  return std::max(1, n - 1);
 }
 
 size_t planes_bytes(const Dims& d, bool decode_only) {
   const size_t plane = align_up(sizeof(float) * (size_t)d.B * d.Ua * d.Dp + 64);
   return (decode_only ? 1 : 6) * plane + align_up(sizeof(float) * (size_t)d.B * d.Tp) +
          4 * align_up(sizeof(float) * (size_t)d.B * d.Ua) +
-         2 * align_up(sizeof(float) * (size_t)d.B * d.Dp * hand_arrays(d));
+         2 * align_up(sizeof(float) * (size_t)d.B * d.Dp * hand_arrays(d, decode_only));
 }
 
 void carve_planes(void* base, const Dims& d, Planes* p, bool decode_only) {
@@ -2879,7 +3060,7 @@ void carve_planes(void* base, const Dims& d, Planes* p, bool decode_only) {
   p->eb = take(align_up(sizeof(float) * (size_t)d.B * d.Tp));
   const size_t bu = align_up(sizeof(float) * (size_t)d.B * d.Ua);
   p->pb = take(bu); p->pl = take(bu); p->gB = take(bu); p->gL = take(bu);
-  const size_t bh = align_up(sizeof(float) * (size_t)d.B * d.Dp * hand_arrays(d));
+  const size_t bh = align_up(sizeof(float) * (size_t)d.B * d.Dp * hand_arrays(d, decode_only));
   p->hand[0] = take(bh); p->hand[1] = take(bh);
 }
 
@@ -2949,6 +3130,15 @@ static __global__ void clear_words_kernel(int* x, int n) {
   if (i < n) x[i] = 0;
 }
 
+// Clears the tagged entries of n blocks side by side.
+static int clear_live(unsigned long long* live, const Dims& d, int n, hipStream_t s) {
+  const int words = 2 * d.B * d.Dp * (n - 1);
+  hipLaunchKernelGGL(clear_words_kernel, dim3((words + 255) / 256), dim3(256), 0, s,
+                     reinterpret_cast<int*>(live), words);
+  RNNT_LAUNCH_CHECK("clear_words_kernel");
+  return kOk;
+}
+
 // Launches the side-by-side form of a walk (K: its kernel, W wavefronts of one position a lane)
 // for n blocks: clears the tagged entries, then one workgroup per utterance and block, eight
 // utterances' blocks in consecutive indices.
@@ -2989,10 +3179,7 @@ static int launch_alpha_walk(const Planes& p, const int* inLen, const int* labLe
   unsigned long long* live = reinterpret_cast<unsigned long long*>(p.hand[0]);
   const int n = alpha_blocks(d);
   if (n > 1) {
-    const int words = 2 * d.B * d.Dp * (n - 1);
-    hipLaunchKernelGGL(clear_words_kernel, dim3((words + 255) / 256), dim3(256), 0, s,
-                       reinterpret_cast<int*>(live), words);
-    RNNT_LAUNCH_CHECK("clear_words_kernel");
+    RNNT_TRY(clear_live(live, d, n, s));
     hipLaunchKernelGGL((alpha_walk_kernel<4, true>), dim3(8 * n * ((d.B + 7) / 8)), dim3(320), 0, s,
                        p, inLen, labLen, costs, d, g_spin_limit, trouble, live, n);
   } else if (d.U <= 64) {
@@ -3079,11 +3266,8 @@ int launch_beta(const Planes& p, const int* labels, const int* inLen, const int*
                 const Dims& d, hipStream_t s) {
   if (d.B == 0 || d.T == 0 || d.U == 0) return kOk;
   const int cpl = block_cells_per_lane(d), nblocks = label_blocks(d);
-  // wavefronts: one up to 128 label positions (a step of this walk is a handful of
-  // instructions a position, and the hand-over would cost as much again), four beyond (two if
-  // only their hand-over array fits LDS); one per block when the axis takes several launches.
-  // (129..256 label positions, B=8 T=2000: 70 ns a step with two wavefronts of two positions, 57
-  // with four of one)
+  // several positions a lane: four wavefronts (two if only their hand-over array fits LDS), one per
+  // block when the axis takes several launches
   const int stride = d.Dp;
   const bool single_block = nblocks == 1;
   const int W = !single_block ? 1
@@ -3092,16 +3276,31 @@ int launch_beta(const Planes& p, const int* labels, const int* inLen, const int*
   const size_t lds = W > 1 ? sizeof(float) * (size_t)(W - 1) * stride : 0;
   int* trouble = nullptr;
   RNNT_TRY(trouble_flag(&trouble));
-  // from 257 label positions in few enough utterances: blocks of 256 positions side by side
-  // (as in launch_alpha)
-  int live_w = 0;
-  if (const int n = live_blocks(d, &live_w)) {
-    if (live_w == 4)
-      return launch_live(beta_kernel<1, 4, false, true>, p, d, n, 4, s, p, labels, inLen, labLen,
-                         d, stride, 0, (const float*)nullptr, (float*)nullptr, g_spin_limit,
-                         trouble);
-    return launch_live(beta_kernel<1, 2, false, true>, p, d, n, 2, s, p, labels, inLen, labLen, d,
-                       stride, 0, (const float*)nullptr, (float*)nullptr, g_spin_limit, trouble);
+  int waves = 0;
+  const int n = beta_blocks(d, &waves);
+  if (d.U <= 256 || n > 1) {
+    unsigned long long* live = reinterpret_cast<unsigned long long*>(p.hand[0]);
+    if (n > 1) {
+      RNNT_TRY(clear_live(live, d, n, s));
+      const dim3 grid(8 * n * ((d.B + 7) / 8));
+      if (waves == 2)
+        hipLaunchKernelGGL((beta_walk_kernel<2, true>), grid, dim3(192), 0, s, p, labels, inLen,
+                           labLen, d, g_spin_limit, trouble, live, n);
+      else
+        hipLaunchKernelGGL((beta_walk_kernel<4, true>), grid, dim3(320), 0, s, p, labels, inLen,
+                           labLen, d, g_spin_limit, trouble, live, n);
+    } else if (d.U <= 64) {
+      hipLaunchKernelGGL((beta_walk_kernel<1, false>), dim3(d.B), dim3(64), 0, s, p, labels, inLen,
+                         labLen, d, g_spin_limit, trouble, live, 1);
+    } else if (d.U <= 128) {
+      hipLaunchKernelGGL((beta_walk_kernel<2, false>), dim3(d.B), dim3(128), 0, s, p, labels, inLen,
+                         labLen, d, g_spin_limit, trouble, live, 1);
+    } else {
+      hipLaunchKernelGGL((beta_walk_kernel<4, false>), dim3(d.B), dim3(256), 0, s, p, labels, inLen,
+                         labLen, d, g_spin_limit, trouble, live, 1);
+    }
+    RNNT_LAUNCH_CHECK("beta_walk_kernel");
+    return kOk;
   }
   for (int k = nblocks - 1; k >= 0; --k) {  // highest block first
     const float* ghin = k == nblocks - 1 ? nullptr : p.hand[(k + 1) & 1];
@@ -3115,11 +3314,10 @@ int launch_beta(const Planes& p, const int* labels, const int* inLen, const int*
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));  \
     hipLaunchKernelGGL((beta_kernel<C, W, M>), dim3(d.B), dim3(64 * W), lds, s, p, labels, \
                        inLen, labLen, d, stride, u_base, ghin, ghout, g_spin_limit,        \
-                       trouble, nullptr, 0);                                                \
+                       trouble);                                                            \
     break;
-      CASE(1, 1, false) CASE(2, 1, false) CASE(4, 1, false) CASE(8, 1, false) CASE(16, 1, false)
-      CASE(2, 2, false) CASE(4, 2, false) CASE(8, 2, false)
-      CASE(1, 4, false) CASE(2, 4, false) CASE(4, 4, false)
+      CASE(8, 1, false) CASE(16, 1, false) CASE(4, 2, false) CASE(8, 2, false)
+      CASE(2, 4, false) CASE(4, 4, false)
       CASE(16, 1, true)
 #undef CASE
       default:
