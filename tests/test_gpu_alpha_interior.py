@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle
-from util import DeviceCase, assert_same_bits, gpu_backward, gpu_forward
+from util import DeviceCase, assert_same_bits, gpu_backward, gpu_forward, gpu_viterbi
 
 pytestmark = pytest.mark.gpu
 
@@ -104,3 +104,41 @@ def test_dalphas_where_the_hand_over_between_wavefronts_wraps(T, U):
     want = oracle.backward(E, P, alphas, LN, labels, il, ll)
     for g, w, what in zip(got, want, ("egrads", "pgrads", "lngrads")):
         assert_same_bits(g, w, what)
+
+
+def check_paths(E, P, il, ll):
+    labels = np.ones((E.shape[0], P.shape[1] - 1), np.int32)
+    LN = np.nan_to_num(oracle.log_norms_naive(E, P, il, ll))
+    got = gpu_viterbi(DeviceCase(E, P, labels, il, ll), LN)
+    want = oracle.viterbi(E, P, LN, il, ll)
+    for b in range(E.shape[0]):
+        assert np.array_equal(got[b, :ll[b]], want[b, :ll[b]]), "path of utterance %d" % b
+
+
+@pytest.mark.parametrize("U", [2, 64, 65, 129, 256, 300, 520])
+@pytest.mark.parametrize("T", [31, 253, 256, 517])
+def test_best_paths_where_the_hand_over_between_wavefronts_wraps(T, U):
+    """Lattices of about 256 steps and of several times as many, utterances whose last label lies
+    in any wavefront or block, with no labels and with one frame."""
+    V = 6
+    il = np.array([T, T - 1, T - 2, T - 3, max(T - 60, 1), 1], np.int32)
+    ll = np.array([U - 1, U // 2, min(64, U - 1), 0, min(63, U - 1), U - 1], np.int32)
+    rng = np.random.default_rng(11000 * T + U)
+    E = rng.standard_normal((6, T, V), dtype=np.float32)
+    P = rng.standard_normal((6, U, V), dtype=np.float32)
+    check_paths(E, P, il, ll)
+
+
+@pytest.mark.parametrize("T,U", [(5200, 4), (2100, 300), (9000, 130), (5200, 60)])
+def test_best_paths_with_thousands_of_frames_between_labels(T, U):
+    """The backtrace looks at 2048 steps at a time: half of the labels in the first frames, the other
+    half in the last ones, blanks only in between; decision columns in LDS and in memory."""
+    V = 4
+    il, ll = np.array([T, T - 37, T], np.int32), np.array([U - 1, U - 1, U // 2], np.int32)
+    rng = np.random.default_rng(T + U)
+    E = rng.standard_normal((3, T, V), dtype=np.float32)
+    P = rng.standard_normal((3, U, V), dtype=np.float32)
+    E[:, U // 2 + 3:T - 40 - U // 2 - 3, 0] += 60.0
+    E[:, :U // 2 + 3, 0] -= 60.0
+    E[:, T - 40 - U // 2 - 3:, 0] -= 60.0
+    check_paths(E, P, il, ll)

@@ -33,9 +33,9 @@
 
 namespace rnnt {
 
-int live_blocks(const Dims& d, int* waves);
 int alpha_blocks(const Dims& d);
 int beta_blocks(const Dims& d, int* waves);
+int viterbi_blocks(const Dims& d);
 
 namespace {
 
@@ -394,8 +394,6 @@ __global__ __launch_bounds__(256) void gather_cells_kernel(const TIO* __restrict
 // null for the last block) and the next one reads them from `ghin` (null for the first block).
 // kMulti: this launch is one of several blocks (the hand-over code is compiled in only then: in
 // the single-block kernel even an unused hand-over load costs the walk its prefetch distance).
-constexpr int kLiveLag = 12;      // groups between blocks that the best-path walk runs side by side
-constexpr int kLiveWaveLag = 2;  // groups between the wavefronts of a live block at the start (8 elsewhere)
 template <int C, int W, bool kMulti>
 __global__ __launch_bounds__(64 * W) void alpha_kernel(Planes p, const int* __restrict__ inLen,
                                                        const int* __restrict__ labLen,
@@ -2468,11 +2466,7 @@ __global__ __launch_bounds__(256) void maxplus_index_kernel(const TIO* __restric
 // afterwards.
 // Dynamic LDS: one int per label position (steps at which labels were taken), the hand-over
 // array (W > 1), the columns (kLdsBits; else they live in global memory).
-// kLive (with kMulti, columns in global memory): live_n blocks of 64 C W label positions side by
-// side, one workgroup each, the boundary column's scores crossing in tagged 64-bit entries as in
-// alpha_kernel (same order of workgroups, same bounded waits).  Such a launch only walks; the
-// path is traced by a launch of its own afterwards (traces != 0, u_base past every label).
-template <int C, int W, bool kLdsBits, bool kMulti, bool kLive = false>
+template <int C, int W, bool kLdsBits, bool kMulti>
 __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* __restrict__ bestS,
                                                          const float* __restrict__ argS,
                                                          const int* __restrict__ inLen,
@@ -2483,21 +2477,13 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
                                                          int* __restrict__ trouble, int u_base,
                                                          const float* __restrict__ ghin,
                                                          float* __restrict__ ghout,
-                                                         int traces,
-                                                         unsigned long long* __restrict__ live,
-                                                         int live_n) {
-  static_assert(!kLive || (kMulti && !kLdsBits), "live blocks keep their columns in global memory");
+                                                         int traces) {
   extern __shared__ __attribute__((aligned(16))) int dyn[];
   __shared__ int done[W];  // steps a wavefront has published
   __shared__ __attribute__((aligned(16))) float nothing[4];
-  const int live_block = kLive ? (int)(blockIdx.x >> 3) % live_n : 0;
-  const int b = kLive ? (int)(blockIdx.x / (8 * live_n)) * 8 + (blockIdx.x & 7) : blockIdx.x;
+  const int b = blockIdx.x;
   const int lane = threadIdx.x & 63, tidx = threadIdx.x;
   const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
-  if (kLive) {
-    if (b >= d.B) return;
-    u_base = live_block * 64 * C * W;
-  }
   int Tb, Ub;
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
   if (Tb == 0 || Ub == 0) return;  // :152-154
@@ -2508,48 +2494,20 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
   if (!walks && !traces) return;
   const int nsteps = Tb + Ub - 1;
   const int ngroups = (nsteps + 3) >> 2;
-  int* taken = dyn;                             // [U rounded up to 4] (not in a live launch)
-  float* hand = reinterpret_cast<float*>(dyn + (kLive ? 0 : (d.U + 3) & ~3));  // [W-1][hand_stride]
+  int* taken = dyn;                             // [U rounded up to 4]
+  float* hand = reinterpret_cast<float*>(dyn + ((d.U + 3) & ~3));  // [W-1][hand_stride]
   unsigned* cols = kLdsBits
       ? reinterpret_cast<unsigned*>(hand + (W - 1) * hand_stride)     // [64 C W][nw]
       : gcols + (size_t)b * d.Ua * nw;                                // [Ua][nw]
-  const float* gin = (kMulti && !kLive && ghin) ? ghin + (size_t)b * hand_stride : nullptr;
-  float* gout = (kMulti && !kLive && ghout && walks) ? ghout + (size_t)b * hand_stride : nullptr;
+  const float* gin = (kMulti && ghin) ? ghin + (size_t)b * hand_stride : nullptr;
+  float* gout = (kMulti && ghout && walks) ? ghout + (size_t)b * hand_stride : nullptr;
   if (kMulti && gout && tidx == 0) gout[0] = kNegInf;  // nothing enters step 0
-  // live blocks: block h reads the entries of boundary h - 1 and writes those of boundary h
-  const bool live_in = kLive && live_block > 0, live_out = kLive && live_block < live_n - 1;
-  const unsigned long long* lrow =
-      kLive ? live + ((size_t)max(live_block - 1, 0) * d.B + b) * hand_stride : nullptr;
-  unsigned long long* lrow_out =
-      kLive ? live + ((size_t)min(live_block, max(live_n - 2, 0)) * d.B + b) * hand_stride
-            : nullptr;
-  auto live_entry = [](int s, float x) -> unsigned long long {
-    return ((unsigned long long)(unsigned)(s + 1) << 32) | (unsigned long long)__float_as_uint(x);
-  };
-  auto live_load = [&](int s) -> unsigned long long {
-    return __hip_atomic_load(lrow + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  // (one opaque statement: see alpha_kernel)
-  auto live_reload = [&](int s) -> unsigned long long {
-    unsigned long long e;
-    const unsigned long long* q = lrow + s;
-    asm volatile("global_load_dwordx2 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)"
-                 : "=&v"(e)
-                 : "v"(q)
-                 : "memory");
-    return e;
-  };
-  unsigned live_sink = 0;
-  if (live_out && tidx == 0)  // nothing enters step 0
-    __hip_atomic_store(lrow_out, live_entry(0, kNegInf), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
   if (W > 1) {
     if (tidx < W) done[tidx] = 0;
     if (tidx < W - 1) hand[tidx * hand_stride] = kNegInf;  // nothing enters step 0
     if (tidx < 4) nothing[tidx] = kNegInf;
   }
-  if (!kLive)
-    for (int u = tidx; u < Ub; u += 64 * W) taken[u] = -1;
+  for (int u = tidx; u < Ub; u += 64 * W) taken[u] = -1;
   __syncthreads();
   float* hand_out = hand + wave * hand_stride;                            // wave < W-1
   // wave > 0; wavefront 0 finds there that nothing comes in
@@ -2595,8 +2553,6 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
     float4 ln[C], bs[C];
     float eb[C + 3];
     float4 gh;  // scores entering the block's first column from the block below
-    unsigned long long lv;  // the same, tagged, from the block running beside this one: lane j
-                            // holds entry 4g + j
   };
   auto load_group = [&](int g) -> Group {
     Group r;
@@ -2610,7 +2566,6 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
     if constexpr (kMulti) {
       r.gh = make_float4(kNegInf, kNegInf, kNegInf, kNegInf);
       if (gin) r.gh = *reinterpret_cast<const float4*>(gin + 4 * g);  // uniform
-      if constexpr (kLive) r.lv = live_load(4 * g + (lane & 3));  // every wavefront asks
     }
     return r;
   };
@@ -2629,7 +2584,6 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
     if constexpr (kMulti) {
       r.gh = make_float4(kNegInf, kNegInf, kNegInf, kNegInf);
       if (gin) r.gh = *reinterpret_cast<const float4*>(gin + 4 * g);  // uniform
-      if constexpr (kLive) r.lv = live_load(4 * g + (lane & 3));
     }
     return r;
   };
@@ -2654,29 +2608,6 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
     constexpr bool kInterior = decltype(interior)::value;
     float4 hin = {kNegInf, kNegInf, kNegInf, kNegInf};
     if constexpr (kMulti) hin = cur.gh;  // wavefront 0: from the block below (or nothing)
-    if constexpr (kLive) {
-      if (live_in && wave == 0) {  // uniform; as in alpha_kernel
-        unsigned long long e = cur.lv;
-        if (__builtin_amdgcn_ballot_w64(lane < 4 &&
-                                        (unsigned)(e >> 32) != (unsigned)(4 * g + lane + 1))) {
-          const int mine = lane < 4 ? 4 * g + lane : min(4 * ngroups, 4 * (g + kLiveLag));
-          int spins = 0;
-          do {
-            if (spins++ >= spin_limit) {
-              if (lane == 0) raise_trouble(trouble);
-              break;
-            }
-            __builtin_amdgcn_s_sleep(4);
-            e = live_reload(mine);
-          } while (__builtin_amdgcn_ballot_w64((unsigned)(e >> 32) != (unsigned)(mine + 1)));
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          f4set(hin, j, __int_as_float(__builtin_amdgcn_readlane((int)(unsigned)e, j)));
-      } else {
-        live_sink ^= (unsigned)cur.lv;
-      }
-    }
     if constexpr (W > 1) {
       if (!kMulti) hin = hand_cur;
       else if (wave > 0) hin = hand_cur;
@@ -2711,14 +2642,6 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
 #pragma unroll
         for (int j = 0; j < 4; ++j) gout[4 * g + 1 + j] = gsend[j];
       }
-      if constexpr (kLive) {
-        if (live_out && wave == W - 1 && lane == 63) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            __hip_atomic_store(lrow_out + 4 * g + 1 + j, live_entry(4 * g + 1 + j, gsend[j]),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
     }
     if ((g & 7) == 7 || g == ngroups - 1) {  // uniform: a word of 32 steps is complete
 #pragma unroll
@@ -2737,24 +2660,11 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
   };
   // four register sets rotate (no copies): a group's loads are requested four groups ahead
   auto clamp_g = [&](int g) { return g < ngroups ? g : ngroups - 1; };
-  if constexpr (kLive) {
-    if (live_in && wave == 0) {  // start kLiveLag groups behind the block below (or when it is done)
-      const int far = min(4 * ngroups, 4 * kLiveLag);
-      int spins = 0;
-      while ((unsigned)(live_load(far) >> 32) != (unsigned)(far + 1)) {
-        if (spins++ >= spin_limit) {
-          if (lane == 0) raise_trouble(trouble);
-          break;
-        }
-        __builtin_amdgcn_s_sleep(8);
-      }
-    }
-  }
   Group q0 = load_group(0), q1 = load_group(clamp_g(1)), q2 = load_group(clamp_g(2)),
         q3 = load_group(clamp_g(3));
   const int nwalk = walks ? ngroups : 0;  // a block past the utterance's labels only traces
   if (W > 1 && wave > 0 && walks)
-    wait_for(min(4 * ngroups, 4 * (kLive ? kLiveWaveLag : 8) * wave));  // fall a few groups behind
+    wait_for(min(4 * ngroups, 4 * 8 * wave));  // fall a few groups behind
   const std::true_type inner;
   const std::false_type edge;
   float4 h0 = make_float4(kNegInf, kNegInf, kNegInf, kNegInf), h1 = h0;
@@ -2780,9 +2690,6 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
     q2 = load_group(clamp_g(g + 6));
     if (g + 3 < ngroups) run_group(g + 3, q3, h1, h0, edge);
     q3 = load_group(clamp_g(g + 7));
-  }
-  if constexpr (kLive) {
-    if (spin_limit < 0 && live_sink == 1u) raise_trouble(trouble);  // never
   }
   if (!kLdsBits) __threadfence();  // the columns in global memory, before another lane reads them
   __syncthreads();
@@ -2814,6 +2721,317 @@ __global__ __launch_bounds__(64 * W) void viterbi_kernel(Planes p, const float* 
     // inside the plane whatever the decision bits hold)
     if (st >= 0) out[u1] = argI[plane_at(d, b, u1, max(st - 1, 0))];
   }
+}
+
+// ------------------------------------------------------------------ backtrace
+// transducer/transducer_cpu.cpp:208-219, from (T_b - 1, U_b - 1): a set bit at (step, u) means
+// "entered from u - 1 with a label", a clear one "entered from t - 1 with a blank", so the step at
+// which position v was entered is the highest set bit at or below the running step in column v.
+// A wavefront finds it with one comparison over 64 words (lane k holds the k-th word down from the
+// path's) and reads kBatch columns at a time; one lane that read a word, tested it and read the next
+// took 100 ns a position from LDS (45 so) and most of a microsecond from memory.
+// taken[v - 1]: the step at which position v was entered; it stays as it is where there is none.
+template <int kBatch, typename Word>
+__device__ inline void trace_path(int v, int s, int* taken, Word word) {
+  const int lane = threadIdx.x & 63;
+  while (v > 0 && s >= 0) {
+    const int w0 = s >> 5;
+    unsigned m[kBatch];
+#pragma unroll
+    for (int c = 0; c < kBatch; ++c)
+      m[c] = word(max(v - c, 0), max(w0 - lane, 0));
+    int step = -1, done = 0;
+    bool more = true;
+#pragma unroll
+    for (int c = 0; c < kBatch; ++c) {
+      if (more && v - c > 0 && s >= 0) {  // uniform
+        const int k0 = w0 - (s >> 5);  // the lane whose word holds step s
+        const unsigned upto = 0xFFFFFFFFu >> (31 - (s & 31));
+        unsigned x = lane == k0 ? m[c] & upto : m[c];
+        x = lane < k0 || lane > w0 ? 0u : x;
+        const unsigned long long any = __builtin_amdgcn_ballot_w64(x != 0u);
+        if (any == 0ull) {  // not in these 2048 steps
+          s = min(s, 32 * (w0 - 63) - 1);
+          more = false;
+        } else {
+          const int f = __builtin_ctzll(any);
+          const unsigned y = __builtin_amdgcn_readlane(x, f);
+          const int st = 32 * (w0 - f) + 31 - __builtin_clz(y);
+          step = lane == c ? st : step;
+          s = st - 1;
+          done = c + 1;
+        }
+      }
+    }
+    if (lane < done) taken[v - 1 - lane] = step;
+    v -= done;
+  }
+}
+// The labels of the path.  (A label is never taken at step 0 on a lattice that was walked; the clamp
+// keeps the read inside the plane whatever the decision bits hold.)
+__device__ inline void put_labels(const int* taken, const float* __restrict__ argS,
+                                  int* __restrict__ labels_out, const Dims& d, int b, int Ub,
+                                  int threads) {
+  int* out = labels_out + (size_t)b * (d.U - 1);
+  const int* argI = reinterpret_cast<const int*>(argS);
+  for (int v = threadIdx.x; v < Ub - 1; v += threads) {
+    const int st = taken[v];
+    if (st >= 0) out[v] = argI[plane_at(d, b, v, max(st - 1, 0))];
+  }
+}
+
+// ------------------------------------------------------------------ best path, one position a lane
+// The same walk with one label position a lane, its wavefronts, blocks and hand-over those of
+// alpha_walk_kernel.  A step is nine instructions: the lane shift, one comparison, two that use it
+// (the larger score; the decision shifted into the lane's word by an addition with carry), the five
+// of the two moves.  Operands are asked for eight groups ahead.  32 ns a step on one wavefront, 43
+// with a neighbour; B=8 T=2000, walk and backtrace: 101 positions 142 -> 107 us, 201 226 -> 129,
+// 401 392 -> 181 (half of that was the backtrace, a word at a time from memory).
+// kLdsBits: the decision columns fit into LDS, and the workgroup traces the path at the end.
+// Otherwise they go to global memory and viterbi_trace_kernel follows.
+template <int W, bool kLive, bool kLdsBits>
+__global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void viterbi_walk_kernel(
+    Planes p, const float* __restrict__ bestS, const float* __restrict__ argS,
+    const int* __restrict__ inLen, const int* __restrict__ labLen, unsigned* __restrict__ gcols,
+    int* __restrict__ labels_out, Dims d, int nw, int spin_limit, int* __restrict__ trouble,
+    unsigned long long* __restrict__ live, int live_n) {
+  static_assert(!kLive || !kLdsBits, "blocks side by side keep their columns in global memory");
+  constexpr bool kHand = W > 1 || kLive;
+  constexpr int kDepth = 8;
+  extern __shared__ __attribute__((aligned(16))) int dyn[];  // kLdsBits: [U up to 4] steps at which
+                                                             // labels were taken, then the columns
+  __shared__ __attribute__((aligned(16))) float ring[W + 1][kHand ? 4 * kRingGroups : 4];
+  __shared__ __attribute__((aligned(16))) float nothing[16];
+  __shared__ __attribute__((aligned(16))) float dump[kHand ? 4 * 64 + 16 : 4];
+  __shared__ int prog[W + 2];
+  const int live_block = kLive ? (int)(blockIdx.x >> 3) % live_n : 0;
+  const int b = kLive ? (int)(blockIdx.x / (8 * live_n)) * 8 + (blockIdx.x & 7) : blockIdx.x;
+  if (kLive && b >= d.B) return;
+  const int u_base = live_block * 64 * W;
+  const int lane = threadIdx.x & 63;
+  const int wave = kHand ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  int Tb, Ub;
+  utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
+  if (Tb == 0 || Ub == 0) return;  // :152-154
+  if (u_base >= Ub) return;
+  const int nsteps = Tb + Ub - 1;
+  const int ngroups = (nsteps + 3) >> 2;
+  const bool live_in = kLive && live_block > 0;
+  const bool live_out = kLive && live_block < live_n - 1 && u_base + 64 * W < Ub;
+  int* taken = dyn;
+  unsigned* cols = kLdsBits ? reinterpret_cast<unsigned*>(dyn + ((d.U + 3) & ~3))  // [64 W][nw]
+                            : gcols + (size_t)b * d.Ua * nw;                       // [Ua][nw]
+  if (threadIdx.x < 16) nothing[threadIdx.x] = kNegInf;
+  if (threadIdx.x < W + 2) {
+    const int w = (int)threadIdx.x - 1;  // the wavefront whose progress this is
+    prog[threadIdx.x] = w < 0 ? (live_in ? 0 : kForever)
+                        : w == W ? (live_out ? 0 : kForever)
+                                 : (u_base + 64 * w < Ub ? 0 : kForever);
+  }
+  if constexpr (kLdsBits)
+    for (int u = threadIdx.x; u < Ub; u += 64 * W) taken[u] = -1;
+  __syncthreads();
+  if (kLive && wave == W) {
+    const unsigned long long* src =
+        live_in ? live + ((size_t)(live_block - 1) * d.B + b) * d.Dp : nullptr;
+    unsigned long long* dst = live_out ? live + ((size_t)live_block * d.B + b) * d.Dp : nullptr;
+    live_carrier<0>(src, dst, ngroups, [](int g, int i) { return 4 * g + 1 + i; }, ring[0], &prog[0],
+                    &prog[1], ring[W], &prog[W], &prog[W + 1], spin_limit, trouble);
+    return;
+  }
+  const int u_lo = u_base + wave * 64;
+  const int u = u_lo + lane;
+  if (u_lo < Ub) {  // uniform: else a wavefront past this utterance's labels
+    if (kLive) __builtin_amdgcn_s_setprio(3);  // ahead of the carrier on the same SIMD
+    const bool first_column = u_lo == 0;
+    const float pb = p.pb[(size_t)b * d.Ua + min(u, d.U - 1)];
+    // cell (0,0) finds 0 coming up from below (:157) and nothing from the left
+    float stay = u == 0 ? 0.0f : kNegInf, emit = kNegInf;
+    unsigned bits = 0;
+    // Groups from in_lo on need not ask whether a cell has started; cells past the utterance run on
+    // whatever the planes hold and are never consulted.
+    const int in_lo = (min(u_lo + 64, Ub) + 2) >> 2;
+    const unsigned gbytes = kLive ? 16u * (unsigned)d.Ua : 1024u * W;  // from a group to the next
+    const size_t plane = (size_t)gbytes * (unsigned)(d.Dp / 4);
+    const char* ln_b = reinterpret_cast<const char*>(p.lnS + plane_group0(d, b, 0));
+    const char* bs_b = reinterpret_cast<const char*>(bestS + plane_group0(d, b, 0));
+    // (buffers that begin at group `origin`, moved on before an offset would outgrow 32 bits)
+    Buffer ln_q(ln_b, plane), bs_q(bs_b, plane);
+    const Buffer eb_q(p.eb + (size_t)b * d.Tp, 4ull * d.Tp);
+    int origin = 0;
+    const int span = (int)((1u << 30) / gbytes);
+    const unsigned lane_o = 16u * (unsigned)min(u, d.U - 1);
+    const unsigned eb_o = 4u * (unsigned)(d.Eo - u);
+    struct Ops {
+      quad_t ln, bs, eb;
+    };
+    auto load = [&](int g) -> Ops {
+      g = min(g, ngroups - 1);
+      const unsigned by = (unsigned)(g - origin) * gbytes;
+      Ops r;
+      r.ln = ln_q.load(lane_o, by);
+      r.bs = bs_q.load(lane_o, by);
+      r.eb = eb_q.load(eb_o, 16u * (unsigned)g);
+      return r;
+    };
+    // ---- hand-over (see alpha_walk_kernel)
+    int ok = kHand ? -1 : kForever;
+    int have_in = 0, have_out = 0;
+    auto refresh = [&](int g) {
+      have_in = bounded_wait(&prog[wave], have_in, min(g + 5, ngroups), spin_limit, trouble);
+      have_out = bounded_wait(&prog[wave + 2], have_out, g + 18 - kRingGroups, spin_limit, trouble);
+      ok = min(have_in >= ngroups ? kForever : have_in - 3,
+               min(have_out, kForever) + kRingGroups - 4);
+    };
+    const float* take = kHand ? (first_column ? nothing : ring[wave]) : nullptr;
+    const int take_mask = first_column ? 0 : kRingGroups / 4 - 1;
+    float* give = kHand ? (lane == 63 ? ring[wave + 1] : dump + 4 * lane) : nullptr;
+    const int give_mask = lane == 63 ? kRingGroups / 4 - 1 : 0;
+    int* give_prog = lane == 63 ? &prog[wave + 1] : reinterpret_cast<int*>(dump + 4 * lane);
+    quad_t pend = {kNegInf, kNegInf, kNegInf, kNegInf}, hand = pend;
+    float carry = kNegInf;
+    auto run_group = [&](int g, const Ops& q, const float* take_next, float* give_last, auto tell,
+                         auto inner) {
+      constexpr bool kInner = decltype(inner)::value;
+      quad_t next = hand;
+      if constexpr (kHand) {
+        *reinterpret_cast<quad_t*>(give_last) = pend;
+        asm volatile("" ::: "memory");  // (LDS serves a wavefront's requests in order)
+        if constexpr (decltype(tell)::value) prog_store(give_prog, g);
+        next = *reinterpret_cast<const quad_t*>(take_next);
+      }
+      float in[4] = {carry, hand[0], hand[1], hand[2]};
+      if constexpr (!kHand) {  // (set well ahead of the lane shifts that fill lane 0 from them)
+        in[0] = in[1] = in[2] = in[3] = kNegInf;
+        asm volatile("" : "+v"(in[0]), "+v"(in[1]), "+v"(in[2]), "+v"(in[3]));
+      }
+      quad_t em;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float left = wave_shr1(emit, in[j]);
+        const bool takes = left > stay;  // :200-206 ties go to blank
+        const float x = takes ? left : stay;
+        bits = bits + bits + (takes ? 1u : 0u);
+        float se = x + q.bs[j];
+        float sb = x + q.eb[j];
+        se = se - q.ln[j];
+        sb = sb + pb;
+        sb = sb - q.ln[j];
+        if constexpr (kInner) {
+          stay = sb;
+          emit = se;
+        } else {
+          const bool started = 4 * g + j >= u;
+          stay = started ? sb : kNegInf;
+          emit = started ? se : kNegInf;
+        }
+        em[j] = emit;
+      }
+      pend = em;
+      carry = hand[3];
+      hand = next;
+    };
+    // a word of 32 steps, the first of them in bit 0 (the last word may hold fewer)
+    auto put_word = [&](int g) {
+      cols[(size_t)u * nw + (g >> 3)] = __brev(bits << (28 - 4 * (g & 7)));
+      bits = 0u;
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    Ops q[kDepth];
+#pragma unroll
+    for (int k = 0; k < kDepth; ++k) q[k] = load(k);
+    if constexpr (kHand) {
+      if (!first_column) {
+        refresh(0);
+        hand = *reinterpret_cast<const quad_t*>(take);
+      }
+    }
+    // groups g .. g + 3, an aligned block of slots; kWhole: all of them exist
+    auto four = [&](int g, Ops* w, auto whole, auto inner) {
+      constexpr bool kWhole = decltype(whole)::value;
+      const float *tk = nullptr, *tk_next = nullptr;
+      float *gv = nullptr, *gv_last = nullptr;
+      if constexpr (kHand) {
+        tk = take + 16 * ((g >> 2) & take_mask);
+        tk_next = take + 16 * (((g >> 2) + 1) & take_mask);
+        gv = give + 16 * ((g >> 2) & give_mask);
+        gv_last = give + 16 * (((g >> 2) - 1) & give_mask) + 12;
+        if (__builtin_expect(g > ok, 0)) refresh(g);
+      }
+      run_group(g, w[0], tk + 4, gv_last, yes, inner);
+      if (kWhole) w[0] = load(g + kDepth);
+      if (kWhole || g + 1 < ngroups) run_group(g + 1, w[1], tk + 8, gv, no, inner);
+      if (kWhole) w[1] = load(g + 1 + kDepth);
+      if (kWhole || g + 2 < ngroups) {
+        if constexpr (kHand) {
+          if (__builtin_expect(g + 2 > ok, 0)) refresh(g + 2);
+        }
+        run_group(g + 2, w[2], tk + 12, gv + 4, yes, inner);
+      }
+      if (kWhole) w[2] = load(g + 2 + kDepth);
+      if (kWhole || g + 3 < ngroups) run_group(g + 3, w[3], tk_next, gv + 8, no, inner);
+      if (kWhole) w[3] = load(g + 3 + kDepth);
+      if constexpr (kHand && kWhole) __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): see alpha
+    };
+    int g = 0;
+    for (; g + 8 <= ngroups && g < in_lo; g += 8) {
+      four(g, q, yes, no);
+      four(g + 4, q + 4, yes, no);
+      put_word(g + 7);
+    }
+    for (; g + 8 <= ngroups; g += 8) {
+      if (g - origin >= span) {
+        origin = g;
+        const size_t by = (size_t)g * gbytes;
+        ln_q = Buffer(ln_b + by, plane - by);
+        bs_q = Buffer(bs_b + by, plane - by);
+      }
+      four(g, q, yes, yes);
+      four(g + 4, q + 4, yes, yes);
+      put_word(g + 7);
+    }
+    if (g < ngroups) {
+      four(g, q, no, no);
+      if (g + 4 < ngroups) four(g + 4, q + 4, no, no);
+      put_word(ngroups - 1);
+    }
+    if constexpr (kHand) {
+      *reinterpret_cast<quad_t*>(give + 16 * (((ngroups - 1) >> 2) & give_mask) +
+                                 4 * ((ngroups - 1) & 3)) = pend;
+      asm volatile("" ::: "memory");
+      prog_store(give_prog, ngroups);
+    }
+  }
+  if constexpr (kLdsBits) {
+    __syncthreads();
+    if (wave == 0)
+      trace_path<8>(Ub - 1, nsteps - 1, taken, [&](int v, int w) { return cols[v * nw + w]; });
+    __syncthreads();
+    put_labels(taken, argS, labels_out, d, b, Ub, 64 * W);
+  }
+}
+
+// The backtrace from decision columns in global memory, one wavefront an utterance.
+// Dynamic LDS: one int per label position.
+__global__ __launch_bounds__(64) void viterbi_trace_kernel(const float* __restrict__ argS,
+                                                           const int* __restrict__ inLen,
+                                                           const int* __restrict__ labLen,
+                                                           const unsigned* __restrict__ gcols,
+                                                           int* __restrict__ labels_out, Dims d,
+                                                           int nw) {
+  extern __shared__ __attribute__((aligned(16))) int taken[];
+  const int b = blockIdx.x;
+  int Tb, Ub;
+  utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
+  if (Tb == 0 || Ub <= 1) return;
+  for (int u = threadIdx.x; u < Ub; u += 64) taken[u] = -1;
+  __syncthreads();
+  const unsigned* cols = gcols + (size_t)b * d.Ua * nw;
+  trace_path<24>(Ub - 1, Tb + Ub - 2, taken,
+                 [&](int v, int w) { return cols[(size_t)v * nw + w]; });
+  __syncthreads();
+  put_labels(taken, argS, labels_out, d, b, Ub, 64);
 }
 
 // ------------------------------------------------------------------ chain-latency floor
@@ -2982,26 +3200,6 @@ int trouble_flag(int** out) {
 // ------------------------------------------------------------------ workspace layout
 static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Blocks of label positions that the alpha and dalpha walks run side by side, one workgroup of
-// `waves` wavefronts (one position a lane) each: four wavefronts, 256 positions, while their
-// three hand-over arrays fit LDS (up to about 12000 anti-diagonals); two wavefronts, 128
-// positions, with their one array up to about 36000.  0 blocks where one workgroup takes the
-// label axis as well or better: up to 256 positions on four wavefronts, up to 128 on two; and,
-// up to 1024 positions, where the batch would need more workgroups than the device has CUs to
-// spare (with that many utterances the planes' traffic holds the walks either way).  Past 1024
-// positions the blocks go side by side whatever the batch: workgroups are dispatched in order,
-// a block after the block it follows, so more workgroups than CUs only queue -- and the other
-// way there, a launch per 1024 positions with sixteen positions a lane, is many times slower.
-int live_blocks(const Dims& d, int* waves) {
-  const size_t one = sizeof(float) * (size_t)d.Dp;
-  const int W = 3 * one <= 144 * 1024 ? 4 : one <= 144 * 1024 ? 2 : 0;
-  if (waves) *waves = W;
-  if (W == 0) return 0;
-  const int n = (d.U + 64 * W - 1) / (64 * W);
-  if (n < 2 || n > 16) return 0;
-  if (d.B * n > 192 && d.U <= 1024) return 0;
-  return n;
-}
 // Blocks of 256 label positions that the alpha walk runs side by side (1: none).  Up to 1024
 // positions the other way is one workgroup with two or four positions a lane, whose one CU holds it:
 // T=2000, 401 positions 663 -> 381 us at B=128, 1000 positions 1724 -> 541 at B=64.  With more
@@ -3031,13 +3229,19 @@ int beta_blocks(const Dims& d, int* waves) {
   *waves = 4;
   return alpha_blocks(d);
 }
+// Blocks of 256 label positions that the best-path walk runs side by side (1: none): alpha's rule,
+// with three blocks or more only up to 192 workgroups, so that the decode's scratch stays what it is.
+int viterbi_blocks(const Dims& d) {
+  const int n = alpha_blocks(d);
+  return n > 2 && (long)d.B * n > 192 && d.U <= 1024 ? 1 : n;
+}
 // The two hand-over vectors of the planes hold the walks' tagged 64-bit entries as well: one
 // array of [B][Dp] entries per boundary between blocks side by side.  In units of [B][Dp] floats
 // each.
 static int hand_arrays(const Dims& d, bool decode_only) {
-  int w, n = live_blocks(d, nullptr);
-  if (!decode_only) n = std::max(n, std::max(alpha_blocks(d), beta_blocks(d, &w)));
-  return std::max(1, n - 1);
+  int w;
+  return std::max(1, (decode_only ? viterbi_blocks(d)
+                                  : std::max(alpha_blocks(d), beta_blocks(d, &w))) - 1);
 }
 
 size_t planes_bytes(const Dims& d, bool decode_only) {
@@ -3136,27 +3340,6 @@ static int clear_live(unsigned long long* live, const Dims& d, int n, hipStream_
   hipLaunchKernelGGL(clear_words_kernel, dim3((words + 255) / 256), dim3(256), 0, s,
                      reinterpret_cast<int*>(live), words);
   RNNT_LAUNCH_CHECK("clear_words_kernel");
-  return kOk;
-}
-
-// Launches the side-by-side form of a walk (K: its kernel, W wavefronts of one position a lane)
-// for n blocks: clears the tagged entries, then one workgroup per utterance and block, eight
-// utterances' blocks in consecutive indices.
-template <typename K, typename... Args>
-static int launch_live(K kernel, const Planes& p, const Dims& d, int n, int W,
-                       hipStream_t s, Args... args) {
-  unsigned long long* live = reinterpret_cast<unsigned long long*>(p.hand[0]);
-  const size_t lds = sizeof(float) * (size_t)(W - 1) * d.Dp;
-  const int words = 2 * d.B * d.Dp * (n - 1);
-  hipLaunchKernelGGL(clear_words_kernel, dim3((words + 255) / 256), dim3(256), 0, s,
-                     reinterpret_cast<int*>(live), words);
-  RNNT_LAUNCH_CHECK("clear_words_kernel");
-  if (lds > 64 * 1024)
-    RNNT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(kernel, dim3(8 * n * ((d.B + 7) / 8)), dim3(64 * W), lds, s, args..., live,
-                     n);
-  RNNT_LAUNCH_CHECK("lattice walk (blocks side by side)");
   return kOk;
 }
 
@@ -3480,6 +3663,47 @@ int launch_maxplus(const f16_t* E, const f16_t* P, const int* inLen, const int* 
 // 32-step words per column of the decision table (one spare)
 static int viterbi_words(const Dims& d) { return (d.T + d.U + 31) / 32 + 1; }
 
+template <int W, bool kLive, bool kLdsBits>
+static int viterbi_walk(const Planes& p, const float* bestS, const float* argS, unsigned* gcols,
+                        const int* inLen, const int* labLen, int* labels_out, const Dims& d, int nw,
+                        hipStream_t s, dim3 grid, size_t lds, int n) {
+  int* trouble = nullptr;
+  RNNT_TRY(trouble_flag(&trouble));
+  unsigned long long* live = reinterpret_cast<unsigned long long*>(p.hand[0]);
+  if (kLive) RNNT_TRY(clear_live(live, d, n, s));
+  const auto kernel = viterbi_walk_kernel<W, kLive, kLdsBits>;
+  if (lds > 48 * 1024)
+    RNNT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(kernel, grid, dim3(64 * (W + (kLive ? 1 : 0))), lds, s, p, bestS, argS, inLen,
+                     labLen, gcols, labels_out, d, nw, g_spin_limit, trouble, live, n);
+  RNNT_LAUNCH_CHECK("viterbi_walk_kernel");
+  if (!kLdsBits) {
+    hipLaunchKernelGGL(viterbi_trace_kernel, dim3(d.B), dim3(64), sizeof(int) * (size_t)d.U, s, argS, inLen, labLen, gcols,
+                       labels_out, d, nw);
+    RNNT_LAUNCH_CHECK("viterbi_trace_kernel");
+  }
+  return kOk;
+}
+
+// One position a lane: one workgroup up to 256 label positions, else blocks of 256 side by side.
+// The decision columns stay in LDS if two workgroups of them fit a CU, or one where there is a CU
+// for each; the path is then traced from there, without a launch of its own.
+static int launch_viterbi_walk(const Planes& p, const float* bestS, const float* argS,
+                               unsigned* gcols, const int* inLen, const int* labLen,
+                               int* labels_out, const Dims& d, int nw, hipStream_t s) {
+  const int W = d.U <= 64 ? 1 : d.U <= 128 ? 2 : 4, n = viterbi_blocks(d);
+  const size_t lds = sizeof(int) * (((size_t)d.U + 3 & ~(size_t)3) + (size_t)64 * W * nw);
+  const bool fits = n == 1 && lds <= (d.B <= 256 ? 140u : 60u) * 1024;
+  const dim3 one(d.B);
+#define WALK(W, LIVE, LDS, GRID, BYTES)                                                               viterbi_walk<W, LIVE, LDS>(p, bestS, argS, gcols, inLen, labLen, labels_out, d, nw, s, GRID, BYTES, n)
+  if (n > 1) return WALK(4, true, false, dim3(8 * n * ((d.B + 7) / 8)), 0);
+  if (W == 1) return fits ? WALK(1, false, true, one, lds) : WALK(1, false, false, one, 0);
+  if (W == 2) return fits ? WALK(2, false, true, one, lds) : WALK(2, false, false, one, 0);
+  return fits ? WALK(4, false, true, one, lds) : WALK(4, false, false, one, 0);
+#undef WALK
+}
+
 int launch_viterbi(const Planes& p, const float* bestS, const float* argS,
                    unsigned long long* gbits, const int* inLen, const int* labLen,
                    int* labels_out, const Dims& d, hipStream_t s) {
@@ -3488,10 +3712,9 @@ int launch_viterbi(const Planes& p, const float* bestS, const float* argS,
   const int cpl = block_cells_per_lane(d), nblocks = label_blocks(d);
   const int stride = d.Dp;
   const int nw = viterbi_words(d);
-  // (four wavefronts from 129 label positions while their hand-over arrays fit: B=8 T=2000,
-  // 209 -> 167 ns a step at 257 positions, 446 -> 254 at 513, 551 -> 340 at 1000)
-  // (B=8 T=10000 U=400, the reference's kernel benchmark: 3.5 ms with one wavefront of eight
-  // positions a lane, which is what 64 KB of LDS allowed)
+  if (d.U <= 256 || viterbi_blocks(d) > 1)
+    return launch_viterbi_walk(p, bestS, argS, gcols, inLen, labLen, labels_out, d, nw, s);
+  // several positions a lane, on four wavefronts while their hand-over arrays fit
   const size_t taken_lds = sizeof(int) * (size_t)((d.U + 3) & ~3);
   const int W = (nblocks == 1 && cpl >= 4 &&
                  taken_lds + 3 * stride * sizeof(float) <= 144 * 1024) ? 4
@@ -3509,22 +3732,6 @@ int launch_viterbi(const Planes& p, const float* bestS, const float* argS,
                 stride, lds);
   int* trouble = nullptr;
   RNNT_TRY(trouble_flag(&trouble));
-  // Blocks of 256 label positions side by side where alpha_kernel takes them so (four wavefronts
-  // whose hand-over arrays fit LDS), then one launch that only traces the path (B=8 T=10000
-  // U=400: 1.65 ms for the walk on one CU, four wavefronts of two positions a lane).
-  int live_w = 0;
-  if (const int n = live_blocks(d, &live_w); n && live_w == 4) {
-    RNNT_TRY(launch_live(viterbi_kernel<1, 4, false, true, true>, p, d, n, 4, s, p, bestS, argS,
-                         inLen, labLen, gcols, labels_out, d, stride, nw, g_spin_limit, trouble, 0,
-                         (const float*)nullptr, (float*)nullptr, 0));
-    const size_t trace_lds = sizeof(int) * (size_t)((d.U + 3) & ~3);
-    hipLaunchKernelGGL((viterbi_kernel<1, 1, false, true>), dim3(d.B), dim3(64), trace_lds, s, p,
-                       bestS, argS, inLen, labLen, gcols, labels_out, d, stride, nw, g_spin_limit,
-                       trouble, d.Ua, (const float*)nullptr, (float*)nullptr, 1,
-                       (unsigned long long*)nullptr, 0);
-    RNNT_LAUNCH_CHECK("viterbi_kernel (trace)");
-    return kOk;
-  }
   for (int k = 0; k < nblocks; ++k) {  // lowest block first; the last launch traces the path
     const float* ghin = k == 0 ? nullptr : p.hand[(k - 1) & 1];
     float* ghout = k == nblocks - 1 ? nullptr : p.hand[k & 1];
@@ -3535,7 +3742,7 @@ int launch_viterbi(const Planes& p, const float* bestS, const float* argS,
     if (use_lds)                                                                               \
       hipLaunchKernelGGL((viterbi_kernel<C, W, true, false>), dim3(d.B), dim3(64 * W), lds,   \
                          s, p, bestS, argS, inLen, labLen, gcols, labels_out, d, stride, nw,   \
-                         g_spin_limit, trouble, u_base, ghin, ghout, traces, nullptr, 0);      \
+                         g_spin_limit, trouble, u_base, ghin, ghout, traces);                  \
     else {                                                                                     \
       if (lds > 64 * 1024)                                                                     \
         RNNT_HIP(hipFuncSetAttribute(                                                          \
@@ -3543,7 +3750,7 @@ int launch_viterbi(const Planes& p, const float* bestS, const float* argS,
             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                            \
       hipLaunchKernelGGL((viterbi_kernel<C, W, false, false>), dim3(d.B), dim3(64 * W), lds,  \
                          s, p, bestS, argS, inLen, labLen, gcols, labels_out, d, stride, nw,   \
-                         g_spin_limit, trouble, u_base, ghin, ghout, traces, nullptr, 0);      \
+                         g_spin_limit, trouble, u_base, ghin, ghout, traces);                  \
     }                                                                                          \
     break;
 #define CASE_MULTI(C, W)                                                                       \
@@ -3554,11 +3761,9 @@ int launch_viterbi(const Planes& p, const float* bestS, const float* argS,
           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                              \
     hipLaunchKernelGGL((viterbi_kernel<C, W, false, true>), dim3(d.B), dim3(64 * W), lds, s,  \
                        p, bestS, argS, inLen, labLen, gcols, labels_out, d, stride, nw,        \
-                       g_spin_limit, trouble, u_base, ghin, ghout, traces, nullptr, 0);        \
+                       g_spin_limit, trouble, u_base, ghin, ghout, traces);                    \
     break;
-      CASE(1, 1) CASE(2, 1) CASE(4, 1) CASE(8, 1) CASE(16, 1)
-      CASE(1, 2) CASE(2, 2) CASE(4, 2) CASE(8, 2)
-      CASE(1, 4) CASE(2, 4) CASE(4, 4)
+      CASE(8, 1) CASE(16, 1) CASE(4, 2) CASE(8, 2) CASE(2, 4) CASE(4, 4)
       CASE_MULTI(16, 1) CASE_MULTI(8, 2)  // several blocks: always 1024 positions each
 #undef CASE
 #undef CASE_MULTI
