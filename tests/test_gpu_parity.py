@@ -663,6 +663,25 @@ def test_whole_loss_cfg1(cfg, seed):
         assert_close(pg, f["pgrads"], what="pgrads vs reference fixture")
 
 
+@pytest.mark.parametrize("V", [3, 20, 31, 33, 64, 95, 100, 129, 161, 300])
+@pytest.mark.parametrize("T,U", [(66, 40), (130, 101), (70, 200)])
+def test_label_scores_picked_out_of_few_slabs_of_columns(T, U, V):
+    """The log-normaliser copies E[t, label] out of the rows it streams, 32 columns at a time: one or
+    two of a slab's columns from registers, more through LDS, 64 entries at a time -- repeated
+    labels, labels that are the blank, more than 64 entries in a slab, one to ten slabs (the
+    requests run four slabs ahead).  A wrong score of one frame would move the cost by far more than
+    the bound: an fp32 sum of T + U moves of rounding 2^-24 each relative to its size."""
+    rng = np.random.default_rng(1000 * T + 10 * U + V)
+    E = rng.standard_normal((3, T, V), dtype=np.float32)
+    P = rng.standard_normal((3, U, V), dtype=np.float32)
+    labels = rng.integers(0, V, (3, U - 1)).astype(np.int32)
+    labels[1] = V - 1
+    il, ll = np.array([T, T - 1, T // 2], np.int32), np.array([U - 1, U // 2, U - 1], np.int32)
+    want = oracle.loss_and_grads(E, P, labels, il, ll, lse="naive")
+    costs, _, _ = gpu_loss(DeviceCase(E, P, labels, il, ll))
+    assert np.all(np.abs(costs - want["costs"]) <= (T + U) * 2.0 ** -24 * np.abs(want["costs"]))
+
+
 @pytest.mark.parametrize("T,U,V", [(60, 150, 36), (60, 150, 37), (40, 260, 16), (33, 113, 520),
                                    (40, 111, 520), (40, 112, 520), (36, 223, 516), (36, 224, 1028),
                                    (20, 500, 64), (33, 113, 528), (70, 100, 528)])

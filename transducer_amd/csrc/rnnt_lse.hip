@@ -161,6 +161,12 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
   constexpr int NR = 4 * kRows / kThreads;  // (row, eight v) items a thread stages per slab
   constexpr int kSlots = kRows * 4;        // 16-byte slots per piece plane: 4 per row
   static_assert(MB >= 1 && NR >= 1, "a tile gives every wavefront a frame block and every thread a row");
+  // Slabs between the request for a slab's emissions (Y fragments) and their use.  Tiles of 64
+  // frames are for grids with about a workgroup per CU, where nothing else covers the round trip to
+  // memory: a slab then took that long, 2 us (B=8 T=2000 U=101 V=1000: 66 us for 32 slabs, half
+  // that with the requests four slabs ahead).  At 128 frames two workgroups cover for each other
+  // and the registers are taken.
+  constexpr int kAhead = kRows == 64 ? 4 : 1, kYAhead = kRows == 64 ? 2 : 1;
   __shared__ uint4 Xs[2][3][kSlots];
   __shared__ float scale[kRows];  // pending factor for a row's sums (1 when its reference stood)
   __shared__ float mfin[kRows];   // final references, for the write-out
@@ -168,12 +174,15 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
   __shared__ int labs[1025];      // columns to pick: the utterance's labels, then the blank
   __shared__ short order[1025];   // their indices sorted by column
   __shared__ int scol[1025];      // and the columns in that order
+  __shared__ float raw[kRows == 64 ? 64 : 1][kSlice + 1];  // a slab's scores (picks)
   // XCD-aware renumbering: physical id n runs on XCD n % 8
   const int n = blockIdx.x, per_xcd = gridDim.x >> 3;
   const int logical = (n & 7) * per_xcd + (n >> 3);
   if (logical >= total) return;
   const int b = logical / (ttiles * utiles);
   const int rem = logical - b * (ttiles * utiles);
+  // (frames first: with the label tiles of the same frames as neighbours all of Y is in use at all
+  // times, B=8 T=10000 U=401 V=1000 630 -> 1029 us)
   const int t0 = (rem % ttiles) * kRows, u0 = (rem / ttiles) * 128;
   int Tb, Ub;
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
@@ -193,40 +202,6 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
         if (t0 + r < d.T) mE[(size_t)b * d.T + t0 + r] = 0.0f;
     return;
   }
-  for (int r = tid; r < kRows; r += kThreads) scale[r] = 1.0f;
-  if (tid == 0) moved = 0;
-  // Picks: the lattice recursions need E[t, blank] and E[t, label_u] in the skewed planes.  Every
-  // element of the tile's rows passes through the staging registers exactly once, so the thread
-  // that holds a wanted column copies it out then (first label tile only; ebv == nullptr: off;
-  // without labels only the blank column is wanted and elS is not touched).
-  const bool picking = ebv != nullptr && u0 == 0;
-  const int nlab = (picking && labels != nullptr) ? min(Ub - 1, 1024) : 0;
-  const int npick = picking ? nlab + 1 : 0;  // entry nlab is the blank column
-  for (int u = tid; u < npick; u += kThreads)
-    labs[u] = u < nlab ? label_at(labels, d, b, u) : d.blank;
-  __syncthreads();
-  // rank every entry by (column, index): the slabs come by in column order, so one cursor into
-  // the sorted list tells each slab which columns to copy, at one LDS read per slab
-  for (int u = tid; u < npick; u += kThreads) {
-    const int c = labs[u];
-    int rank = 0;
-    for (int w = 0; w < npick; ++w) {
-      const int cw = labs[w];
-      rank += (cw < c || (cw == c && w < u)) ? 1 : 0;
-    }
-    order[rank] = (short)u;
-    scol[rank] = c;
-  }
-  int cursor = 0;   // uniform: entries before it have been copied
-  int ncol = -1;    // column and index of entry `cursor`, -1 past the last: read one entry ahead, so
-  int nu = 0;       // that a slab without a pick costs one scalar comparison
-  auto next_pick = [&]() {
-    const bool more = cursor < npick;
-    const int c = more ? scol[cursor] : -1, u = more ? order[cursor] : 0;
-    ncol = __builtin_amdgcn_readfirstlane(c);
-    nu = __builtin_amdgcn_readfirstlane(u);
-  };
-
   // staging: thread -> rows srow (+ 64 with four wavefronts) of the tile, v = slab start +
   // 8*c8 .. +7.  Rows past the utterance repeat its last frame, columns past V repeat earlier
   // ones of the row (its last group of four or eight, or its last element when the values are
@@ -251,9 +226,81 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
       r.x[i] = kVec ? load8(px[i], k0 + 8 * c8, d.V) : load8_any(px[i], k0 + 8 * c8, d.V);
     return r;
   };
+  // this wavefront's block of 32 label positions and first frame block; a label block past the
+  // utterance only helps staging
+  const int ublock = (u0 >> 5) + (wave & 3);
+  const int mb0 = (wave >> 2) * MB;
+  const bool active = 32 * ublock < Ub;
+  const uint4* yw = Yp + ((size_t)b * nub + (active ? ublock : 0)) * nks * 3 * 64 + lane;
+  // Y fragments of step `ks` (16 v): three coalesced 16-byte loads
+  auto fetch_y = [&](int ks) -> Frag3 {
+    const uint4* p = yw + (size_t)ks * 3 * 64;
+    Frag3 y;
+    y.h = p[0]; y.m = p[64]; y.l = p[128];
+    return y;
+  };
+
+  const int nk = (d.V + kSlice - 1) / kSlice;
+  // The first slabs' requests go out ahead of everything else: in a grid of about a workgroup per CU
+  // the start, a chain of round trips to memory that nobody has touched lately, is half the time
+  // (B=8 T=2000 U=101 V=100, four slabs: 43 us inside a training step, 18 called by itself).
+  XRegs xq[kAhead];
+  const XRegs x0 = fetch(0);
+  if constexpr (kAhead > 1) {
+    xq[1] = fetch(min(1, nk - 1) * kSlice);
+    xq[2 % kAhead] = fetch(min(2, nk - 1) * kSlice);
+    xq[3 % kAhead] = fetch(min(3, nk - 1) * kSlice);
+    xq[0] = fetch(min(4, nk - 1) * kSlice);
+  }
+  struct YRegs { Frag3 s0, s1; };
+  YRegs y0[kYAhead];
+  if (active) {
+    y0[0].s0 = fetch_y(0);
+    y0[0].s1 = fetch_y(1);
+    if constexpr (kYAhead > 1) {
+      y0[1].s0 = fetch_y(2 * min(1, nk - 1));
+      y0[1].s1 = fetch_y(2 * min(1, nk - 1) + 1);
+    }
+  }
+  for (int r = tid; r < kRows; r += kThreads) scale[r] = 1.0f;
+  if (tid == 0) moved = 0;
+  // Picks: the lattice recursions need E[t, blank] and E[t, label_u] in the skewed planes.  Every
+  // element of the tile's rows passes through the staging registers exactly once, so the thread
+  // that holds a wanted column copies it out then (first label tile only; ebv == nullptr: off;
+  // without labels only the blank column is wanted and elS is not touched).
+  const bool picking = ebv != nullptr && u0 == 0;
+  const int nlab = (picking && labels != nullptr) ? min(Ub - 1, 1024) : 0;
+  const int npick = picking ? nlab + 1 : 0;  // entry nlab is the blank column
+  for (int u = tid; u < npick; u += kThreads)
+    labs[u] = u < nlab ? label_at(labels, d, b, u) : d.blank;
+  __syncthreads();
+  // rank every entry by (column, index): the slabs come by in column order, so one cursor into
+  // the sorted list tells each slab which columns to copy, at one LDS read per slab
+  for (int u = tid; u < npick; u += kThreads) {
+    const int c = labs[u];
+    int rank = 0;
+#pragma unroll 8
+    for (int w = 0; w < npick; ++w) {  // (eight reads under way at once)
+      const int cw = labs[w];
+      rank += (cw < c || (cw == c && w < u)) ? 1 : 0;
+    }
+    order[rank] = (short)u;
+    scol[rank] = c;
+  }
+  int cursor = 0;  // uniform: entries before it have been copied
+  int ncol = -1;   // column of entry `cursor`, -1 past the last: read one entry ahead, so that a slab
+                   // without a pick costs one scalar comparison
+  int nidx = 0;    // its index (tiles of 128 frames)
+  auto next_pick = [&]() {
+    const bool more = cursor < npick;
+    const int c = more ? scol[cursor] : -1, u = kRows != 64 && more ? order[cursor] : 0;
+    ncol = __builtin_amdgcn_readfirstlane(c);
+    if constexpr (kRows != 64) nidx = __builtin_amdgcn_readfirstlane(u);
+  };
+
   // copies column `col` (which lies in the slab held in r) of this thread's rows to the blank
   // vector (nu_plane < 0: dst[t]) or to label position nu_plane of the skewed plane dst
-  auto pick = [&](const XRegs& r, int col, float* dst, int nu_plane) {
+  auto pick = [&](const XRegs& r, int col, float* dst, int nu_plane) __attribute__((always_inline)) {
     if (c8 != ((col & 31) >> 3)) return;
     const int e = col & 7;  // uniform
 #pragma unroll
@@ -274,15 +321,60 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
       if (t < Tb) dst[nu_plane < 0 ? (size_t)t : plane_at(d, b, nu_plane, t + nu_plane)] = v;
     }
   };
-  auto picks = [&](const XRegs& r, int kslab) {
+  // The columns of slab `kslab` that are picked, copied out of the registers by the threads that hold
+  // them, one after the other: 0.2 us each, most of it the two LDS reads of the next entry.  Tiles
+  // of 64 frames read the entries 64 at a time, one a lane, and send three or more through LDS, a
+  // row a lane and a column a wavefront: B=8 T=2000 U=101 V=100 45 -> 26 us, V=1000 69 -> 58.  (Tiles
+  // of 128 have no registers for that: B=32 U=101 V=10000 885 -> 915 us, T=10000 U=401 V=1000
+  // 720 -> 684, with either part of it.)
+  auto picks = [&](const XRegs& r, int kslab) __attribute__((always_inline)) {
+    if constexpr (kRows != 64) {
+      while ((ncol >> 5) == kslab) {  // uniform
+        if (nidx == nlab) pick(r, ncol, ebv + (size_t)b * d.Tp + d.Eo, -1);
+        else pick(r, ncol, elS, nidx);
+        ++cursor;
+        next_pick();
+      }
+      return;
+    }
+    bool staged = false;
     while ((ncol >> 5) == kslab) {  // uniform
-      if (nu == nlab) pick(r, ncol, ebv + (size_t)b * d.Tp + d.Eo, -1);
-      else pick(r, ncol, elS, nu);
-      ++cursor;
+      const int mine = cursor + lane;
+      const int c = mine < npick ? scol[mine] : -1, o = mine < npick ? order[mine] : 0;
+      const int cnt = __builtin_popcountll(__builtin_amdgcn_ballot_w64((c >> 5) == kslab));
+      if (cnt <= 2 && !staged) {
+        for (int i = 0; i < cnt; ++i) {
+          const int col = __builtin_amdgcn_readlane(c, i), nu = __builtin_amdgcn_readlane(o, i);
+          if (nu == nlab) pick(r, col, ebv + (size_t)b * d.Tp + d.Eo, -1);
+          else pick(r, col, elS, nu);
+        }
+      } else if constexpr (kRows == 64) {
+        if (!staged) {  // (what was read of the last such slab lies behind the barrier of its end)
+#pragma unroll
+          for (int i = 0; i < NR; ++i) {
+            float x[8];
+            expand(r.x[i], x);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) raw[srow + (kThreads / 4) * i][8 * c8 + j] = x[j];
+          }
+          __syncthreads();
+          staged = true;
+        }
+        for (int i = tid; i < cnt * kRows; i += kThreads) {
+          const int e = cursor + i / kRows, row = i % kRows, t = t0 + row;
+          const int col = scol[e], nu = order[e];
+          const float v = raw[row][col & 31];
+          if (t < Tb) {
+            if (nu == nlab) ebv[(size_t)b * d.Tp + d.Eo + t] = v;
+            else elS[plane_at(d, b, nu, t + nu)] = v;
+          }
+        }
+      }
+      cursor += cnt;
       next_pick();
     }
   };
-  auto stash = [&](int buf, const XRegs& r, bool first, int kslab) {
+  auto stash = [&](int buf, const XRegs& r, bool first, int kslab) __attribute__((always_inline)) {
     // maximum of each row's 32 values of this slab (values past V repeat earlier ones); taken
     // before the picks so that the loads are waited for here and not inside the pick loop
     float lm[NR];
@@ -331,20 +423,6 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
     }
   };
 
-  // this wavefront's block of 32 label positions and first frame block; a label block past the
-  // utterance only helps staging
-  const int ublock = (u0 >> 5) + (wave & 3);
-  const int mb0 = (wave >> 2) * MB;
-  const bool active = 32 * ublock < Ub;
-  const uint4* yw = Yp + ((size_t)b * nub + (active ? ublock : 0)) * nks * 3 * 64 + lane;
-  // Y fragments of step `ks` (16 v): three coalesced 16-byte loads
-  auto fetch_y = [&](int ks) -> Frag3 {
-    const uint4* p = yw + (size_t)ks * 3 * 64;
-    Frag3 y;
-    y.h = p[0]; y.m = p[64]; y.l = p[128];
-    return y;
-  };
-
   floatx16 acc[MB], tot[MB];
 #pragma unroll
   for (int m = 0; m < MB; ++m)
@@ -358,7 +436,6 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
 #pragma unroll
     for (int m = 0; m < MB; ++m) aslot[s][m] = xslot(32 * (mb0 + m) + l32, 2 * s + h);
 
-  const int nk = (d.V + kSlice - 1) / kSlice;
   int cur = 0;
   // One slab: request the next slab's emissions, multiply the current one, stage the next.
   // Inside the matrix part the order is pinned with scheduling fences: the fragments of the
@@ -367,14 +444,16 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
   // step's Y fragments are re-requested for the next slab right after their last use (one set
   // again).  Left to itself the compiler reads every fragment just before its first use and the
   // matrix instructions wait for LDS one by one.
-  struct YRegs { Frag3 s0, s1; };
-  auto slab = [&](int kt, YRegs& y, auto act) {
+  // xq: the next slab's emissions (kAhead == 1: requested here; else already under way, and
+  // replaced by those of kAhead slabs on once they are staged).  y: this slab's fragments.
+  auto slab = [&](int kt, XRegs& xq, YRegs& y, auto act) __attribute__((always_inline)) {
     constexpr bool kAct = decltype(act)::value;
     const int ktn = min(kt + 1, nk - 1);
+    const int kty = min(kt + kYAhead, nk - 1);  // whose fragments are requested
     // did a row's reference move while this slab was staged?  Read together with the fragments
     // (LDS answers in order), so the flag costs no round trip of its own.
     const int mv = moved;
-    const XRegs xs = fetch(ktn * kSlice);
+    if constexpr (kAhead == 1) xq = fetch(ktn * kSlice);
     if (kAct) {
       uint4 ah[MB], am[MB], al[MB];
 #pragma unroll
@@ -417,7 +496,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int m = 0; m < MB; ++m) ah[m] = Xs[cur][0][aslot[1][m]];
-      y.s0 = fetch_y(2 * ktn);
+      y.s0 = fetch_y(2 * kty);
 #pragma unroll
       for (int m = 0; m < MB; ++m) acc[m] = mfma_bf16(al[m], y.s1.h, acc[m]);
       __builtin_amdgcn_sched_barrier(0);
@@ -432,7 +511,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
 #pragma unroll
       for (int m = 0; m < MB; ++m) acc[m] = mfma_bf16(ah[m], y.s1.h, acc[m]);
       __builtin_amdgcn_sched_barrier(0);
-      y.s1 = fetch_y(2 * ktn + 1);
+      y.s1 = fetch_y(2 * kty + 1);
     }
     __builtin_amdgcn_sched_barrier(0);
     if (mv) {  // every wavefront has used the factors: back to 1 before the staging sets new ones
@@ -441,35 +520,48 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
       if (tid == 0) moved = 0;
       __syncthreads();
     }
-    stash(cur ^ 1, xs, false, min(kt + 1, nk - 1));
+    stash(cur ^ 1, xq, false, ktn);
+    if constexpr (kAhead > 1) xq = fetch(min(kt + 1 + kAhead, nk - 1) * kSlice);
     __syncthreads();
     cur ^= 1;
   };
   __syncthreads();  // order
   next_pick();
-  stash(0, fetch(0), true, 0);
-  YRegs y0;
-  if (active) {
-    y0.s0 = fetch_y(0);
-    y0.s1 = fetch_y(1);
-  }
+  stash(0, x0, true, 0);
   __syncthreads();
   // Two copies of the loop, so that a wavefront with nothing to multiply is a path of its own:
   // inside one loop the counted waits for the emission loads would have to hold on both paths,
   // and the one without Y requests in flight makes the multiplying wavefronts wait for theirs.
-  if (active) {
-    for (int kt = 0; kt < nk; ++kt) {
-      slab(kt, y0, std::true_type{});
-      if ((kt + 1) % kFlush == 0) {
+  auto flush = [&]() {
 #pragma unroll
-        for (int m = 0; m < MB; ++m)
+    for (int m = 0; m < MB; ++m)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) { tot[m][r] += acc[m][r]; acc[m][r] = 0.0f; }
+      for (int r = 0; r < 16; ++r) { tot[m][r] += acc[m][r]; acc[m][r] = 0.0f; }
+  };
+  auto walk = [&](auto act) __attribute__((always_inline)) {
+    constexpr bool kAct = decltype(act)::value;
+    int kt = 0;
+    if constexpr (kAhead > 1) {
+      static_assert(kAhead == 4 && kYAhead == 2 && kFlush % kAhead == 0, "as written out here");
+      for (; kt + 4 <= nk; kt += 4) {
+        slab(kt, xq[1], y0[0], act);
+        slab(kt + 1, xq[2], y0[1], act);
+        slab(kt + 2, xq[3], y0[0], act);
+        slab(kt + 3, xq[0], y0[1], act);
+        if (kAct && (kt + 4) % kFlush == 0) flush();
+      }
+      if (kt < nk) slab(kt, xq[1], y0[0], act);
+      if (kt + 1 < nk) slab(kt + 1, xq[2], y0[1], act);
+      if (kt + 2 < nk) slab(kt + 2, xq[3], y0[0], act);
+    } else {
+      for (; kt < nk; ++kt) {
+        slab(kt, xq[0], y0[0], act);
+        if (kAct && (kt + 1) % kFlush == 0) flush();
       }
     }
-  } else {
-    for (int kt = 0; kt < nk; ++kt) slab(kt, y0, std::false_type{});
-  }
+  };
+  if (active) walk(std::true_type{});
+  else walk(std::false_type{});
 
   // final references: to LDS for the write-out below, to mE for the kernels that come later
 #pragma unroll
