@@ -885,6 +885,12 @@ static int egrads_window(const TIO* E, const TIO* P, const float* mE, const floa
   chunks = chunks < 1 ? 1 : chunks;
   const int max_chunks = (ntiles + 7) / 8;
   if (chunks > max_chunks) chunks = max_chunks;
+  // ... but where that leaves a workgroup per CU or less, shorter runs until there are two: the Y
+  // fragments then cost less than the tiles that follow one another (us, runs of eight tiles and
+  // now: B=8 T=2000 U=101 V=100 30 -> 16, B=32 33 -> 28; B=1 T=500 U=41 V=1000 29 -> 11; from more
+  // workgroups on the other way round: B=8 U=101 V=1000 53 with runs of eight, 57 of four)
+  if ((long)chunks * vtiles * d.B <= 256)
+    chunks = std::max(chunks, std::min(ntiles, 512 / (vtiles * d.B)));
   const int per = (ntiles + chunks - 1) / chunks;
   chunks = (ntiles + per - 1) / per;
   // A launch contracts 16 * kEsMaxS label positions (what a wavefront keeps of Y in registers);
