@@ -25,6 +25,7 @@ HIP_SOURCES = [("rnnt_dp.hip", ["-DRNNT_DP_PART=%d" % part], "rnnt_dp_%d.o" % pa
                for part in range(6)] + \
               [(src, [], src.replace(".hip", ".o"))
                for src in ("rnnt_capi.hip", "rnnt_lse.hip", "rnnt_cand.hip", "rnnt_fused.hip",
+                           "rnnt_egrads_long.hip",
                            "rnnt_prep.hip")]
 
 # -ffp-contract=off: the lattice recursions must round like the reference's scalar code.

@@ -523,9 +523,13 @@ int lowp_loss_backward(const TIO* E, const TIO* P, const int* labels, const int*
   auto dense = [&]() -> int {
     // a label axis of more than one slice: the slices add up in fp32, in the part of the workspace
     // that held the log-normaliser's Y pieces during the forward pass (free by now)
-    RNNT_STAGE(kEgrads, launch_egrads_stream(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen,
-                                             d, false, sp, s, static_cast<float*>(w.lse_scratch),
-                                             lse_scratch_bytes(d)));
+    if (egrads_long_takes(d))
+      RNNT_STAGE(kEgrads, launch_egrads_long(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen, d,
+                                             sp, w.lse_scratch, s));
+    else
+      RNNT_STAGE(kEgrads, launch_egrads_stream(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen,
+                                               d, false, sp, s, static_cast<float*>(w.lse_scratch),
+                                               lse_scratch_bytes(d)));
     return kOk;
   };
   auto across = [&]() -> int {
@@ -991,8 +995,13 @@ int rnnt_hip_loss_backward(const float* E, const float* P, const int* labels, co
     return kOk;
   }
   auto dense = [&]() -> int {
-    RNNT_STAGE(kEgrads, launch_egrads(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen, d,
-                                      false, sp, s));
+    // (the pieces of Y go where the log-normaliser's were during the forward pass)
+    if (egrads_long_takes(d))
+      RNNT_STAGE(kEgrads, launch_egrads_long(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen, d,
+                                             sp, w.lse_scratch, s));
+    else
+      RNNT_STAGE(kEgrads, launch_egrads(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen, d,
+                                        false, sp, s));
     return kOk;
   };
   auto across = [&]() -> int {

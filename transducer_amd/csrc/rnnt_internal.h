@@ -366,6 +366,21 @@ int launch_grads_fused(const float* E, const float* P, const float* mE, const fl
 // at least 32 frames of B * V values), a window of frames at a time, so that each value is still
 // rounded once.
 bool egrads_one_pass(const Dims& d);
+// ---- (rnnt_egrads_long.hip) A longer label axis in one launch, where the pieces of Y have room:
+// scratch of lse_scratch_bytes(d).  out = delta * (dense + sparse), egrads written once.
+bool egrads_long_takes(const Dims& d);
+int launch_egrads_long(const float* E, const float* P, const float* mE, const float* mP,
+                       const float* Wn, const float* deltas, float* egrads, const int* inLen,
+                       const int* labLen, const Dims& d, const SparseTerms& sparse, void* scratch,
+                       hipStream_t s);
+int launch_egrads_long(const bf16_t* E, const bf16_t* P, const float* mE, const float* mP,
+                       const float* Wn, const float* deltas, bf16_t* egrads, const int* inLen,
+                       const int* labLen, const Dims& d, const SparseTerms& sparse, void* scratch,
+                       hipStream_t s);
+int launch_egrads_long(const f16_t* E, const f16_t* P, const float* mE, const float* mP,
+                       const float* Wn, const float* deltas, f16_t* egrads, const int* inLen,
+                       const int* labLen, const Dims& d, const SparseTerms& sparse, void* scratch,
+                       hipStream_t s);
 int launch_egrads_stream(const float* E, const float* P, const float* mE, const float* mP,
                          const float* Wn, const float* deltas, float* egrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
