@@ -126,12 +126,12 @@ SHAPES = [
     (4, 50, 11, 32),
     (2, 130, 112, 520),
     (3, 96, 20, 1000),
-    # label axes of more than one slice of 112 positions: the slices add up in fp32, a window of
-    # frames at a time, and each gradient entry is still rounded once
+    # label axes of more than the 112 positions that egrads keeps in registers: each gradient entry
+    # is still rounded once
     (2, 40, 113, 24),
     (2, 70, 225, 520),
     (1, 33, 401, 40),
-    (2, 300, 113, 40),  # two windows of frames (288 + 12)
+    (2, 300, 113, 40),  # three tiles of 128 frames, the last one short
     # vocabularies off the eight-element vector width: the rows are read element by element
     (1, 8, 3, 12),
     (2, 9, 4, 5),
@@ -164,6 +164,13 @@ def test_16bit_against_the_fp32_entry_points_and_the_oracle(B, T, U, V, kind):
         frac, worst = violations(got.float().cpu().numpy(), ref, rtol=LOWP_RTOL, atol=ATOL)
         assert frac == 0.0, "%s: %.4g%% outside rtol=%g atol=%g (max abs err %g)" % (
             what, 100 * frac, LOWP_RTOL, ATOL, worst)
+
+
+@pytest.mark.parametrize("kind", KIND_NAMES)
+@pytest.mark.parametrize("B,T,U,V", [(2, 1, 113, 31), (2, 127, 113, 33), (2, 128, 128, 127),
+                                     (2, 129, 129, 129), (2, 257, 161, 600)])
+def test_16bit_egrads_of_long_label_axes_at_the_edges_of_their_tiles(B, T, U, V, kind):
+    test_16bit_against_the_fp32_entry_points_and_the_oracle(B, T, U, V, kind)
 
 
 @pytest.mark.parametrize("kind", KIND_NAMES)

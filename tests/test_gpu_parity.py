@@ -900,6 +900,32 @@ def test_sparse_terms_either_side_of_every_split_of_frames_and_positions(T, U, V
             assert_same_bits(g, w, what)
 
 
+@pytest.mark.parametrize("T,U,V", [(1, 113, 31), (127, 113, 33), (128, 128, 127), (129, 129, 129),
+                                   (130, 160, 32), (257, 161, 600), (64, 225, 520)])
+def test_egrads_of_long_label_axes_at_the_edges_of_their_tiles(T, U, V):
+    """Tiles of 128 frames, 128 columns and slabs of 32 label positions, each one short, full and
+    one over; utterances that end inside, at the end of and a tile before the frame axis; labels
+    that meet each other and the blank.  With the device's log-normaliser on both sides, at the
+    tolerance of the other whole-loss tests."""
+    rng = np.random.default_rng(T + U + V)
+    B = 3
+    E = rng.standard_normal((B, T, V), dtype=np.float32)
+    P = rng.standard_normal((B, U, V), dtype=np.float32)
+    labels = rng.integers(0, V, (B, U - 1)).astype(np.int32)
+    labels[1] = np.arange(U - 1) % 3  # in one block of 32 columns, one of them the blank
+    il = np.array([T, max(T - 1, 1), max(T - 128, 1)], np.int32)
+    ll = np.array([U - 1, U - 2, 5], np.int32)
+    c = DeviceCase(E, P, labels, il, ll)
+    _, eg, _ = gpu_loss(c)
+    LN = np.nan_to_num(gpu_log_norms(c))
+    _, alphas = oracle.forward(E, P, LN, labels, il, ll)
+    weg, wpg, lng = oracle.backward(E, P, np.nan_to_num(alphas), LN, labels, il, ll)
+    weg, _ = oracle.accumulate_grads(E, P, weg, wpg, lng, LN, il, ll)
+    assert_close(eg, weg, what="egrads")
+    for b in range(B):
+        assert not eg[b, il[b]:].any()
+
+
 @pytest.mark.parametrize("U,V", [(113, 512), (130, 514), (250, 700), (401, 515)])
 def test_label_terms_of_label_axes_of_several_slices(U, V):
     """Dozens of labels in one block of 32 columns, the same label many times, labels that are the

@@ -264,7 +264,7 @@ size_t loss_workspace_layout(const Dims& d, void* base, LossWorkspace* w) {
   float* bsum = take(sizeof(float) * (size_t)d.B * d.T);
   float* emT = take(btu);  // label-move terms of egrads, [B][U][T]
   // One piece of memory with three uses after one another on the call's stream: the Y pieces
-  // (forward pass), the first partial sums of pgrads, the fp32 window of 16-bit egrads.  Sums past
+  // (forward pass), the first partial sums of pgrads, the Y pieces of egrads of a long label axis.  Sums past
   // its end go where nothing else is wanted any more once W is formed: the dalpha walk's planes
   // (which every backward pass forms anew), then the array of egrads (both_gradients).  So the
   // workspace has no B*T*V term for them, however long the utterances.
@@ -521,15 +521,14 @@ int lowp_loss_backward(const TIO* E, const TIO* P, const int* labels, const int*
   SparsePTerms spp;
   spp.gB = w.planes.gB; spp.gL = w.planes.gL; spp.labels = lab;
   auto dense = [&]() -> int {
-    // a label axis of more than one slice: the slices add up in fp32, in the part of the workspace
-    // that held the log-normaliser's Y pieces during the forward pass (free by now)
-    if (egrads_long_takes(d))
+    // a longer label axis: the pieces of Y go into the part of the workspace that held the
+    // log-normaliser's during the forward pass (free by now)
+    if (egrads_one_pass(d))
+      RNNT_STAGE(kEgrads, launch_egrads_stream(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen,
+                                               d, false, sp, s));
+    else
       RNNT_STAGE(kEgrads, launch_egrads_long(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen, d,
                                              sp, w.lse_scratch, s));
-    else
-      RNNT_STAGE(kEgrads, launch_egrads_stream(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen,
-                                               d, false, sp, s, static_cast<float*>(w.lse_scratch),
-                                               lse_scratch_bytes(d)));
     return kOk;
   };
   auto across = [&]() -> int {
@@ -996,12 +995,12 @@ int rnnt_hip_loss_backward(const float* E, const float* P, const int* labels, co
   }
   auto dense = [&]() -> int {
     // (the pieces of Y go where the log-normaliser's were during the forward pass)
-    if (egrads_long_takes(d))
-      RNNT_STAGE(kEgrads, launch_egrads_long(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen, d,
-                                             sp, w.lse_scratch, s));
-    else
+    if (egrads_one_pass(d))
       RNNT_STAGE(kEgrads, launch_egrads(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen, d,
                                         false, sp, s));
+    else
+      RNNT_STAGE(kEgrads, launch_egrads_long(E, P, w.mE, w.mP, w.Wn, deltas, egrads, inLen, labLen, d,
+                                             sp, w.lse_scratch, s));
     return kOk;
   };
   auto across = [&]() -> int {

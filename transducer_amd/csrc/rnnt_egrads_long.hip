@@ -327,7 +327,6 @@ int egrads_long_any(const TIO* E, const TIO* P, const float* mE, const float* mP
 // V=1000, four slices 942 -> 515; T=2000 U=129 V=1000, two 88 -> 63; B=32 T=1000 U=150 V=5000
 // 763 -> 569; B=1 T=1000 U=300 V=600 122 -> 37.  With one slice it is the streamed form, whose Y stays
 // in registers: B=32 T=2000 U=101 V=10000 1190 against 1890, V=1000 190 against 222.)
-bool egrads_long_takes(const Dims& d) { return !egrads_one_pass(d); }
 
 int launch_egrads_long(const float* E, const float* P, const float* mE, const float* mP,
                        const float* Wn, const float* deltas, float* egrads, const int* inLen,

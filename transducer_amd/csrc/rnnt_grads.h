@@ -29,8 +29,6 @@ constexpr int kEsPitch = 16 * kEsMaxS + 8;  // LDS row pitch of a W-slab plane i
                                             // 16-byte reads of 8 consecutive rows spread over all banks)
 constexpr int kEsPlane = 32 * kEsPitch;
 constexpr int kEsPrefetch = 2;          // labels per 32-column block whose sparse terms are prefetched
-constexpr int kEsManyPrefetch = 7;      // the same for long transcripts, two labels to a register
-constexpr int kEsBlockPitch = 36;       // floats between columns of the LDS block they add up in
 constexpr int kMaxLabels = 1024;        // labels whose terms the egrads write-out can fold in
 
 // Row of the 32x32 output block that register r of lane-half h holds.

@@ -52,13 +52,6 @@ struct SlabRegs {
   float m;
 };
 
-// The frames one egrads launch covers and where they go: tiles [tile_begin, tile_end) of 32
-// frames; frame t of utterance b lands in row b * out_T + (t - t_base) of the output array.  The
-// whole frame axis into the caller's array: {0, tiles of T, T, 0}.
-struct EgradsWindow {
-  int tile_begin, tile_end, out_T, t_base;
-};
-
 // The walk of one workgroup over its frame tiles with NS steps of sixteen label positions
 // (a template parameter, so the matrix instructions of a tile form one straight-line block).
 // Label positions past the utterance contribute exact zeros: their Y rows are masked and the
@@ -66,20 +59,18 @@ struct EgradsWindow {
 // kMode: what a launch does with the sums of its slice of the label axis.
 //   kEgWhole    out = delta (X sums + sparse terms)         the only slice
 //   kEgAdd      out = delta (out + X sums)                  onto what the caller's array holds
-//   kEgPartial  out = sums (first slice) or out + sums      a slice but the last of several:
-//                                                           no emissions read, no exponentials
-//   kEgFinal    out = delta (X (out + sums) + sparse terms) the last of several slices
-constexpr int kEgWhole = 0, kEgAdd = 1, kEgPartial = 2, kEgFinal = 3;
+// (A label axis of several slices is added to the caller's array slice by slice; where the array is
+// only written, it goes through rnnt_egrads_long.hip.)
+constexpr int kEgWhole = 0, kEgAdd = 1;
 // kManyLabels: compiled for transcripts that put more than two labels into most blocks of 32
 // columns (the launcher decides by U * 32 > 2 V); see where the terms are fetched.
-template <int NS, int kMode, bool kManyLabels, typename TIO, typename TOUT>
+template <int NS, int kMode, bool kManyLabels, typename TIO>
 __device__ __forceinline__ void egrads_walk(
     const TIO* __restrict__ E, const TIO* __restrict__ P, const float* __restrict__ mE,
     const float* __restrict__ mP, const float* __restrict__ Wn, const float* __restrict__ deltas,
-    TOUT* __restrict__ egrads, unsigned short (*As)[3][kEsPlane], float (*Ms)[32], const Dims& d,
+    TIO* __restrict__ egrads, unsigned short (*As)[3][kEsPlane], float (*Ms)[32], const Dims& d,
     int Up, int Tw, int tiles_per_chunk, int u_lo, int b, int Tb, int Ub, const SparseTerms& sp,
-    const unsigned short* match, int nmatch, float (*Sp)[32], float* block,
-    const EgradsWindow& win) {
+    const unsigned short* match, int nmatch, float (*Sp)[32]) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, h = lane >> 5;
   const int wave_col0 = blockIdx.x * 128 + wave * 32;  // this wavefront's 32 columns
   const int vcol = wave_col0 + l32;
@@ -87,19 +78,15 @@ __device__ __forceinline__ void egrads_walk(
   const int vc = vok ? vcol : d.V - 1;  // always readable
   const bool cols_full = wave_col0 + 32 <= d.V;
   // lane that owns the blank column, if it is one of this wavefront's and terms are folded in
-  constexpr bool kSparse = kMode == kEgWhole || kMode == kEgFinal;  // may fold sparse terms in
-  constexpr bool kScores = kMode != kEgPartial;                     // reads the emissions
-  // reads what the output holds (a first partial slice starts from nothing)
-  const bool reads_out = kMode == kEgAdd || kMode == kEgFinal || (kMode == kEgPartial && u_lo > 0);
+  constexpr bool kSparse = kMode == kEgWhole;  // may fold sparse terms in
   const int blank_lane = (sp.labels && d.blank >= wave_col0 && d.blank < wave_col0 + 32)
                              ? d.blank - wave_col0 : -1;
-  const int tile_lo = win.tile_begin + blockIdx.y * tiles_per_chunk;
-  const int tile_hi = min(tile_lo + tiles_per_chunk, win.tile_end);
+  const int tile_lo = blockIdx.y * tiles_per_chunk;
+  const int tile_hi = min(tile_lo + tiles_per_chunk, (d.T + 31) >> 5);
   const int tile_valid = min(tile_hi, (Tb + 31) >> 5);  // tiles that hold frames of the utterance
   const float delta = deltas ? deltas[b] : 1.0f;
   const TIO* Eb = E + (size_t)b * d.T * d.V;
-  // frame t of the utterance is row t - win.t_base of its block of win.out_T rows in `egrads`
-  TOUT* out = egrads + (size_t)b * win.out_T * d.V;
+  TIO* out = egrads + (size_t)b * d.T * d.V;
   const float* mEb = mE + (size_t)b * d.T;
 
   // Y fragments for this wavefront's columns (branch-free: clamped address, masked value):
@@ -183,27 +170,12 @@ __device__ __forceinline__ void egrads_walk(
   if (tile_lo < tile_valid) store_slab(0, fetch_slab(tile_lo));
   __syncthreads();
 
-  // the first matches, resolved once: label position and target lane.  (kBlocks: each half of the
-  // wavefront keeps every second one)
-  constexpr bool kBlocks = kManyLabels && kMode == kEgFinal;
-  constexpr int kPre = kBlocks ? kEsManyPrefetch : kEsPrefetch;
-  constexpr int kPerReg = kBlocks ? 2 : 1;
-  int mu[kPre], mc[kPre];
+  // the first matches, resolved once: label position and target lane
+  int mu[kEsPrefetch], mc[kEsPrefetch];
 #pragma unroll
-  for (int i = 0; i < kPre; ++i) {
-    const int m = kPerReg * i + (kBlocks ? h : 0);
-    mu[i] = (sp.labels && m < nmatch) ? match[m] : 0;
-    mc[i] = (sp.labels && m < nmatch) ? label_at(sp.labels, d, b, mu[i]) - wave_col0 : -1;
-  }
-  // (kBlocks) pairs that are the same label twice: bit i
-  unsigned twins = 0;
-  auto is_twin = [&](int col) {
-    const int other = __shfl_xor(col, 32);  // (by all lanes: one that is off would hand over 0)
-    return __ballot(col >= 0 && other == col) != 0;  // uniform
-  };
-  if constexpr (kBlocks) {
-#pragma unroll
-    for (int i = 0; i < kPre; ++i) twins |= is_twin(mc[i]) ? 1u << i : 0u;
+  for (int i = 0; i < kEsPrefetch; ++i) {
+    mu[i] = (sp.labels && i < nmatch) ? match[i] : 0;
+    mc[i] = (sp.labels && i < nmatch) ? label_at(sp.labels, d, b, mu[i]) - wave_col0 : -1;
   }
 
   // bf16 only: with half the bytes the kernel is held by how long a request takes, not by how
@@ -233,11 +205,10 @@ __device__ __forceinline__ void egrads_walk(
     const SlabRegs nxt = fetch_slab(min(ti + 1, tile_valid - 1));
     const bool interior = cols_full && (t0 + 32 <= Tb);  // no row or column needs a guard
     const TIO* Etile = Eb + (size_t)t0 * d.V;
-    TOUT* Otile = out + (size_t)(t0 - win.t_base) * d.V;
+    TIO* Otile = out + (size_t)t0 * d.V;
     float evl[16];
     float (&ev)[16] = pick_set(ahead, evc, evl);
-    if constexpr (!kScores) {
-    } else if constexpr (decltype(ahead)::value) {
+    if constexpr (decltype(ahead)::value) {
       load_e(min(ti + 1, tile_valid - 1), evn);
     } else if (interior) {
       // the emissions of this tile, requested before the matrix work so they arrive under it
@@ -255,10 +226,7 @@ __device__ __forceinline__ void egrads_walk(
     // slice of 112 label positions at B=8 T=10000 V=1000, where the first slice takes 0.30)
     float ov[16];
     if constexpr (kMode != kEgWhole) {
-      if (!reads_out) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) ov[r] = 0.0f;
-      } else if (interior) {
+      if (interior) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
           ov[r] = ldf(Otile + (lane_off + (unsigned)(8 * (r >> 2) + (r & 3)) * (unsigned)d.V));
@@ -266,20 +234,17 @@ __device__ __forceinline__ void egrads_walk(
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int t = t0 + mfma_row(r, h);
-          ov[r] = (t < d.T && vok) ? ldf(out + (size_t)(t - win.t_base) * d.V + vcol) : 0.0f;
+          ov[r] = (t < d.T && vok) ? ldf(out + (size_t)t * d.V + vcol) : 0.0f;
         }
       }
     }
-    // sparse terms of this tile for the first labels that fall into this wavefront's columns: one coalesced load per plane, requested here so it arrives under the matrix work
-    float sd[kPre], sbl = 0.0f;
+    // sparse terms of this tile for the first labels that fall into this wavefront's columns:
+    // one coalesced load per plane, requested here so it arrives under the matrix work
+    float sd[kEsPrefetch], sbl = 0.0f;
     if (kSparse && (nmatch > 0 || blank_lane >= 0)) {
       const int tr = min(t0 + l32, Tb - 1);
 #pragma unroll
-      for (int i = 0; i < kPre; ++i) {
-        sd[i] = 0.0f;
-        if (!kBlocks || kPerReg * i < nmatch)
-          sd[i] = sp.emT[((size_t)b * d.U + mu[i]) * d.T + tr];
-      }
+      for (int i = 0; i < kEsPrefetch; ++i) sd[i] = sp.emT[((size_t)b * d.U + mu[i]) * d.T + tr];
       if (blank_lane >= 0) sbl = sp.bsum[(size_t)b * d.T + tr];
     }
     // two accumulators, so that consecutive matrix instructions never wait on each other
@@ -315,10 +280,7 @@ __device__ __forceinline__ void egrads_walk(
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const int r = 4 * g + k;
-        float x;
-        if constexpr (kMode == kEgPartial) x = ov[r] + acc[r];
-        else if constexpr (kMode == kEgFinal) x = exp_minus_scaled(ev[r], f4at(m4, k)) * (ov[r] + acc[r]);
-        else x = exp_minus_scaled(ev[r], f4at(m4, k)) * acc[r];
+        const float x = exp_minus_scaled(ev[r], f4at(m4, k)) * acc[r];
         v[r] = (interior || t0 + mfma_row(r, h) < Tb) ? x : 0.0f;
       }
     }
@@ -341,66 +303,11 @@ __device__ __forceinline__ void egrads_walk(
           }
         }
       };
-      if constexpr (kBlocks) {
-        // label axes of several slices (400 labels and 1000 columns put a dozen into every block):
-        // the terms are added up in a 32 x 32 block in LDS, a label to each half of the wavefront
-        // at a time and nothing waited for, and a lane takes its column's sixteen frames from
-        // there once; the first fourteen are asked for before the matrix block.  The order of the
-        // additions is the order of the pairs: LDS takes a wavefront's instructions one after the
-        // other, and a pair of the same label, whose halves would meet at one address within an
-        // instruction, is added up first and goes in from the lower half alone (13 us of the 4754 of
-        // a training step of B=8 T=10000 U=400 V=1000).  All slices of egrads at B=8 T=10000 U=401
-        // V=1000 1026 -> 934 us before that, B=4 T=2000 U=300 V=2000 145 -> 126; with one slice there are
-        // few labels a block, and filling and reading it costs more than it saves (B=32 T=2000 U=101
-        // V=1000: 197 -> 213).
-        auto add_pair = [&](int col, float x, bool twin) {
-          if (twin) x += __shfl_xor(x, 32);
-          if (col >= 0 && row_ok && !(twin && h))
-            unsafeAtomicAdd(&block[col * kEsBlockPitch + l32], x);
-        };
-        if (nmatch > 0) {
 #pragma unroll
-          for (int k = 0; k < (32 * kEsBlockPitch / 4 + 63) / 64; ++k)
-            if (64 * k + lane < 32 * kEsBlockPitch / 4)
-              reinterpret_cast<float4*>(block)[64 * k + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-#pragma unroll
-          for (int i = 0; i < kPre; ++i)
-            if (2 * i < nmatch) add_pair(mc[i], sd[i], (twins >> i) & 1u);
-          constexpr int kBatch = 4;
-          for (int i0 = 2 * kPre; i0 < nmatch; i0 += 2 * kBatch) {
-            float term[kBatch];
-            int col[kBatch];
-#pragma unroll
-            for (int k = 0; k < kBatch; ++k) {
-              const int m = i0 + 2 * k + h, u = match[min(m, nmatch - 1)];
-              term[k] = sp.emT[((size_t)b * d.U + u) * d.T + min(t0 + l32, Tb - 1)];
-              col[k] = m < nmatch ? label_at(sp.labels, d, b, u) - wave_col0 : -1;
-            }
-#pragma unroll
-            for (int k = 0; k < kBatch; ++k) add_pair(col[k], term[k], is_twin(col[k]));
-          }
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const float4 x =
-                *reinterpret_cast<const float4*>(&block[l32 * kEsBlockPitch + 8 * g + 4 * h]);
-            v[4 * g + 0] -= x.x;
-            v[4 * g + 1] -= x.y;
-            v[4 * g + 2] -= x.z;
-            v[4 * g + 3] -= x.w;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < kEsPrefetch; ++i)
-          if (i < nmatch) apply(row_ok ? sd[i] : 0.0f, mc[i], -1.0f);
-      }
+      for (int i = 0; i < kEsPrefetch; ++i)
+        if (i < nmatch) apply(row_ok ? sd[i] : 0.0f, mc[i], -1.0f);
       // more labels in one 32-column block
-      if constexpr (kBlocks) {
-      } else if constexpr (kManyLabels) {
+      if constexpr (kManyLabels) {
         // long transcripts over a small vocabulary: their terms are asked for four at a time, so
         // that a tile waits one memory round trip per four, not one per label.  A kernel of its
         // own: compiled into the kernel of the large vocabularies, where it hardly ever runs, it
@@ -431,9 +338,8 @@ __device__ __forceinline__ void egrads_walk(
     if (interior) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        TOUT* o = Otile + (lane_off + (unsigned)(8 * (r >> 2) + (r & 3)) * (unsigned)d.V);
+        TIO* o = Otile + (lane_off + (unsigned)(8 * (r >> 2) + (r & 3)) * (unsigned)d.V);
         if constexpr (kMode == kEgAdd) stf(o, delta * (ov[r] + v[r]));
-        else if constexpr (kMode == kEgPartial) stf(o, v[r]);
         else stf(o, delta * v[r]);
       }
     } else {
@@ -441,9 +347,8 @@ __device__ __forceinline__ void egrads_walk(
       for (int r = 0; r < 16; ++r) {
         const int t = t0 + mfma_row(r, h);
         if (t < d.T && vok) {
-          TOUT* o = out + (size_t)(t - win.t_base) * d.V + vcol;
+          TIO* o = out + (size_t)t * d.V + vcol;
           if constexpr (kMode == kEgAdd) stf(o, delta * (ov[r] + v[r]));
-          else if constexpr (kMode == kEgPartial) stf(o, v[r]);
           else stf(o, delta * v[r]);
         }
       }
@@ -453,7 +358,7 @@ __device__ __forceinline__ void egrads_walk(
     cur ^= 1;
   };
   float evA[16], evB[16];
-  if constexpr (kAhead && kScores) {
+  if constexpr (kAhead) {
     // two tiles per trip, the two register sets swapping roles (a copy from one set to the other
     // would wait for the requests a tile too early)
     if (tile_lo < tile_valid) load_e(tile_lo, evA);
@@ -465,15 +370,14 @@ __device__ __forceinline__ void egrads_walk(
     for (int ti = tile_lo; ti < tile_valid; ++ti) tile(ti, evA, evB, std::false_type());
   }
 
-  // frames past the utterance: the dense part is exactly zero (of several slices the first
-  // writes the zeros and the later ones leave them)
-  if (kMode == kEgWhole || kMode == kEgAdd || (kMode == kEgPartial && u_lo == 0)) {
+  // frames past the utterance: the dense part is exactly zero
+  {
     for (int ti = max(tile_lo, tile_valid); ti < tile_hi; ++ti) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int t = ti * 32 + mfma_row(r, h);
         if (t < d.T && vok) {
-          TOUT* o = out + (size_t)(t - win.t_base) * d.V + vcol;
+          TIO* o = out + (size_t)t * d.V + vcol;
           stf(o, kMode == kEgAdd ? delta * ldf(o) : 0.0f);
         }
       }
@@ -481,18 +385,15 @@ __device__ __forceinline__ void egrads_walk(
   }
 }
 
-template <int kMode, bool kManyLabels, typename TIO, typename TOUT>
+template <int kMode, bool kManyLabels, typename TIO>
 __global__ __launch_bounds__(256, 2) void egrads_stream_kernel(
     const TIO* __restrict__ E, const TIO* __restrict__ P, const float* __restrict__ mE,
     const float* __restrict__ mP, const float* __restrict__ Wn, const float* __restrict__ deltas,
-    TOUT* __restrict__ egrads, const int* __restrict__ inLen, const int* __restrict__ labLen,
-    Dims d, int Up, int Tw, int tiles_per_chunk, int u_lo, SparseTerms sp, EgradsWindow win) {
+    TIO* __restrict__ egrads, const int* __restrict__ inLen, const int* __restrict__ labLen,
+    Dims d, int Up, int Tw, int tiles_per_chunk, int u_lo, SparseTerms sp) {
   __shared__ __attribute__((aligned(16))) unsigned short As[2][3][kEsPlane];
   __shared__ __attribute__((aligned(16))) float Ms[2][32];  // mE * log2(e) of the slab's frames
   __shared__ __attribute__((aligned(16))) float Strip[4][32];  // per wavefront: sparse terms
-  constexpr bool kBlocks = kManyLabels && kMode == kEgFinal;
-  __shared__ __attribute__((aligned(16))) float Block[kBlocks ? 4 : 1]
-                                                     [kBlocks ? 32 * kEsBlockPitch : 1];
   __shared__ unsigned short Match[4][kMaxLabels];  // per wavefront: label positions whose label
                                                    // is one of its 32 columns
   const int b = blockIdx.z;
@@ -500,7 +401,6 @@ __global__ __launch_bounds__(256, 2) void egrads_stream_kernel(
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
   // a later slice of the label axis that lies past this utterance adds nothing; only the last
   // slice (the one that is given the factors) still has to finish what is there
-  if (kMode == kEgPartial && u_lo > 0 && u_lo >= Ub) return;
   if (kMode == kEgAdd && u_lo > 0 && u_lo >= Ub && deltas == nullptr) return;
   int nmatch = 0;
   if (sp.labels) {
@@ -524,7 +424,7 @@ __global__ __launch_bounds__(256, 2) void egrads_stream_kernel(
 #define RNNT_EG_WALK(NS)                                                                      \
   egrads_walk<NS, kMode, kManyLabels>(E, P, mE, mP, Wn, deltas, egrads, As, Ms, d, Up, Tw,   \
                                tiles_per_chunk, u_lo, b, Tb, Ub, sp, Match[threadIdx.x >> 6], \
-                               nmatch, &Strip[threadIdx.x >> 6], Block[kBlocks ? threadIdx.x >> 6 : 0], win)
+                               nmatch, &Strip[threadIdx.x >> 6])
   if (nsteps <= 2) RNNT_EG_WALK(2);
   else if (nsteps <= 4) RNNT_EG_WALK(4);
   else if (nsteps == 5) RNNT_EG_WALK(5);
@@ -870,15 +770,20 @@ __global__ __launch_bounds__(256) void pgrads_combine_kernel(
 bool egrads_one_pass(const Dims& d) { return wplane_up(d.U) <= 16 * kEsMaxS; }
 #endif
 
-// One pass of the egrads kernels over the frames of `win` (all slices of the label axis), into
-// `out` (the caller's array, or a wide copy of a window of it).
-template <typename TIO, typename TOUT>
-static int egrads_window(const TIO* E, const TIO* P, const float* mE, const float* mP,
-                         const float* Wn, const float* deltas, TOUT* out, const int* inLen,
-                         const int* labLen, const Dims& d, bool accumulate,
-                         const SparseTerms& sparse, const EgradsWindow& win, hipStream_t s) {
+template <typename TIO>
+static int egrads_stream_any(const TIO* E, const TIO* P, const float* mE, const float* mP,
+                             const float* Wn, const float* deltas, TIO* egrads, const int* inLen,
+                             const int* labLen, const Dims& d, bool accumulate,
+                             const SparseTerms& sparse, hipStream_t s) {
+  if (sparse.labels && accumulate)
+    return fail(kInvalid, "sparse-term folding and accumulation are mutually exclusive");
+  if (sparse.labels && d.U - 1 > kMaxLabels)  // the per-wavefront match list of the folded terms
+    return fail(kInvalid, "egrads: blank/label terms can be folded in for at most %d labels",
+                kMaxLabels);
+  if (!accumulate && !egrads_one_pass(d))
+    return fail(kInvalid, "egrads: %d label positions take more than one slice", d.U);
   const int Up = wplane_up(d.U), Tw = wplane_tw(d.T);
-  const int vtiles = (d.V + 127) / 128, ntiles = win.tile_end - win.tile_begin;
+  const int vtiles = (d.V + 127) / 128, ntiles = (d.T + 31) / 32;
   // enough workgroups to fill 256 CUs two deep several times over, but long enough runs of
   // frames per workgroup to amortise loading the Y fragments
   int chunks = (2048 + vtiles * d.B - 1) / (vtiles * d.B);
@@ -893,92 +798,28 @@ static int egrads_window(const TIO* E, const TIO* P, const float* mE, const floa
     chunks = std::max(chunks, std::min(ntiles, 512 / (vtiles * d.B)));
   const int per = (ntiles + chunks - 1) / chunks;
   chunks = (ntiles + per - 1) / per;
-  // A launch contracts 16 * kEsMaxS label positions (what a wavefront keeps of Y in registers);
-  // a longer label axis goes slice by slice.  Into an array of the caller's that is added to,
-  // every slice adds X times its sums and the last one scales the whole.  Otherwise the slices
-  // but the last leave their bare sums in the output -- no emissions read, no exponentials --
-  // and the last one finishes them: X times the total, the sparse terms, the factor (B=8
-  // T=10000 U=400 V=1000, four slices: 1.91 ms with every slice adding X times its sums and
-  // asking for the output where it is stored, 1.49 asking for it at the start of a tile).
+  // A launch contracts 16 * kEsMaxS label positions (what a wavefront keeps of Y in registers).  Into
+  // an array of the caller's that is added to, a longer label axis goes slice by slice: every slice
+  // adds X times its sums and the last one scales the whole.
   const SparseTerms none;
   const int slice = 16 * kEsMaxS;
   const bool many = (long)d.U * 32 > 2 * (long)d.V;  // labels per block of 32 columns
-#define RNNT_EG_LAUNCH_(MODE, MANY, DL, SP)                                                   \
-  hipLaunchKernelGGL((egrads_stream_kernel<MODE, MANY, TIO, TOUT>), dim3(vtiles, chunks, d.B), \
-                     dim3(256), 0, s, E, P, mE, mP, Wn, DL, out, inLen, labLen, d, Up, Tw,    \
-                     per, u_lo, SP, win)
-  // (only the kernels that fold sparse terms in come in both forms)
-#define RNNT_EG_LAUNCH(MODE, DL, SP)                                                          \
-  do {                                                                                        \
-    if constexpr (sizeof(TOUT) == 2 && MODE != kEgWhole) {                                    \
-      /* 16-bit gradients of several slices add up in a wide window: never reached */        \
-      return fail(kInvalid, "egrads: slices of 16-bit gradients need a wide window");        \
-    } else if constexpr (MODE == kEgWhole || MODE == kEgFinal) {                              \
-      if (many) RNNT_EG_LAUNCH_(MODE, true, DL, SP);                                          \
-      else RNNT_EG_LAUNCH_(MODE, false, DL, SP);                                              \
-    } else {                                                                                  \
-      RNNT_EG_LAUNCH_(MODE, false, DL, SP);                                                   \
-    }                                                                                         \
-  } while (0)
+#define RNNT_EG_LAUNCH(MODE, MANY, DL, SP)                                                     \
+  hipLaunchKernelGGL((egrads_stream_kernel<MODE, MANY, TIO>), dim3(vtiles, chunks, d.B),       \
+                     dim3(256), 0, s, E, P, mE, mP, Wn, DL, egrads, inLen, labLen, d, Up, Tw, \
+                     per, u_lo, SP)
   for (int u_lo = 0; u_lo < Up; u_lo += slice) {
-    const bool last = u_lo + slice >= Up;
-    if (accumulate) RNNT_EG_LAUNCH(kEgAdd, (last ? deltas : nullptr), none);
-    else if (Up <= slice) RNNT_EG_LAUNCH(kEgWhole, deltas, sparse);
-    else if (!last) RNNT_EG_LAUNCH(kEgPartial, nullptr, none);
-    else RNNT_EG_LAUNCH(kEgFinal, deltas, sparse);
+    if constexpr (sizeof(TIO) == 4) {
+      if (accumulate) RNNT_EG_LAUNCH(kEgAdd, false, (u_lo + slice >= Up ? deltas : nullptr), none);
+    } else if (accumulate) {
+      return fail(kInvalid, "egrads: 16-bit gradients cannot be added to");
+    }
+    // (only the kernels that fold sparse terms in come in both forms)
+    if (!accumulate && many) RNNT_EG_LAUNCH(kEgWhole, true, deltas, sparse);
+    else if (!accumulate) RNNT_EG_LAUNCH(kEgWhole, false, deltas, sparse);
     RNNT_LAUNCH_CHECK("egrads_stream_kernel");
   }
 #undef RNNT_EG_LAUNCH
-#undef RNNT_EG_LAUNCH_
-  return kOk;
-}
-
-// rows [t_lo, t_lo + n) of every utterance of dst[B][T][V] = the rows [0, n) of src[B][Tc][V],
-// each value rounded once
-template <typename TIO>
-__global__ void narrow_rows_kernel(const float* __restrict__ src, TIO* __restrict__ dst, int T,
-                                   int Tc, int V, int t_lo, int per_row) {
-  const int b = blockIdx.y, t = blockIdx.x / per_row;
-  const int v = (blockIdx.x - t * per_row) * 256 + threadIdx.x;
-  if (v < V) stf(dst + ((size_t)b * T + t_lo + t) * V + v, src[((size_t)b * Tc + t) * V + v]);
-}
-
-// `wide`, `wide_bytes`: fp32 scratch for 16-bit gradients whose label axis needs more than one
-// slice.  Slices add up in the output array, which for a 16-bit array would round every partial
-// sum; so the frames are taken a window at a time, the slices add up in an fp32 copy of the
-// window, and the finished window is rounded once on its way into the caller's array.
-template <typename TIO>
-static int egrads_stream_any(const TIO* E, const TIO* P, const float* mE, const float* mP,
-                             const float* Wn, const float* deltas, TIO* egrads, const int* inLen,
-                             const int* labLen, const Dims& d, bool accumulate,
-                             const SparseTerms& sparse, hipStream_t s, float* wide = nullptr,
-                             size_t wide_bytes = 0) {
-  if (sparse.labels && accumulate)
-    return fail(kInvalid, "sparse-term folding and accumulation are mutually exclusive");
-  if (sparse.labels && d.U - 1 > kMaxLabels)  // the per-wavefront match list of the folded terms
-    return fail(kInvalid, "egrads: blank/label terms can be folded in for at most %d labels",
-                kMaxLabels);
-  const int ntiles = (d.T + 31) / 32;
-  if (sizeof(TIO) == sizeof(float) || egrads_one_pass(d)) {
-    const EgradsWindow all{0, ntiles, d.T, 0};
-    return egrads_window(E, P, mE, mP, Wn, deltas, egrads, inLen, labLen, d, accumulate, sparse,
-                         all, s);
-  }
-  if (accumulate) return fail(kInvalid, "egrads: 16-bit gradients cannot be added to");
-  const size_t row_bytes = sizeof(float) * (size_t)d.B * d.V;
-  const int Tc = (int)std::min<size_t>(wide ? wide_bytes / row_bytes / 32 * 32 : 0, (size_t)ntiles * 32);
-  if (Tc < 32)
-    return fail(kWorkspace, "egrads: no room for a window of 32 frames of fp32 gradients");
-  for (int t_lo = 0; t_lo < d.T; t_lo += Tc) {
-    const EgradsWindow win{t_lo / 32, std::min(ntiles, (t_lo + Tc) / 32), Tc, t_lo};
-    RNNT_TRY(egrads_window(E, P, mE, mP, Wn, deltas, wide, inLen, labLen, d, false, sparse, win,
-                           s));
-    const int n = std::min(Tc, d.T - t_lo);
-    const unsigned per_row = (unsigned)((d.V + 255) / 256);
-    hipLaunchKernelGGL((narrow_rows_kernel<TIO>), dim3(per_row * (unsigned)n, d.B), dim3(256), 0,
-                       s, wide, egrads, d.T, Tc, d.V, t_lo, (int)per_row);
-    RNNT_LAUNCH_CHECK("narrow_rows_kernel");
-  }
   return kOk;
 }
 #if RNNT_IN_PART(0)
@@ -994,20 +835,18 @@ int launch_egrads_stream(const float* E, const float* P, const float* mE, const 
 int launch_egrads_stream(const bf16_t* E, const bf16_t* P, const float* mE, const float* mP,
                          const float* Wn, const float* deltas, bf16_t* egrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
-                         const SparseTerms& sparse, hipStream_t s, float* wide,
-                         size_t wide_bytes) {
+                         const SparseTerms& sparse, hipStream_t s) {
   return egrads_stream_any(E, P, mE, mP, Wn, deltas, egrads, inLen, labLen, d, accumulate, sparse,
-                           s, wide, wide_bytes);
+                           s);
 }
 #endif
 #if RNNT_IN_PART(2)
 int launch_egrads_stream(const f16_t* E, const f16_t* P, const float* mE, const float* mP,
                          const float* Wn, const float* deltas, f16_t* egrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
-                         const SparseTerms& sparse, hipStream_t s, float* wide,
-                         size_t wide_bytes) {
+                         const SparseTerms& sparse, hipStream_t s) {
   return egrads_stream_any(E, P, mE, mP, Wn, deltas, egrads, inLen, labLen, d, accumulate, sparse,
-                           s, wide, wide_bytes);
+                           s);
 }
 #endif
 

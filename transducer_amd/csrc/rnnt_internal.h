@@ -361,14 +361,12 @@ int launch_grads_fused(const float* E, const float* P, const float* mE, const fl
                        const WImages& img, const float* deltas, float* egrads, float* pgrads,
                        const int* inLen, const int* labLen, const Dims& d, const SparseTerms& sp,
                        const SparsePTerms& spp, hipStream_t s);
-// Whether one launch covers the label axis.  A longer axis goes slice by slice, the slices adding
-// up in the output array; 16-bit gradients then go through `wide` (fp32 scratch of wide_bytes,
-// at least 32 frames of B * V values), a window of frames at a time, so that each value is still
-// rounded once.
+// Whether launch_egrads_stream's workgroups can hold the whole label axis.  A longer one goes
+// through launch_egrads_long; only where it is added to fp32 values of the caller's
+// (accumulate) does launch_egrads_stream take it too, slice by slice.
 bool egrads_one_pass(const Dims& d);
-// ---- (rnnt_egrads_long.hip) A longer label axis in one launch, where the pieces of Y have room:
-// scratch of lse_scratch_bytes(d).  out = delta * (dense + sparse), egrads written once.
-bool egrads_long_takes(const Dims& d);
+// ---- (rnnt_egrads_long.hip) A longer label axis in one launch, the pieces of Y in scratch of
+// lse_scratch_bytes(d).  out = delta * (dense + sparse), egrads written once.
 int launch_egrads_long(const float* E, const float* P, const float* mE, const float* mP,
                        const float* Wn, const float* deltas, float* egrads, const int* inLen,
                        const int* labLen, const Dims& d, const SparseTerms& sparse, void* scratch,
@@ -388,13 +386,11 @@ int launch_egrads_stream(const float* E, const float* P, const float* mE, const 
 int launch_egrads_stream(const bf16_t* E, const bf16_t* P, const float* mE, const float* mP,
                          const float* Wn, const float* deltas, bf16_t* egrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
-                         const SparseTerms& sparse, hipStream_t s, float* wide = nullptr,
-                         size_t wide_bytes = 0);
+                         const SparseTerms& sparse, hipStream_t s);
 int launch_egrads_stream(const f16_t* E, const f16_t* P, const float* mE, const float* mP,
                          const float* Wn, const float* deltas, f16_t* egrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
-                         const SparseTerms& sparse, hipStream_t s, float* wide = nullptr,
-                         size_t wide_bytes = 0);
+                         const SparseTerms& sparse, hipStream_t s);
 int launch_pgrads_stream(const float* E, const float* P, const float* mE, const float* mP,
                          const float* Wt, const float* deltas, float* pgrads, const int* inLen,
                          const int* labLen, const Dims& d, bool accumulate,
