@@ -900,6 +900,26 @@ def test_sparse_terms_either_side_of_every_split_of_frames_and_positions(T, U, V
             assert_same_bits(g, w, what)
 
 
+@pytest.mark.parametrize("V,step", [(9, 1), (40, 4), (300, 0)])
+@pytest.mark.parametrize("U", [9, 10, 64, 65, 66, 129, 130])
+def test_label_terms_of_a_small_vocabulary_at_the_edges_of_64_positions(U, V, step):
+    """Labels picked 64 positions at a time and taken eight at a time by the wavefront of their column's
+    remainder by four: every label in one column (step 0), in one remainder (4) or across all (1)."""
+    rng = np.random.default_rng(U + V)
+    B, T = 2, 37
+    E = rng.standard_normal((B, T, V), dtype=np.float32)
+    P = rng.standard_normal((B, U, V), dtype=np.float32)
+    labels = np.broadcast_to((1 + step * np.arange(U - 1)) % V, (B, U - 1)).astype(np.int32).copy()
+    il, ll = np.array([T, T - 5], np.int32), np.array([U - 1, U - 2], np.int32)
+    LN = oracle.log_norms_naive(E, P, il, ll)
+    c = DeviceCase(E, P, labels, il, ll)
+    _, alphas = gpu_forward(c, np.nan_to_num(LN))
+    got = gpu_backward(c, np.nan_to_num(alphas), np.nan_to_num(LN))
+    want = oracle.backward(E, P, np.nan_to_num(alphas), LN, labels, il, ll)
+    for g, w, what in zip(got, want, ("egrads", "pgrads", "lngrads")):
+        assert_same_bits(g, w, what)
+
+
 @pytest.mark.parametrize("T,U,V", [(1, 113, 31), (127, 113, 33), (128, 128, 127), (129, 129, 129),
                                    (130, 160, 32), (257, 161, 600), (64, 225, 520)])
 def test_egrads_of_long_label_axes_at_the_edges_of_their_tiles(T, U, V):

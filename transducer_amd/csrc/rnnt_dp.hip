@@ -1735,10 +1735,13 @@ __global__ __launch_bounds__(256) void sparse_e_kernel(const float* __restrict__
 // dense part.  With few columns the hardware adds of sparse_e_kernel all land in a few cache
 // lines per row and queue up at L2 (B=8, T=2000, U=100, V=100: 0.08 ms for 1.6 M adds), so
 // here a workgroup keeps its frames' rows in LDS (64 x V floats, odd pitch: lane t owns row t, all
-// lanes hit column l together, no conflicts).  Its first wavefront subtracts the terms there in the
-// reference's order, the next sixteen requested ahead; then all four add the rows to egrads, which are
-// one contiguous piece of memory (B=8 T=2000 U=101 V=100: 34 us with one wavefront doing it all, a
-// round trip per eight rows and 64 columns, 21 now).
+// lanes hit column l together, no conflicts).  Each of the four wavefronts takes the columns of one
+// remainder by four: it picks their positions out of 64 labels at a time with a ballot and subtracts
+// their terms in the reference's order, the next eight requested ahead (a subtraction in LDS waits
+// for the one before it, 0.1 us; LDS adds that nothing waits for are no faster: B=8 T=10000 U=401
+// V=32 the whole step 2073 us with one wavefront subtracting, 2165 with one adding).  Then all four add
+// the rows to egrads, one contiguous piece of memory (B=8 T=2000 U=101 V=100: 20 us with one
+// wavefront subtracting, 15 with four; T=10000 U=401 V=32 53 and 45).
 // `frames` (at most 64) rows a workgroup; 32 where the LDS of 64 would pass 64 KB (B=16 T=2000 U=101
 // V=500: 162 us with hardware adds, 58 so).  Dynamic LDS: frames * (V | 1) floats.
 __global__ __launch_bounds__(256) void sparse_e_rows_kernel(const float* __restrict__ bsum,
@@ -1757,34 +1760,47 @@ __global__ __launch_bounds__(256) void sparse_e_rows_kernel(const float* __restr
   const int pitch = d.V | 1;
   for (int i = tid; i < frames * pitch; i += 256) rows[i] = 0.0f;
   __syncthreads();
-  if (tid < frames) {
-    const int t = min(t0 + tid, Tb - 1);  // lanes past the utterance walk its last frame, unused
-    float* mine = rows + tid * pitch;
+  {
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t = min(t0 + lane, Tb - 1);  // lanes past the utterance walk its last frame, unused
+    const bool own = lane < frames;
+    float* mine = rows + min(lane, frames - 1) * pitch;
     const int* __restrict__ lab = labels + (size_t)b * (d.U - 1);
     const float* __restrict__ em = emT + (size_t)b * d.U * d.T + t;
-    constexpr int kChunk = 16;
-    struct Terms { float e[kChunk]; };
-    auto request = [&](int uhi) -> Terms {
-      Terms r;
-#pragma unroll
-      for (int k = 0; k < kChunk; ++k) r.e[k] = em[(size_t)max(uhi - k, 0) * d.T];
-      return r;
+    if (wave == 0 && own) mine[d.blank] += bsum[(size_t)b * d.T + t];
+    constexpr int kBatch = 8;
+    struct Batch { float e[kBatch]; int l[kBatch]; };
+    // lane k of a look holds the label of position c0 + k (the blank's where there is none)
+    auto look = [&](int c0) -> int {
+      const int u = c0 + lane, l = clampi(lab[clampi(u, 0, Ub - 2)], 0, d.V - 1);
+      return u < Ub - 1 ? l : d.blank;
     };
-    const float blanks = bsum[(size_t)b * d.T + t];
-    Terms cur = request(Ub - 2);
-    for (int uhi = Ub - 2; uhi >= 0; uhi -= kChunk) {
-      const Terms nxt = request(uhi - kChunk);
+    const int last = Ub >= 2 ? (Ub - 2) & ~63 : -1;
+    int next = last >= 0 ? look(last) : 0;
+    for (int c0 = last; c0 >= 0; c0 -= 64) {
+      const int here = next;
+      next = look(max(c0 - 64, 0));
+      unsigned long long m = __ballot(here != d.blank && (here & 3) == wave);
+      auto request = [&]() -> Batch {  // the next moves, highest position first; l = -1: no more
+        Batch x;
 #pragma unroll
-      for (int k = 0; k < kChunk; ++k) {
-        const int u = uhi - k;
-        if (u >= 0) {  // uniform
-          const int l = clampi(lab[u], 0, d.V - 1);
-          if (l != d.blank) mine[l] -= cur.e[k];
+        for (int k = 0; k < kBatch; ++k) {
+          const int at = m ? 63 - __builtin_clzll(m) : 0;
+          x.l[k] = m ? __builtin_amdgcn_readlane(here, at) : -1;
+          x.e[k] = em[(size_t)(c0 + at) * d.T];
+          m &= ~(1ull << at);
         }
+        return x;
+      };
+      Batch cur = request();
+      while (cur.l[0] >= 0) {
+        const Batch nxt = request();
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k)
+          if (cur.l[k] >= 0 && own) mine[cur.l[k]] -= cur.e[k];
+        cur = nxt;
       }
-      cur = nxt;
     }
-    mine[d.blank] += blanks;
   }
   __syncthreads();
   const float sc = scale ? scale[b] : 1.0f;
@@ -3679,8 +3695,8 @@ static int viterbi_walk(const Planes& p, const float* bestS, const float* argS, 
                      labLen, gcols, labels_out, d, nw, g_spin_limit, trouble, live, n);
   RNNT_LAUNCH_CHECK("viterbi_walk_kernel");
   if (!kLdsBits) {
-    hipLaunchKernelGGL(viterbi_trace_kernel, dim3(d.B), dim3(64), sizeof(int) * (size_t)d.U, s, argS, inLen, labLen, gcols,
-                       labels_out, d, nw);
+    hipLaunchKernelGGL(viterbi_trace_kernel, dim3(d.B), dim3(64), sizeof(int) * (size_t)d.U, s, argS,
+                       inLen, labLen, gcols, labels_out, d, nw);
     RNNT_LAUNCH_CHECK("viterbi_trace_kernel");
   }
   return kOk;
@@ -3696,7 +3712,9 @@ static int launch_viterbi_walk(const Planes& p, const float* bestS, const float*
   const size_t lds = sizeof(int) * (((size_t)d.U + 3 & ~(size_t)3) + (size_t)64 * W * nw);
   const bool fits = n == 1 && lds <= (d.B <= 256 ? 140u : 60u) * 1024;
   const dim3 one(d.B);
-#define WALK(W, LIVE, LDS, GRID, BYTES)                                                               viterbi_walk<W, LIVE, LDS>(p, bestS, argS, gcols, inLen, labLen, labels_out, d, nw, s, GRID, BYTES, n)
+#define WALK(W, LIVE, LDS, GRID, BYTES)                                                          \
+  viterbi_walk<W, LIVE, LDS>(p, bestS, argS, gcols, inLen, labLen, labels_out, d, nw, s, GRID,   \
+                             BYTES, n)
   if (n > 1) return WALK(4, true, false, dim3(8 * n * ((d.B + 7) / 8)), 0);
   if (W == 1) return fits ? WALK(1, false, true, one, lds) : WALK(1, false, false, one, 0);
   if (W == 2) return fits ? WALK(2, false, true, one, lds) : WALK(2, false, false, one, 0);
