@@ -578,6 +578,28 @@ def test_log_norms_reference_moves_late_in_the_row():
     assert np.abs(got - truth).max() < 4e-6 * max(1.0, np.abs(truth).max())
 
 
+@pytest.mark.parametrize("B,T,V", [(1, 70, 700), (1, 130, 701), (128, 129, 200)])
+@pytest.mark.parametrize("U", [9, 33, 65, 97, 128])
+def test_log_norms_references_that_move_from_slab_to_slab(B, T, U, V):
+    """References that jump in one slab of 32 columns after another, in all rows, in those that one
+    wavefront stages (16 of 64) or in every third, while one to four wavefronts have label positions
+    to multiply: a factor that is applied a slab early or late leaves sums that are exp(50) off.
+    The bound is the one above.  (The last shape takes tiles of 128 frames, the others of 64.)"""
+    rng = np.random.default_rng(B + T + U + V)
+    E = rng.standard_normal((B, T, V), dtype=np.float32)
+    P = rng.standard_normal((B, U, V), dtype=np.float32)
+    slab = np.arange(V) // 32
+    t = np.arange(T)[:, None]
+    E[:, :, :] += np.where(t % 64 // 16 == slab % 5, 50.0 * slab,      # one wavefront's rows a slab
+                           np.where(t % 3 == 0, 50.0 * slab,           # every slab
+                                    np.where(t % 3 == 1, 50.0 * (slab // 2), 0.0))).astype(np.float32)
+    c = DeviceCase(E, P, np.zeros((B, U - 1), np.int32), np.full(B, T, np.int32),
+                   np.full(B, U - 1, np.int32))
+    got = gpu_log_norms(c, with_lengths=False)
+    truth = oracle.log_norms_truth(E, P)
+    assert np.abs(got - truth).max() < 4e-6 * np.abs(truth).max()
+
+
 @pytest.mark.parametrize("off_e,off_p", [(300.0, 0.0), (-300.0, 150.0), (120.0, -400.0)])
 @pytest.mark.parametrize("V", [200, 700])
 def test_gradients_of_scores_far_from_zero(off_e, off_p, V):

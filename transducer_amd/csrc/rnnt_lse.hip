@@ -168,9 +168,11 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
   // and the registers are taken.
   constexpr int kAhead = kRows == 64 ? 4 : 1, kYAhead = kRows == 64 ? 2 : 1;
   __shared__ uint4 Xs[2][3][kSlots];
-  __shared__ float scale[kRows];  // pending factor for a row's sums (1 when its reference stood)
+  // By the buffer of the slab they belong to: a wavefront that is done with a slab says what moved
+  // while it stages the next one, and others may not have looked at this slab's flag yet.
+  __shared__ float scale[2][kRows];  // pending factor for a row's sums (1 when its reference stood)
   __shared__ float mfin[kRows];   // final references, for the write-out
-  __shared__ int moved;           // some row's reference moved while the last slab was staged
+  __shared__ int moved[2];           // some row's reference moved while the slab was staged
   __shared__ int labs[1025];      // columns to pick: the utterance's labels, then the blank
   __shared__ short order[1025];   // their indices sorted by column
   __shared__ int scol[1025];      // and the columns in that order
@@ -262,8 +264,8 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
       y0[1].s1 = fetch_y(2 * min(1, nk - 1) + 1);
     }
   }
-  for (int r = tid; r < kRows; r += kThreads) scale[r] = 1.0f;
-  if (tid == 0) moved = 0;
+  for (int r = tid; r < 2 * kRows; r += kThreads) scale[r / kRows][r % kRows] = 1.0f;
+  if (tid < 2) moved[tid] = 0;
   // Picks: the lattice recursions need E[t, blank] and E[t, label_u] in the skewed planes.  Every
   // element of the tile's rows passes through the staging registers exactly once, so the thread
   // that holds a wanted column copies it out then (first label tile only; ebv == nullptr: off;
@@ -417,8 +419,8 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
 #pragma unroll
       for (int i = 0; i < NR; ++i)
         if (need[i]) {
-          if (c8 == 0) scale[srow + (kThreads / 4) * i] = __expf(was[i] - mx[i]);
-          moved = 1;
+          if (c8 == 0) scale[buf][srow + (kThreads / 4) * i] = __expf(was[i] - mx[i]);
+          moved[buf] = 1;
         }
     }
   };
@@ -452,7 +454,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
     const int kty = min(kt + kYAhead, nk - 1);  // whose fragments are requested
     // did a row's reference move while this slab was staged?  Read together with the fragments
     // (LDS answers in order), so the flag costs no round trip of its own.
-    const int mv = moved;
+    const int mv = moved[cur];
     if constexpr (kAhead == 1) xq = fetch(ktn * kSlice);
     if (kAct) {
       uint4 ah[MB], am[MB], al[MB];
@@ -468,7 +470,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
         for (int m = 0; m < MB; ++m)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const float f = scale[32 * (mb0 + m) + mfma_row(r, h)];
+            const float f = scale[cur][32 * (mb0 + m) + mfma_row(r, h)];
             acc[m][r] *= f;
             tot[m][r] *= f;
           }
@@ -514,11 +516,10 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
       y.s1 = fetch_y(2 * kty + 1);
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (mv) {  // every wavefront has used the factors: back to 1 before the staging sets new ones
+    if (mv) {  // every wavefront has used the factors: back to 1, for the slab after the next
       __syncthreads();
-      for (int r = tid; r < kRows; r += kThreads) scale[r] = 1.0f;
-      if (tid == 0) moved = 0;
-      __syncthreads();
+      for (int r = tid; r < kRows; r += kThreads) scale[cur][r] = 1.0f;
+      if (tid == 0) moved[cur] = 0;
     }
     stash(cur ^ 1, xq, false, ktn);
     if constexpr (kAhead > 1) xq = fetch(min(kt + 1 + kAhead, nk - 1) * kSlice);
