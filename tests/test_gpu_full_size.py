@@ -8,8 +8,8 @@ configurations go through the oracle whole."""
 import numpy as np
 import pytest
 
-from util import (RTOL, ATOL, DeviceCase, assert_close, dev, gpu_log_norms, gpu_loss, ptr,
-                  violations)
+from util import (RTOL, ATOL, DeviceCase, assert_close, dev, gpu_backward, gpu_forward,
+                  gpu_log_norms, gpu_loss, gpu_viterbi, ptr, violations)
 
 pytestmark = pytest.mark.gpu
 
@@ -463,3 +463,23 @@ def test_arrays_past_two_to_the_31_elements_index_like_small_ones():
         alone = viterbi_on_device(one, LN[b:b + 1].contiguous())
         n = int(c.ll_h[b])
         assert torch.equal(alone[0, :n], paths[b, :n]), b
+
+
+def test_planes_of_more_than_4_gib_carry_the_reference_bits():
+    """An utterance so long that its lattice planes pass 2^32 bytes each (64 label positions are the
+    least a plane holds, so few label positions and many frames do): the walks move their buffers
+    four times on the way, and what lies past 4 GiB is walked like the rest."""
+    T, U, V = 16777300, 2, 2
+    rng = np.random.default_rng(T)
+    E = rng.standard_normal((1, T, V), dtype=np.float32)
+    P = rng.standard_normal((1, U, V), dtype=np.float32)
+    LN = np.logaddexp(E[:, :, None, 0] + P[:, None, :, 0], E[:, :, None, 1] + P[:, None, :, 1])
+    labels, il, ll = np.ones((1, 1), np.int32), np.array([T], np.int32), np.array([1], np.int32)
+    c = DeviceCase(E, P, labels, il, ll)
+    costs, alphas = gpu_forward(c, LN)
+    want_costs, want = oracle.forward(E, P, LN, labels, il, ll)
+    assert np.array_equal(costs, want_costs) and np.array_equal(alphas, want)
+    assert np.array_equal(gpu_viterbi(c, LN), oracle.viterbi(E, P, LN, il, ll))
+    got = gpu_backward(c, want, LN)
+    for g, w in zip(got, oracle.backward(E, P, want, LN, labels, il, ll)):
+        assert np.array_equal(g, w)

@@ -837,7 +837,7 @@ typedef float quad4_t __attribute__((ext_vector_type(4), aligned(4)));
 struct Buffer {
   __amdgpu_buffer_rsrc_t r;
   __device__ Buffer(const void* p, size_t bytes) {
-    int n = (int)(unsigned)bytes, flags = 0x00020000;
+    int n = (int)buffer_bytes(bytes), flags = 0x00020000;
     // (opaque: words that several descriptors have in common would be copied around at every use)
     asm volatile("" : "+s"(n), "+s"(flags));
     r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, n, flags);

@@ -87,6 +87,13 @@ __host__ __device__ inline size_t plane_group0(const Dims& d, int b, int u) {
 }
 __host__ __device__ inline int plane_group_stride(const Dims& d) { return 4 * d.Ua; }
 
+// What a buffer descriptor can say of a piece of memory: its size in 32 bits, so all of it or, of a
+// longer piece, its first 4 GiB less a byte.  (The walks move their buffers on every GiB of a plane
+// and never look further than that and a few groups ahead.)
+__host__ __device__ constexpr unsigned buffer_bytes(size_t bytes) {
+  return bytes < 0xffffffffu ? (unsigned)bytes : 0xffffffffu;
+}
+
 __device__ inline int clampi(int x, int lo, int hi) { return x < lo ? lo : (x > hi ? hi : x); }
 
 // Per-utterance extents, clamped to the padded array so a bad length can never index past it.
