@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "rnnt_internal.h"
+#include "rnnt_blocks.h"
 #include "rnnt_libm.h"
 #include "rnnt_split.h"
 
@@ -32,10 +33,6 @@
 #define RNNT_IN_PART(n) (RNNT_DP_PART < 0 || RNNT_DP_PART == (n))
 
 namespace rnnt {
-
-int alpha_blocks(const Dims& d);
-int beta_blocks(const Dims& d, int* waves);
-int viterbi_blocks(const Dims& d);
 
 namespace {
 
@@ -3216,41 +3213,6 @@ int trouble_flag(int** out) {
 // ------------------------------------------------------------------ workspace layout
 static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Blocks of 256 label positions that the alpha walk runs side by side (1: none).  Up to 1024
-// positions the other way is one workgroup with two or four positions a lane, whose one CU holds it:
-// T=2000, 401 positions 663 -> 381 us at B=128, 1000 positions 1724 -> 541 at B=64.  With more
-// workgroups than fit two to a CU side by side (about three if the axis takes three blocks or more,
-// which leaves the other way as many cells a lane) the walks only share issue slots: T=500,
-// 300 positions, B=300: 307 -> 413.  Past 1024 positions the other way is a launch per 1024, many
-// times slower whatever the batch; workgroups beyond the device's CUs queue in order.
-int alpha_blocks(const Dims& d) {
-  const int n = (d.U + 255) / 256;
-  if (n < 2 || n > 16 || ((long)d.B * n > (n == 2 ? 512 : 900) && d.U <= 1024)) return 1;
-  return n;
-}
-// Blocks that the dalpha walk runs side by side, and the wavefronts (64 positions each) of a block.
-// A cell is six instructions and 12 bytes, and what one CU's memory path moves holds the walk, so
-// blocks are narrower than alpha's: 128 positions (B=8 T=10000, 401 positions: 610 us with blocks
-// of 256, 372 with 128; T=2000 100 either way).  129 to 256 positions, which four wavefronts
-// of one workgroup can take as well, go side by side where the three planes of the walk are more
-// than the memory-side cache keeps beside everything else (B=8, 201 positions: T=2000 80 us on one
-// workgroup, 84 as two; T=4000 142 and 142; T=6000 314 and 202; B=32 T=2000 152 and 106).
-// Up to 512 positions that holds for any batch (B=512 T=300, 300 positions: 378 -> 266 against two
-// positions a lane on one CU); on longer axes with more than 512 such blocks, alpha's.
-int beta_blocks(const Dims& d, int* waves) {
-  const int n2 = (d.U + 127) / 128;
-  *waves = 2;
-  if (d.U > 256 && n2 <= 16 && (d.U <= 512 || (long)d.B * n2 <= 512)) return n2;
-  if (d.U > 128 && d.U <= 256 && 12ull * d.B * d.Ua * d.Dp > 100ull << 20) return n2;
-  *waves = 4;
-  return alpha_blocks(d);
-}
-// Blocks of 256 label positions that the best-path walk runs side by side (1: none): alpha's rule,
-// with three blocks or more only up to 192 workgroups, so that the decode's scratch stays what it is.
-int viterbi_blocks(const Dims& d) {
-  const int n = alpha_blocks(d);
-  return n > 2 && (long)d.B * n > 192 && d.U <= 1024 ? 1 : n;
-}
 // The two hand-over vectors of the planes hold the walks' tagged 64-bit entries as well: one
 // array of [B][Dp] entries per boundary between blocks side by side.  In units of [B][Dp] floats
 // each.
@@ -3336,14 +3298,6 @@ int launch_gather(const f16_t* E, const f16_t* P, const int* labels, const int* 
 }
 
 #endif
-
-// Label positions one launch of a lattice walk covers: the whole axis up to 1024, else blocks of
-// 1024 (64 lanes x 16 positions), one launch per block.
-static int block_cells_per_lane(const Dims& d) { return min(cells_per_lane(d.U), 16); }
-static int label_blocks(const Dims& d) {
-  const int width = 64 * block_cells_per_lane(d);
-  return (d.U + width - 1) / width;
-}
 
 static __global__ void clear_words_kernel(int* x, int n) {
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -3676,9 +3630,6 @@ int launch_maxplus(const f16_t* E, const f16_t* P, const int* inLen, const int* 
 #endif
 
 #if RNNT_IN_PART(4)
-// 32-step words per column of the decision table (one spare)
-static int viterbi_words(const Dims& d) { return (d.T + d.U + 31) / 32 + 1; }
-
 template <int W, bool kLive, bool kLdsBits>
 static int viterbi_walk(const Planes& p, const float* bestS, const float* argS, unsigned* gcols,
                         const int* inLen, const int* labLen, int* labels_out, const Dims& d, int nw,
@@ -3733,18 +3684,10 @@ int launch_viterbi(const Planes& p, const float* bestS, const float* argS,
   if (d.U <= 256 || viterbi_blocks(d) > 1)
     return launch_viterbi_walk(p, bestS, argS, gcols, inLen, labLen, labels_out, d, nw, s);
   // several positions a lane, on four wavefronts while their hand-over arrays fit
-  const size_t taken_lds = sizeof(int) * (size_t)((d.U + 3) & ~3);
-  const int W = (nblocks == 1 && cpl >= 4 &&
-                 taken_lds + 3 * stride * sizeof(float) <= 144 * 1024) ? 4
-                : (cpl >= 2 && taken_lds + stride * sizeof(float) <= 144 * 1024) ? 2 : 1;
-  // dynamic LDS: one int per label position, the hand-over arrays between the wavefronts,
-  // and the decision columns when they fit (one block only: with several, every block's columns
-  // must be there for the backtrace of the last launch)
-  const size_t base_lds = sizeof(int) * (size_t)((d.U + 3) & ~3) +
-                          (W > 1 ? sizeof(float) * (size_t)(W - 1) * stride : 0);
-  const size_t cols_lds = sizeof(unsigned) * (size_t)64 * cpl * nw;
-  const bool use_lds = nblocks == 1 && base_lds + cols_lds <= 60 * 1024;
-  const size_t lds = base_lds + (use_lds ? cols_lds : 0);
+  const ViterbiOne one = viterbi_one(d);
+  const int W = one.wavefronts;
+  const bool use_lds = one.columns;
+  const size_t lds = one.lds;
   if (lds > 150 * 1024)
     return fail(kInvalid, "viterbi: %d label positions and %d steps need %zu bytes of LDS", d.U,
                 stride, lds);
