@@ -313,8 +313,7 @@ def test_label_axes_dealt_to_several_wavefronts_carry_the_reference_bits(T, U):
     """From 65 label positions the alpha walk and from 129 the dalpha walk deal the label axis to
     two or four wavefronts of one workgroup, which hand the boundary column's score on through
     LDS and wait for each other's progress counters (four from 129 positions; from 257 a small
-    batch like this one is walked as two halves side by side, and past 512 a lane owns two to
-    four positions, those of the dalpha walk 64 apart).  U counts the rows of predictions and sits on
+    batch like this one is walked as blocks side by side).  U counts the rows of predictions and sits on
     either side of every change of that split; T = 1 and 6 leave most wavefronts with less than
     one or two groups of four steps, 45 lets them fall the few groups behind that they run at.
     Same bars as everywhere: the reference's bits in every alpha, dalpha and sparse term, the
@@ -338,15 +337,17 @@ def test_label_axes_dealt_to_several_wavefronts_carry_the_reference_bits(T, U):
 
 
 @pytest.mark.parametrize("B,T,U", [(11, 300, 400), (3, 700, 258), (17, 150, 512), (96, 40, 300),
-                                   (97, 40, 300)])
+                                   (128, 8, 300), (129, 8, 300), (65, 30, 500), (129, 8, 500),
+                                   (257, 8, 400)])
 def test_two_halves_of_a_label_axis_walked_side_by_side_carry_the_reference_bits(B, T, U):
-    """257 .. 512 label positions in a batch of at most 96 utterances: the alpha and the dalpha
-    walk run the two halves of the label axis as two workgroups at the same time; the values of
-    the boundary column cross through memory, each with the number of its step beside it, and
-    the half that follows asks again for what was not there yet.  Long enough lattices that it
-    runs its steady state a few groups of steps behind the half that leads; batches that fill the last eight
-    workgroup slots only partly; 97 utterances take the one-workgroup walk again.  U counts the
-    rows of predictions."""
+    """257 .. 512 label positions: the alpha and the best-path walk run the two halves of the label
+    axis as two workgroups at the same time, the dalpha walk blocks of 128 or 256 positions; the values
+    of the boundary column cross through memory, each with the number of its step beside it, and a
+    wavefront of the block that follows asks again for what was not there yet.  Lattices short and long;
+    batches that fill the last eight workgroup slots only partly.  On lattices this short 128 utterances
+    are the last that go side by side: 129 take one workgroup each again, two positions a lane (the
+    dalpha walk from 385 positions on; 65 utterances of those are its first with blocks of 256).  U
+    counts the rows of predictions."""
     cfg = small_config(B, T, U - 1, 5, ragged=True)
     E, P, labels, il, ll = unpack(make_inputs(cfg, seed=B * 1000 + U))
     il[0], ll[0] = T, U - 1                  # one utterance uses both halves to the end
@@ -364,23 +365,26 @@ def test_two_halves_of_a_label_axis_walked_side_by_side_carry_the_reference_bits
         assert_same_bits(lng, lng_o, what="lngrads")
         assert_same_bits(eg, eg_o, what="egrads (sparse)")
         assert_same_bits(pg, pg_o, what="pgrads (sparse)")
+        assert np.array_equal(gpu_viterbi(c, LN), oracle.viterbi(E, P, LN, il, ll))
     from transducer_amd import capi
     assert capi.load().rnnt_hip_check_kernels(None) == 0
 
 
 @pytest.mark.parametrize("B,T,U", [(5, 200, 513), (9, 120, 700), (3, 60, 1000), (4, 90, 1025),
                                    (2, 40, 2100), (70, 6, 600), (40, 5, 1025), (12, 4, 4200),
-                                   (300, 3, 1100)])
+                                   (300, 3, 1100), (49, 20, 1000), (101, 4, 1000), (171, 4, 700),
+                                   (201, 4, 1000), (301, 4, 700)])
 def test_label_axis_as_a_chain_of_blocks_side_by_side_and_where_it_is_not(B, T, U):
-    """From 513 label positions the alpha and dalpha walks run three and more blocks of 256
-    positions side by side, each following the one before it through its own array of tagged
-    entries -- up to 1024 positions as long as the batch leaves the device the CUs for it
-    (utterances x blocks at most 192), beyond whatever the batch (40 x 5 workgroups, 300 x 5:
-    more than the device runs at once, so later utterances' blocks queue behind earlier ones).
-    70 x 3 workgroups for 600 positions are too many and 17 blocks too long: those take one
-    workgroup per utterance again, a lane owning several positions, or a launch per 1024
-    positions.  Either way the reference's bits.  U counts the rows of
-    predictions; ragged batches, so that some utterances end blocks below the top one."""
+    """From 513 label positions the walks run three and more blocks of 256 positions (the dalpha walk
+    of 128 in small batches) side by side, each following the one before it through its own array of
+    tagged entries -- up to 1024 positions as long as the batch leaves the device room for it, beyond
+    whatever the batch (40 x 5 workgroups, 300 x 5: more than the device runs at once, so later
+    utterances' blocks queue behind earlier ones).  Batches past that room take one workgroup per
+    utterance, a lane owning four positions: here the best path of 70 x 600, 49 x 1000 and all
+    larger ones, alpha of 171 x 700, 201 x 1000 and 301 x 700, dalpha of 101 x 1000, 201 x 1000 and
+    301 x 700.  17 blocks are too many: a launch per 1024 positions.  Either way the reference's bits.  U
+    counts the rows of predictions; ragged batches, so that some utterances end blocks below the top
+    one."""
     cfg = small_config(B, T, U - 1, 4, ragged=True)
     E, P, labels, il, ll = unpack(make_inputs(cfg, seed=B * 7 + U))
     il[0], ll[0] = T, U - 1
@@ -397,18 +401,19 @@ def test_label_axis_as_a_chain_of_blocks_side_by_side_and_where_it_is_not(B, T, 
         assert_same_bits(lng, lng_o, what="lngrads")
         assert_same_bits(eg, eg_o, what="egrads (sparse)")
         assert_same_bits(pg, pg_o, what="pgrads (sparse)")
+        assert np.array_equal(gpu_viterbi(c, LN), oracle.viterbi(E, P, LN, il, ll))
     from transducer_amd import capi
     assert capi.load().rnnt_hip_check_kernels(None) == 0
 
 
 @pytest.mark.parametrize("B,T,U", [(2, 13000, 70), (2, 12500, 200), (1, 20000, 300), (3, 12400, 129),
-                                   (1, 40000, 30), (1, 37000, 150)])
+                                   (1, 40000, 30), (1, 37000, 150), (1, 12300, 4100),
+                                   (1, 33000, 4100)])
 def test_very_long_utterances_keep_their_wavefronts(B, T, U):
-    """Past about 12000 anti-diagonals the three hand-over arrays of four wavefronts no longer fit
-    LDS: the walks then deal the label axis to workgroups of two wavefronts (one array, good for
-    36000 anti-diagonals), up to 128 positions one workgroup, beyond blocks of 128 side by side;
-    past 36000 anti-diagonals one wavefront per utterance walks the whole label axis.
-    The reference's bits and the exact path, as everywhere."""
+    """One position a lane the walks hand over through rings of fixed size, whatever the length.  Past 4096
+    positions, a launch per 1024, whole hand-over arrays lie in LDS: two wavefronts share them up to
+    about 36000 anti-diagonals (12300 + 4100 here), one walks alone beyond (33000 + 4100).  The
+    reference's bits and the exact path, as everywhere."""
     cfg = small_config(B, T, U - 1, 4, ragged=True)
     E, P, labels, il, ll = unpack(make_inputs(cfg, seed=T + U))
     il[0], ll[0] = T, U - 1
