@@ -948,10 +948,14 @@ def test_label_terms_of_a_small_vocabulary_at_the_edges_of_64_positions(U, V, st
 
 
 @pytest.mark.parametrize("T,U,V", [(1, 113, 31), (127, 113, 33), (128, 128, 127), (129, 129, 129),
-                                   (130, 160, 32), (257, 161, 600), (64, 225, 520)])
+                                   (130, 160, 32), (257, 161, 600), (64, 225, 520), (32, 129, 33),
+                                   (33, 160, 160), (63, 401, 40), (65, 161, 96), (160, 128, 31),
+                                   (161, 129, 65), (193, 130, 64), (400, 113, 40), (401, 129, 33),
+                                   (448, 113, 65), (449, 160, 31), (512, 128, 128)])
 def test_egrads_of_long_label_axes_at_the_edges_of_their_tiles(T, U, V):
-    """Tiles of 128 frames, 128 columns and slabs of 32 label positions, each one short, full and
-    one over; utterances that end inside, at the end of and a tile before the frame axis; labels
+    """Tiles of 64 frames (128 past 400 frames, with exp(P) prepared), 128 columns and slabs of 32 label
+    positions, each one short, full and one over; one, two and four blocks of 32 frames left for the
+    last tile; utterances that end inside, at the end of and a tile before the frame axis; labels
     that meet each other and the blank.  With the device's log-normaliser on both sides, at the
     tolerance of the other whole-loss tests."""
     rng = np.random.default_rng(T + U + V)

@@ -8,10 +8,13 @@
 // the matrix instruction's operand order (yt_planes_kernel, 6 bytes per element of the predictions,
 // in the memory that held the log-normaliser's Y pieces), a workgroup turns 128 frames x 32 label
 // positions of W at a time into pieces in LDS, and a wavefront owns 32 columns and all 128 frames, so
-// that E is read and egrads written once.
+// that E is read and egrads written once.  Where frames are few, the pieces are multiplied too few
+// times to be worth writing and reading: a wavefront then forms them from the predictions as it
+// goes, with tiles of 64 frames.
 // Bound by the matrix instructions with the W pieces' staging beside them (B=8 T=10000 U=401
 // V=1000: 384 GFLOP of bf16 products), then by E and egrads (0.64 GB).
 #include <algorithm>
+#include <type_traits>
 
 #include "rnnt_internal.h"
 #include "rnnt_io.h"
@@ -22,8 +25,9 @@ namespace rnnt {
 
 namespace {
 
-constexpr int kElRows = 128;  // frames of a tile
-constexpr int kElSlice = 32;  // label positions of a slab
+constexpr int kElRows = 128;       // frames of a tile
+constexpr int kElDirectRows = 64;  // ... where Y is not prepared
+constexpr int kElDirect = 400;     // frames up to which it is not (launch_egrads_long)
 constexpr int kElBlockPitch = 68;  // floats between columns of the block label terms add up in
 
 inline int el_vblocks(const Dims& d) { return (d.V + 31) / 32; }
@@ -59,16 +63,19 @@ __global__ __launch_bounds__(256) void yt_planes_kernel(const TIO* __restrict__ 
   dst[128] = f.l;
 }
 
-template <typename TIO>
+// kDirect: Y is formed here, from the predictions (Yt is not there).
+template <typename TIO, bool kDirect>
 __global__ __launch_bounds__(256, 2) void egrads_long_kernel(
-    const TIO* __restrict__ E, const uint4* __restrict__ Yt, const float* __restrict__ mE,
-    const float* __restrict__ Wn, const float* __restrict__ deltas, TIO* __restrict__ egrads,
-    const int* __restrict__ inLen, const int* __restrict__ labLen, Dims d, int Up, int Tw, int nvb,
-    int nus, int tile0, SparseTerms sp) {
+    const TIO* __restrict__ E, const TIO* __restrict__ P, const uint4* __restrict__ Yt,
+    const float* __restrict__ mE, const float* __restrict__ mP, const float* __restrict__ Wn,
+    const float* __restrict__ deltas, TIO* __restrict__ egrads, const int* __restrict__ inLen,
+    const int* __restrict__ labLen, Dims d, int Up, int Tw, int nvb, int nus, int tile0,
+    SparseTerms sp) {
   __shared__ __attribute__((aligned(16))) uint4 Xs[2][3][kElRows * 4];
   __shared__ float Ms[kElRows];                   // mE log2(e) of the tile's frames
   __shared__ unsigned short Match[4][kMaxLabels];  // per wavefront: labels among its columns
-  const int b = blockIdx.z, t0 = (tile0 + (int)blockIdx.y) * kElRows;
+  constexpr int kTile = kDirect ? kElDirectRows : kElRows, kM = kTile / 32;  // blocks of 32 frames
+  const int b = blockIdx.z, t0 = (tile0 + (int)blockIdx.y) * kTile;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, h = lane >> 5;
   int Tb, Ub;
   utt_extent(inLen, labLen, b, d.T, d.U, Tb, Ub);
@@ -76,7 +83,7 @@ __global__ __launch_bounds__(256, 2) void egrads_long_kernel(
   const bool vok = vcol < d.V;
   TIO* out = egrads + (size_t)b * d.T * d.V;
   if (t0 >= Tb) {  // frames past the utterance: exactly zero
-    for (int r = 0; r < kElRows / 2; ++r) {
+    for (int r = 0; r < kTile / 2; ++r) {
       const int t = t0 + 2 * r + h;
       if (t < d.T && vok) stf(out + (size_t)t * d.V + vcol, 0.0f);
     }
@@ -93,125 +100,162 @@ __global__ __launch_bounds__(256, 2) void egrads_long_kernel(
       nmatch += __popcll(m);
     }
   }
-  if (tid < kElRows) Ms[tid] = mE[(size_t)b * d.T + min(t0 + tid, Tb - 1)] * kLog2e;
+  if (tid < kTile) Ms[tid] = mE[(size_t)b * d.T + min(t0 + tid, Tb - 1)] * kLog2e;
 
   // staging: rows srow and srow + 64 of the tile, label positions 8 c8 .. 8 c8 + 7 of the slab
   const int srow = tid >> 2, c8 = tid & 3;
-  const float* pw[2];
-  int slot[2];
+  constexpr int kRowsEach = (kM + 1) / 2;
+  const float* pw[kRowsEach];
+  int slot[kRowsEach];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < kRowsEach; ++i) {
     const int row = srow + 64 * i;
     pw[i] = Wn + ((size_t)b * Tw + min(t0 + row, Tb - 1)) * Up;
     slot[i] = wslot(row, c8);
   }
-  struct WRegs { float4 lo[2], hi[2]; };
-  auto fetch = [&](int k) -> WRegs {  // (Up is a multiple of eight; Y is zero past the utterance)
-    const int u = min(32 * k + 8 * c8, Up - 8);
-    WRegs r;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      r.lo[i] = *reinterpret_cast<const float4*>(pw[i] + u);
-      r.hi[i] = *reinterpret_cast<const float4*>(pw[i] + u + 4);
-    }
-    return r;
-  };
-  auto stash = [&](int buf, const WRegs& r) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const float x[8] = {r.lo[i].x, r.lo[i].y, r.lo[i].z, r.lo[i].w,
-                          r.hi[i].x, r.hi[i].y, r.hi[i].z, r.hi[i].w};
-      const Frag3 f = split8(x);
-      Xs[buf][0][slot[i]] = f.h;
-      Xs[buf][1][slot[i]] = f.m;
-      Xs[buf][2][slot[i]] = f.l;
-    }
-  };
   const uint4* yw = Yt + ((size_t)b * nvb + min(vcol0 >> 5, nvb - 1)) * nus * 3 * 64 + lane;
-  auto fetch_y = [&](int ks) -> Frag3 {
-    const uint4* p = yw + (size_t)ks * 3 * 64;
-    Frag3 y;
-    y.h = p[0]; y.m = p[64]; y.l = p[128];
-    return y;
+  // what a step's fragment of Y is made from, and the fragment (zero past the utterance)
+  struct YRaw { float e[8], m[8]; };
+  const TIO* Pv = P + (size_t)b * d.U * d.V + min(vcol, d.V - 1);
+  const float* mPb = mP + (size_t)b * d.U;
+  auto request_y = [&](int ks) {
+    if constexpr (kDirect) {
+      YRaw r;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int u = min(16 * ks + 8 * h + i, Ub - 1);
+        r.e[i] = ldf(Pv + (size_t)u * d.V);
+        r.m[i] = mPb[u];
+      }
+      return r;
+    } else {
+      const uint4* p = yw + (size_t)ks * 3 * 64;
+      Frag3 y;
+      y.h = p[0]; y.m = p[64]; y.l = p[128];
+      return y;
+    }
   };
-  int aslot[2][4];
+  auto make_y = [&](const YRaw& r, int ks) -> Frag3 {
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] = 16 * ks + 8 * h + i < Ub ? __expf(r.e[i] - r.m[i]) : 0.0f;
+    return split8(y);
+  };
+  int aslot[2][kM];
 #pragma unroll
   for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int m = 0; m < 4; ++m) aslot[s][m] = wslot(32 * m + l32, 2 * s + h);
+    for (int m = 0; m < kM; ++m) aslot[s][m] = wslot(32 * m + l32, 2 * s + h);
 
   // The instruction truncates what falls below its accumulator's last bit; every two slabs (24
   // instructions, 64 label positions) the sums go into a second set, rounded, and start again.
-  floatx16 acc[4], tot[4];
+  floatx16 acc[kM], tot[kM];
 #pragma unroll
-  for (int m = 0; m < 4; ++m)
+  for (int m = 0; m < kM; ++m)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[m][r] = tot[m][r] = 0.0f;
   const int nk = (Ub + 31) >> 5;
-  Frag3 y0, y1;
-  // One slab, its order pinned as in the log-normaliser's: the second step's fragments are read under
-  // the first step's instructions, a step's Y fragments are asked for again right after their last use.
-  auto slab = [&](int kt, int cur) __attribute__((always_inline)) {
-    const int ktn = min(kt + 1, nk - 1);
-    const WRegs ws = fetch(ktn);
-    uint4 ah[4], am[4], al[4];
+  // The walk over the slabs with M blocks of 32 frames, one, two or four: what the utterance has left
+  // for this tile (a last tile or a short utterance is multiplied at its own size).
+  auto walk = [&](auto blocks) __attribute__((always_inline)) {
+    constexpr int M = decltype(blocks)::value, kRows = (M + 1) / 2;  // (rows a thread stages)
+    struct WRegs { float4 lo[kRows], hi[kRows]; };
+    auto fetch = [&](int k) -> WRegs {  // (Up is a multiple of eight; Y is zero past the utterance)
+      const int u = min(32 * k + 8 * c8, Up - 8);
+      WRegs r;
 #pragma unroll
-    for (int m = 0; m < 4; ++m) al[m] = Xs[cur][2][aslot[0][m]];
+      for (int i = 0; i < kRows; ++i) {
+        r.lo[i] = *reinterpret_cast<const float4*>(pw[i] + u);
+        r.hi[i] = *reinterpret_cast<const float4*>(pw[i] + u + 4);
+      }
+      return r;
+    };
+    auto stash = [&](int buf, const WRegs& r) __attribute__((always_inline)) {
 #pragma unroll
-    for (int m = 0; m < 4; ++m) ah[m] = Xs[cur][0][aslot[0][m]];
+      for (int i = 0; i < kRows; ++i) {
+        const float x[8] = {r.lo[i].x, r.lo[i].y, r.lo[i].z, r.lo[i].w,
+                            r.hi[i].x, r.hi[i].y, r.hi[i].z, r.hi[i].w};
+        const Frag3 f = split8(x);
+        Xs[buf][0][slot[i]] = f.h;
+        Xs[buf][1][slot[i]] = f.m;
+        Xs[buf][2][slot[i]] = f.l;
+      }
+    };
+    Frag3 y0, y1;
+    YRaw n0, n1;  // (kDirect: the next slab's)
+    // One slab, its order pinned as in the log-normaliser's: the second step's fragments are read under
+    // the first step's instructions, a step's Y fragments are asked for again right after their last use.
+    auto slab = [&](int kt, int cur) __attribute__((always_inline)) {
+      const int ktn = min(kt + 1, nk - 1);
+      const WRegs ws = fetch(ktn);
+      if constexpr (kDirect) {
+        y0 = make_y(n0, 2 * kt);
+        y1 = make_y(n1, 2 * kt + 1);
+        n0 = request_y(2 * ktn);
+        n1 = request_y(2 * ktn + 1);
+      }
+      uint4 ah[M], am[M], al[M];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) am[m] = Xs[cur][1][aslot[0][m]];
-    __builtin_amdgcn_sched_barrier(0);
+      for (int m = 0; m < M; ++m) al[m] = Xs[cur][2][aslot[0][m]];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(al[m], y0.h, acc[m]);
-    __builtin_amdgcn_sched_barrier(0);
+      for (int m = 0; m < M; ++m) ah[m] = Xs[cur][0][aslot[0][m]];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) al[m] = Xs[cur][2][aslot[1][m]];
+      for (int m = 0; m < M; ++m) am[m] = Xs[cur][1][aslot[0][m]];
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(ah[m], y0.l, acc[m]);
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(al[m], y0.h, acc[m]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(am[m], y0.m, acc[m]);
+      for (int m = 0; m < M; ++m) al[m] = Xs[cur][2][aslot[1][m]];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(am[m], y0.h, acc[m]);
-    __builtin_amdgcn_sched_barrier(0);
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(ah[m], y0.l, acc[m]);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) am[m] = Xs[cur][1][aslot[1][m]];
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(am[m], y0.m, acc[m]);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(ah[m], y0.m, acc[m]);
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(am[m], y0.h, acc[m]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(ah[m], y0.h, acc[m]);
-    __builtin_amdgcn_sched_barrier(0);
+      for (int m = 0; m < M; ++m) am[m] = Xs[cur][1][aslot[1][m]];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) ah[m] = Xs[cur][0][aslot[1][m]];
-    y0 = fetch_y(2 * ktn);
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(ah[m], y0.m, acc[m]);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(al[m], y1.h, acc[m]);
-    __builtin_amdgcn_sched_barrier(0);
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(ah[m], y0.h, acc[m]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(ah[m], y1.l, acc[m]);
+      for (int m = 0; m < M; ++m) ah[m] = Xs[cur][0][aslot[1][m]];
+      if constexpr (!kDirect) y0 = request_y(2 * ktn);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(am[m], y1.m, acc[m]);
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(al[m], y1.h, acc[m]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(am[m], y1.h, acc[m]);
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(ah[m], y1.l, acc[m]);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(ah[m], y1.m, acc[m]);
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(am[m], y1.m, acc[m]);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) acc[m] = mfma_bf16(ah[m], y1.h, acc[m]);
-    __builtin_amdgcn_sched_barrier(0);
-    y1 = fetch_y(2 * ktn + 1);
-    stash(cur ^ 1, ws);
-    __syncthreads();
-  };
-  auto flush = [&]() __attribute__((always_inline)) {
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(am[m], y1.h, acc[m]);
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(ah[m], y1.m, acc[m]);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) { tot[m][r] += acc[m][r]; acc[m][r] = 0.0f; }
-  };
-  if (nk > 0) {
+      for (int m = 0; m < M; ++m) acc[m] = mfma_bf16(ah[m], y1.h, acc[m]);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!kDirect) y1 = request_y(2 * ktn + 1);
+      stash(cur ^ 1, ws);
+      __syncthreads();
+    };
+    auto flush = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { tot[m][r] += acc[m][r]; acc[m][r] = 0.0f; }
+    };
     stash(0, fetch(0));
-    y0 = fetch_y(0);
-    y1 = fetch_y(1);
+    if constexpr (kDirect) {
+      n0 = request_y(0);
+      n1 = request_y(1);
+    } else {
+      y0 = request_y(0);
+      y1 = request_y(1);
+    }
     __syncthreads();
     int kt = 0;
     for (; kt + 2 <= nk; kt += 2) {
@@ -223,9 +267,11 @@ __global__ __launch_bounds__(256, 2) void egrads_long_kernel(
       slab(kt, 0);
       flush();
     }
-  } else {
-    __syncthreads();
-  }
+  };
+  if (nk == 0) __syncthreads();
+  else if (t0 + 32 >= Tb) walk(std::integral_constant<int, 1>{});
+  else if (kDirect || t0 + 64 >= Tb) walk(std::integral_constant<int, 2>{});
+  else walk(std::integral_constant<int, kM>{});
 
   // Write-out, 64 frames at a time: the tile's own scores are asked for, the label terms among this
   // wavefront's columns are added up in a block of LDS (a frame a lane, one label after the other, so
@@ -238,7 +284,8 @@ __global__ __launch_bounds__(256, 2) void egrads_long_kernel(
   const bool blank_here = terms && d.blank >= vcol0 && d.blank < vcol0 + 32;
   // (the last slab's barrier lies behind every read of the pieces)
 #pragma unroll
-  for (int p = 0; p < 2; ++p) {
+  for (int p = 0; p < kM / 2; ++p) {
+    if (t0 + 64 * p >= d.T) break;
     const int tl = t0 + 64 * p + lane;  // this lane's frame where lanes are frames
     float e[2][16];
 #pragma unroll
@@ -307,15 +354,24 @@ int egrads_long_any(const TIO* E, const TIO* P, const float* mE, const float* mP
     return fail(kInvalid, "egrads: blank/label terms can be folded in for at most %d labels",
                 kMaxLabels);
   const int nvb = el_vblocks(d), nus = el_steps(d);
-  const int ttiles = (d.T + kElRows - 1) / kElRows;
+  const bool direct = d.T <= kElDirect;
+  const int rows = direct ? kElDirectRows : kElRows, ttiles = (d.T + rows - 1) / rows, Up = wplane_up(d.U), Tw = wplane_tw(d.T);
+  const uint4* Yt = static_cast<const uint4*>(scratch);
+  if (direct) {
+    hipLaunchKernelGGL((egrads_long_kernel<TIO, true>), dim3((d.V + 127) / 128, ttiles, d.B), dim3(256), 0,
+                       s, E, P, Yt, mE, mP, Wn, deltas, egrads, inLen, labLen, d, Up, Tw, nvb, nus, 0,
+                       sparse);
+    RNNT_LAUNCH_CHECK("egrads_long_kernel");
+    return kOk;
+  }
   hipLaunchKernelGGL(yt_planes_kernel<TIO>, dim3(nvb, (nus + 3) / 4, d.B), dim3(256), 0, s, P, mP,
                      static_cast<uint4*>(scratch), labLen, d, nvb, nus);
   RNNT_LAUNCH_CHECK("yt_planes_kernel");
   for (int tile0 = 0; tile0 < ttiles; tile0 += 65535) {  // (what a grid's y holds)
-    hipLaunchKernelGGL(egrads_long_kernel<TIO>,
+    hipLaunchKernelGGL((egrads_long_kernel<TIO, false>),
                        dim3((d.V + 127) / 128, std::min(ttiles - tile0, 65535), d.B), dim3(256), 0, s,
-                       E, static_cast<const uint4*>(scratch), mE, Wn, deltas, egrads, inLen, labLen,
-                       d, wplane_up(d.U), wplane_tw(d.T), nvb, nus, tile0, sparse);
+                       E, P, Yt, mE, mP, Wn, deltas, egrads, inLen, labLen, d, Up, Tw, nvb, nus, tile0,
+                       sparse);
     RNNT_LAUNCH_CHECK("egrads_long_kernel");
   }
   return kOk;
@@ -327,6 +383,11 @@ int egrads_long_any(const TIO* E, const TIO* P, const float* mE, const float* mP
 // V=1000, four slices 942 -> 515; T=2000 U=129 V=1000, two 88 -> 63; B=32 T=1000 U=150 V=5000
 // 763 -> 569; B=1 T=1000 U=300 V=600 122 -> 37.  With one slice it is the streamed form, whose Y stays
 // in registers: B=32 T=2000 U=101 V=10000 1190 against 1890, V=1000 190 against 222.)
+// Y is prepared past 400 frames: with few frames the form that prepares it was slower than slices (B=64
+// V=2500, ragged, slices, prepared, not: T=20 U=401 150, 232, 80; T=130 U=201 151, 180, 114; T=256
+// U=201 220, 222, 177; T=400 U=401 627, 457, 401).  Time prepared over not, U=113 .. 700, V=100 .. 5000:
+// up to 400 frames 0.92 .. 3.05, all below 1.03 where both take about 30 us; 600 frames 0.85 .. 1.52;
+// from 1000 on mostly below 1 (2000: 0.75 .. 1.36, 10000: 0.66 .. 0.93).
 
 int launch_egrads_long(const float* E, const float* P, const float* mE, const float* mP,
                        const float* Wn, const float* deltas, float* egrads, const int* inLen,
