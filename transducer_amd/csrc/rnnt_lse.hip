@@ -246,9 +246,12 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
   // The first slabs' requests go out ahead of everything else: in a grid of about a workgroup per CU
   // the start, a chain of round trips to memory that nobody has touched lately, is half the time
   // (B=8 T=2000 U=101 V=100, four slabs: 43 us inside a training step, 18 called by itself).
-  XRegs xq[kAhead];
-  const XRegs x0 = fetch(0);
+  // (Tiles of 128 frames have neighbours to cover it and ask when the picks are sorted, so that these
+  // registers are not taken meanwhile: B=64 T=130 U=201 V=2500 201 -> 199, B=128 T=400 U=101 V=1001
+  // 147 -> 144.)
+  XRegs xq[kAhead], x0;
   if constexpr (kAhead > 1) {
+    x0 = fetch(0);
     xq[1] = fetch(min(1, nk - 1) * kSlice);
     xq[2 % kAhead] = fetch(min(2, nk - 1) * kSlice);
     xq[3 % kAhead] = fetch(min(3, nk - 1) * kSlice);
@@ -256,13 +259,11 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
   }
   struct YRegs { Frag3 s0, s1; };
   YRegs y0[kYAhead];
-  if (active) {
+  if (kYAhead > 1 && active) {
     y0[0].s0 = fetch_y(0);
     y0[0].s1 = fetch_y(1);
-    if constexpr (kYAhead > 1) {
-      y0[1].s0 = fetch_y(2 * min(1, nk - 1));
-      y0[1].s1 = fetch_y(2 * min(1, nk - 1) + 1);
-    }
+    y0[1 % kYAhead].s0 = fetch_y(2 * min(1, nk - 1));
+    y0[1 % kYAhead].s1 = fetch_y(2 * min(1, nk - 1) + 1);
   }
   for (int r = tid; r < 2 * kRows; r += kThreads) scale[r / kRows][r % kRows] = 1.0f;
   if (tid < 2) moved[tid] = 0;
@@ -528,7 +529,12 @@ __global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
   };
   __syncthreads();  // order
   next_pick();
+  if constexpr (kAhead == 1) x0 = fetch(0);
   stash(0, x0, true, 0);
+  if (kYAhead == 1 && active) {
+    y0[0].s0 = fetch_y(0);
+    y0[0].s1 = fetch_y(1);
+  }
   __syncthreads();
   // Two copies of the loop, so that a wavefront with nothing to multiply is a path of its own:
   // inside one loop the counted waits for the emission loads would have to hold on both paths,
