@@ -465,20 +465,27 @@ def test_arrays_past_two_to_the_31_elements_index_like_small_ones():
         assert torch.equal(alone[0, :n], paths[b, :n]), b
 
 
-def test_planes_of_more_than_4_gib_carry_the_reference_bits():
-    """An utterance so long that its lattice planes pass 2^32 bytes each (64 label positions are the
-    least a plane holds, so few label positions and many frames do): the walks move their buffers
-    four times on the way, and what lies past 4 GiB is walked like the rest."""
-    T, U, V = 16777300, 2, 2
+@pytest.mark.parametrize("T,U", [(16777300, 2), (1060000, 130), (530000, 300)])
+def test_planes_that_take_more_than_one_window_carry_the_reference_bits(T, U):
+    """The walks address an utterance's planes through windows of a GiB.  Two label positions (64 are the
+    least a plane holds) and 16.8 million frames: past 2^32 bytes a plane, five windows on one
+    wavefront; 130 positions: two windows, four wavefronts and blocks of two; 300: blocks side by side
+    in all three walks."""
+    V = 2
     rng = np.random.default_rng(T)
     E = rng.standard_normal((1, T, V), dtype=np.float32)
     P = rng.standard_normal((1, U, V), dtype=np.float32)
-    LN = np.logaddexp(E[:, :, None, 0] + P[:, None, :, 0], E[:, :, None, 1] + P[:, None, :, 1])
-    labels, il, ll = np.ones((1, 1), np.int32), np.array([T], np.int32), np.array([1], np.int32)
+    LN = np.empty((1, T, U), np.float32)
+    for t in range(0, T, 1 << 17):
+        s = E[:, t:t + (1 << 17), None] + P[:, None]
+        LN[:, t:t + (1 << 17)] = np.logaddexp(s[..., 0], s[..., 1])
+    labels = np.ones((1, U - 1), np.int32)
+    il, ll = np.array([T], np.int32), np.array([U - 1], np.int32)
     c = DeviceCase(E, P, labels, il, ll)
     costs, alphas = gpu_forward(c, LN)
     want_costs, want = oracle.forward(E, P, LN, labels, il, ll)
     assert np.array_equal(costs, want_costs) and np.array_equal(alphas, want)
+    del alphas
     assert np.array_equal(gpu_viterbi(c, LN), oracle.viterbi(E, P, LN, il, ll))
     got = gpu_backward(c, want, LN)
     for g, w in zip(got, oracle.backward(E, P, want, LN, labels, il, ll)):
