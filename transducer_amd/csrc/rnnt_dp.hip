@@ -699,6 +699,22 @@ __device__ inline void prog_store(int* p, int x) {
   __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// Waits for the neighbours of a wavefront that is about to run group g of n, and returns the group up
+// to which it need not look again.  `in`: groups handed on to it, `out`: how far the taker of its own has
+// got (both as far as known in have_in, have_out).  Asked ahead of every second group: groups g and
+// g + 1 take in the quads up to g + 2, each asking for the next group's, so g + 3 have to be there;
+// two more are waited for, so that the next look finds what it needs.  They write the quads up to g,
+// over those up to g - kRingGroups, and a taker that tells x has read every quad below x: up to
+// x + kRingGroups nothing unread is lost, and four less is allowed.  A walk that had to wait goes on
+// fourteen groups ahead of that line.
+__device__ __forceinline__ int hand_over_until(const int* in, const int* out, int& have_in,
+                                               int& have_out, int g, int n, int spin_limit,
+                                               int* __restrict__ trouble) {
+  have_in = bounded_wait(in, have_in, min(g + 5, n), spin_limit, trouble);
+  have_out = bounded_wait(out, have_out, g + 18 - kRingGroups, spin_limit, trouble);
+  return min(have_in >= n ? kForever : have_in - 3, min(have_out, kForever) + kRingGroups - 4);
+}
+
 // The wavefront beside the walking ones of a block that runs side by side with others: brings what
 // the block before it has left in memory (`src`) into the ring of the first walking wavefront, and
 // takes what the last one hands on out to `dst`, up to 64 quads in a turn.  It keeps the
@@ -971,12 +987,9 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
   // ---- hand-over
   int ok = kHand ? -1 : kForever;  // groups up to here may run without looking at the neighbours
   int have_in = 0, have_out = 0;
-  // before groups g and g + 1, which ask for the quads up to g + 2 and write those up to g + 1
   auto refresh = [&](int g) {
-    have_in = bounded_wait(&prog[wave], have_in, min(g + 5, ngroups), spin_limit, trouble);
-    have_out = bounded_wait(&prog[wave + 2], have_out, g + 18 - kRingGroups, spin_limit, trouble);
-    ok = min(have_in >= ngroups ? kForever : have_in - 3,
-             min(have_out, kForever) + kRingGroups - 4);
+    ok = hand_over_until(&prog[wave], &prog[wave + 2], have_in, have_out, g, ngroups, spin_limit,
+                         trouble);
   };
   const float* take = kHand ? (first_column ? nothing : ring[wave]) : nullptr;
   const int take_mask = first_column ? 0 : kRingGroups / 4 - 1;
@@ -1232,15 +1245,11 @@ __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __res
   }
   const int nsteps = Tb + Ub - 1;
   const int last = nsteps - 1;  // diagonal of the last cell
-  // kSpread: a lane's C positions are 64 apart (u0 + 64 c), so that the 64 lanes of a load or
-  // store touch neighbouring 16-byte pieces of the plane, whole cache lines together; the price
-  // is a lane-to-scalar move per position and step (lane 63's right neighbour is lane 0's next
-  // position).  With two positions a lane next to each other (u0 + c) a load still fills half
-  // of every line it touches, and the walk of up to 128 label positions is faster that way
-  // (B=32 T=2000 U=100: 38.6 against 45.4 ns a step; two wavefronts of one position: 52.5).
-  constexpr bool kSpread = W > 1 || C > 2;
-  constexpr int kApart = kSpread ? 64 : 1;
-  const int u0 = u_base + wave * 64 * C + (kSpread ? lane : lane * C);
+  // A lane's C positions are 64 apart (u0 + 64 c), so that the 64 lanes of a load or store touch
+  // neighbouring 16-byte pieces of the plane, whole cache lines together; the price is a
+  // lane-to-scalar move per position and step (lane 63's right neighbour is lane 0's next position).
+  constexpr int kApart = 64;
+  const int u0 = u_base + wave * 64 * C + lane;
   const int gstride = plane_group_stride(d);
   float* hand_out = hand + (wave > 0 ? wave - 1 : 0) * hand_stride;  // wave > 0
   const float* hand_in = hand + wave * hand_stride;                  // wave < W-1
@@ -1324,17 +1333,12 @@ __global__ __launch_bounds__(64 * W) void beta_kernel(Planes p, const int* __res
         float above = 0.0f;  // right of the wavefront's last position
         if constexpr (kMulti) above = gin ? w.gh[j] : 0.0f;
         if (W > 1) above = wave < W - 1 ? hh[j] : 0.0f;
-        if constexpr (kSpread) {
 #pragma unroll
-          for (int c = 0; c < C; ++c) {
-            const float past =  // what lane 63 receives
-                c < C - 1 ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dcol[c + 1]), 0))
-                          : above;
-            right[c] = wave_shl1(dcol[c], past);
-          }
-        } else {
-#pragma unroll
-          for (int c = 0; c < C; ++c) right[c] = c < C - 1 ? dcol[c + 1] : wave_shl1(dcol[0], above);
+        for (int c = 0; c < C; ++c) {
+          const float past =  // what lane 63 receives
+              c < C - 1 ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dcol[c + 1]), 0))
+                        : above;
+          right[c] = wave_shl1(dcol[c], past);
         }
 #pragma unroll
         for (int c = 0; c < C; ++c) {
@@ -1532,7 +1536,7 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void beta_walk_kernel(
   // ---- hand-over (see alpha_walk_kernel)
   int ok = kHand ? -1 : kForever;
   int have_in = 0, have_out = 0;
-  auto refresh = [&](int i) {
+  auto refresh = [&](int i) {  // hand_over_until written out: called, the walk is scheduled 1.5 % worse
     have_in = bounded_wait(&prog[order], have_in, min(i + 5, n), spin_limit, trouble);
     have_out = bounded_wait(&prog[order + 2], have_out, i + 18 - kRingGroups, spin_limit, trouble);
     ok = min(have_in >= n ? kForever : have_in - 3, min(have_out, kForever) + kRingGroups - 4);
@@ -2891,10 +2895,8 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void viterbi_walk_kerne
     int ok = kHand ? -1 : kForever;
     int have_in = 0, have_out = 0;
     auto refresh = [&](int g) {
-      have_in = bounded_wait(&prog[wave], have_in, min(g + 5, ngroups), spin_limit, trouble);
-      have_out = bounded_wait(&prog[wave + 2], have_out, g + 18 - kRingGroups, spin_limit, trouble);
-      ok = min(have_in >= ngroups ? kForever : have_in - 3,
-               min(have_out, kForever) + kRingGroups - 4);
+      ok = hand_over_until(&prog[wave], &prog[wave + 2], have_in, have_out, g, ngroups, spin_limit,
+                           trouble);
     };
     const float* take = kHand ? (first_column ? nothing : ring[wave]) : nullptr;
     const int take_mask = first_column ? 0 : kRingGroups / 4 - 1;
@@ -3053,7 +3055,7 @@ __global__ __launch_bounds__(64) void viterbi_trace_kernel(const float* __restri
 //   kind 0: a cell of alpha_walk_kernel -- DPP hand-over, log-sum-exp on the hardware units with
 //           the check that its sum is the C library's (alpha_cell; the operands are large, so no lane
 //           falls back), the additions of its two moves;
-//   kind 1: a cell of beta_kernel -- DPP hand-over, two multiplies and an add;
+//   kind 1: a cell of the dalpha walk -- DPP hand-over, two multiplies and an add;
 //   kind 2: kind 0 with every lane on the library path (rnnt_libm.h: ~100 instructions, two of
 //           them divisions): what a step costs while any lane of the wavefront falls back.
 // The walks cannot run faster than steps x this; the ratio is what the prefetch, the stores and
@@ -3419,8 +3421,8 @@ int launch_beta(const Planes& p, const int* labels, const int* inLen, const int*
                 const Dims& d, hipStream_t s) {
   if (d.B == 0 || d.T == 0 || d.U == 0) return kOk;
   const int cpl = block_cells_per_lane(d), nblocks = label_blocks(d);
-  // several positions a lane: four wavefronts (two if only their hand-over array fits LDS), one per
-  // block when the axis takes several launches
+  // several positions a lane (2 or, from 513 positions on, 4): four wavefronts; there two or one if
+  // only that many hand-over arrays fit LDS; one per block when the axis takes several launches
   const int stride = d.Dp;
   const bool single_block = nblocks == 1;
   const int W = !single_block ? 1
@@ -3469,8 +3471,7 @@ int launch_beta(const Planes& p, const int* labels, const int* inLen, const int*
                        inLen, labLen, d, stride, u_base, ghin, ghout, g_spin_limit,        \
                        trouble);                                                            \
     break;
-      CASE(8, 1, false) CASE(16, 1, false) CASE(4, 2, false) CASE(8, 2, false)
-      CASE(2, 4, false) CASE(4, 4, false)
+      CASE(2, 4, false) CASE(4, 4, false) CASE(8, 2, false) CASE(16, 1, false)
       CASE(16, 1, true)
 #undef CASE
       default:
