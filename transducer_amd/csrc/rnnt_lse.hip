@@ -141,22 +141,23 @@ __global__ __launch_bounds__(256) void yplanes_kernel(const TIO* __restrict__ P,
 }
 
 // ------------------------------------------------------------------ contraction
-// kRows frames x 128 label positions per workgroup: each of its four wavefronts owns one block of
-// 32 label positions and all kRows frames (four accumulators at 128 frames, two at 64).  64 frames
-// for grids that 128 would leave below one workgroup per CU (each workgroup walks all columns, so a
-// small grid is a long walk on a few CUs: B=32 T=400 U=101 V=4096 0.25 -> 0.18 ms, B=8 T=2000 U=101
-// V=2000 0.147 -> 0.096).
+// kRows frames x 128 label positions per workgroup.  kWaves = 4: a wavefront owns one block of
+// 32 label positions and all kRows frames (four accumulators at 128 frames, two at 64).
+// kWaves = 8: two wavefronts share a block, half the frames each (half the registers, twice the
+// wavefronts to hide each other's staging).  64 frames for grids that 128 would leave below one
+// workgroup per CU (each workgroup walks all columns, so a small grid is a long walk on a few
+// CUs: B=32 T=400 U=101 V=4096 0.25 -> 0.18 ms, B=8 T=2000 U=101 V=2000 0.147 -> 0.096).
 // kVec: rows start 16-byte aligned and hold a multiple of the vector width, so a thread's eight
 // values are one or two 16-byte loads; otherwise they are fetched one by one.
-constexpr int kThreads = 256;
-template <typename TIO, bool kVec, int kRows>
-__global__ __launch_bounds__(kThreads, 2) void lse_stream_kernel(
+template <int kWaves, typename TIO, bool kVec, int kRows>
+__global__ __launch_bounds__(64 * kWaves, kWaves / 2) void lse_stream_kernel(
     const TIO* __restrict__ E, float* __restrict__ mE, const float* __restrict__ mP,
     const uint4* __restrict__ Yp, float* __restrict__ LN, const int* __restrict__ inLen,
     const int* __restrict__ labLen, Dims d, int ttiles, int utiles, int total, int nub, int nks,
     const int* __restrict__ labels, float* __restrict__ elS, float* __restrict__ ebv,
     float* __restrict__ lnS) {
-  constexpr int MB = kRows / 32;            // 32-frame blocks per wavefront
+  constexpr int kThreads = 64 * kWaves;
+  constexpr int MB = kRows / 8 / kWaves;   // 32-frame blocks per wavefront
   constexpr int NR = 4 * kRows / kThreads;  // (row, eight v) items a thread stages per slab
   constexpr int kSlots = kRows * 4;        // 16-byte slots per piece plane: 4 per row
   static_assert(MB >= 1 && NR >= 1, "a tile gives every wavefront a frame block and every thread a row");
@@ -227,8 +228,10 @@ __global__ __launch_bounds__(kThreads, 2) void lse_stream_kernel(
       r.x[i] = kVec ? load8(px[i], k0 + 8 * c8, d.V) : load8_any(px[i], k0 + 8 * c8, d.V);
     return r;
   };
-  // this wavefront's block of 32 label positions; one past the utterance only helps staging
-  const int ublock = (u0 >> 5) + wave;
+  // this wavefront's block of 32 label positions and first frame block; a label block past the
+  // utterance only helps staging
+  const int ublock = (u0 >> 5) + (wave & 3);
+  const int mb0 = (wave >> 2) * MB;
   const bool active = 32 * ublock < Ub;
   const uint4* yw = Yp + ((size_t)b * nub + (active ? ublock : 0)) * nks * 3 * 64 + lane;
   // Y fragments of step `ks` (16 v): three coalesced 16-byte loads
@@ -429,12 +432,12 @@ __global__ __launch_bounds__(kThreads, 2) void lse_stream_kernel(
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[m][r] = tot[m][r] = 0.0f;
 
-  // fragment slots of this lane: row 32 m + l32, v-eights 2*s + h
+  // fragment slots of this lane: row 32*(mb0 + m) + l32, v-eights 2*s + h
   int aslot[2][MB];
 #pragma unroll
   for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int m = 0; m < MB; ++m) aslot[s][m] = xslot(32 * m + l32, 2 * s + h);
+    for (int m = 0; m < MB; ++m) aslot[s][m] = xslot(32 * (mb0 + m) + l32, 2 * s + h);
 
   int cur = 0;
   // One slab: request the next slab's emissions, multiply the current one, stage the next.
@@ -468,7 +471,7 @@ __global__ __launch_bounds__(kThreads, 2) void lse_stream_kernel(
         for (int m = 0; m < MB; ++m)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const float f = scale[cur][32 * m + mfma_row(r, h)];
+            const float f = scale[cur][32 * (mb0 + m) + mfma_row(r, h)];
             acc[m][r] *= f;
             tot[m][r] *= f;
           }
@@ -582,7 +585,7 @@ __global__ __launch_bounds__(kThreads, 2) void lse_stream_kernel(
     // label positions past the utterance (but inside U) are written as zeros
     if (u < d.U && lnS == nullptr)
       for (int r = 0; r < 16 * MB; ++r) {
-        const int t = t0 + 32 * (r >> 4) + mfma_row(r & 15, h);
+        const int t = t0 + 32 * (mb0 + (r >> 4)) + mfma_row(r & 15, h);
         if (t < d.T) LNb[(size_t)t * d.U + u] = 0.0f;
       }
     return;
@@ -592,7 +595,7 @@ __global__ __launch_bounds__(kThreads, 2) void lse_stream_kernel(
   for (int m = 0; m < MB; ++m)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int row = 32 * m + mfma_row(r, h), t = t0 + row;
+      const int row = 32 * (mb0 + m) + mfma_row(r, h), t = t0 + row;
       if (t < d.T && u < d.U) {
         float v = 0.0f;
         if (t < Tb && u < Ub)
@@ -658,11 +661,12 @@ static int lse_stream_any(const TIO* E, float* mE, const float* mP, float* LN,
   const int ttiles = (d.T + rows - 1) / rows;
   const long total = (long)ttiles * utiles * d.B;
   const int grid = (int)((total + 7) / 8 * 8);
+  constexpr int kWaves = 4;
   constexpr int kA = RowAlign<TIO>::kElems;
   const bool vec = d.V % kA == 0 && d.V >= kA && (reinterpret_cast<uintptr_t>(E) & 15) == 0;
 #define RNNT_LSE_LAUNCH(VEC, ROWS)                                                            \
-  hipLaunchKernelGGL((lse_stream_kernel<TIO, VEC, ROWS>), dim3(grid),                 \
-                     dim3(kThreads), 0, s, E, mE, mP, static_cast<const uint4*>(scratch),  \
+  hipLaunchKernelGGL((lse_stream_kernel<kWaves, TIO, VEC, ROWS>), dim3(grid),                 \
+                     dim3(64 * kWaves), 0, s, E, mE, mP, static_cast<const uint4*>(scratch),  \
                      LN, inLen, labLen, d, ttiles, utiles, (int)total, nub, nks, labels, elS, \
                      eb, lnS)
   if (vec && low) RNNT_LSE_LAUNCH(true, 64);
