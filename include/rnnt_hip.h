@@ -121,13 +121,11 @@ int rnnt_hip_loss_backward(const float* emissions, const float* predictions, con
  * for a caller whose projection layers emit 16-bit logits, and they halve the traffic of the two
  * [B,T,V] arrays.  A score converts to fp32 exactly and all arithmetic is the fp32 path's; each
  * gradient element is the fp32 result (dense + blank/label terms, times deltas[b]) rounded once
- * to nearest-even (an fp16 gradient past 65504 becomes infinity).  A label axis of more than
- * 112 positions is contracted in slices that add up in fp32 (in the workspace, a window of frames
- * at a time) before the one rounding; the loss takes at most 1025 label positions (U <= 1025) in
- * these types and refuses more with an error.  Any V; 16-byte loads are
- * used when V is a multiple of 8 and the arrays are 16-byte aligned.  Workspace as for the fp32
- * calls.  The best path of
- * rnnt_hip_viterbi_decode_* is the one rnnt_hip_viterbi_decode finds on the same values. */
+ * to nearest-even (an fp16 gradient past 65504 becomes infinity), however long the label axis; the
+ * loss takes at most 1025 label positions (U <= 1025) in these types and refuses more with an
+ * error.  Any V; 16-byte loads are used when V is a multiple of 8 and the arrays are 16-byte
+ * aligned.  Workspace as for the fp32 calls.  The best path of rnnt_hip_viterbi_decode_* is the one
+ * rnnt_hip_viterbi_decode finds on the same values. */
 int rnnt_hip_loss_forward_bf16(const uint16_t* emissions, const uint16_t* predictions,
                                const int* labels, const int* input_lengths,
                                const int* label_lengths, float* costs, void* workspace,
@@ -214,10 +212,10 @@ int rnnt_hip_profile_read(double* total_ms, int* launches, int n);
 
 /* ---- diagnostics of the lattice walks (no counterpart in the reference) ------------------ */
 
-/* The lattice walks deal a long label axis to several wavefronts of a workgroup (from 257
- * label positions in a small batch the alpha and dalpha walks also to several workgroups); each
- * waits, with a trip bound, for what its neighbour hands over.  Should the bound ever run out
- * the kernel still finishes, with invalid results, and raises a flag on its device.  This call waits for `stream`, reads the current device's flag and clears it:
+/* The lattice walks deal a long label axis to several wavefronts of a workgroup (a longer one also
+ * to several workgroups); each waits, with a trip bound, for what its neighbour hands over.  Should
+ * the bound ever run out the kernel still finishes, with invalid results, and raises a flag on its
+ * device.  This call waits for `stream`, reads the current device's flag and clears it:
  * RNNT_OK if no kernel gave up since the last check, else RNNT_HIP_FAILURE with a message.
  * (The reference's kernels synchronise with __syncthreads and cannot hang this way,
  * transducer/transducer_cuda.cu:65-90.) */

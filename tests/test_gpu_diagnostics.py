@@ -20,9 +20,9 @@ KEYS = ("emissions", "predictions", "labels", "input_lengths", "label_lengths")
 
 @pytest.mark.parametrize("U", [100, 400])
 def test_a_wait_that_runs_out_raises_the_flag_and_the_kernel_still_finishes(U):
-    """101 label positions: two wavefronts of one workgroup wait for each other; 401: the alpha
-    walk also runs the two halves of the label axis as two workgroups side by side, the upper
-    one waiting (with the same bound) for the scores the lower one writes to memory."""
+    """101 label positions: two wavefronts of one workgroup wait for each other; 401: the walks also run
+    blocks of the label axis as workgroups side by side, one waiting (with the same bound) for
+    what its neighbour writes to memory."""
     lib = capi.load()
     d = make_inputs(small_config(2, 300, U, 16, ragged=False), seed=9)
     E, P, labels, il, ll = (d[k] for k in KEYS)
@@ -34,7 +34,7 @@ def test_a_wait_that_runs_out_raises_the_flag_and_the_kernel_still_finishes(U):
     try:
         _, alphas = gpu_forward(c, LN)          # returns: the walk finishes on whatever it finds
         gpu_viterbi(c, LN)
-        if U > 256:                             # the dalpha walk of two halves waits the same way
+        if U > 256:                             # the dalpha walk of several blocks waits the same way
             assert lib.rnnt_hip_check_kernels(None) == 2
             gpu_backward(c, np.nan_to_num(alphas, posinf=0.0, neginf=0.0), LN)
         assert lib.rnnt_hip_check_kernels(None) == 2

@@ -124,8 +124,9 @@ struct Planes {
   float* pl;    // P[u, label_u]         [B, Ua]
   float* gB;    // per-(b,u) blank-column sum of the sparse pgrads term   [B, Ua]
   float* gL;    // per-(b,u) label-column sum of the sparse pgrads term   [B, Ua]
-  float* hand[2];  // [B, Dp] each: what crosses from one block of 1024 label positions to the
-                   // next when a lattice walk takes the label axis block by block
+  float* hand[2];  // what crosses from one block of label positions to the next: [B, Dp] each when a
+                   // walk takes the axis a launch per 1024 positions; both together [B, Dp] tagged
+                   // entries of 8 bytes a boundary when it takes blocks side by side
 };
 
 // Trips a wavefront of the lattice kernels may spend waiting for its neighbour's progress

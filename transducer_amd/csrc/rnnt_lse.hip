@@ -143,8 +143,9 @@ __global__ __launch_bounds__(256) void yplanes_kernel(const TIO* __restrict__ P,
 // ------------------------------------------------------------------ contraction
 // kRows frames x 128 label positions per workgroup.  kWaves = 4: a wavefront owns one block of
 // 32 label positions and all kRows frames (four accumulators at 128 frames, two at 64).
-// kWaves = 8: two wavefronts share a block, half the frames each (half the registers, twice the
-// wavefronts to hide each other's staging).  64 frames for grids that 128 would leave below one
+// (kWaves = 8, two wavefronts to a block with half the frames each, is launched nowhere.  With the
+// count written out of the code the 64-frame tiles of odd 16-bit rows are scheduled worse, B=32 T=400
+// U=102 V=4097 fp16 150.5 -> 154 us, for 1 % on tiles of 128.)  64 frames for grids that 128 would leave below one
 // workgroup per CU (each workgroup walks all columns, so a small grid is a long walk on a few
 // CUs: B=32 T=400 U=101 V=4096 0.25 -> 0.18 ms, B=8 T=2000 U=101 V=2000 0.147 -> 0.096).
 // kVec: rows start 16-byte aligned and hold a multiple of the vector width, so a thread's eight
