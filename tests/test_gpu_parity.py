@@ -381,8 +381,7 @@ def test_label_axis_as_a_chain_of_blocks_side_by_side_and_where_it_is_not(B, T, 
     whatever the batch (40 x 5 workgroups, 300 x 5: more than the device runs at once, so later
     utterances' blocks queue behind earlier ones).  Batches past that room take one workgroup per
     utterance, a lane owning four positions: here the best path of 70 x 600, 49 x 1000 and all
-    larger ones, alpha of 171 x 700, 201 x 1000 and 301 x 700, dalpha of 101 x 1000, 201 x 1000 and
-    301 x 700.  17 blocks are too many: a launch per 1024 positions.  Either way the reference's bits.  U
+    larger ones, alpha of 201 x 1000 and 301 x 700, dalpha of 101 x 1000, 201 x 1000 and 301 x 700.  17 blocks are too many: a launch per 1024 positions.  Either way the reference's bits.  U
     counts the rows of predictions; ragged batches, so that some utterances end blocks below the top
     one."""
     cfg = small_config(B, T, U - 1, 4, ragged=True)

@@ -27,12 +27,10 @@ inline int label_blocks(const Dims& d) {
 }
 
 // Blocks of 256 label positions that the alpha walk runs side by side (1: none).
-//   two      256 workgroups (1.29 .. 2.10); up to 512 from 2000 frames on (0.97 .. 1.22, below that
-//            0.72 .. 1.09)
-//   three    512 workgroups (1.13 .. 2.93); between 171 and 256 utterances from 500 frames on (1.00 ..
-//            1.38, below 0.82 .. 1.13); past 256 utterances, where one workgroup an utterance takes some
-//            CUs twice, again, up to 900 workgroups (1.26 .. 1.62)
-//   four     800 workgroups (0.98 .. 1.93); up to 900 from 2000 frames on (1.01, below 0.78 .. 0.96)
+//   two      256 workgroups (1.30 .. 2.10); up to 512 from 1000 frames on (1.04 .. 1.16, below that
+//            0.77 .. 1.35, on 257 positions 0.77 .. 0.99)
+//   three    900 workgroups (0.99 .. 3.42)
+//   four     800 workgroups (1.11 .. 3.16); up to 900 from 1000 frames on (1.04, below 0.88 .. 1.31)
 // Past 1024 positions the other way is a launch per 1024, many times slower whatever the batch;
 // workgroups beyond the device's CUs queue in order.
 inline int alpha_blocks(const Dims& d) {
@@ -40,8 +38,8 @@ inline int alpha_blocks(const Dims& d) {
   if (n < 2 || n > 16) return 1;
   if (d.U > 1024) return n;
   const long workgroups = (long)d.B * n;
-  const bool alone = workgroups <= (n == 2 ? 256 : n == 3 ? 512 : 800) || (n == 3 && d.B > 256);
-  return (alone || d.T >= (n == 3 ? 500 : 2000)) && workgroups <= (n == 2 ? 512 : 900) ? n : 1;
+  const int alone = n == 2 ? 256 : n == 3 ? 900 : 800, at_length = n == 2 ? 512 : 900;
+  return workgroups <= (d.T >= 1000 ? at_length : alone) ? n : 1;
 }
 
 // Blocks that the dalpha walk runs side by side, and the wavefronts (64 positions each) of a block.

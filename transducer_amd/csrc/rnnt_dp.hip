@@ -719,31 +719,33 @@ __device__ __forceinline__ int hand_over_until(const int* in, const int* out, in
 // the block before it has left in memory (`src`) into the ring of the first walking wavefront, and
 // takes what the last one hands on out to `dst`, up to 64 quads in a turn.  It keeps the
 // tagged entries, their waits and their addresses out of the walk.  at(g, i): the step of value
-// i = 0..3 of group g (four steps in a row).  Groups are numbered in walking order, n of them on either side; group g's quad
-// lies in slot g + kShift of a ring.  Bounded
-// like every wait here: when nothing has moved for spin_limit turns it raises the trouble flag and
-// lets everybody go on with whatever the rings hold.
+// i = 0..3 of group g (four steps in a row).  Groups are numbered in walking order; quads [in, n_in) are
+// brought, [out, n_out) taken; group g's lies in slot g + kShift of a ring.  Bounded like every wait
+// here: when nothing has moved for spin_limit turns it raises the trouble flag and lets everybody go
+// on with whatever the rings hold.
 template <int kShift, typename At>
 __device__ inline void live_carrier(const unsigned long long* __restrict__ src,
-                                    unsigned long long* __restrict__ dst, int n, At at,
-                                    float* ring_in, int* prog_in, const int* prog_first,
+                                    unsigned long long* __restrict__ dst, int in, int n_in, int out,
+                                    int n_out, At at, float* ring_in, int* prog_in, const int* prog_first,
                                     const float* ring_out, const int* prog_last, int* prog_out,
                                     int spin_limit, int* __restrict__ trouble) {
   const int lane = threadIdx.x & 63, quad = lane >> 2, value = lane & 3;
-  int in = src ? 0 : n, out = dst ? 0 : n, idle = 0;
-  while (in < n || out < n) {
+  int idle = 0;
+  in = src ? in : n_in;
+  out = dst ? out : n_out;
+  while (in < n_in || out < n_out) {
     bool moved = false;
     unsigned long long e[4];
-    const int room = in < n ? min(prog_load(prog_first) + kRingGroups - 4, n) - in : 0;
+    const int room = in < n_in ? min(prog_load(prog_first) + kRingGroups - 4, n_in) - in : 0;
     asm volatile("" ::: "memory");
     if (room > 0) {  // (asked for ahead of the other side's work: the answer takes a microsecond)
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        e[k] = __hip_atomic_load(src + at(min(in + 16 * k + quad, n - 1), value), __ATOMIC_RELAXED,
+        e[k] = __hip_atomic_load(src + at(min(in + 16 * k + quad, n_in - 1), value), __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (out < n) {
-      const int m = min(min(prog_load(prog_last), n) - out, 64);
+    if (out < n_out) {
+      const int m = min(min(prog_load(prog_last), n_out) - out, 64);
       asm volatile("" ::: "memory");
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
@@ -775,7 +777,7 @@ __device__ inline void live_carrier(const unsigned long long* __restrict__ src,
       if (ready > 0) {
         in += ready;
         asm volatile("" ::: "memory");  // (LDS serves a wavefront's requests in order)
-        if (lane == 0) prog_store(prog_in, in);
+        if (lane == 0) prog_store(prog_in, in < n_in ? in : kForever);
         moved = true;
       }
     }
@@ -877,6 +879,10 @@ struct Buffer {
 // at 101 (93 and 111 with 29 instructions, the comparison right ahead of its branch, whole
 // hand-over arrays in LDS whose writes the next group waited for); B=8 T=10000, 401
 // positions 84 (128 with the entries between blocks asked for and checked inside the walk).
+// A wavefront runs the groups from its first position's first cell to its last one's last.  While all of
+// them ran all groups, most instructions of a lattice with more label positions than frames were for
+// cells outside, and two workgroups on a CU, short of issue slots, were slower than the walk before
+// this one: B=64 T=100, 1025 positions 317 us then, 371 with all groups, 239 so; B=4 238 and 206.
 template <int W, bool kLive>
 __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
     Planes p, const int* __restrict__ inLen, const int* __restrict__ labLen,
@@ -904,18 +910,21 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
     return;
   }
   if (u_base >= Ub) return;  // a block past this utterance's labels: nobody reads what it would leave
-  const int nsteps = Tb + Ub - 1;
-  const int ngroups = (nsteps + 3) >> 2;
+  // groups a wavefront of positions u .. u + 63 runs
+  auto begin_of = [](int u) { return u >> 2; };
+  auto end_of = [&](int u) { return ((Tb - 1 + min(u + 63, Ub - 1)) >> 2) + 1; };
   // a block below and a block above this one (for this utterance)
   const bool live_in = kLive && live_block > 0;
   const bool live_out = kLive && live_block < live_n - 1 && u_base + 64 * W < Ub;
   exp2_table_to_lds(etab);
   if (threadIdx.x < 16) nothing[threadIdx.x] = kNegInf;
   if (threadIdx.x < W + 2) {
+    // (counted from where each of them starts; a wavefront also needs the quad ahead of its first
+    // group, whose last value enters its first step)
     const int w = (int)threadIdx.x - 1;  // the wavefront whose progress this is
-    prog[threadIdx.x] = w < 0 ? (live_in ? 0 : kForever)
-                        : w == W ? (live_out ? 0 : kForever)
-                                 : (u_base + 64 * w < Ub ? 0 : kForever);
+    prog[threadIdx.x] = w < 0 ? (live_in ? begin_of(u_base) - 1 : kForever)
+                        : w == W ? (live_out ? begin_of(u_base + 64 * W) - 1 : kForever)
+                                 : (u_base + 64 * w < Ub ? begin_of(u_base + 64 * w) : kForever);
   }
   __syncthreads();
   if (kLive && wave == W) {
@@ -923,8 +932,9 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
         live_in ? live + ((size_t)(live_block - 1) * d.B + b) * d.Dp : nullptr;
     unsigned long long* dst = live_out ? live + ((size_t)live_block * d.B + b) * d.Dp : nullptr;
     // what enters step s: value i of group g is what enters step 4g + 1 + i (nothing enters step 0)
-    live_carrier<0>(src, dst, ngroups, [](int g, int i) { return 4 * g + 1 + i; }, ring[0], &prog[0],
-                 &prog[1], ring[W], &prog[W], &prog[W + 1], spin_limit, trouble);
+    live_carrier<0>(src, dst, begin_of(u_base) - 1, end_of(u_base - 64), begin_of(u_base + 64 * W) - 1,
+                    end_of(u_base + 64 * (W - 1)), [](int g, int i) { return 4 * g + 1 + i; }, ring[0],
+                    &prog[0], &prog[1], ring[W], &prog[W], &prog[W + 1], spin_limit, trouble);
     return;
   }
   const int u_lo = u_base + wave * 64;
@@ -948,8 +958,9 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
   // Interior groups [in_lo, in_hi): step 4g is past the first frame of the wavefront's last
   // position, step 4g + 3 not past the last frame of its first one.
   const unsigned gbytes = kLive ? 16u * (unsigned)d.Ua : 1024u * W;  // from a group to the next
+  const int g_begin = begin_of(u_lo), g_end = end_of(u_lo);
   const int in_lo = (min(u_lo + 64, Ub) + 2) >> 2;
-  const int in_hi = Ub > 1 ? min((Tb + u_lo) >> 2, ngroups - 1) : 0;
+  const int in_hi = Ub > 1 ? min((Tb + u_lo) >> 2, g_end - 1) : 0;
   // The planes as buffers that begin at group `origin` of the utterance (moved on before an offset
   // would outgrow 32 bits).  E[t,blank] of step s, lane by lane, sits at eb[Eo + s - u].
   const size_t plane = (size_t)gbytes * (unsigned)(d.Dp / 4);
@@ -982,14 +993,13 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
     r.eb = eb_q.load(eb_o, 16u * (unsigned)g);
     return r;
   };
-  auto load_to_end = [&](int g) -> Ops { return load(min(g, ngroups - 1)); };
+  auto load_to_end = [&](int g) -> Ops { return load(min(g, g_end - 1)); };
 
   // ---- hand-over
   int ok = kHand ? -1 : kForever;  // groups up to here may run without looking at the neighbours
   int have_in = 0, have_out = 0;
   auto refresh = [&](int g) {
-    ok = hand_over_until(&prog[wave], &prog[wave + 2], have_in, have_out, g, ngroups, spin_limit,
-                         trouble);
+    ok = hand_over_until(&prog[wave], &prog[wave + 2], have_in, have_out, g, g_end, spin_limit, trouble);
   };
   const float* take = kHand ? (first_column ? nothing : ring[wave]) : nullptr;
   const int take_mask = first_column ? 0 : kRingGroups / 4 - 1;
@@ -1024,8 +1034,9 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
           inside[j] = __builtin_amdgcn_ballot_w64((unsigned)(4 * g + j - u) < tlim);
           // what enters the lattice's own first column: nothing, which is -inf while its cells are
           // inside the lattice (:49-52 adds nothing there, so a -inf blank score must come out as
-          // -inf) and kOutside once they are past the last frame (see kOutside)
-          if (first_column && 4 * g + j >= Tb) in[j] = kOutside;
+          // -inf) and, as in any first column, kOutside once they are past the last frame (see
+          // kOutside; nobody hands anything on for those steps)
+          if (4 * g + j >= Tb + u_lo) in[j] = kOutside;
         }
       }
       // (set well ahead of the lane shifts that fill lane 0 from them)
@@ -1067,16 +1078,18 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
 
   // four sets of operands rotate: a group's loads are requested four groups (16 steps, more than a
   // microsecond) ahead -- the planes of a long batch do not fit L2
-  Ops q0 = load_to_end(0), q1 = load_to_end(1), q2 = load_to_end(2), q3 = load_to_end(3);
+  Ops q0 = load_to_end(g_begin), q1 = load_to_end(g_begin + 1), q2 = load_to_end(g_begin + 2),
+      q3 = load_to_end(g_begin + 3);
   if constexpr (kHand) {
-    if (!first_column) {
-      refresh(0);
-      hand = *reinterpret_cast<const quad_t*>(take);
+    if (!first_column) {  // (g_begin is a multiple of sixteen)
+      refresh(g_begin);
+      carry = take[16 * (((g_begin >> 2) - 1) & take_mask) + 15];
+      hand = *reinterpret_cast<const quad_t*>(take + 16 * ((g_begin >> 2) & take_mask));
     }
   }
   const std::true_type yes;
   const std::false_type no;
-  int g = 0;
+  int g = g_begin;
   auto block = [&](auto inner) {
     constexpr bool kInner = decltype(inner)::value;
     const float *tk = nullptr, *tk_next = nullptr;
@@ -1108,10 +1121,10 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
     if constexpr (kHand) __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     g += 4;
   };
-  while (g + 4 < ngroups) {
+  while (g + 4 < g_end) {
     if (g - origin >= span) move_on(g);
-    if (g >= in_lo && g + 4 <= in_hi && g + 8 <= ngroups) {
-      const int end = min(min(in_hi, ngroups - 4), origin + span);
+    if (g >= in_lo && g + 4 <= in_hi && g + 8 <= g_end) {
+      const int end = min(min(in_hi, g_end - 4), origin + span);
       do block(yes);
       while (g + 4 <= end);
     } else {
@@ -1119,7 +1132,7 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
     }
   }
   // the last one to four groups
-  while (g < ngroups) {
+  while (g < g_end) {
     const float* tk = nullptr;
     float* gv = nullptr;
     if constexpr (kHand) {
@@ -1134,9 +1147,9 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void alpha_walk_kernel(
     ++g;
   }
   if constexpr (kHand) {
-    *reinterpret_cast<quad_t*>(give + 16 * (((ngroups - 1) >> 2) & give_mask) + 4 * ((ngroups - 1) & 3)) = pend;
+    *reinterpret_cast<quad_t*>(give + 16 * (((g_end - 1) >> 2) & give_mask) + 4 * ((g_end - 1) & 3)) = pend;
     asm volatile("" ::: "memory");
-    prog_store(give_prog, ngroups);
+    prog_store(give_prog, kForever);
   }
   // :73-78 the blank move out of the last cell, negated
   if (u == Ub - 1) costs[b] = -final;
@@ -1483,7 +1496,7 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void beta_walk_kernel(
         live_in ? live + ((size_t)live_block * d.B + b) * d.Dp : nullptr;
     unsigned long long* dst =
         live_out ? live + ((size_t)(live_block - 1) * d.B + b) * d.Dp : nullptr;
-    live_carrier<3>(src, dst, n, [&](int i, int k) { return 4 * (g_first - i) + k; }, ring[0],
+    live_carrier<3>(src, dst, 0, n, 0, n, [&](int i, int k) { return 4 * (g_first - i) + k; }, ring[0],
                     &prog[0], &prog[1], ring[W], &prog[W], &prog[W + 1], spin_limit, trouble);
     return;
   }
@@ -2852,8 +2865,8 @@ __global__ __launch_bounds__(64 * (W + (kLive ? 1 : 0))) void viterbi_walk_kerne
     const unsigned long long* src =
         live_in ? live + ((size_t)(live_block - 1) * d.B + b) * d.Dp : nullptr;
     unsigned long long* dst = live_out ? live + ((size_t)live_block * d.B + b) * d.Dp : nullptr;
-    live_carrier<0>(src, dst, ngroups, [](int g, int i) { return 4 * g + 1 + i; }, ring[0], &prog[0],
-                    &prog[1], ring[W], &prog[W], &prog[W + 1], spin_limit, trouble);
+    live_carrier<0>(src, dst, 0, ngroups, 0, ngroups, [](int g, int i) { return 4 * g + 1 + i; },
+                    ring[0], &prog[0], &prog[1], ring[W], &prog[W], &prog[W + 1], spin_limit, trouble);
     return;
   }
   const int u_lo = u_base + wave * 64;
