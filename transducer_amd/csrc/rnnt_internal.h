@@ -131,7 +131,8 @@ struct Planes {
 
 // Trips a wavefront of the lattice kernels may spend waiting for its neighbour's progress
 // counter before it gives up and raises the trouble flag (each trip is an LDS read and a short
-// sleep, roughly 50 ns; the longest legitimate wait is a few dozen trips).
+// sleep, roughly 50 ns; the longest legitimate wait is an alpha wavefront's for the lattice to reach its
+// first position, up to 4095 steps or some ten thousand trips; others are a few dozen).
 constexpr int kDefaultSpinLimit = 1 << 20;
 extern int g_spin_limit;
 // Device address of the current device's trouble flag (a static device int, looked up once per
